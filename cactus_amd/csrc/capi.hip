@@ -92,7 +92,7 @@ bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 // and that kernel loads with 2-byte aligned vectors throughout.
 // The types of 32-value blocks also come with rows of K % 64 == 0 elements (hidden sizes such as 576, 896, 960): such
 // rows are multiples of 4 bytes only, and only the kernels that load with 4-byte aligned vectors take them (the
-// dot-product GEMV; the GEMM, whose staging reads single blocks, when K % 128 == 0).
+// dot-product GEMV; the GEMM, whose staging reads single blocks).
 bool is_block32_type(int t) { return t == T_Q4_0 || t == T_Q8_0 || t == T_Q5_0 || t == T_IQ4_NL || t == T_Q4_1 || t == T_Q5_1; }
 bool weights_aligned(int type, const void *W, size_t nb01, int64_t K = 256) {
     // (Q3_K: 110-byte super-blocks, as Q6_K's 210; Q2_K: 84 bytes; IQ4_XS: 136 bytes, loaded as an 8-byte and 4-byte aligned pieces)

@@ -210,7 +210,12 @@ __device__ __forceinline__ void load16_into_lds(const uint8_t *src, uint32_t lds
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_addr) : "memory");
 }
 
-template <int WT, int TM, int TN, int WR, int WC, int OCC, bool GATHER>
+// TAIL: K is an odd multiple of 64, so the last stage of a row holds two blocks instead of four.  Its other two are read from
+// the blocks in front of them (in bounds) with both scales set to zero, which adds 0 * (a finite sum): a template argument,
+// because the selects that zero the activation scales would sit in every stage of the K % 128 == 0 shapes too.  Before this form
+// such rows ran through the dot-product GEMV, a pass per 8 tokens (Q4_0, 133 tokens, 960 and 2560 rows of 960 values: 17 passes
+// of 6 - 8 us, 110 - 140 us a matrix; one launch of 8 - 12 us with this kernel; an 8-layer step 5818 -> 995 us).
+template <int WT, int TM, int TN, int WR, int WC, int OCC, bool GATHER, bool TAIL>
 __global__ __launch_bounds__(WR *WC * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 void gemm_blk32_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64_t N, const uint8_t *__restrict__ ws,
                               size_t ws_stride, int64_t M, float *__restrict__ y, int64_t ldy, TileMap map, RowGather rg,
@@ -231,10 +236,13 @@ void gemm_blk32_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, in
     if (gv.tok_tile < 0) return;
     const int64_t tok_base = (int64_t)(GATHER ? gv.tok_tile : tc.tok_tile) * C::BN;
     if (tok_base >= M) return;
-    int stage0 = 0, nstages = (int)(K / (32 * GEMM_KB));
+    static_assert(!(GATHER && TAIL), "expert rows are whole stages");
+    int stage0 = 0, nstages = (int)(TAIL ? ceil_div(K, (int64_t)(32 * GEMM_KB)) : K / (32 * GEMM_KB));
+    int tail_stage = nstages - 1;                                                  // TAIL: the short stage, counted from this slice's first
     if (!GATHER && slice_stages > 0) {
         stage0 = (int)blockIdx.y * slice_stages;
         nstages = min(slice_stages, nstages - stage0);
+        tail_stage -= stage0;
         y += (size_t)blockIdx.y * (size_t)M * (size_t)ldy;
     }
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
@@ -273,13 +281,20 @@ void gemm_blk32_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, in
 #pragma unroll
         for (int i = 0; i < C::W_PER_T; i++) {
             const uint8_t *p = wsrc[i] + (size_t)s * (GEMM_KB * T::BYTES);
+            const bool dead = TAIL && s == tail_stage && ((tid + i * C::NT) % GEMM_KB) >= 2;
+            if (TAIL && dead) p -= 2 * T::BYTES;
             if constexpr (T::HAS_MIN) wd[i] = *reinterpret_cast<const uint32_t *>(p);
             else wd[i] = *reinterpret_cast<const unsigned short *>(p);
             T::fetch(wq[i], p);
+            if (TAIL && dead) wd[i] = 0u;
         }
         if constexpr (T::HAS_MIN) {
 #pragma unroll
-            for (int i = 0; i < C::S_PER_T; i++) xm[i] = *reinterpret_cast<const float *>(msrc[i] + (size_t)s * (4 * GEMM_KB));
+            for (int i = 0; i < C::S_PER_T; i++) {
+                const bool dead = TAIL && s == tail_stage && ((tid + i * C::NT) % GEMM_KB) >= 2;
+                xm[i] = *reinterpret_cast<const float *>(msrc[i] + (size_t)s * (4 * GEMM_KB) - (TAIL && dead ? 8 : 0));
+                if (TAIL && dead) xm[i] = 0.f;
+            }
         }
     };
     auto issue_direct = [&](int s, uint32_t buf_off) {
@@ -344,7 +359,7 @@ void gemm_blk32_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, in
     for (int b = 0; b < GEMM_KB; b++) b_rd[b] = (uint32_t)C::OFF_B + (uint32_t)(n0 + l32) * 128u + 16u * (uint32_t)((2 * b + half) ^ ((l32 >> 1) & 7));
 
     // one stage from the buffer at byte offset BUF
-    auto compute = [&](auto buf_tag) {
+    auto compute = [&](auto buf_tag, int s) {
         constexpr uint32_t BUF = decltype(buf_tag)::value ? (uint32_t)C::STAGE : 0u;
         const uint8_t *base = lds + BUF;
         if constexpr (T::HAS_MIN) {
@@ -369,6 +384,8 @@ void gemm_blk32_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, in
         for (int c = 0; c < TN; c++) {
             const float4 t = *reinterpret_cast<const float4 *>(base + sx_rd + c * 512);
             dxs[c][0] = t.x; dxs[c][1] = t.y; dxs[c][2] = t.z; dxs[c][3] = t.w;
+            // the scale cell of the short stage ends in two words of the sums plane: any bits, NaN patterns among them
+            if constexpr (TAIL) { dxs[c][2] = s == tail_stage ? 0.f : dxs[c][2]; dxs[c][3] = s == tail_stage ? 0.f : dxs[c][3]; }
             if constexpr (T::HAS_MIN) {
 #pragma unroll
                 for (int b = 0; b < GEMM_KB; b++) dxs[c][b] *= T::INV_MULT;       // the min term has no power of two to take back
@@ -458,7 +475,7 @@ void gemm_blk32_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, in
             commit_w((uint32_t)C::STAGE);
             issue_direct(min(s + 1, last), (uint32_t)C::STAGE);
             fetch_w(min(s + 2, last));
-            compute(std::false_type{});
+            compute(std::false_type{}, s);
             __builtin_amdgcn_s_waitcnt(WAIT_ACTS);
             __syncthreads();
         }
@@ -466,7 +483,7 @@ void gemm_blk32_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, in
             commit_w(0u);
             issue_direct(min(s + 2, last), 0u);
             fetch_w(min(s + 3, last));
-            compute(std::true_type{});
+            compute(std::true_type{}, s + 1);
             __builtin_amdgcn_s_waitcnt(WAIT_ACTS);
             __syncthreads();
         }
@@ -518,7 +535,7 @@ static int64_t gemm_blk32_min_tokens(int wtype, int64_t K, int64_t N, bool can_s
 }
 bool gemm_blk32_supported(int wtype, int64_t K, int64_t N, int64_t n, bool can_split) {
     if (!(wtype == T_Q4_0 || wtype == T_Q8_0 || wtype == T_Q5_0 || wtype == T_IQ4_NL || wtype == T_Q4_1 || wtype == T_Q5_1)) return false;
-    if (K % (32 * GEMM_KB) != 0 || N < 1) return false;
+    if (K < 64 || K % 64 != 0 || N < 1) return false;
     const int64_t forced = tune("CHIP_GEMM_MIN_TOKENS", 0);
     if (forced > 0) return n >= forced;
     return n >= gemm_blk32_min_tokens(wtype, K, N, can_split);
@@ -576,7 +593,7 @@ hipError_t launch_sum_slices(const float *part, int slices, int64_t n, int64_t N
 // grow with the token count), at least eight stages each.
 static int blk32_slices_for(int64_t K, int64_t N, int64_t M, int64_t cus) {
     const int forced = (int)tune("CHIP_GEMM_SLICES", 0);
-    const int64_t units = K / (32 * GEMM_KB), tiles = ceil_div(N, (int64_t)64) * ceil_div(M, (int64_t)64);
+    const int64_t units = ceil_div(K, (int64_t)(32 * GEMM_KB)), tiles = ceil_div(N, (int64_t)64) * ceil_div(M, (int64_t)64);
     if (forced > 0) {
         const int64_t per = ceil_div(units, (int64_t)(forced < units ? forced : units));
         return (int)ceil_div(units, per);
@@ -590,20 +607,24 @@ static int blk32_slices_for(int64_t K, int64_t N, int64_t M, int64_t cus) {
     return (int)ceil_div(units, per);                                   // no empty slice
 }
 
-template <int WT, int TM, int TN, int WR, int WC, int OCC, bool GATHER>
+template <int WT, int TM, int TN, int WR, int WC, int OCC, bool GATHER, bool TAIL = false>
 static hipError_t launch_direct(const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, int64_t M,
                                 float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t n_as,
                                 int slices = 1, float *part = nullptr) {
+    if constexpr (!GATHER && !TAIL) {
+        if (K % (32 * GEMM_KB) != 0)
+            return launch_direct<WT, TM, TN, WR, WC, OCC, GATHER, true>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as, slices, part);
+    }
     using C = DirectCfg<TM, TN, WR, WC, Blk32<WT>::HAS_MIN>;
     const size_t lds_bytes = 2 * C::STAGE;
     if ((int64_t)lds_bytes > lim.max_lds_per_block) return hipErrorInvalidValue;
-    auto kfn = gemm_blk32_kernel<WT, TM, TN, WR, WC, OCC, GATHER>;
+    auto kfn = gemm_blk32_kernel<WT, TM, TN, WR, WC, OCC, GATHER, TAIL>;
     static LdsGrant grant;
     if (hipError_t e = grant_dynamic_lds(kfn, lds_bytes, lim, grant); e != hipSuccess) return e;
     const int per_cu = (int)(lds_bytes > 80 * 1024 ? 1 : (4 * OCC / C::NW > 0 ? 4 * OCC / C::NW : 1));
     const TileMap map = make_tile_map(ceil_div(N, C::BM), GATHER ? 1 : ceil_div(M, C::BN), 32 * per_cu);
     if (!GATHER && slices > 1) {
-        const int slice_stages = (int)ceil_div(K / (32 * GEMM_KB), (int64_t)slices);
+        const int slice_stages = (int)ceil_div(ceil_div(K, (int64_t)(32 * GEMM_KB)), (int64_t)slices);
         hipLaunchKernelGGL(kfn, dim3(map.grid, (unsigned)slices), dim3(C::NT), lds_bytes, st, (const uint8_t *)W, nb01, K, N,
                            (const uint8_t *)ws, ws_stride, M, part, N, map, rg, slice_stages);
         if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
