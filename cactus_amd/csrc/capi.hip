@@ -788,9 +788,8 @@ int chip_mul_mat_id(int type, const void *W, size_t nb01, size_t nb02, int64_t K
     const size_t stride = act_stride(chip_vec_dot_type(type), K);
     hipStream_t st = (hipStream_t)stream;
 
-    const bool kq = type == T_Q4_K || type == T_Q5_K || type == T_Q6_K;
-    // (the 2- and 3-bit K-quants have no GEMM of their own: every pair takes the GEMV)
-    const bool have_gemm = (type == T_Q3_K || type == T_Q2_K || type == T_IQ4_XS) ? false : type == T_F16 ? K % 64 == 0 : (kq ? true : K % 128 == 0);
+    const bool kq = gemm_kq_type(type);
+    const bool have_gemm = type == T_F16 ? K % 64 == 0 : (kq ? true : K % 128 == 0);
     if (pairs >= MOE_GEMM_MIN_PAIRS && have_gemm && moe_group_supported(n_as, pairs)) {
         rc = chip_mul_mat_prepare(type, K, x, ldx, rows, workspace, workspace_bytes, stream);
         if (rc) return rc;

@@ -1,5 +1,5 @@
-// Prefill GEMM for gfx950 over K-quant weights (Q4_K, Q5_K, Q6_K) and Q8_K activations: the batched form of
-// lm_ggml_vec_dot_q4_K_q8_K / _q5_K_q8_K / _q6_K_q8_K (reference ggml-cpu/ggml-cpu-quants.c) as driven by
+// Prefill GEMM for gfx950 over K-quant weights (Q2_K .. Q6_K, IQ4_XS) and Q8_K activations: the batched form of
+// lm_ggml_vec_dot_q2_K_q8_K .. _q6_K_q8_K, _iq4_xs_q8_K (reference ggml-cpu/ggml-cpu-quants.c) as driven by
 // lm_ggml_compute_forward_mul_mat (ggml-cpu/ggml-cpu.c:1257-1449).
 //
 // Per 256-value super-block the reference forms two integers per (row, token),
@@ -11,6 +11,9 @@
 //
 //   Q4_K   sc = 8*sh + sl (3-bit digits): planes q*sh and q*sl (both <= 105), sumi = 8*P0 + P1
 //   Q5_K   the same digits on (q - 16) in -16..15 (products in -112..105), sumi = 8*P0 + P1 + 16 * sum_j sc_j * bsum_j
+//   Q3_K   (4 - q)*sc (q = 0..7, sc = -32..31) lies in -128..124: one plane, sumi = -P0
+//   Q2_K   q*sc <= 45: one plane, sumi = P0; its sixteen mins stand against one bsum each in the fp16 product below
+//   IQ4_XS (code point)*sc + 4064 in 127..8128: the two digits of Q6_K's form
 //   Q6_K   (q - 32)*sc + 4064 = 64*hi + lo with hi in 0..127, lo in 0..63: the digits of the biased product,
 //          sumi = 64*P0 + P1 - 4064 * (sum of the token's 256 quants, i.e. of its 16 bsums)
 //
@@ -40,8 +43,7 @@ typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int KQ_KB = 4;                      // 32-value k-blocks per LDS stage
 constexpr int KQ_TN = 2;                      // 32-token tiles per wave
-constexpr int KQ_NPL = 2;                     // int8 digit planes per weight type
-constexpr int Q6_BIAS = 4064;                 // 32 * 127: makes (q - 32) * sc + bias >= 0 for every int8 sc
+constexpr int Q6_BIAS = 4064;                 // 32 * 127: makes (q - 32) * sc + bias >= 0 for every int8 sc; IQ4_XS: -127..113 times -32..31
 
 // two independent 16-bit products / multiply-adds per dword (v_pk_mul_lo_u16, v_pk_mad_u16)
 __device__ __forceinline__ uint32_t pk_mul16(uint32_t a, uint32_t b) {
@@ -90,13 +92,20 @@ __device__ __forceinline__ u32x4 i16x8_to_f16(const u32x4 &v) {
 // One staging item = (row, x) of a stage h (half of a super-block): 16 bytes of packed quants that expand into
 // the 16-value k-half hf = x & 1 of two k-blocks kb0(x), kb1(x) of the stage, for both digit planes.
 struct Emit {
-    u32x4 cell[KQ_NPL][2]; // [plane][0: k-block kb0, 1: k-block kb1]
+    u32x4 cell[2][2];      // [plane][0: k-block kb0, 1: k-block kb1]  (IQ4_XS: the two k-halves of k-block x)
 };
+// LDS position [k-block][k-half] of an item's two cells
+template <class T> __device__ __forceinline__ int cell_pos(int x, int c) {
+    if constexpr (T::HALVES) return 2 * x + c;
+    else return (c ? T::kb1(x) : T::kb0(x)) * 2 + (x & 1);
+}
 
 template <int WT> struct KQ;
 
 template <> struct KQ<T_Q4_K> {
     static constexpr int BYTES = BYTES_Q4_K, NF16 = 1;             // fp16 products: summ
+    static constexpr int NPL = 2;                                  // int8 digit planes
+    static constexpr bool HALVES = false;
     static constexpr bool HAS_BSUM = false;
     // what item x of a row needs from one super-block: the 16 header bytes and 16 quant bytes per half
     struct Raw { u32x4 hdr, q[2]; };
@@ -134,6 +143,8 @@ template <> struct KQ<T_Q4_K> {
 
 template <> struct KQ<T_Q5_K> {
     static constexpr int BYTES = BYTES_Q5_K, NF16 = 2;             // fp16 products: summ, sum_j sc_j * bsum_j
+    static constexpr int NPL = 2;                                  // int8 digit planes
+    static constexpr bool HALVES = false;
     static constexpr bool HAS_BSUM = false;
     struct Raw { u32x4 hdr, qh, q[2]; };
     __device__ static __forceinline__ void fetch(Raw &r, const uint8_t *blk, int x) {
@@ -182,6 +193,8 @@ template <> struct KQ<T_Q5_K> {
 
 template <> struct KQ<T_Q6_K> {
     static constexpr int BYTES = BYTES_Q6_K, NF16 = 0;
+    static constexpr int NPL = 2;                                  // int8 digit planes
+    static constexpr bool HALVES = false;
     static constexpr bool HAS_BSUM = true;
     struct Raw { u32x4 ql[2], qh[2], sc; uint32_t d; };
     // Half h of a super-block holds, for l = 0..31, the elements 128h + 32b + l of k-blocks b = 0..3 as
@@ -234,6 +247,133 @@ template <> struct KQ<T_Q6_K> {
     }
 };
 
+template <> struct KQ<T_Q3_K> {
+    static constexpr int BYTES = BYTES_Q3_K, NF16 = 0, NPL = 1;
+    static constexpr bool HAS_BSUM = false, HALVES = false;
+    // hmask[32] | qs[64] | scales[12] | d.  Element 128h + 32v + l: bits 2v of qs[32h + l], bit 4h + v of hmask[l], scale 8h + 2v + l/16.
+    // Item x: the 16 bytes l = 16*(x & 1) + [0,16), k-blocks v = x / 2 and x / 2 + 2 (the two items of a k-half read the same bytes).
+    struct Raw { u32x4 hm, q[2]; uint32_t s[3], d; };
+    __device__ static __forceinline__ void fetch(Raw &r, const uint8_t *blk, int x) {
+        const int hf = x & 1;
+        r.hm = *reinterpret_cast<const u32x4_a2 *>(blk + 16 * hf);
+        r.q[0] = *reinterpret_cast<const u32x4_a2 *>(blk + 32 + 16 * hf);
+        r.q[1] = *reinterpret_cast<const u32x4_a2 *>(blk + 64 + 16 * hf);
+#pragma unroll
+        for (int i = 0; i < 3; i++) r.s[i] = *reinterpret_cast<const u32_a2 *>(blk + 96 + 4 * i);
+        r.d = *reinterpret_cast<const unsigned short *>(blk + 108);
+    }
+    __device__ static __forceinline__ int kb0(int x) { return x >> 1; }
+    __device__ static __forceinline__ int kb1(int x) { return (x >> 1) + 2; }
+    __device__ static __forceinline__ void emit(Emit &e, const Raw &r, int h, int x) {
+        const int p = x >> 1, hf = x & 1;
+        // 6-bit scale 4w + i is byte i of word w (reference ggml-quants.c:1062-1071): words 2h and 2h + 1 hold k-blocks 0, 1 and 2, 3
+        const uint32_t hi2 = r.s[2] >> (4 * h);
+        const uint32_t wa = ((r.s[0] >> (4 * h)) & 0x0f0f0f0fu) | ((hi2 & 0x03030303u) << 4);
+        const uint32_t wb = ((r.s[1] >> (4 * h)) & 0x0f0f0f0fu) | (((hi2 >> 2) & 0x03030303u) << 4);
+        const int b = 8 * (2 * p + hf);
+        const int sc[2] = {(int)((wa >> b) & 0xffu) - 32, (int)((wb >> b) & 0xffu) - 32};
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const int v = p + 2 * c;
+            // byte = 128 + (4 - q)*sc in 0..252: the two bytes of a 16-bit lane never carry into each other, whatever the sign of
+            // the multiplier (arithmetic modulo 2^16); flipping bit 7 gives the signed byte
+            const uint32_t mul = splat16((uint32_t)(-sc[c])), add = splat16((uint32_t)((128 + 4 * sc[c]) * 0x101));
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint32_t q = ((r.q[h][i] >> (2 * v)) & 0x03030303u) | (((r.hm[i] >> (4 * h + v)) & 0x01010101u) << 2);
+                e.cell[0][c][i] = pk_mad16(q, mul, add) ^ 0x80808080u;
+            }
+        }
+    }
+    __device__ static __forceinline__ uint32_t scales(const Raw &r) { return r.d; }
+    __device__ static __forceinline__ u32x4 f16_cell(const Raw &, int) { return u32x4{0u, 0u, 0u, 0u}; }
+    __device__ static __forceinline__ float value(int p0, int, const float (&)[2], uint32_t dd, int) {
+        return __builtin_fmaf(h2f(dd), (float)-p0, 0.f);
+    }
+};
+
+template <> struct KQ<T_Q2_K> {
+    static constexpr int BYTES = BYTES_Q2_K, NF16 = 1, NPL = 1;    // fp16 product: sum_j m_j * bsum_j over the 16 sub-blocks
+    static constexpr bool HAS_BSUM = false, HALVES = false;
+    // scales[16] (low nibble scale, high nibble min) | qs[64] | d | dmin; quants, scales and items placed as in Q3_K
+    struct Raw { u32x4 sc, q[2]; uint32_t dd; };
+    __device__ static __forceinline__ void fetch(Raw &r, const uint8_t *blk, int x) {
+        const int hf = x & 1;
+        r.sc = *reinterpret_cast<const u32x4_a4 *>(blk);
+        r.q[0] = *reinterpret_cast<const u32x4_a4 *>(blk + 16 + 16 * hf);
+        r.q[1] = *reinterpret_cast<const u32x4_a4 *>(blk + 48 + 16 * hf);
+        r.dd = *reinterpret_cast<const uint32_t *>(blk + 80);
+    }
+    __device__ static __forceinline__ int kb0(int x) { return x >> 1; }
+    __device__ static __forceinline__ int kb1(int x) { return (x >> 1) + 2; }
+    __device__ static __forceinline__ void emit(Emit &e, const Raw &r, int h, int x) {
+        const int p = x >> 1, b = 8 * (2 * p + (x & 1));
+        const uint32_t s0 = splat16((r.sc[2 * h] >> b) & 15u), s1 = splat16((r.sc[2 * h + 1] >> b) & 15u);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            e.cell[0][0][i] = pk_mul16((r.q[h][i] >> (2 * p)) & 0x03030303u, s0);           // byte products <= 45
+            e.cell[0][1][i] = pk_mul16((r.q[h][i] >> (2 * p + 4)) & 0x03030303u, s1);
+        }
+    }
+    __device__ static __forceinline__ uint32_t scales(const Raw &r) { return r.dd; }
+    // fp16 operand cell of item x < 2: mins of sub-blocks 8x .. 8x+7
+    __device__ static __forceinline__ u32x4 f16_cell(const Raw &r, int x) {
+        u32x4 c;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint32_t w = ((i < 2 ? r.sc[2 * (x & 1)] : r.sc[2 * (x & 1) + 1]) >> (16 * (i & 1) + 4)) & 0x0f0fu;
+            c[i] = (uint32_t)__half_as_ushort(__float2half_rn((float)(w & 0xffu))) |
+                   ((uint32_t)__half_as_ushort(__float2half_rn((float)(w >> 8))) << 16);    // exact
+        }
+        return c;
+    }
+    __device__ static __forceinline__ float value(int p0, int, const float (&f)[2], uint32_t dd, int) {
+        return __builtin_fmaf(-h2f(dd >> 16), f[0], __builtin_fmaf(h2f(dd), (float)p0, 0.f));
+    }
+};
+
+template <> struct KQ<T_IQ4_XS> {
+    static constexpr int BYTES = BYTES_IQ4_XS, NF16 = 0, NPL = 2;
+    static constexpr bool HAS_BSUM = true, HALVES = true;
+    // d | u16 scales_h | scales_l[4] | qs[128]: sub-block ib is qs[16 ib ..], low nibbles elements 0..15, high nibbles 16..31.
+    // Item x of stage h is sub-block 4h + x, both k-halves of k-block x.
+    struct Raw { u32x2 h; u32x4 q[2]; };
+    __device__ static __forceinline__ void fetch(Raw &r, const uint8_t *blk, int x) {
+        r.h = *reinterpret_cast<const u32x2 *>(blk);
+        r.q[0] = *reinterpret_cast<const u32x4_a4 *>(blk + 8 + 16 * x);
+        r.q[1] = *reinterpret_cast<const u32x4_a4 *>(blk + 72 + 16 * x);
+    }
+    __device__ static __forceinline__ int kb0(int x) { return x; }
+    __device__ static __forceinline__ int kb1(int x) { return x; }
+    // four code indices (one per byte) -> code point + 128 of kvalues_iq4nl (reference ggml-common.h), 1..241
+    __device__ static __forceinline__ uint32_t lookup4(uint32_t idx) {
+        constexpr uint32_t F = 0x80808080u, T0 = 0xbfad9881u ^ F, T1 = 0xf6eaddcfu ^ F, T2 = 0x26190d01u ^ F, T3 = 0x71594535u ^ F;
+        const uint32_t sel = idx & 0x07070707u;
+        const uint32_t lo = __builtin_amdgcn_perm(T1, T0, sel), hi = __builtin_amdgcn_perm(T3, T2, sel);
+        const uint32_t m = ((idx >> 3) & 0x01010101u) * 0xffu;
+        return (lo & ~m) | (hi & m);
+    }
+    __device__ static __forceinline__ void emit(Emit &e, const Raw &r, int h, int x) {
+        const int ib = 4 * h + x;
+        const uint32_t nib = (r.h.y >> (4 * ib)) & 15u, top = (r.h.x >> (16 + 2 * ib)) & 3u;
+        const int ls = (int)(nib | (top << 4)) - 32;
+        const uint32_t mul = splat16((uint32_t)ls), bias = splat16((uint32_t)(Q6_BIAS - 128 * ls));
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            uint32_t hi, lo;
+            KQ<T_Q6_K>::digits(lookup4(r.q[h][i] & 0x0f0f0f0fu), mul, bias, hi, lo);
+            e.cell[0][0][i] = hi; e.cell[1][0][i] = lo;
+            KQ<T_Q6_K>::digits(lookup4((r.q[h][i] >> 4) & 0x0f0f0f0fu), mul, bias, hi, lo);
+            e.cell[0][1][i] = hi; e.cell[1][1][i] = lo;
+        }
+    }
+    __device__ static __forceinline__ uint32_t scales(const Raw &r) { return r.h.x & 0xffffu; }
+    __device__ static __forceinline__ u32x4 f16_cell(const Raw &, int) { return u32x4{0u, 0u, 0u, 0u}; }
+    __device__ static __forceinline__ float value(int p0, int p1, const float (&)[2], uint32_t dd, int corr) {
+        return __builtin_fmaf(h2f(dd), (float)((p0 << 6) + p1 + corr), 0.f);
+    }
+};
+
 constexpr int KQ_PRODUCERS = 4;               // staging waves per workgroup, one per SIMD
 
 template <int WT, int WR, int WC>
@@ -244,10 +384,10 @@ struct KqCfg {
     static constexpr int NPT = KQ_PRODUCERS * 64;                  // staging threads
     static constexpr int BM = 32 * WR;                             // weight rows per workgroup
     static constexpr int BN = 32 * KQ_TN * WC;                     // tokens per workgroup
-    static constexpr int NF = T::NF16 > 0 ? T::NF16 : 1;
+    static constexpr int NF = T::NF16 > 0 ? T::NF16 : 1, NPL = T::NPL;
     // plane stride 2 mod 16 cells: the staging threads of one wave spread over the bank groups
     static constexpr int A_PLANE = BM + 2, B_PLANE = BN + 2;
-    static constexpr int A_CELLS = KQ_NPL * KQ_KB * 2 * A_PLANE;   // 16-byte cells
+    static constexpr int A_CELLS = NPL * KQ_KB * 2 * A_PLANE;   // 16-byte cells
     static constexpr int B_CELLS = KQ_KB * 2 * B_PLANE;
     // one stage buffer (two of them, by stage parity)
     static constexpr size_t OFF_A = 0;
@@ -373,14 +513,14 @@ void gemm_kq_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64
 #pragma unroll
             for (int i = 0; i < C::W_PER_T; i++) {
                 const int item = pt + i * C::NPT;
-                const int r = item >> 2, x = item & 3, hf = x & 1;
+                const int r = item >> 2, x = item & 3;
                 Emit e;
                 T::emit(e, RW.w[i], h, x);
-                const int k0 = T::kb0(x), k1 = T::kb1(x);
+                const int c0 = cell_pos<T>(x, 0), c1 = cell_pos<T>(x, 1);
 #pragma unroll
-                for (int pl = 0; pl < KQ_NPL; pl++) {
-                    A[((pl * KQ_KB + k0) * 2 + hf) * C::A_PLANE + r] = e.cell[pl][0];
-                    A[((pl * KQ_KB + k1) * 2 + hf) * C::A_PLANE + r] = e.cell[pl][1];
+                for (int pl = 0; pl < C::NPL; pl++) {
+                    A[(pl * KQ_KB * 2 + c0) * C::A_PLANE + r] = e.cell[pl][0];
+                    A[(pl * KQ_KB * 2 + c1) * C::A_PLANE + r] = e.cell[pl][1];
                 }
                 if constexpr (even) {
                     // the lane that owns MFMA result register v of a 32-row tile holds row 8*(v/4) + 4*half + v%4:
@@ -445,7 +585,7 @@ void gemm_kq_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64
     const int half = lane >> 5, l32 = lane & 31;
     const int r0 = wr * 32, n0 = wc * TN * 32;
 
-    i32x16 P[KQ_NPL][TN];
+    i32x16 P[C::NPL][TN];
     float out[TN][16];
 #pragma unroll
     for (int c = 0; c < TN; c++)
@@ -460,9 +600,9 @@ void gemm_kq_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64
         const u32x4 *B = reinterpret_cast<const u32x4 *>(base + C::OFF_B);
 #pragma unroll
         for (int b = 0; b < KQ_KB; b++) {
-            i32x4 af[KQ_NPL], bf[TN];
+            i32x4 af[C::NPL], bf[TN];
 #pragma unroll
-            for (int pl = 0; pl < KQ_NPL; pl++) {
+            for (int pl = 0; pl < C::NPL; pl++) {
                 const u32x4 t = A[((pl * KQ_KB + b) * 2 + half) * C::A_PLANE + r0 + l32];
                 af[pl] = i32x4{(int)t.x, (int)t.y, (int)t.z, (int)t.w};
             }
@@ -472,7 +612,7 @@ void gemm_kq_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64
                 bf[c] = i32x4{(int)t.x, (int)t.y, (int)t.z, (int)t.w};
             }
 #pragma unroll
-            for (int pl = 0; pl < KQ_NPL; pl++)
+            for (int pl = 0; pl < C::NPL; pl++)
 #pragma unroll
                 for (int c = 0; c < TN; c++) {
                     if (first && b == 0) {
@@ -515,7 +655,7 @@ void gemm_kq_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64
                 float f[2] = {0.f, 0.f};
 #pragma unroll
                 for (int j = 0; j < T::NF16; j++) f[j] = F[j][v];
-                out[c][v] = __builtin_fmaf(T::value(P[0][c][v], P[1][c][v], f, sd[v], corr), dx, out[c][v]);
+                out[c][v] = __builtin_fmaf(T::value(P[0][c][v], P[C::NPL - 1][c][v], f, sd[v], corr), dx, out[c][v]);
             }
         }
     };
@@ -866,10 +1006,12 @@ void gemm_ks_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64
 // memory speed.  Up to 128 tokens on a matrix with few row tiles the walk is cut into slices (kq_slices_for below:
 // 16 - 19 us at K = 4096, 36 - 41 us at K = 14336).  The token count from which the GEMM is ahead, measured on 4096 x 4096,
 // 14336 x 4096 (too many row tiles to split) and 4096 x 14336:
+// (Q3_K, Q2_K and IQ4_XS, us at 16 tokens: two GEMV passes against the GEMM at 17: Q3_K 21 / 14, 44 / 24 and 41 / 28, IQ4_XS
+// 20 / 17, 40 / 35 and 40 / 38; 201 tokens of Q3_K on 4096 x 14336: 26 passes, 499 us, against 46.)
 static bool kq_splittable(int64_t N) { return ceil_div(N, (int64_t)64) <= 128; }
 static int64_t gemm_kq_min_tokens(int wtype, int64_t K, int64_t N, bool can_split) {
     if (can_split || !kq_splittable(N)) {
-        if (wtype == T_Q6_K) return 9;                               // its GEMV passes take 8 tokens
+        if (wtype != T_Q4_K && wtype != T_Q5_K) return 9;            // their GEMV passes take 8 tokens
         return kq_splittable(N) ? 17 : 33;                           // Q4_K, Q5_K: passes of 16 tokens
     }
     // the caller's workspace has no room for the partial outputs: the unsplit walk
@@ -880,8 +1022,11 @@ static int64_t gemm_kq_min_tokens(int wtype, int64_t K, int64_t N, bool can_spli
         default:     return long_rows ? 41 : 25;
     }
 }
+bool gemm_kq_type(int wtype) {
+    return wtype == T_Q4_K || wtype == T_Q5_K || wtype == T_Q6_K || wtype == T_Q3_K || wtype == T_Q2_K || wtype == T_IQ4_XS;
+}
 bool gemm_kq_supported(int wtype, int64_t K, int64_t N, int64_t n, bool can_split) {
-    if (!(wtype == T_Q4_K || wtype == T_Q5_K || wtype == T_Q6_K) || K < QK_K || K % QK_K != 0 || N < 1) return false;
+    if (!gemm_kq_type(wtype) || K < QK_K || K % QK_K != 0 || N < 1) return false;
     const int64_t forced = tune("CHIP_GEMM_MIN_TOKENS", 0);
     if (forced > 0) return n >= forced;
     return n >= gemm_kq_min_tokens(wtype, K, N, can_split);
@@ -937,7 +1082,7 @@ template <int WT, int TM, int TN, int WR, int WC, int OCC, bool GATHER>
 static hipError_t launch_ks(const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, int64_t M,
                             float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t n_as,
                             int slices = 1, float *part = nullptr) {
-    if constexpr (WT == T_Q6_K) return hipErrorInvalidValue;
+    if constexpr (WT != T_Q4_K && WT != T_Q5_K) return hipErrorInvalidValue;
     else {
         using C = KsCfg<WT, TM, TN, WR, WC>;
         const size_t lds_bytes = C::TOTAL;
@@ -977,7 +1122,7 @@ static hipError_t launch_kq_type(const void *W, size_t nb01, int64_t K, int64_t 
     // Measured (us, K = 4096, tokens x rows; two-plane kernel -> single plane): Q4_K 2048 x 14336 432 -> 385, 2048 x 4096
     // 118 -> 108, 512 x 4096 36 -> 39 (stays); Q5_K 553 -> 455, 150 -> 125, 43 -> 42; Q4_K 512 x 4096 with K = 14336 107 -> 124 (stays).
     const int64_t g128 = ceil_div(N, 128) * ceil_div(M, 128), g64x128 = ceil_div(N, 64) * ceil_div(M, 128);
-    const bool single_plane = WT != T_Q6_K && g64x128 >= (WT == T_Q5_K ? 1 : 2) * cus;
+    const bool single_plane = (WT == T_Q4_K || WT == T_Q5_K) && g64x128 >= (WT == T_Q5_K ? 1 : 2) * cus;
     const int cfg = (int)tune("CHIP_GEMM_KQ_CFG", single_plane ? 11 : g128 >= cus ? 0 : 2);
     switch (cfg) {
         case 0: return launch_kq<WT, 4, 2, 3, false>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);      // 128 x 128, 8 + 4 waves
@@ -999,6 +1144,9 @@ hipError_t launch_gemm_kq(int wtype, const void *W, size_t nb01, int64_t K, int6
         case T_Q4_K: return launch_kq_type<T_Q4_K>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as, split);
         case T_Q5_K: return launch_kq_type<T_Q5_K>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as, split);
         case T_Q6_K: return launch_kq_type<T_Q6_K>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as, split);
+        case T_Q3_K: return launch_kq_type<T_Q3_K>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as, split);
+        case T_Q2_K: return launch_kq_type<T_Q2_K>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as, split);
+        case T_IQ4_XS: return launch_kq_type<T_IQ4_XS>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as, split);
         default: return hipErrorInvalidValue;
     }
 }

@@ -244,8 +244,9 @@ hipError_t launch_gemm_f16(const void *W, size_t nb01, int64_t K, int64_t N, con
                            int64_t n_as = 1, int gather_tile = 64,        // gather_tile: tokens per list entry, 64 or 128
                            const F32Rows *f32_rows = nullptr);
 
-// gemm_kquant.hip: int8-MFMA prefill GEMM over Q4_K / Q5_K / Q6_K weights, activations in the split Q8_K workspace
+// gemm_kquant.hip: int8-MFMA prefill GEMM over Q2_K .. Q6_K and IQ4_XS weights, activations in the split Q8_K workspace
 // layout; the integer sub-block scales ride in the MFMA operand.
+bool       gemm_kq_type(int wtype);
 bool       gemm_kq_supported(int wtype, int64_t K, int64_t N, int64_t n, bool can_split = false);
 hipError_t launch_gemm_kq(int wtype, const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride,
                           int64_t n, float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st, const RowGather *rg = nullptr,

@@ -38,3 +38,69 @@ def test_block32_rows_with_a_short_last_stage(dev, orc, wt, K, N, n):
     ref = orc.mul_mat(wt, wq[rows], x[toks], nthreads=8, want=("sum_abs",))
     check(y[np.ix_(toks, rows)], ref, "short last stage")
     assert np.isfinite(y).all()
+
+
+# ---- Q3_K, Q2_K and IQ4_XS on the matrix cores ----
+LOW_BIT = (O.Q3_K, O.Q2_K, O.IQ4_XS)
+
+
+def random_rows(wt, rng, N, nsb):
+    """Raw super-blocks: random bytes (every scale and quant occurs), d = dmin = 1; the first rows saturated."""
+    w = rng.integers(0, 256, (N, nsb, O.BLOCK_BYTES[wt]), dtype=np.uint8)
+    for r, fill in enumerate((0xFF, 0x00, 0x80, 0x7F)):
+        w[r] = fill
+    one = np.array([1.0], np.float16).view(np.uint8)
+    w[..., slice(108, 110) if wt == O.Q3_K else slice(80, 82) if wt == O.Q2_K else slice(0, 2)] = one
+    if wt == O.Q2_K:
+        w[..., 82:84] = one
+    return w.reshape(N, -1)
+
+
+# (K, N, n): the fewest tokens; ragged tiles; K split over workgroups with uneven slices; 128 x 128 tiles; many tokens, few rows
+@pytest.mark.parametrize("wt", LOW_BIT, ids=lambda t: O.TYPE_NAMES[t])
+@pytest.mark.parametrize("K,N,n", [(256, 5, 41), (1024, 131, 65), (2304, 131, 70), (4096, 300, 9), (512, 4100, 1030), (768, 33, 1100)])
+def test_low_bit_kquant_gemm(dev, orc, wt, K, N, n):
+    rng = np.random.default_rng(K + N + wt)
+    w = random_rows(wt, rng, N, K // 256)
+    x = common.activations_f32(K + n, n, K)
+    x[3] = 0
+    x[4] = 127.0
+    x[5] = -127.0
+    x[4:6, ::256] = -127.0
+    y = dev.mul_mat(wt, w, x)
+    rows = np.unique(np.concatenate([[0, 1, 2, 3, N - 1], rng.choice(N, min(N, 200), replace=False)]))
+    toks = np.unique(np.concatenate([[0, 3, 4, 5, n - 1], rng.choice(n, min(n, 64), replace=False)]))
+    ref = orc.mul_mat(wt, w[rows], x[toks], nthreads=8, want=("sum_abs",))
+    check(y[np.ix_(toks, rows)], ref, "low-bit k-quant gemm")
+
+
+@pytest.mark.parametrize("wt", LOW_BIT, ids=lambda t: O.TYPE_NAMES[t])
+def test_low_bit_kquant_integer_sums_bit_exact(dev, orc, wt):
+    """d = dmin = 1 and activation scale 1: the output of one super-block is the integer sumi - summ itself (below 2^24)."""
+    K, N, n = 256, 150, 56
+    rng = np.random.default_rng(77 + wt)
+    w = random_rows(wt, rng, N, 1)
+    x = rng.integers(-127, 128, (n, K)).astype(np.float32)
+    x[:, 0] = -127.0
+    x[7, 1:] = 0.0
+    aq = orc.quantize_activation(O.Q8_K, x)
+    y = dev.mul_mat(wt, w, x)
+    want = np.zeros((n, N), np.int64)
+    for t in range(n):
+        for i in range(N):
+            _, isum, imin = orc.vec_dot(wt, K, w[i], aq[t], want_sums=True)
+            want[t, i] = int(isum.sum()) - (int(imin.sum()) if wt == O.Q2_K else 0)
+    assert np.abs(want).max() < 2 ** 24
+    assert np.array_equal(y.astype(np.int64), want)
+
+
+@pytest.mark.parametrize("wt", LOW_BIT, ids=lambda t: O.TYPE_NAMES[t])
+def test_low_bit_kquant_expert_groups(dev, orc, wt):
+    """64 pairs and more: the pairs grouped by expert and run through the GEMM (ragged groups, an expert nobody picks)."""
+    K, N, n_as, n_used, n_tokens = 512, 70, 5, 2, 90
+    rng = np.random.default_rng(wt)
+    experts = np.stack([random_rows(wt, rng, N, K // 256) for _ in range(n_as)])
+    x = common.activations_f32(wt, n_tokens, K).reshape(n_tokens, 1, K)
+    ids = np.stack([rng.permutation(4)[:n_used] for _ in range(n_tokens)]).astype(np.int32)
+    ref = orc.mul_mat_id(wt, experts, x, ids, want=("sum_abs",))
+    check(dev.mul_mat_id(wt, experts, x, ids), ref, "expert groups")
