@@ -18,8 +18,8 @@
 //   long rows (kqv): a workgroup takes four rows, its four waves a quarter of K each; the activations are read once for
 //     the four rows; partial sums meet in LDS.
 // Many columns (prefill): the columns of a KV head are the token rows of a GEMM against that head's cache rows, so
-//   the work goes to the fp16 MFMA GEMM in its row-gather mode (the mode MUL_MAT_ID uses): activations rounded to fp16
-//   into a workspace, one (KV head, 64-column tile) list entry per workgroup column.
+//   the work goes to the fp16 MFMA GEMM in its batch mode: kqv rounds the activations to fp16 in its staging, kq reads an
+//   fp16 copy of them from the workspace.
 // Activations are rounded with v_cvt_f16_f32 (nearest even) and multiplied as halves by v_fma_mix_f32 with an fp32
 // accumulator.  The summation order differs from the reference's 4 x 8-lane accumulators, so parity is a tolerance
 // (1e-5 of sum |terms|), as for the other fp32-accumulating kernels.
@@ -422,8 +422,8 @@ __global__ __launch_bounds__(AM_THREADS) void mm_f16_slice_sum_kernel(BatchedArg
     col_y(a, b0, c)[row] = v;
 }
 
-// ---- many columns: fp16 rows for the GEMM and its (KV head, tile) list ----
-// Row R = b * n + t of the workspace and of y is column (query head b, token t); the pairs of KV head e are the rows
+// ---- many columns: fp16 rows for the GEMM ----
+// Row R = b * n + t of the workspace and of y is column (query head b, token t); the columns of KV head e are the rows
 // e * r2 * n ... (e + 1) * r2 * n - 1, in order.
 __global__ __launch_bounds__(AM_THREADS) void mm_f16_round_rows_kernel(const float *__restrict__ x, int64_t ldx1, int64_t ldx2,
                                                                        int64_t n, int64_t K, uint8_t *__restrict__ ws, size_t ws_stride) {
@@ -439,38 +439,21 @@ __global__ __launch_bounds__(AM_THREADS) void mm_f16_round_rows_kernel(const flo
         reinterpret_cast<u32x4 *>(ws + (size_t)(b * n + t) * ws_stride)[ch] = round8(xp[0], xp[1]);
     }
 }
-__global__ __launch_bounds__(AM_THREADS) void mm_f16_tile_list_kernel(int64_t ne02, int64_t per_head, int tile_tokens,
-                                                                      int32_t *__restrict__ perm, int32_t *__restrict__ offsets,
-                                                                      int32_t *__restrict__ tiles) {
-    const int64_t i0 = (int64_t)blockIdx.x * AM_THREADS + threadIdx.x, step = (int64_t)gridDim.x * AM_THREADS;
-    const int64_t tiles_per_head = ceil_div(per_head, (int64_t)tile_tokens);
-    for (int64_t i = i0; i < ne02 * per_head; i += step) perm[i] = (int32_t)i;
-    for (int64_t i = i0; i <= ne02; i += step) offsets[i] = (int32_t)(i * per_head);
-    for (int64_t i = i0; i < ne02 * tiles_per_head; i += step)
-        tiles[1 + i] = (int32_t)(i / tiles_per_head) | (int32_t)((i % tiles_per_head) << MOE_EXPERT_BITS);
-    if (i0 == 0) tiles[0] = (int32_t)(ne02 * tiles_per_head);
-}
-
 constexpr int64_t GEMM_MIN_COLS = 64;        // columns per KV head from which the GEMM route is taken
 
-struct GemmPlan { bool use; size_t act_stride, off_perm, off_offsets, off_tiles, bytes; int64_t n_tiles; int tile; };
+struct GemmPlan { bool use, direct; size_t act_stride, bytes; };
 GemmPlan gemm_plan(int64_t K, int64_t N, int64_t ne02, int64_t r2, int64_t n) {
     GemmPlan p{};
     const int64_t per_head = r2 * n;
     const int64_t min_cols = tune("CHIP_ATTN_GEMM_MIN", GEMM_MIN_COLS);
-    p.use = K >= 64 && K % 8 == 0 && N >= 32 && per_head >= min_cols && ne02 < (1 << MOE_EXPERT_BITS) && ne02 * per_head < (1LL << 30);
+    p.use = K >= 64 && K % 8 == 0 && N >= 32 && per_head >= min_cols && ne02 * per_head < (1LL << 30) &&
+            ne02 * ceil_div(per_head, (int64_t)32) * ceil_div(N, (int64_t)64) < (1LL << 31);          // workgroups of the one-dimensional grid
     if (!p.use) return p;
     p.act_stride = f16_stride(K);
-    // 128 x 128 tiles once they still give every CU four workgroups, else 64 x 64
-    const int forced = (int)tune("CHIP_ATTN_TILE", 0);
-    p.tile = (N >= 128 && per_head >= 128 && ne02 * ceil_div(per_head, (int64_t)128) * ceil_div(N, (int64_t)128) >= 1024) ? 128 : 64;
-    if (forced == 64 || forced == 128) p.tile = forced;
-    p.n_tiles = ne02 * ceil_div(per_head, (int64_t)p.tile);
-    if (p.n_tiles > 65535) { p.use = false; return p; }                  // one grid row per list entry
-    p.off_perm = align128((size_t)(ne02 * per_head) * p.act_stride);
-    p.off_offsets = p.off_perm + align128((size_t)(ne02 * per_head) * 4);
-    p.off_tiles = p.off_offsets + align128((size_t)(ne02 + 1) * 4);
-    p.bytes = p.off_tiles + align128((size_t)(1 + p.n_tiles) * 4);
+    // kqv (a head's 64 - 256 rows, one or two row tiles): the GEMM reads the fp32 activations itself.  kq, with thousands of
+    // cache positions as rows, reads the activations back once per row tile: it gets an fp16 copy first.
+    p.direct = N <= 256;
+    p.bytes = (size_t)(ne02 * per_head) * p.act_stride;
     return p;
 }
 
@@ -520,26 +503,15 @@ hipError_t launch_mul_mat_f16_batched(const void *W, size_t nb01, size_t nb02, i
     // the GEMM writes row R of y at R * ldy1: the batches of y must follow each other without a gap
     if (plan.use && !y2 && workspace && workspace_bytes >= plan.bytes && ldy2 == n * ldy1 && n <= 65535 && ne02 * r2 <= 65535) {
         uint8_t *ws = (uint8_t *)workspace;
-        int32_t *perm = (int32_t *)(ws + plan.off_perm), *offsets = (int32_t *)(ws + plan.off_offsets), *tiles = (int32_t *)(ws + plan.off_tiles);
-        // one row tile, or two with at most 1024 columns per KV head (kqv: a head's rows): the GEMM reads the fp32 activations
-        // itself and rounds them while staging (measured: 1.3 % of a 128-token step over 4096 positions; with 2048 columns and two
-        // row tiles the doubled staging traffic costs more than the rounding pass, and kq, with thousands of cache positions
-        // as rows, reads the activations back once per row tile): the others get an fp16 copy first
-        const bool f32_direct = tune("CHIP_ATTN_F32_ROWS", 1) != 0;
-        const int64_t row_tiles = ceil_div(N, (int64_t)plan.tile);
-        const bool direct = f32_direct && (row_tiles == 1 || (row_tiles == 2 && r2 * n <= 1024)) && n <= 0x7fffffff &&
-                            ne02 * r2 * n <= 0x7fffffff;
+        const bool direct = plan.direct && n <= 0x7fffffff && ne02 * r2 * n <= 0x7fffffff;
         if (!direct) {
             const int64_t chunks = K / 8, per = chunks >= AM_THREADS ? 1 : AM_THREADS / chunks;
             hipLaunchKernelGGL(mm_f16_round_rows_kernel, dim3((unsigned)ceil_div(n, per), (unsigned)(ne02 * r2)), dim3(AM_THREADS), 0, st, x,
                                ldx1, ldx2, n, K, ws, plan.act_stride);
+            if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
         }
-        hipLaunchKernelGGL(mm_f16_tile_list_kernel, dim3(64), dim3(AM_THREADS), 0, st, ne02, r2 * n, plan.tile, perm, offsets, tiles);
-        if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-        const RowGather rg{perm, offsets, tiles, 1, 1, nb02};
-        const F32Rows fr{x, ldx1, ldx2, n};
-        return launch_gemm_f16(W, nb01, K, N, ws, plan.act_stride, ne02 * r2 * n, y, ldy1, lim, st, &rg, plan.n_tiles, plan.tile,
-                               direct ? &fr : nullptr);
+        const F16Batch fb{ne02, r2 * n, nb02, direct ? x : nullptr, ldx1, ldx2, n};
+        return launch_gemm_f16_batch(W, nb01, K, N, ws, plan.act_stride, y, ldy1, lim, st, fb);
     }
     const BatchedArgs a{(const uint8_t *)W, nb01, nb02, K, N, x, ldx1, ldx2, n, r2, y, ldy1, ldy2, y2, ld2y1, ld2y2};
     const int cus = lim.compute_units > 0 ? lim.compute_units : 256;

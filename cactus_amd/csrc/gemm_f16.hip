@@ -36,10 +36,13 @@ struct F16Cfg {
     static_assert(W_ITEMS % NT == 0 && X_ITEMS % NT == 0, "staging items divide evenly over the threads");
 };
 
-// XF32 (row-gather mode only): the activations are read as fp32 from their own tensor - row R of the gather is token
-// R % n of batch R / n - and rounded to fp16 (nearest even) on their way into LDS, instead of from an fp16 copy in the
-// workspace.  Pays when the output has one or two row tiles (kqv: a head's 64 - 256 rows), so that the fp32 rows are read
-// once or twice; with many row tiles the fp16 copy, read back many times, is the cheaper source.
+// MODE: plain MUL_MAT, the expert groups of MUL_MAT_ID (RowGather), or the batches of an attention matmul over an F16 cache
+// (F16Batch): KV head e owns activation and output rows e * per_head ... + per_head - 1 and the weights W + e * nb02.
+// XF32 (attention only): the activations are read as fp32 from their own tensor - row R is token R % n of batch R / n - and
+// rounded to fp16 (nearest even) on their way into LDS, instead of from an fp16 copy in the workspace.  Pays when the output
+// has one or two row tiles (kqv: a head's 64 - 256 rows), so that the fp32 rows are read once or twice; with many row tiles
+// the fp16 copy, read back many times, is the cheaper source.
+enum F16Mode { F16_PLAIN, F16_EXPERTS, F16_BATCH };
 __device__ __forceinline__ u32x4 round8_f16(const float4 a, const float4 b) {
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
     const h2 h0 = {(_Float16)a.x, (_Float16)a.y}, h1 = {(_Float16)a.z, (_Float16)a.w};
@@ -50,29 +53,43 @@ __device__ __forceinline__ u32x4 round8_f16(const float4 a, const float4 b) {
     return r;
 }
 
-template <int TM, int TN, int WR, int WC, int OCC, bool GATHER, bool XF32 = false>
+template <int TM, int TN, int WR, int WC, int OCC, F16Mode MODE, bool XF32 = false>
 __global__ __launch_bounds__(WR *WC * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 void gemm_f16_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64_t N, const uint8_t *__restrict__ ws,
-                     size_t ws_stride, int64_t M, float *__restrict__ y, int64_t ldy, TileMap map, RowGather rg, F32Rows fs) {
-    static_assert(!XF32 || GATHER, "fp32 activation rows come with the row-gather mode");
+                     size_t ws_stride, int64_t M, float *__restrict__ y, int64_t ldy, TileMap map, RowGather rg, F16Batch fb) {
+    static_assert(!XF32 || MODE == F16_BATCH, "fp32 activation rows come with the attention mode");
     using C = F16Cfg<TM, TN, WR, WC>;
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = wave / WC, wc = wave % WC;
     const int half = lane >> 5, l32 = lane & 31;
-    const TileCoord tc = xcd_tile(blockIdx.x, map);
-    if (tc.row_tile >= map.row_tiles || tc.tok_tile >= map.tok_tiles) return;
-    const int64_t row_base = (int64_t)tc.row_tile * C::BM;
-    size_t w_offset;
-    const GatherView gv = resolve_gather<GATHER>(rg, w_offset, M);                   // MUL_MAT_ID: this expert's rows
-    W += w_offset;
-    if (gv.tok_tile < 0) return;
-    const int64_t tok_base = (int64_t)(GATHER ? gv.tok_tile : tc.tok_tile) * C::BN;
+    int64_t row_base, tok_base, row0 = 0;                            // row0: first activation and output row of this batch
+    GatherView gv{nullptr, 1, 1, 0};
+    if constexpr (MODE == F16_BATCH) {
+        // One-dimensional grid, the KV head fastest: workgroups are handed to the 8 XCDs in turn, so with 8 KV heads every XCD
+        // works on one head and that head's cache rows stay in its L2; whatever the head count, all XCDs get the same share.
+        const uint32_t rest = blockIdx.x / (uint32_t)fb.heads, e = blockIdx.x - rest * (uint32_t)fb.heads;
+        const uint32_t ct = rest / (uint32_t)map.row_tiles;
+        row_base = (int64_t)(rest - ct * (uint32_t)map.row_tiles) * C::BM;
+        tok_base = (int64_t)ct * C::BN;
+        M = fb.per_head;
+        row0 = (int64_t)e * fb.per_head;
+        W += (size_t)e * fb.nb02;
+    } else {
+        const TileCoord tc = xcd_tile(blockIdx.x, map);
+        if (tc.row_tile >= map.row_tiles || tc.tok_tile >= map.tok_tiles) return;
+        row_base = (int64_t)tc.row_tile * C::BM;
+        size_t w_offset;
+        gv = resolve_gather<MODE == F16_EXPERTS>(rg, w_offset, M);                   // MUL_MAT_ID: this expert's rows
+        W += w_offset;
+        if (gv.tok_tile < 0) return;
+        tok_base = (int64_t)(MODE == F16_EXPERTS ? gv.tok_tile : tc.tok_tile) * C::BN;
+    }
     if (tok_base >= M) return;
-    // The row-gather instantiation also takes K that is not a multiple of the 64-value stage (the attention matmul over
-    // n_kv cache positions, a multiple of 8): cells of the last stage that lie past K are zeroed on both sides.
-    constexpr bool KTAIL = GATHER;
+    // The attention mode also takes K that is not a multiple of the 64-value stage (n_kv cache positions, a multiple of 8):
+    // cells of the last stage that lie past K are zeroed on both sides.
+    constexpr bool KTAIL = MODE == F16_BATCH;
     const int nstages = (int)(KTAIL ? ceil_div(K, (int64_t)(16 * F16_KG)) : K / (16 * F16_KG));
     constexpr int STAGE_BYTES = 16 * F16_KG * 2;                   // bytes of one row per stage
     static_assert(C::NT % C::CELLS == 0, "a thread's items all have the same cell index");
@@ -88,48 +105,48 @@ void gemm_f16_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int6
 #pragma unroll
     for (int i = 0; i < C::X_PER_T; i++) {
         const int item = tid + i * C::NT;
-        const int64_t arow = gv.act_row(min(tok_base + item / C::CELLS, M - 1));
+        const int64_t arow = row0 + gv.act_row(min(tok_base + item / C::CELLS, M - 1));
         if constexpr (XF32) {
-            const uint32_t b = (uint32_t)arow / (uint32_t)fs.n, t = (uint32_t)arow - b * (uint32_t)fs.n;
-            xsrc[i] = reinterpret_cast<const uint8_t *>(fs.x + (int64_t)b * fs.ldx2 + (int64_t)t * fs.ldx1) + 32 * (item % C::CELLS);
+            const uint32_t b = (uint32_t)arow / (uint32_t)fb.n, t = (uint32_t)arow - b * (uint32_t)fb.n;
+            xsrc[i] = reinterpret_cast<const uint8_t *>(fb.x + (int64_t)b * fb.ldx2 + (int64_t)t * fb.ldx1) + 32 * (item % C::CELLS);
         } else {
             xsrc[i] = ws + (size_t)arow * ws_stride + 16 * (item % C::CELLS);
         }
     }
     u32x4 wq[C::W_PER_T], xq[C::X_PER_T];
+    float4 xf[XF32 ? C::X_PER_T : 1][2];                             // rounded when they are committed: nothing waits in fetch
+    bool live = true;
 
     auto fetch = [&](int stage) {
-        const bool live = !KTAIL || (int64_t)stage * (16 * F16_KG) + 8 * my_cell < K;
+        live = !KTAIL || (int64_t)stage * (16 * F16_KG) + 8 * my_cell < K;
         const size_t off = live ? (size_t)stage * STAGE_BYTES : 0;                   // a dead cell re-reads stage 0 (in bounds) and is zeroed
-        const u32x4 z = {0u, 0u, 0u, 0u};
 #pragma unroll
-        for (int i = 0; i < C::W_PER_T; i++) {
-            wq[i] = *reinterpret_cast<const u32x4 *>(wsrc[i] + off);
-            if (KTAIL && !live) wq[i] = z;
-        }
+        for (int i = 0; i < C::W_PER_T; i++) wq[i] = *reinterpret_cast<const u32x4 *>(wsrc[i] + off);
 #pragma unroll
         for (int i = 0; i < C::X_PER_T; i++) {
             if constexpr (XF32) {
                 const float4 *xp = reinterpret_cast<const float4 *>(xsrc[i] + 2 * off);      // a stage is twice the bytes in fp32
-                xq[i] = round8_f16(xp[0], xp[1]);
+                xf[i][0] = xp[0];
+                xf[i][1] = xp[1];
             } else {
                 xq[i] = *reinterpret_cast<const u32x4 *>(xsrc[i] + off);
             }
-            if (KTAIL && !live) xq[i] = z;
         }
     };
     auto commit = [&](int buf) {
+        const u32x4 z = {0u, 0u, 0u, 0u};
         u32x4 *A = reinterpret_cast<u32x4 *>(lds + (size_t)buf * C::STAGE + C::OFF_A);
         u32x4 *B = reinterpret_cast<u32x4 *>(lds + (size_t)buf * C::STAGE + C::OFF_B);
 #pragma unroll
         for (int i = 0; i < C::W_PER_T; i++) {
             const int item = tid + i * C::NT;
-            A[(item % C::CELLS) * C::A_PLANE + item / C::CELLS] = wq[i];
+            A[(item % C::CELLS) * C::A_PLANE + item / C::CELLS] = KTAIL && !live ? z : wq[i];
         }
 #pragma unroll
         for (int i = 0; i < C::X_PER_T; i++) {
             const int item = tid + i * C::NT;
-            B[(item % C::CELLS) * C::B_PLANE + item / C::CELLS] = xq[i];
+            if constexpr (XF32) xq[i] = round8_f16(xf[i][0], xf[i][1]);
+            B[(item % C::CELLS) * C::B_PLANE + item / C::CELLS] = KTAIL && !live ? z : xq[i];
         }
     };
 
@@ -173,7 +190,7 @@ void gemm_f16_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int6
         for (int c = 0; c < TN; c++) {
             const int64_t tok = tok_base + (wc * TN + c) * 32 + l32;
             if (tok >= M) continue;
-            const int64_t orow = gv.out_row(tok);
+            const int64_t orow = row0 + gv.out_row(tok);
 #pragma unroll
             for (int g = 0; g < 4; g++) {
                 const int64_t row = row_base + (wr * TM + a) * 32 + 8 * g + 4 * half;
@@ -351,47 +368,60 @@ static hipError_t launch_f16_direct(const void *W, size_t nb01, int64_t K, int64
 // rows must be 16-byte aligned (the weight alignment rule of the C-ABI) and K a multiple of the 64-value stage
 bool gemm_f16_supported(int64_t K, int64_t N, int64_t n) { return K >= 64 && K % (16 * F16_KG) == 0 && N >= 1 && n >= 32; }
 
-template <int TM, int TN, int WR, int WC, int OCC, bool GATHER, bool XF32 = false>
+template <int TM, int TN, int WR, int WC, int OCC, F16Mode MODE, bool XF32 = false>
 static hipError_t launch_f16(const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, int64_t M,
                              float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t n_as,
-                             const F32Rows &fs = F32Rows{nullptr, 0, 0, 1}) {
+                             const F16Batch &fb = F16Batch{1, 0, 0, nullptr, 0, 0, 1}) {
     using C = F16Cfg<TM, TN, WR, WC>;
     const size_t lds_bytes = 2 * C::STAGE;
-    auto kfn = gemm_f16_kernel<TM, TN, WR, WC, OCC, GATHER, XF32>;
+    auto kfn = gemm_f16_kernel<TM, TN, WR, WC, OCC, MODE, XF32>;
     static LdsGrant grant;
     if (hipError_t e = grant_dynamic_lds(kfn, lds_bytes, lim, grant); e != hipSuccess) return e;
-    const TileMap map = make_tile_map(ceil_div(N, C::BM), GATHER ? 1 : ceil_div(M, C::BN), 32 * (4 * OCC / C::NW > 0 ? 4 * OCC / C::NW : 1));
+    TileMap map = make_tile_map(ceil_div(N, C::BM), MODE == F16_PLAIN ? ceil_div(M, C::BN) : 1, 32 * (4 * OCC / C::NW > 0 ? 4 * OCC / C::NW : 1));
+    if (MODE == F16_BATCH) map.grid = (unsigned)(fb.heads * ceil_div(fb.per_head, (int64_t)C::BN) * map.row_tiles);      // < 2^31, checked by the caller
     hipLaunchKernelGGL(kfn, dim3(map.grid, (unsigned)n_as), dim3(C::NT), lds_bytes, st, (const uint8_t *)W, nb01, K, N,
-                       (const uint8_t *)ws, ws_stride, M, y, ldy, map, rg, fs);
+                       (const uint8_t *)ws, ws_stride, M, y, ldy, map, rg, fb);
     return hipGetLastError();
+}
+
+// The attention matmuls of a prompt.  Tiles (rows x columns of a KV head):
+//   kqv (fp32 activations, at most 256 rows): all rows of a head (64 or 128) in one tile, so that the probabilities are read
+//     once, by 64 columns - 32 while that leaves CUs without a workgroup.
+//   kq: 128 x 128 once they give every CU four workgroups, else 64 x 64.
+// Measured (us, 32 query heads over 8 KV heads of 128, 512 tokens, 4096 positions): kqv 67 (fp16 copy) + 157 (64 x 64 tiles, whose
+// padded two-tile grid rows all fell on two of the eight XCDs) + 5 (tile list) -> 117; kq 91 + 5 -> 84.
+hipError_t launch_gemm_f16_batch(const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, float *y, int64_t ldy,
+                                 const DeviceLimits &lim, hipStream_t st, const F16Batch &fb) {
+    const RowGather rg{nullptr, nullptr, nullptr, 1, 1, 0};
+    const int64_t cus = lim.compute_units > 0 ? lim.compute_units : 256, c64 = ceil_div(fb.per_head, (int64_t)64);
+#define BATCH_CASE(TM, TN, WR, WC, OCC, XF) \
+    return launch_f16<TM, TN, WR, WC, OCC, F16_BATCH, XF>(W, nb01, K, N, ws, ws_stride, fb.per_head, y, ldy, lim, st, rg, 1, fb)
+    if (fb.x) {
+        const int bn = (int)tune("CHIP_ATTN_BN", fb.heads * c64 * ceil_div(N, (int64_t)128) >= cus ? 64 : 32);
+        if (N > 64) { if (bn == 64) BATCH_CASE(2, 1, 2, 2, 2, true); else BATCH_CASE(1, 1, 4, 1, 3, true); }
+        if (bn == 64) BATCH_CASE(1, 1, 2, 2, 4, true); else BATCH_CASE(1, 1, 2, 1, 3, true);
+    }
+    const bool big = N >= 128 && fb.per_head >= 128 && fb.heads * ceil_div(fb.per_head, (int64_t)128) * ceil_div(N, (int64_t)128) >= 4 * cus;
+    if (big) BATCH_CASE(2, 2, 2, 2, 2, false);
+    BATCH_CASE(1, 1, 2, 2, 4, false);
+#undef BATCH_CASE
 }
 
 int gemm_f16_moe_tile_tokens() { return F16Cfg<1, 1, 2, 2>::BN; }      // the 64 x 64 shape serves the expert groups
 
 hipError_t launch_gemm_f16(const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, int64_t M,
-                           float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st, const RowGather *rgp, int64_t n_as,
-                           int gather_tile, const F32Rows *f32_rows) {
+                           float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st, const RowGather *rgp, int64_t n_as) {
     if (M <= 0 || N <= 0 || n_as <= 0) return hipSuccess;
     const RowGather rg = rgp ? *rgp : RowGather{nullptr, nullptr, nullptr, 1, 1, 0};
     const int64_t cus = lim.compute_units > 0 ? lim.compute_units : 256;
-    if (rg.perm) {                                                                   // row groups: the tile list was built for 64 or 128 tokens
-        if (f32_rows) {
-            if (gather_tile == 128) return launch_f16<2, 2, 2, 2, 2, true, true>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as, *f32_rows);
-            if (gather_tile != 64) return hipErrorInvalidValue;
-            return launch_f16<1, 1, 2, 2, 4, true, true>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as, *f32_rows);
-        }
-        if (gather_tile == 128) return launch_f16<2, 2, 2, 2, 2, true>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
-        if (gather_tile != 64) return hipErrorInvalidValue;
-        return launch_f16<1, 1, 2, 2, 4, true>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
-    }
-    if (f32_rows) return hipErrorInvalidValue;
+    if (rg.perm) return launch_f16<1, 1, 2, 2, 4, F16_EXPERTS>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);      // expert groups: 64 x 64 tiles
     const int64_t g128 = ceil_div(N, 128) * ceil_div(M, 128), g256 = ceil_div(N, 256) * ceil_div(M, 256);
     const int cfg = (int)tune("CHIP_GEMM_F16_CFG", 2 * g256 >= cus && K >= 4 * BIG_K && n_as == 1 ? 9 : g128 >= cus ? 0 : 1);
     switch (cfg) {
-        case 0: return launch_f16<2, 2, 2, 2, 2, false>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);       // 128 x 128, 4 waves
-        case 1: return launch_f16<1, 1, 2, 2, 4, false>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);       // 64 x 64, 4 waves
-        case 2: return launch_f16<2, 2, 2, 4, 2, false>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);       // 128 x 256, 8 waves
-        case 3: return launch_f16<2, 4, 2, 2, 2, false>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);       // 128 x 256, 4 waves
+        case 0: return launch_f16<2, 2, 2, 2, 2, F16_PLAIN>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);       // 128 x 128, 4 waves
+        case 1: return launch_f16<1, 1, 2, 2, 4, F16_PLAIN>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);       // 64 x 64, 4 waves
+        case 2: return launch_f16<2, 2, 2, 4, 2, F16_PLAIN>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);       // 128 x 256, 8 waves
+        case 3: return launch_f16<2, 4, 2, 2, 2, F16_PLAIN>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);       // 128 x 256, 4 waves
         case 9: return launch_f16_direct(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st);                             // 256 x 256, 4 waves, direct to LDS
         default: return hipErrorInvalidValue;
     }

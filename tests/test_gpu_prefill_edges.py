@@ -104,3 +104,21 @@ def test_low_bit_kquant_expert_groups(dev, orc, wt):
     ids = np.stack([rng.permutation(4)[:n_used] for _ in range(n_tokens)]).astype(np.int32)
     ref = orc.mul_mat_id(wt, experts, x, ids, want=("sum_abs",))
     check(dev.mul_mat_id(wt, experts, x, ids), ref, "expert groups")
+
+
+# ---- attention matmuls of a prompt: head size, heads, KV heads, tokens, cached positions ----
+# one 64-row tile by 64 and by 32 columns; 96 and 256 rows (a ragged and two row tiles); 3 KV heads; K no multiple of a stage;
+# kq with 128 x 128 tiles and with n_kv below and above the fp32 rule's 256 rows
+@pytest.mark.parametrize("hd,nh,nkv,n,kv", [(64, 32, 8, 512, 1064), (64, 15, 5, 133, 160), (96, 24, 8, 260, 104), (256, 6, 3, 75, 264),
+                                            (128, 8, 8, 257, 2056), (128, 4, 2, 70, 256)])
+def test_attention_matmuls_of_a_prompt(dev, orc, hd, nh, nkv, n, kv):
+    rng = np.random.default_rng(hd + n + kv)
+    q = rng.standard_normal((nh, n, hd)).astype(np.float32)
+    kc = rng.standard_normal((nkv, kv, hd)).astype(np.float16)
+    vt = rng.standard_normal((nkv, hd, kv)).astype(np.float16)
+    p = rng.random((nh, n, kv)).astype(np.float32)
+    toks = np.unique(np.concatenate([[0, n - 1], rng.choice(n, 40, replace=False)]))
+    for w, x in ((kc, q), (vt, p)):
+        y = dev.mul_mat_f16_batched(w, x)
+        ref = orc.mul_mat_f16_batched(w, np.ascontiguousarray(x[:, toks]), want=("sum_abs",))
+        check(y[:, toks], ref, "attention matmul")
