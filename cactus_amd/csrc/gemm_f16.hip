@@ -12,6 +12,7 @@
 #include "act_layout.h"
 #include "kernels.h"
 #include <cstdlib>
+#include <type_traits>
 
 namespace chip {
 
@@ -43,6 +44,12 @@ struct F16Cfg {
 // has one or two row tiles (kqv: a head's 64 - 256 rows), so that the fp32 rows are read once or twice; with many row tiles
 // the fp16 copy, read back many times, is the cheaper source.
 enum F16Mode { F16_PLAIN, F16_EXPERTS, F16_BATCH };
+// AHEAD: stages whose loads are in flight, each in a register set of its own.  With few tiles the kernel is bound by the latency
+// of its loads: a stage's 4 (16) MFMAs a wave end long before the next stage's weights have come from HBM.  One stage ahead -> AHEAD
+// (us, a different 4096 x 4096 F16 matrix each call, which no cache holds): 64 x 64 tiles, AHEAD 3: 64 tokens 38.4 -> 26.6, 201
+// tokens 41.3 -> 30.0, 512 tokens 61.7 -> 45.2 (AHEAD 2: 29.8, 33.3, 44.6; AHEAD 4 at three workgroups a CU: 26.0, 28.7, 45.8;
+// at four it spills: 66.9, 70.7, 111); 128 tokens of 14336 x 4096: 179 -> 106.  128 x 128 tiles, AHEAD 2: 1024 tokens 83.8 -> 66.6,
+// 300 tokens of 4096 x 14336 89.7 -> 85.7.
 __device__ __forceinline__ u32x4 round8_f16(const float4 a, const float4 b) {
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
     const h2 h0 = {(_Float16)a.x, (_Float16)a.y}, h1 = {(_Float16)a.z, (_Float16)a.w};
@@ -53,7 +60,7 @@ __device__ __forceinline__ u32x4 round8_f16(const float4 a, const float4 b) {
     return r;
 }
 
-template <int TM, int TN, int WR, int WC, int OCC, F16Mode MODE, bool XF32 = false>
+template <int TM, int TN, int WR, int WC, int OCC, F16Mode MODE, bool XF32, int AHEAD>
 __global__ __launch_bounds__(WR *WC * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 void gemm_f16_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64_t N, const uint8_t *__restrict__ ws,
                      size_t ws_stride, int64_t M, float *__restrict__ y, int64_t ldy, TileMap map, RowGather rg, F16Batch fb) {
@@ -113,11 +120,13 @@ void gemm_f16_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int6
             xsrc[i] = ws + (size_t)arow * ws_stride + 16 * (item % C::CELLS);
         }
     }
-    u32x4 wq[C::W_PER_T], xq[C::X_PER_T];
-    float4 xf[XF32 ? C::X_PER_T : 1][2];                             // rounded when they are committed: nothing waits in fetch
-    bool live = true;
+    u32x4 wqs[AHEAD][C::W_PER_T], xqs[AHEAD][C::X_PER_T];
+    float4 xfs[AHEAD][XF32 ? C::X_PER_T : 1][2];                     // rounded when they are committed: nothing waits in fetch
+    bool lives[AHEAD];
 
-    auto fetch = [&](int stage) {
+    auto fetch = [&](auto set, int stage) {
+        auto &wq = wqs[decltype(set)::value]; auto &xq = xqs[decltype(set)::value]; auto &xf = xfs[decltype(set)::value];
+        bool &live = lives[decltype(set)::value];
         live = !KTAIL || (int64_t)stage * (16 * F16_KG) + 8 * my_cell < K;
         const size_t off = live ? (size_t)stage * STAGE_BYTES : 0;                   // a dead cell re-reads stage 0 (in bounds) and is zeroed
 #pragma unroll
@@ -133,7 +142,9 @@ void gemm_f16_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int6
             }
         }
     };
-    auto commit = [&](int buf) {
+    auto commit = [&](auto set, int buf) {
+        auto &wq = wqs[decltype(set)::value]; auto &xq = xqs[decltype(set)::value]; auto &xf = xfs[decltype(set)::value];
+        const bool live = lives[decltype(set)::value];
         const u32x4 z = {0u, 0u, 0u, 0u};
         u32x4 *A = reinterpret_cast<u32x4 *>(lds + (size_t)buf * C::STAGE + C::OFF_A);
         u32x4 *B = reinterpret_cast<u32x4 *>(lds + (size_t)buf * C::STAGE + C::OFF_B);
@@ -158,13 +169,12 @@ void gemm_f16_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int6
 #pragma unroll
             for (int v = 0; v < 16; v++) acc[a][c][v] = 0.f;
 
-    fetch(0);
-    commit(0);
-    __syncthreads();
-
-    for (int s = 0; s < nstages; s++) {
+    // stage s: its registers are in LDS already, so they take stage s + AHEAD (unconditional: the last stage is loaded again)
+    const int last = nstages - 1;
+    auto step = [&](auto set, int s) {
+        constexpr int J = decltype(set)::value;
         const int buf = s & 1;
-        fetch(min(s + 1, nstages - 1));                              // unconditional: the last stage is loaded twice
+        fetch(set, min(s + AHEAD, last));
         const f16x8 *A = reinterpret_cast<const f16x8 *>(lds + (size_t)buf * C::STAGE + C::OFF_A);
         const f16x8 *B = reinterpret_cast<const f16x8 *>(lds + (size_t)buf * C::STAGE + C::OFF_B);
 #pragma unroll
@@ -179,8 +189,25 @@ void gemm_f16_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int6
 #pragma unroll
                 for (int c = 0; c < TN; c++) acc[a][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[a], bf[c], acc[a][c], 0, 0, 0);
         }
-        commit(buf ^ 1);
+        commit(std::integral_constant<int, (J + 1) % AHEAD>{}, buf ^ 1);
         __syncthreads();
+    };
+
+    fetch(std::integral_constant<int, 0>{}, 0);
+    if constexpr (AHEAD > 1) fetch(std::integral_constant<int, 1 % AHEAD>{}, min(1, last));
+    if constexpr (AHEAD > 2) fetch(std::integral_constant<int, 2 % AHEAD>{}, min(2, last));
+    commit(std::integral_constant<int, 0>{}, 0);
+    __syncthreads();
+    for (int s = 0; s < nstages; s += AHEAD) {
+        step(std::integral_constant<int, 0>{}, s);
+        if constexpr (AHEAD > 1) {
+            if (s + 1 >= nstages) break;
+            step(std::integral_constant<int, 1 % AHEAD>{}, s + 1);
+        }
+        if constexpr (AHEAD > 2) {
+            if (s + 2 >= nstages) break;
+            step(std::integral_constant<int, 2 % AHEAD>{}, s + 2);
+        }
     }
 
     // ---- epilogue: register v of tile (a, c) is row 8*(v/4) + 4*half + v%4, token l32 ----
@@ -368,13 +395,13 @@ static hipError_t launch_f16_direct(const void *W, size_t nb01, int64_t K, int64
 // rows must be 16-byte aligned (the weight alignment rule of the C-ABI) and K a multiple of the 64-value stage
 bool gemm_f16_supported(int64_t K, int64_t N, int64_t n) { return K >= 64 && K % (16 * F16_KG) == 0 && N >= 1 && n >= 32; }
 
-template <int TM, int TN, int WR, int WC, int OCC, F16Mode MODE, bool XF32 = false>
+template <int TM, int TN, int WR, int WC, int OCC, F16Mode MODE, bool XF32 = false, int AHEAD = 1>
 static hipError_t launch_f16(const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, int64_t M,
                              float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t n_as,
                              const F16Batch &fb = F16Batch{1, 0, 0, nullptr, 0, 0, 1}) {
     using C = F16Cfg<TM, TN, WR, WC>;
     const size_t lds_bytes = 2 * C::STAGE;
-    auto kfn = gemm_f16_kernel<TM, TN, WR, WC, OCC, MODE, XF32>;
+    auto kfn = gemm_f16_kernel<TM, TN, WR, WC, OCC, MODE, XF32, AHEAD>;
     static LdsGrant grant;
     if (hipError_t e = grant_dynamic_lds(kfn, lds_bytes, lim, grant); e != hipSuccess) return e;
     TileMap map = make_tile_map(ceil_div(N, C::BM), MODE == F16_PLAIN ? ceil_div(M, C::BN) : 1, 32 * (4 * OCC / C::NW > 0 ? 4 * OCC / C::NW : 1));
@@ -418,8 +445,8 @@ hipError_t launch_gemm_f16(const void *W, size_t nb01, int64_t K, int64_t N, con
     const int64_t g128 = ceil_div(N, 128) * ceil_div(M, 128), g256 = ceil_div(N, 256) * ceil_div(M, 256);
     const int cfg = (int)tune("CHIP_GEMM_F16_CFG", 2 * g256 >= cus && K >= 4 * BIG_K && n_as == 1 ? 9 : g128 >= cus ? 0 : 1);
     switch (cfg) {
-        case 0: return launch_f16<2, 2, 2, 2, 2, F16_PLAIN>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);       // 128 x 128, 4 waves
-        case 1: return launch_f16<1, 1, 2, 2, 4, F16_PLAIN>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);       // 64 x 64, 4 waves
+        case 0: return launch_f16<2, 2, 2, 2, 2, F16_PLAIN, false, 2>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);       // 128 x 128, 4 waves
+        case 1: return launch_f16<1, 1, 2, 2, 4, F16_PLAIN, false, 3>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);       // 64 x 64, 4 waves
         case 2: return launch_f16<2, 2, 2, 4, 2, F16_PLAIN>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);       // 128 x 256, 8 waves
         case 3: return launch_f16<2, 4, 2, 2, 2, F16_PLAIN>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);       // 128 x 256, 4 waves
         case 9: return launch_f16_direct(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st);                             // 256 x 256, 4 waves, direct to LDS

@@ -122,3 +122,18 @@ def test_attention_matmuls_of_a_prompt(dev, orc, hd, nh, nkv, n, kv):
         y = dev.mul_mat_f16_batched(w, x)
         ref = orc.mul_mat_f16_batched(w, np.ascontiguousarray(x[:, toks]), want=("sum_abs",))
         check(y[:, toks], ref, "attention matmul")
+
+
+# ---- F16 weights: the loads run two or three stages of 64 values ahead of the products ----
+# four to twenty stages (every remainder of two and three), ragged 64 x 64 tiles; the same over 128 x 128 tiles
+@pytest.mark.parametrize("N,n", [(131, 70), (2050, 2049)])
+@pytest.mark.parametrize("K", (256, 512, 768, 1280))
+def test_f16_gemm_stage_counts(dev, orc, K, N, n):
+    rng = np.random.default_rng(K + N)
+    w = orc.quantize_weights(O.F16, common.weights_f32(K + N, N, K))
+    x = common.activations_f32(K + n, n, K)
+    y = dev.mul_mat(O.F16, w, x)
+    rows = np.unique(np.concatenate([[0, N - 1], rng.choice(N, min(N, 200), replace=False)]))
+    toks = np.unique(np.concatenate([[0, n - 1], rng.choice(n, min(n, 64), replace=False)]))
+    ref = orc.mul_mat(O.F16, w[rows], x[toks], nthreads=8, want=("sum_abs",))
+    check(y[np.ix_(toks, rows)], ref, "F16 gemm, %d stages" % (K // 64))
