@@ -417,12 +417,14 @@ static hipError_t launch_f16(const void *W, size_t nb01, int64_t K, int64_t N, c
 //   kq: 128 x 128 once they give every CU four workgroups, else 64 x 64.
 // Measured (us, 32 query heads over 8 KV heads of 128, 512 tokens, 4096 positions): kqv 67 (fp16 copy) + 157 (64 x 64 tiles, whose
 // padded two-tile grid rows all fell on two of the eight XCDs) + 5 (tile list) -> 117; kq 91 + 5 -> 84.
+// kqv loads two stages ahead: a one-layer step of that size 793 -> 742 us (three ahead 743), 300 tokens at position 3000 (15 heads
+// over 5 of 64, 8 layers) 1502 -> 1414 (three ahead 1732: registers).  kq, two stages of K in all, keeps one (two: 802, three: 834).
 hipError_t launch_gemm_f16_batch(const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, float *y, int64_t ldy,
                                  const DeviceLimits &lim, hipStream_t st, const F16Batch &fb) {
     const RowGather rg{nullptr, nullptr, nullptr, 1, 1, 0};
     const int64_t cus = lim.compute_units > 0 ? lim.compute_units : 256, c64 = ceil_div(fb.per_head, (int64_t)64);
 #define BATCH_CASE(TM, TN, WR, WC, OCC, XF) \
-    return launch_f16<TM, TN, WR, WC, OCC, F16_BATCH, XF>(W, nb01, K, N, ws, ws_stride, fb.per_head, y, ldy, lim, st, rg, 1, fb)
+    return launch_f16<TM, TN, WR, WC, OCC, F16_BATCH, XF, XF ? 2 : 1>(W, nb01, K, N, ws, ws_stride, fb.per_head, y, ldy, lim, st, rg, 1, fb)
     if (fb.x) {
         const int bn = (int)tune("CHIP_ATTN_BN", fb.heads * c64 * ceil_div(N, (int64_t)128) >= cus ? 64 : 32);
         if (N > 64) { if (bn == 64) BATCH_CASE(2, 1, 2, 2, 2, true); else BATCH_CASE(1, 1, 4, 1, 3, true); }
