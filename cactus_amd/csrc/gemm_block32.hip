@@ -542,27 +542,31 @@ bool gemm_blk32_supported(int wtype, int64_t K, int64_t N, int64_t n, bool can_s
 }
 
 // ---- split K: the partial outputs [slice][token][row] added in slice order ----
-__global__ __launch_bounds__(256) void sum_slices_kernel(const float *__restrict__ part, int slices, int64_t per_slice, int64_t n,
-                                                         int64_t N, float *__restrict__ y, int64_t ldy) {
-    const int64_t e0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;                // four consecutive rows of one token
-    if (e0 >= n * N) return;
-    const uint32_t t = (uint32_t)(e0 / N);
-    const int64_t r = e0 - (int64_t)t * N;
-    const bool vec = (N & 3) == 0 && (((uintptr_t)part) & 15) == 0;
+// Bound by the reads of the partial outputs.  A thread adds four consecutive rows of one token; the groups of four are counted
+// per token, so that none straddles two, and with N not a multiple of 4 they lie at 4-byte alignment and each token's last one is
+// short.  One launch for every N: such an N used to take a launch per token (us of the whole product, before -> now: Q3_K
+// 4352 x 694 at 363 tokens 909 -> 22, Q2_K 13056 x 1159 at 69 tokens 331 -> 27, Q8_0 5312 x 670 at 1107 tokens 2403 -> 42).
+__global__ __launch_bounds__(256) void sum_slices_kernel(const float *__restrict__ part, int slices, int64_t n, int64_t N,
+                                                         float *__restrict__ y, int64_t ldy) {
+    typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+    const int64_t groups = ceil_div(N, (int64_t)4), g = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (g >= n * groups) return;
+    const int64_t t = g / groups, r = (g - t * groups) * 4, per_slice = n * N;
+    const float *src0 = part + t * N + r;
+    const bool whole = r + 3 < N;
     float v[4] = {0.f, 0.f, 0.f, 0.f};
     for (int s0 = 0; s0 < slices; s0 += 8) {
-        float4 p[8];
+        f32x4_a4 p[8];
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-            p[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+            p[j] = f32x4_a4{0.f, 0.f, 0.f, 0.f};
             if (s0 + j < slices) {
-                const float *src = part + (size_t)(s0 + j) * per_slice + e0;
-                if (vec) p[j] = *reinterpret_cast<const float4 *>(src);
+                const float *src = src0 + (size_t)(s0 + j) * per_slice;
+                if (whole) p[j] = *reinterpret_cast<const f32x4_a4 *>(src);
                 else {
                     p[j].x = src[0];
                     if (r + 1 < N) p[j].y = src[1];
                     if (r + 2 < N) p[j].z = src[2];
-                    if (r + 3 < N) p[j].w = src[3];
                 }
             }
         }
@@ -577,15 +581,8 @@ __global__ __launch_bounds__(256) void sum_slices_kernel(const float *__restrict
 }
 hipError_t launch_sum_slices(const float *part, int slices, int64_t n, int64_t N, float *y, int64_t ldy, hipStream_t st) {
     if (n <= 0 || N <= 0 || slices <= 0) return hipSuccess;
-    // a token's rows in fours: with N not a multiple of 4 a group of four would straddle two tokens, so pad per token
-    if ((N & 3) != 0) {
-        for (int64_t t = 0; t < n; t++) {
-            hipLaunchKernelGGL(sum_slices_kernel, dim3((unsigned)ceil_div(N, (int64_t)1024)), dim3(256), 0, st, part + t * N, slices, n * N,
-                               (int64_t)1, N, y + t * ldy, ldy);
-        }
-        return hipGetLastError();
-    }
-    hipLaunchKernelGGL(sum_slices_kernel, dim3((unsigned)ceil_div(n * N, (int64_t)1024)), dim3(256), 0, st, part, slices, n * N, n, N, y, ldy);
+    hipLaunchKernelGGL(sum_slices_kernel, dim3((unsigned)ceil_div(n * ceil_div(N, (int64_t)4), (int64_t)256)), dim3(256), 0, st, part, slices,
+                       n, N, y, ldy);
     return hipGetLastError();
 }
 

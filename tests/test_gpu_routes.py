@@ -1,0 +1,54 @@
+"""Which kernels a call takes: the launches of a call are counted as the nodes of a graph that records it."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import common
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    import cactus_amd
+    return cactus_amd.Device(0)
+
+
+def launches(dev, call):
+    """Kernel launches of call(stream), which is made once before it is recorded (a kernel's first launch raises its LDS limit)."""
+    hip = C.CDLL("libamdhip64.so")
+    st, graph, count = C.c_void_p(), C.c_void_p(), C.c_size_t()
+    dev.check(dev.lib.chip_stream_create(C.byref(st)))
+    dev.check(call(st))
+    dev.sync(st)
+    assert hip.hipStreamBeginCapture(st, 0) == 0
+    rc = call(st)
+    assert hip.hipStreamEndCapture(st, C.byref(graph)) == 0 and rc == 0
+    assert hip.hipGraphGetNodes(graph, None, C.byref(count)) == 0
+    hip.hipGraphDestroy(graph)
+    dev.check(dev.lib.chip_stream_destroy(st))
+    return count.value
+
+
+def mul_mat_launches(dev, wt, W, x, split_k=True):
+    n, K = x.shape
+    N, L = W.shape[0], dev.lib
+    dW, dx, dy = dev.to_device(W), dev.to_device(x), dev.alloc(n * N * 4)
+    wsz = L.chip_mul_mat_workspace_size_n(wt, K, N, n) if split_k else L.chip_mul_mat_workspace_size(wt, K, n)
+    ws = dev.alloc(wsz)
+    return launches(dev, lambda st: L.chip_mul_mat(wt, dW.ptr, W.shape[1], K, N, dx.ptr, K, n, dy.ptr, N, ws.ptr, wsz, st))
+
+
+# quantizer, GEMM over slices of K, slice sum; rows in fours, and one, two and three rows in a token's last group
+@pytest.mark.parametrize("N", (300, 301, 302, 303, 3))
+@pytest.mark.parametrize("wt", (O.Q3_K, O.Q4_K, O.Q8_0), ids=lambda t: O.TYPE_NAMES[t])
+def test_split_k_takes_three_launches_whatever_the_rows(dev, orc, wt, N):
+    K, n = 4096, 70
+    wq = orc.quantize_weights(wt, common.weights_f32(K + N, N, K))
+    x = common.activations_f32(K + n, n, K)
+    assert mul_mat_launches(dev, wt, wq, x) == 3
+    ref = orc.mul_mat(wt, wq, x, nthreads=8, want=("sum_abs",))
+    err = np.abs(dev.mul_mat(wt, wq, x).astype(np.float64) - ref["y"].astype(np.float64))
+    assert (err <= 1e-5 * ref["sum_abs"]).all()
