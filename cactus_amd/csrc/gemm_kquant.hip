@@ -1006,12 +1006,10 @@ void gemm_ks_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64
 // memory speed.  Up to 128 tokens on a matrix with few row tiles the walk is cut into slices (kq_slices_for below:
 // 16 - 19 us at K = 4096, 36 - 41 us at K = 14336).  The token count from which the GEMM is ahead, measured on 4096 x 4096,
 // 14336 x 4096 (too many row tiles to split) and 4096 x 14336:
-// (Q3_K, Q2_K and IQ4_XS, us at 16 tokens: two GEMV passes against the GEMM at 17: Q3_K 21 / 14, 44 / 24 and 41 / 28, IQ4_XS
-// 20 / 17, 40 / 35 and 40 / 38; 201 tokens of Q3_K on 4096 x 14336: 26 passes, 499 us, against 46.)
 static bool kq_splittable(int64_t N) { return ceil_div(N, (int64_t)64) <= 128; }
 static int64_t gemm_kq_min_tokens(int wtype, int64_t K, int64_t N, bool can_split) {
     if (can_split || !kq_splittable(N)) {
-        if (wtype != T_Q4_K && wtype != T_Q5_K) return 9;            // their GEMV passes take 8 tokens
+        if (wtype == T_Q6_K) return 9;                               // its GEMV passes take 8 tokens
         return kq_splittable(N) ? 17 : 33;                           // Q4_K, Q5_K: passes of 16 tokens
     }
     // the caller's workspace has no room for the partial outputs: the unsplit walk
@@ -1021,15 +1019,6 @@ static int64_t gemm_kq_min_tokens(int wtype, int64_t K, int64_t N, bool can_spli
         case T_Q5_K: return long_rows ? 33 : 49;
         default:     return long_rows ? 41 : 25;
     }
-}
-bool gemm_kq_type(int wtype) {
-    return wtype == T_Q4_K || wtype == T_Q5_K || wtype == T_Q6_K || wtype == T_Q3_K || wtype == T_Q2_K || wtype == T_IQ4_XS;
-}
-bool gemm_kq_supported(int wtype, int64_t K, int64_t N, int64_t n, bool can_split) {
-    if (!gemm_kq_type(wtype) || K < QK_K || K % QK_K != 0 || N < 1) return false;
-    const int64_t forced = tune("CHIP_GEMM_MIN_TOKENS", 0);
-    if (forced > 0) return n >= forced;
-    return n >= gemm_kq_min_tokens(wtype, K, N, can_split);
 }
 
 // Slices of K for the 64 x 128 shape: up to two workgroups per CU with one token tile, one per CU with more (the partial
@@ -1048,6 +1037,37 @@ static int kq_slices_for(int64_t K, int64_t N, int64_t M, int64_t cus) {
     if (s < 2) return 1;
     const int64_t per = ceil_div(units, s);
     return (int)ceil_div(units, per);                                   // no empty slice
+}
+// Q3_K, Q2_K and IQ4_XS: the dot-product GEMV passes of 8 tokens, whose time grows with the tokens, against the GEMM, whose time
+// below 128 tokens does not.  A token count alone does not part them (GEMV / GEMM, us, split K: IQ4_XS 8192 x 8192 at 12
+// tokens 36 / 43, 14336 x 1024 at 9 tokens 20 / 19; Q2_K 4096 x 1024 at 10 tokens 12 / 14, 4096 x 4096 at 9 tokens 16 / 15;
+// unsplit: IQ4_XS 7168 x 748 at 32 tokens 34 / 58, 1024 x 4096 at 25 tokens 32 / 14), so both times are estimated, in us, with terms
+// fitted to 5000 measured products (to 12 and 7 per cent for nine in ten of them):
+//   GEMV   a launch per pass, then per token the rounds of 1024 rows (four a CU) and of 4096 values of a row
+//   GEMM   quantizer and launch (and slice sum), then the super-blocks a workgroup walks times the rounds of 256 workgroups; split K
+//          has most of the weights in flight at once and pays for their bytes too
+static bool low_bit_gemm_ahead(int wtype, int64_t K, int64_t N, int64_t n, int slices) {
+    if (n < 9) return false;                                         // one GEMV pass
+    const int64_t group = gemv_max_tokens(wtype, K, DeviceLimits{256, 160 * 1024});      // 8, fewer on very long rows
+    if (group < 1) return true;
+    const float passes = (float)ceil_div(n, group), rows = (float)ceil_div(N, (int64_t)1024), parts = (float)ceil_div(K, (int64_t)4096);
+    const float gemv = passes * (4.6f + 0.235f * rows) + (float)n * parts * (0.135f + 0.103f * rows);
+    const int64_t tiles = ceil_div(N, (int64_t)64) * ceil_div(n, (int64_t)128) * slices;
+    const float walk = (wtype == T_Q3_K ? 1.12f : wtype == T_Q2_K ? 1.23f : 1.84f) * (float)ceil_div(K / QK_K, (int64_t)slices) *
+                       (float)ceil_div(tiles, (int64_t)256);
+    const float gemm = slices == 1 ? 7.1f + walk : 9.2f + 0.82f * walk + 0.14f * (float)N * (float)K / 1048576.f;
+    return gemm < gemv;
+}
+bool gemm_kq_type(int wtype) {
+    return wtype == T_Q4_K || wtype == T_Q5_K || wtype == T_Q6_K || wtype == T_Q3_K || wtype == T_Q2_K || wtype == T_IQ4_XS;
+}
+bool gemm_kq_supported(int wtype, int64_t K, int64_t N, int64_t n, bool can_split) {
+    if (!gemm_kq_type(wtype) || K < QK_K || K % QK_K != 0 || N < 1) return false;
+    const int64_t forced = tune("CHIP_GEMM_MIN_TOKENS", 0);
+    if (forced > 0) return n >= forced;
+    if (wtype == T_Q3_K || wtype == T_Q2_K || wtype == T_IQ4_XS)
+        return low_bit_gemm_ahead(wtype, K, N, n, can_split ? kq_slices_for(K, N, n, 256) : 1);
+    return n >= gemm_kq_min_tokens(wtype, K, N, can_split);
 }
 int gemm_kq_slices(int wtype, int64_t K, int64_t N, int64_t n, int compute_units) {
     if (!gemm_kq_supported(wtype, K, N, n, true)) return 1;

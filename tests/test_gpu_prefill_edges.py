@@ -56,9 +56,11 @@ def random_rows(wt, rng, N, nsb):
     return w.reshape(N, -1)
 
 
-# (K, N, n): the fewest tokens; ragged tiles; K split over workgroups with uneven slices; 128 x 128 tiles; many tokens, few rows
+# (K, N, n): one super-block; ragged tiles; K split over workgroups with uneven slices; the GEMV passes that 9 tokens take on few
+# short rows; 128 x 128 tiles; many tokens, few rows; the GEMM at the fewest tokens it is taken from
 @pytest.mark.parametrize("wt", LOW_BIT, ids=lambda t: O.TYPE_NAMES[t])
-@pytest.mark.parametrize("K,N,n", [(256, 5, 41), (1024, 131, 65), (2304, 131, 70), (4096, 300, 9), (512, 4100, 1030), (768, 33, 1100)])
+@pytest.mark.parametrize("K,N,n", [(256, 5, 41), (1024, 131, 65), (2304, 131, 70), (4096, 300, 9), (512, 4100, 1030), (768, 33, 1100),
+                                   (14336, 70, 9)])
 def test_low_bit_kquant_gemm(dev, orc, wt, K, N, n):
     rng = np.random.default_rng(K + N + wt)
     w = random_rows(wt, rng, N, K // 256)

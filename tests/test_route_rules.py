@@ -1,0 +1,32 @@
+"""CPU-only: which kernels a shape is sent to, as the workspace size queries show it (256 compute units where no device is present)."""
+import pytest
+
+import cactus_amd as ca
+
+
+@pytest.fixture(scope="module")
+def lib():
+    return ca.load_library()
+
+
+def splits_k(lib, t, K, N, n):
+    return lib.chip_mul_mat_workspace_size_n(t, K, N, n) > lib.chip_mul_mat_workspace_size(t, K, n)
+
+
+# Measured on either side of the rule (us, GEMV passes / GEMM): the low-bit types take the GEMM, with K split, only where it is ahead
+@pytest.mark.parametrize("t,K,N,n,gemm", [
+    (ca.IQ4_XS, 4096, 1024, 10, False), (ca.IQ4_XS, 8192, 8192, 12, False), (ca.IQ4_XS, 2048, 692, 9, False),        # 12 / 17, 36 / 43, 12 / 16
+    (ca.IQ4_XS, 14336, 1024, 12, True), (ca.IQ4_XS, 4096, 4096, 17, True),                                           # 23 / 19, 24 / 18
+    (ca.Q3_K, 2816, 300, 10, False), (ca.Q3_K, 3840, 612, 9, False), (ca.Q3_K, 4096, 4096, 9, True), (ca.Q3_K, 14336, 1024, 9, True),
+    (ca.Q3_K, 14336, 70, 9, True), (ca.Q2_K, 14336, 70, 9, True), (ca.IQ4_XS, 14336, 70, 9, True),
+    (ca.Q2_K, 2304, 280, 11, False), (ca.Q2_K, 4096, 1024, 10, False), (ca.Q2_K, 4096, 4096, 12, True)])
+def test_low_bit_types_take_the_gemm_where_it_is_ahead(lib, t, K, N, n, gemm):
+    assert splits_k(lib, t, K, N, n) == gemm
+    assert splits_k(lib, t, K, N, 70)
+    assert not splits_k(lib, t, K, N, 8)
+
+
+def test_rows_too_long_for_the_gemv_stay_accepted(lib):
+    """K = 2^18: no token's activations fit a workgroup's local memory, so only the GEMM can run it."""
+    for t in (ca.Q3_K, ca.Q2_K, ca.IQ4_XS):
+        assert splits_k(lib, t, 1 << 18, 64, 9)
