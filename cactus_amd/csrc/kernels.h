@@ -330,6 +330,7 @@ hipError_t launch_moe_group(const int32_t *ids, int64_t ids_stride, int64_t n_us
                             int tile_tokens, int32_t *offsets, int32_t *perm, int32_t *tiles, hipStream_t st);
 int        gemm_blk32_moe_tile_tokens();
 int        gemm_kq_moe_tile_tokens();
+bool       gemm_kq_moe_ahead(int wtype, int64_t K, int64_t N, int64_t n_as, int64_t pairs);   // the GEMM by expert groups against a GEMV per pair
 int        gemm_f16_moe_tile_tokens();
 
 }  // namespace chip

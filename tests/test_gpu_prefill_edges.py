@@ -96,10 +96,12 @@ def test_low_bit_kquant_integer_sums_bit_exact(dev, orc, wt):
     assert np.array_equal(y.astype(np.int64), want)
 
 
+@pytest.mark.parametrize("n_tokens", (90, 700))
 @pytest.mark.parametrize("wt", LOW_BIT, ids=lambda t: O.TYPE_NAMES[t])
-def test_low_bit_kquant_expert_groups(dev, orc, wt):
-    """64 pairs and more: the pairs grouped by expert and run through the GEMM (ragged groups, an expert nobody picks)."""
-    K, N, n_as, n_used, n_tokens = 512, 70, 5, 2, 90
+def test_low_bit_kquant_expert_groups(dev, orc, wt, n_tokens):
+    """64 pairs and more, an expert nobody picks: a GEMV per pair while that is ahead (90 tokens here), then the pairs grouped by
+    expert and run through the GEMM (700 tokens; ragged groups of several token tiles)."""
+    K, N, n_as, n_used = 512, 70, 5, 2
     rng = np.random.default_rng(wt)
     experts = np.stack([random_rows(wt, rng, N, K // 256) for _ in range(n_as)])
     x = common.activations_f32(wt, n_tokens, K).reshape(n_tokens, 1, K)

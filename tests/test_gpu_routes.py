@@ -52,3 +52,22 @@ def test_split_k_takes_three_launches_whatever_the_rows(dev, orc, wt, N):
     ref = orc.mul_mat(wt, wq, x, nthreads=8, want=("sum_abs",))
     err = np.abs(dev.mul_mat(wt, wq, x).astype(np.float64) - ref["y"].astype(np.float64))
     assert (err <= 1e-5 * ref["sum_abs"]).all()
+
+
+# A GEMV per pair is two launches (quantizer, GEMV), the expert groups three (quantizer, grouping, GEMM).  Measured on either side of
+# the rule: few pairs an expert, many pairs, and short rows, where the GEMM is ahead with a pair an expert
+@pytest.mark.parametrize("wt", (O.Q3_K, O.Q2_K, O.IQ4_XS), ids=lambda t: O.TYPE_NAMES[t])
+@pytest.mark.parametrize("K,N,n_as,n_used,n_tokens,gemm", [(2048, 768, 128, 8, 8, False), (1024, 256, 64, 2, 32, False), (2048, 768, 128, 8, 192, True),
+                                                           (512, 2048, 32, 4, 100, True), (1024, 256, 8, 8, 40, True), (512, 70, 5, 2, 90, False), (512, 70, 5, 2, 700, True)])
+def test_low_bit_expert_matmul_takes_the_gemm_where_it_is_ahead(dev, wt, K, N, n_as, n_used, n_tokens, gemm):
+    L, row = dev.lib, dev.row_size(wt, K)
+    rng = np.random.default_rng(K + N)
+    dW = dev.alloc(n_as * N * row)
+    dev.check(L.chip_memset(dW.ptr, 0, n_as * N * row, None))
+    dx = dev.to_device(common.activations_f32(K, n_tokens, K))
+    ids = dev.to_device(np.stack([rng.permutation(n_as)[:n_used] for _ in range(n_tokens)]).astype(np.int32))
+    dy = dev.alloc(n_tokens * n_used * N * 4)
+    wsz = L.chip_mul_mat_id_workspace_size(wt, K, n_as, n_used, n_tokens, 1)
+    ws = dev.alloc(wsz)
+    assert launches(dev, lambda st: L.chip_mul_mat_id(wt, dW.ptr, row, N * row, K, N, n_as, dx.ptr, K, 1, ids.ptr, n_used, n_used, n_tokens,
+                                                      dy.ptr, N, ws.ptr, wsz, st)) == (3 if gemm else 2)
