@@ -526,8 +526,18 @@ void gemm_blk32_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, in
 static bool blk32_splittable(int64_t N) { return ceil_div(N, (int64_t)64) <= 384; }
 static int64_t gemm_blk32_min_tokens(int wtype, int64_t K, int64_t N, bool can_split) {
     const bool long_rows = K > 8192, big = N * K >= ((int64_t)48 << 20);
-    if (can_split && blk32_splittable(N)) return (wtype == T_Q8_0 && long_rows) ? 9 : 17;
+    if (can_split && blk32_splittable(N)) {
+        // Rows with a short last stage, where these three types are also slower to unpack: on a small matrix a third GEMV pass over
+        // one or two tokens is the cheaper (us, passes / GEMM at 17 tokens: Q4_1 320 x 2624 14.7 / 17.4, Q5_0 960 x 3648 15.8 / 18.4,
+        // Q5_1 192 x 3264 at 18 tokens 15.2 / 16.2; rows beyond 4096 values 20 / 16, 2560 x 2496 22 / 17)
+        if (K % (32 * GEMM_KB) != 0 && K <= 4096 && N <= 1024 && (wtype == T_Q5_0 || wtype == T_Q4_1 || wtype == T_Q5_1)) return 19;
+        return (wtype == T_Q8_0 && long_rows) ? 9 : 17;
+    }
     // too many row tiles to split, or no room for the partial outputs in the caller's workspace: the unsplit walk
+    // (long rows with a short last stage, few of them: the walk is slower than the passes up to some 60 tokens - us, passes / GEMM,
+    // 320 x 12352: Q5_0 48 tokens 67 / 97, 65 tokens 93 / 97, Q4_1 64 tokens 85 / 93, IQ4_NL 48 tokens 69 / 77, 56 tokens 78 / 77, Q8_0
+    // 49 tokens 68 / 73; 320 x 8256: IQ4_NL 49 tokens 61 / 57; 2560 x 8256 at 48 tokens the GEMM is ahead)
+    if (K % (32 * GEMM_KB) != 0 && long_rows && N <= 1024) return !(wtype == T_Q8_0 || wtype == T_IQ4_NL) ? 65 : K > 10240 ? 57 : 49;
     switch (wtype) {
         case T_Q8_0: return long_rows ? 49 : big ? 17 : 49;
         case T_Q4_0: return long_rows ? 65 : big ? 33 : 49;

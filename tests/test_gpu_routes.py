@@ -71,3 +71,10 @@ def test_low_bit_expert_matmul_takes_the_gemm_where_it_is_ahead(dev, wt, K, N, n
     ws = dev.alloc(wsz)
     assert launches(dev, lambda st: L.chip_mul_mat_id(wt, dW.ptr, row, N * row, K, N, n_as, dx.ptr, K, 1, ids.ptr, n_used, n_used, n_tokens,
                                                       dy.ptr, N, ws.ptr, wsz, st)) == (3 if gemm else 2)
+
+
+# long rows with a short last stage, no room to split K: quantizer and six GEMV passes while they are ahead of the GEMM's walk
+@pytest.mark.parametrize("wt,n,count", [(O.Q5_0, 48, 7), (O.Q4_1, 48, 7), (O.Q5_1, 48, 7), (O.IQ4_NL, 48, 7), (O.Q5_0, 65, 2), (O.IQ4_NL, 57, 2), (O.Q8_0, 57, 2)])
+def test_unsplit_short_last_stage_takes_the_gemm_where_it_is_ahead(dev, orc, wt, n, count):
+    wq = orc.quantize_weights(wt, common.weights_f32(5, 64, 8256))
+    assert mul_mat_launches(dev, wt, wq, common.activations_f32(6, n, 8256), split_k=False) == count

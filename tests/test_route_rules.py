@@ -26,6 +26,14 @@ def test_low_bit_types_take_the_gemm_where_it_is_ahead(lib, t, K, N, n, gemm):
     assert not splits_k(lib, t, K, N, 8)
 
 
+# the third GEMV pass over one or two tokens against the GEMM (us: 14.7 / 17.4, 15.8 / 18.4, 15.2 / 16.2; 20 / 16, 22 / 15, 17 / 16)
+@pytest.mark.parametrize("t,K,N,n,gemm", [(ca.Q4_1, 2624, 320, 17, False), (ca.Q5_0, 3648, 960, 17, False), (ca.Q5_1, 3264, 192, 18, False),
+                                          (ca.Q5_1, 4160, 320, 17, True), (ca.Q4_0, 2112, 2560, 18, True), (ca.Q4_0, 2624, 960, 17, True),
+                                          (ca.Q4_1, 2624, 320, 19, True), (ca.Q4_1, 2560, 320, 17, True)])
+def test_short_last_stage_takes_the_gemm_where_it_is_ahead(lib, t, K, N, n, gemm):
+    assert splits_k(lib, t, K, N, n) == gemm
+
+
 def test_rows_too_long_for_the_gemv_stay_accepted(lib):
     """K = 2^18: no token's activations fit a workgroup's local memory, so only the GEMM can run it."""
     for t in (ca.Q3_K, ca.Q2_K, ca.IQ4_XS):
