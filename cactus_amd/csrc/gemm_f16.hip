@@ -48,8 +48,8 @@ enum F16Mode { F16_PLAIN, F16_EXPERTS, F16_BATCH };
 // of its loads: a stage's 4 (16) MFMAs a wave end long before the next stage's weights have come from HBM.  One stage ahead -> AHEAD
 // (us, a different 4096 x 4096 F16 matrix each call, which no cache holds): 64 x 64 tiles, AHEAD 3: 64 tokens 38.4 -> 26.6, 201
 // tokens 41.3 -> 30.0, 512 tokens 61.7 -> 45.2 (AHEAD 2: 29.8, 33.3, 44.6; AHEAD 4 at three workgroups a CU: 26.0, 28.7, 45.8;
-// at four it spills: 66.9, 70.7, 111); 128 tokens of 14336 x 4096: 179 -> 106.  128 x 128 tiles, AHEAD 2: 1024 tokens 83.8 -> 66.6,
-// 300 tokens of 4096 x 14336 89.7 -> 85.7.
+// at four it spills: 66.9, 70.7, 111); 128 tokens of 14336 x 4096: 179 -> 106.  128 x 128 tiles, AHEAD 2: 1024 tokens 83.8 -> 66.6.
+// More workgroups a CU cover each other's loads, and the deeper prefetch then only crowds the caches (launch_gemm_f16).
 __device__ __forceinline__ u32x4 round8_f16(const float4 a, const float4 b) {
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
     const h2 h0 = {(_Float16)a.x, (_Float16)a.y}, h1 = {(_Float16)a.z, (_Float16)a.w};
@@ -444,11 +444,18 @@ hipError_t launch_gemm_f16(const void *W, size_t nb01, int64_t K, int64_t N, con
     const RowGather rg = rgp ? *rgp : RowGather{nullptr, nullptr, nullptr, 1, 1, 0};
     const int64_t cus = lim.compute_units > 0 ? lim.compute_units : 256;
     if (rg.perm) return launch_f16<1, 1, 2, 2, 4, F16_EXPERTS>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);      // expert groups: 64 x 64 tiles
-    const int64_t g128 = ceil_div(N, 128) * ceil_div(M, 128), g256 = ceil_div(N, 256) * ceil_div(M, 256);
+    // Stages ahead, by the workgroups a CU runs (400 drawn products, median of the times against the other depth): 128 x 128, one
+    // a CU: 2 (1 is 14 % slower), more: 1 (3 % faster than 2 for K > 2048, the same below); 64 x 64, up to one and a half a CU: 3, more: 2
+    // (up to 2 a CU 1 %, from 2.5 a CU 3 % faster than 3; 1 is 5 to 35 % slower up to 2.5 a CU and no faster beyond).
+    const int64_t g128 = ceil_div(N, 128) * ceil_div(M, 128), g256 = ceil_div(N, 256) * ceil_div(M, 256), g64 = ceil_div(N, 64) * ceil_div(M, 64);
     const int cfg = (int)tune("CHIP_GEMM_F16_CFG", 2 * g256 >= cus && K >= 4 * BIG_K && n_as == 1 ? 9 : g128 >= cus ? 0 : 1);
     switch (cfg) {
-        case 0: return launch_f16<2, 2, 2, 2, 2, F16_PLAIN, false, 2>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);       // 128 x 128, 4 waves
-        case 1: return launch_f16<1, 1, 2, 2, 4, F16_PLAIN, false, 3>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);       // 64 x 64, 4 waves
+        case 0:                                                                                                         // 128 x 128, 4 waves
+            if (g128 > cus) return launch_f16<2, 2, 2, 2, 2, F16_PLAIN, false, 1>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
+            return launch_f16<2, 2, 2, 2, 2, F16_PLAIN, false, 2>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
+        case 1:                                                                                                         // 64 x 64, 4 waves
+            if (2 * g64 > 3 * cus) return launch_f16<1, 1, 2, 2, 4, F16_PLAIN, false, 2>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
+            return launch_f16<1, 1, 2, 2, 4, F16_PLAIN, false, 3>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
         case 2: return launch_f16<2, 2, 2, 4, 2, F16_PLAIN>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);       // 128 x 256, 8 waves
         case 3: return launch_f16<2, 4, 2, 2, 2, F16_PLAIN>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);       // 128 x 256, 4 waves
         case 9: return launch_f16_direct(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st);                             // 256 x 256, 4 waves, direct to LDS
