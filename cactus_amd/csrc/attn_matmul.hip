@@ -446,13 +446,13 @@ GemmPlan gemm_plan(int64_t K, int64_t N, int64_t ne02, int64_t r2, int64_t n) {
     GemmPlan p{};
     const int64_t per_head = r2 * n;
     const int64_t min_cols = tune("CHIP_ATTN_GEMM_MIN", GEMM_MIN_COLS);
-    p.use = K >= 64 && K % 8 == 0 && N >= 32 && per_head >= min_cols && ne02 * per_head < (1LL << 30) &&
-            ne02 * ceil_div(per_head, (int64_t)32) * ceil_div(N, (int64_t)64) < (1LL << 31);          // workgroups of the one-dimensional grid
-    if (!p.use) return p;
-    p.act_stride = f16_stride(K);
     // kqv (a head's 64 - 256 rows, one or two row tiles): the GEMM reads the fp32 activations itself.  kq, with thousands of
     // cache positions as rows, reads the activations back once per row tile: it gets an fp16 copy first.
     p.direct = N <= 256;
+    p.use = K >= 64 && K % 8 == 0 && N >= 32 && per_head >= min_cols && ne02 * per_head < (1LL << 30) &&
+            gemm_f16_batch_threads(ne02, per_head, N, p.direct, 256) < (1LL << 32);
+    if (!p.use) return p;
+    p.act_stride = f16_stride(K);
     p.bytes = (size_t)(ne02 * per_head) * p.act_stride;
     return p;
 }

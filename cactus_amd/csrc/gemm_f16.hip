@@ -405,33 +405,46 @@ static hipError_t launch_f16(const void *W, size_t nb01, int64_t K, int64_t N, c
     static LdsGrant grant;
     if (hipError_t e = grant_dynamic_lds(kfn, lds_bytes, lim, grant); e != hipSuccess) return e;
     TileMap map = make_tile_map(ceil_div(N, C::BM), MODE == F16_PLAIN ? ceil_div(M, C::BN) : 1, 32 * (4 * OCC / C::NW > 0 ? 4 * OCC / C::NW : 1));
-    if (MODE == F16_BATCH) map.grid = (unsigned)(fb.heads * ceil_div(fb.per_head, (int64_t)C::BN) * map.row_tiles);      // < 2^31, checked by the caller
+    if (MODE == F16_BATCH) map.grid = (unsigned)(fb.heads * ceil_div(fb.per_head, (int64_t)C::BN) * map.row_tiles);      // gemm_f16_batch_threads, checked by the caller
     hipLaunchKernelGGL(kfn, dim3(map.grid, (unsigned)n_as), dim3(C::NT), lds_bytes, st, (const uint8_t *)W, nb01, K, N,
                        (const uint8_t *)ws, ws_stride, M, y, ldy, map, rg, fb);
     return hipGetLastError();
 }
 
+struct BatchTile { int rows, columns, threads; };
 // The attention matmuls of a prompt.  Tiles (rows x columns of a KV head):
-//   kqv (fp32 activations, at most 256 rows): all rows of a head (64 or 128) in one tile, so that the probabilities are read
-//     once, by 64 columns - 32 while that leaves CUs without a workgroup.
+//   kqv (fp32 activations, at most 256 rows): all rows of a head in one tile of 64 or 128, so that the probabilities are read
+//     once, by 64 columns - 32 while that leaves CUs without a workgroup.  Head sizes of 129 to 256 take two tiles that read them from
+//     the same L2 (8 heads over 2 of 256, 512 tokens, 4096 positions: 36 us, with an fp16 copy and 64 x 64 tiles 65; 16 heads over 8,
+//     2048 tokens 161 against 420).
 //   kq: 128 x 128 once they give every CU four workgroups, else 64 x 64.
 // Measured (us, 32 query heads over 8 KV heads of 128, 512 tokens, 4096 positions): kqv 67 (fp16 copy) + 157 (64 x 64 tiles, whose
 // padded two-tile grid rows all fell on two of the eight XCDs) + 5 (tile list) -> 117; kq 91 + 5 -> 84.
 // kqv loads two stages ahead: a one-layer step of that size 793 -> 742 us (three ahead 743), 300 tokens at position 3000 (15 heads
 // over 5 of 64, 8 layers) 1502 -> 1414 (three ahead 1732: registers).  kq, two stages of K in all, keeps one (two: 802, three: 834).
+static BatchTile batch_tile(int64_t heads, int64_t per_head, int64_t N, bool f32_rows, int64_t cus) {
+    if (!f32_rows) {
+        const bool big = N >= 128 && per_head >= 128 && heads * ceil_div(per_head, (int64_t)128) * ceil_div(N, (int64_t)128) >= 4 * cus;
+        return big ? BatchTile{128, 128, 256} : BatchTile{64, 64, 256};
+    }
+    const int bn = (int)tune("CHIP_ATTN_BN", heads * ceil_div(per_head, (int64_t)64) * ceil_div(N, (int64_t)128) >= cus ? 64 : 32);
+    return N > 64 ? BatchTile{128, bn, 256} : BatchTile{64, bn, bn == 64 ? 256 : 128};
+}
+int64_t gemm_f16_batch_threads(int64_t heads, int64_t per_head, int64_t N, bool f32_rows, int64_t cus) {
+    const BatchTile t = batch_tile(heads, per_head, N, f32_rows, cus);
+    return heads * ceil_div(per_head, (int64_t)t.columns) * ceil_div(N, (int64_t)t.rows) * t.threads;
+}
 hipError_t launch_gemm_f16_batch(const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, float *y, int64_t ldy,
                                  const DeviceLimits &lim, hipStream_t st, const F16Batch &fb) {
     const RowGather rg{nullptr, nullptr, nullptr, 1, 1, 0};
-    const int64_t cus = lim.compute_units > 0 ? lim.compute_units : 256, c64 = ceil_div(fb.per_head, (int64_t)64);
+    const BatchTile t = batch_tile(fb.heads, fb.per_head, N, fb.x != nullptr, lim.compute_units > 0 ? lim.compute_units : 256);
 #define BATCH_CASE(TM, TN, WR, WC, OCC, XF) \
     return launch_f16<TM, TN, WR, WC, OCC, F16_BATCH, XF, XF ? 2 : 1>(W, nb01, K, N, ws, ws_stride, fb.per_head, y, ldy, lim, st, rg, 1, fb)
     if (fb.x) {
-        const int bn = (int)tune("CHIP_ATTN_BN", fb.heads * c64 * ceil_div(N, (int64_t)128) >= cus ? 64 : 32);
-        if (N > 64) { if (bn == 64) BATCH_CASE(2, 1, 2, 2, 2, true); else BATCH_CASE(1, 1, 4, 1, 3, true); }
-        if (bn == 64) BATCH_CASE(1, 1, 2, 2, 4, true); else BATCH_CASE(1, 1, 2, 1, 3, true);
+        if (t.rows == 128) { if (t.columns == 64) BATCH_CASE(2, 1, 2, 2, 2, true); else BATCH_CASE(1, 1, 4, 1, 3, true); }
+        if (t.columns == 64) BATCH_CASE(1, 1, 2, 2, 4, true); else BATCH_CASE(1, 1, 2, 1, 3, true);
     }
-    const bool big = N >= 128 && fb.per_head >= 128 && fb.heads * ceil_div(fb.per_head, (int64_t)128) * ceil_div(N, (int64_t)128) >= 4 * cus;
-    if (big) BATCH_CASE(2, 2, 2, 2, 2, false);
+    if (t.rows == 128) BATCH_CASE(2, 2, 2, 2, 2, false);
     BATCH_CASE(1, 1, 2, 2, 4, false);
 #undef BATCH_CASE
 }

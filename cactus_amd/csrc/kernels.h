@@ -242,7 +242,9 @@ hipError_t launch_gemm_f16(const void *W, size_t nb01, int64_t K, int64_t N, con
 // The attention matmuls with many columns: `heads` products of one shape.  Batch e takes the weights W + e * nb02 and rows
 // e * per_head ... of the workspace and of y.  x (optional): the activation rows as fp32, row R = token R % n of batch R / n,
 // rounded to fp16 in the kernel's staging instead of being read from the fp16 workspace.
+// gemm_f16_batch_threads: threads of its one-dimensional grid, which HIP takes below 2^32.
 struct F16Batch { int64_t heads, per_head; size_t nb02; const float *x; int64_t ldx1, ldx2, n; };
+int64_t    gemm_f16_batch_threads(int64_t heads, int64_t per_head, int64_t N, bool f32_rows, int64_t cus);
 hipError_t launch_gemm_f16_batch(const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, float *y, int64_t ldy,
                                  const DeviceLimits &lim, hipStream_t st, const F16Batch &fb);
 

@@ -38,3 +38,11 @@ def test_rows_too_long_for_the_gemv_stay_accepted(lib):
     """K = 2^18: no token's activations fit a workgroup's local memory, so only the GEMM can run it."""
     for t in (ca.Q3_K, ca.Q2_K, ca.IQ4_XS):
         assert splits_k(lib, t, 1 << 18, 64, 9)
+
+
+def test_attention_grids_stay_below_the_launch_limit(lib):
+    """kq through the GEMM needs room for fp16 activations; a grid of 2^32 threads or more cannot be launched and is not planned."""
+    size = lib.chip_mul_mat_f16_batched_workspace_size
+    assert size(64, 1 << 20, 8, 8, 100) == 800 * 128
+    assert size(64, 1 << 28, 8, 8, 100) == 0                   # 8 x 2 x 2^22 workgroups of 256 threads
+    assert size(64, 1 << 24, 8, 8, 1024) == 8192 * 128         # 8 x 8 x 2^17 of the larger tiles
