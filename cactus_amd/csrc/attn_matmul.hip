@@ -453,7 +453,10 @@ GemmPlan gemm_plan(int64_t K, int64_t N, int64_t ne02, int64_t r2, int64_t n) {
             gemm_f16_batch_threads(ne02, per_head, N, p.direct, 256) < (1LL << 32);
     if (!p.use) return p;
     p.act_stride = f16_stride(K);
-    p.bytes = (size_t)(ne02 * per_head) * p.act_stride;
+    // The direct form writes nothing to the workspace and asks for no more than that there is one: a caller without any keeps the kernels
+    // that cut K over their lanes, slower but closer to the 64-bit sums (kqv of 300 tokens over 4096 positions: 1.0e-7 relative, the
+    // GEMM's accumulation along K 4.0e-7).
+    p.bytes = p.direct ? 256 : (size_t)(ne02 * per_head) * p.act_stride;
     return p;
 }
 
@@ -503,14 +506,13 @@ hipError_t launch_mul_mat_f16_batched(const void *W, size_t nb01, size_t nb02, i
     // the GEMM writes row R of y at R * ldy1: the batches of y must follow each other without a gap
     if (plan.use && !y2 && workspace && workspace_bytes >= plan.bytes && ldy2 == n * ldy1 && n <= 65535 && ne02 * r2 <= 65535) {
         uint8_t *ws = (uint8_t *)workspace;
-        const bool direct = plan.direct && n <= 0x7fffffff && ne02 * r2 * n <= 0x7fffffff;
-        if (!direct) {
+        if (!plan.direct) {
             const int64_t chunks = K / 8, per = chunks >= AM_THREADS ? 1 : AM_THREADS / chunks;
             hipLaunchKernelGGL(mm_f16_round_rows_kernel, dim3((unsigned)ceil_div(n, per), (unsigned)(ne02 * r2)), dim3(AM_THREADS), 0, st, x,
                                ldx1, ldx2, n, K, ws, plan.act_stride);
             if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
         }
-        const F16Batch fb{ne02, r2 * n, nb02, direct ? x : nullptr, ldx1, ldx2, n};
+        const F16Batch fb{ne02, r2 * n, nb02, plan.direct ? x : nullptr, ldx1, ldx2, n};
         return launch_gemm_f16_batch(W, nb01, K, N, ws, plan.act_stride, y, ldy1, lim, st, fb);
     }
     const BatchedArgs a{(const uint8_t *)W, nb01, nb02, K, N, x, ldx1, ldx2, n, r2, y, ldy1, ldy2, y2, ld2y1, ld2y2};

@@ -78,3 +78,25 @@ def test_low_bit_expert_matmul_takes_the_gemm_where_it_is_ahead(dev, wt, K, N, n
 def test_unsplit_short_last_stage_takes_the_gemm_where_it_is_ahead(dev, orc, wt, n, count):
     wq = orc.quantize_weights(wt, common.weights_f32(5, 64, 8256))
     assert mul_mat_launches(dev, wt, wq, common.activations_f32(6, n, 8256), split_k=False) == count
+
+
+# kqv of more than 128 columns per KV head: one launch of the GEMM with the 256 bytes it asks for, the same bits whatever lies behind
+# them, and nothing written there; one launch of the dot-product kernel without a workspace
+@pytest.mark.parametrize("hd,nh,nkv,n,kv", [(128, 8, 2, 70, 264), (64, 6, 3, 133, 1064), (256, 4, 1, 65, 520), (96, 8, 4, 80, 136)])
+def test_kqv_of_a_prompt_with_a_small_workspace(dev, orc, hd, nh, nkv, n, kv):
+    L, rng = dev.lib, np.random.default_rng(hd + n + kv)
+    vt = rng.standard_normal((nkv, hd, kv)).astype(np.float16)
+    p = rng.random((nh, n, kv)).astype(np.float32)
+    ref = orc.mul_mat_f16_batched(vt, p, want=("sum_abs",))
+    dv, dp, dy = dev.to_device(vt), dev.to_device(p), dev.alloc(nh * n * hd * 4)
+    outs = []
+    for wsz in (0, 256, nh * n * kv * 2 + 4096):
+        ws = dev.to_device(np.full(max(wsz, 16), 0x5A, np.uint8))
+        assert launches(dev, lambda st: L.chip_mul_mat_f16_batched(dv.ptr, 2 * kv, 2 * kv * hd, kv, hd, nkv, dp.ptr, kv, kv * n, n, nh, dy.ptr,
+                                                                   hd, hd * n, ws.ptr if wsz else None, wsz, st)) == 1
+        y = dy.download(np.float32, nh * n * hd).reshape(nh, n, hd)
+        assert (np.abs(y - ref["y"]) <= 1e-5 * ref["sum_abs"]).all()
+        assert (ws.download(np.uint8, max(wsz, 16)) == 0x5A).all()
+        outs.append(y)
+    assert outs[1].tobytes() == outs[2].tobytes()
+    assert outs[0].tobytes() != outs[1].tobytes()

@@ -46,3 +46,10 @@ def test_attention_grids_stay_below_the_launch_limit(lib):
     assert size(64, 1 << 20, 8, 8, 100) == 800 * 128
     assert size(64, 1 << 28, 8, 8, 100) == 0                   # 8 x 2 x 2^22 workgroups of 256 threads
     assert size(64, 1 << 24, 8, 8, 1024) == 8192 * 128         # 8 x 8 x 2^17 of the larger tiles
+
+
+def test_kqv_of_a_prompt_asks_for_no_copy(lib):
+    """Its GEMM reads the fp32 probabilities; up to 128 pairs per KV head the split-K kernels still want room for partial outputs."""
+    size = lib.chip_mul_mat_f16_batched_workspace_size
+    assert size(4096, 128, 8, 32, 512) == 256 and size(4096, 256, 2, 8, 2048) == 256
+    assert size(4096, 128, 8, 32, 32) > 256 and size(128, 4096, 8, 32, 512) == 8 * 2048 * 256
