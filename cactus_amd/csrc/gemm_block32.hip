@@ -554,41 +554,40 @@ bool gemm_blk32_supported(int wtype, int64_t K, int64_t N, int64_t n, bool can_s
 
 // ---- split K: the partial outputs [slice][token][row] added in slice order ----
 // Bound by the reads of the partial outputs.  A thread adds four consecutive rows of one token; the groups of four are counted
-// per token, so that none straddles two, and with N not a multiple of 4 they lie at 4-byte alignment and each token's last one is
-// short.  One launch for every N: such an N used to take a launch per token (us of the whole product, before -> now: Q3_K
-// 4352 x 694 at 363 tokens 909 -> 22, Q2_K 13056 x 1159 at 69 tokens 331 -> 27, Q8_0 5312 x 670 at 1107 tokens 2403 -> 42).
+// per token, so that none straddles two.  With N not a multiple of 4 they lie at 4-byte alignment, and a token's last group starts
+// at N - 4 and stores only the rows that the group before it has not, so that every load is a whole one.  One launch for every N: such
+// an N used to take a launch per token (us of the whole product, before -> now: Q3_K 4352 x 694 at 363 tokens 909 -> 22, Q2_K 13056 x 1159
+// at 69 tokens 331 -> 27, Q8_0 5312 x 670 at 1107 tokens 2403 -> 42).
 __global__ __launch_bounds__(256) void sum_slices_kernel(const float *__restrict__ part, int slices, int64_t n, int64_t N,
                                                          float *__restrict__ y, int64_t ldy) {
     typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
     const int64_t groups = ceil_div(N, (int64_t)4), g = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (g >= n * groups) return;
     const int64_t t = g / groups, r = (g - t * groups) * 4, per_slice = n * N;
-    const float *src0 = part + t * N + r;
-    const bool whole = r + 3 < N;
-    float v[4] = {0.f, 0.f, 0.f, 0.f};
+    if (N < 4) {                                                                     // one group of one to three rows
+        for (int64_t k = 0; k < N; k++) {
+            float v = 0.f;
+            for (int s = 0; s < slices; s++) v += part[(size_t)s * per_slice + t * N + k];
+            y[(size_t)t * ldy + k] = v;
+        }
+        return;
+    }
+    const int64_t first = r < N - 4 ? r : N - 4;
+    const float *src = part + t * N + first;
+    f32x4_a4 v = {0.f, 0.f, 0.f, 0.f};
     for (int s0 = 0; s0 < slices; s0 += 8) {
         f32x4_a4 p[8];
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            p[j] = f32x4_a4{0.f, 0.f, 0.f, 0.f};
-            if (s0 + j < slices) {
-                const float *src = src0 + (size_t)(s0 + j) * per_slice;
-                if (whole) p[j] = *reinterpret_cast<const f32x4_a4 *>(src);
-                else {
-                    p[j].x = src[0];
-                    if (r + 1 < N) p[j].y = src[1];
-                    if (r + 2 < N) p[j].z = src[2];
-                }
-            }
-        }
+        for (int j = 0; j < 8; j++)
+            if (s0 + j < slices) p[j] = *reinterpret_cast<const f32x4_a4 *>(src + (size_t)(s0 + j) * per_slice);
 #pragma unroll
         for (int j = 0; j < 8; j++)
-            if (s0 + j < slices) { v[0] += p[j].x; v[1] += p[j].y; v[2] += p[j].z; v[3] += p[j].w; }
+            if (s0 + j < slices) v += p[j];
     }
-    float *dst = y + (size_t)t * ldy + r;
+    float *dst = y + (size_t)t * ldy + first;
 #pragma unroll
     for (int k = 0; k < 4; k++)
-        if (r + k < N) dst[k] = v[k];
+        if (first + k >= r) dst[k] = v[k];
 }
 hipError_t launch_sum_slices(const float *part, int slices, int64_t n, int64_t N, float *y, int64_t ldy, hipStream_t st) {
     if (n <= 0 || N <= 0 || slices <= 0) return hipSuccess;
