@@ -19,7 +19,8 @@
 //
 //   F16 activations (for F16 weights), token stride = f16_stride(K): K halves, nothing else.
 //
-// K is a multiple of 256, so every plane starts 16-byte aligned.  Token strides are multiples of 128 bytes: a token's
+// With K a multiple of 256 every plane starts 16-byte aligned; Q8_0 rows also come with K % 64 == 0, where qs and d still do and sum
+// starts at a multiple of 8 bytes.  Token strides are multiples of 128 bytes: a token's
 // 128-byte stretches of quants then coincide with cache lines, which halves the lines the GEMM kernels touch.
 #pragma once
 #include <stdint.h>

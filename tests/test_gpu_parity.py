@@ -533,7 +533,8 @@ def test_mul_mat_with_transposed_fp16_store(dev, wt):
 def test_block32_rows_of_k_not_a_multiple_of_256(dev, orc, wt, K, N):
     """Hidden sizes such as 576, 896 and 960 (K % 64 == 0): the rows of the 32-value block types are then multiples of 4
     bytes only.  Every token count class: prologue-quantizing GEMV (1, 2, 4), GEMV over the workspace (3, 5, 8), several
-    passes (11, 20), and from 17 tokens the GEMM where K % 128 == 0 (896, 960 is not: passes)."""
+    passes (11, and 20 where K is too short to be split), and the GEMM: at 70 tokens for every K, at 20 tokens with K = 4160 split.
+    Its last stage is short where K is an odd multiple of 64 (all but 896)."""
     import cactus_amd as ca
     assert dev.lib.chip_mul_mat_supported(wt, K) == 1
     wq = quantized_weights(wt, 7 * K + N, N, K)
