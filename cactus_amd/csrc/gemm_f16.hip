@@ -469,8 +469,6 @@ hipError_t launch_gemm_f16(const void *W, size_t nb01, int64_t K, int64_t N, con
         case 1:                                                                                                         // 64 x 64, 4 waves
             if (2 * g64 > 3 * cus) return launch_f16<1, 1, 2, 2, 4, F16_PLAIN, false, 2>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
             return launch_f16<1, 1, 2, 2, 4, F16_PLAIN, false, 3>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
-        case 2: return launch_f16<2, 2, 2, 4, 2, F16_PLAIN>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);       // 128 x 256, 8 waves
-        case 3: return launch_f16<2, 4, 2, 2, 2, F16_PLAIN>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);       // 128 x 256, 4 waves
         case 9: return launch_f16_direct(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st);                             // 256 x 256, 4 waves, direct to LDS
         default: return hipErrorInvalidValue;
     }

@@ -1147,7 +1147,6 @@ static hipError_t launch_kq_type(const void *W, size_t nb01, int64_t K, int64_t 
     const int cfg = (int)tune("CHIP_GEMM_KQ_CFG", single_plane ? 11 : g128 >= cus ? 0 : 2);
     switch (cfg) {
         case 0: return launch_kq<WT, 4, 2, 3, false>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);      // 128 x 128, 8 + 4 waves
-        case 1: return launch_kq<WT, 4, 1, 2, false>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);      // 128 x 64, 4 + 4 waves
         case 2: return launch_kq<WT, 2, 2, 2, false>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);      // 64 x 128, 4 + 4 waves
         case 11: return launch_ks<WT, 1, 2, 2, 2, 2, false>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);   // single plane, 64 x 128, 4 waves
         default: return hipErrorInvalidValue;
