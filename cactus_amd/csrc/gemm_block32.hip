@@ -556,8 +556,8 @@ bool gemm_blk32_supported(int wtype, int64_t K, int64_t N, int64_t n, bool can_s
 // Bound by the reads of the partial outputs.  A thread adds four consecutive rows of one token; the groups of four are counted
 // per token, so that none straddles two.  With N not a multiple of 4 they lie at 4-byte alignment, and a token's last group starts
 // at N - 4 and stores only the rows that the group before it has not, so that every load is a whole one.  One launch for every N: such
-// an N used to take a launch per token (us of the whole product, before -> now: Q3_K 4352 x 694 at 363 tokens 909 -> 22, Q2_K 13056 x 1159
-// at 69 tokens 331 -> 27, Q8_0 5312 x 670 at 1107 tokens 2403 -> 42).
+// an N used to take a launch per token (us of the whole product, before -> now: Q3_K 694 x 4352 at 363 tokens 909 -> 22, Q2_K 1159 x 13056
+// at 69 tokens 331 -> 27, Q8_0 670 x 5312 at 1107 tokens 2403 -> 42).
 __global__ __launch_bounds__(256) void sum_slices_kernel(const float *__restrict__ part, int slices, int64_t n, int64_t N,
                                                          float *__restrict__ y, int64_t ldy) {
     typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));

@@ -1041,9 +1041,9 @@ static int kq_slices_for(int64_t K, int64_t N, int64_t M, int64_t cus) {
 }
 // Q3_K, Q2_K and IQ4_XS: the dot-product GEMV passes of 8 tokens, whose time grows with the tokens, against the GEMM, whose time
 // below 128 tokens does not.  A token count alone does not part them (GEMV / GEMM, us, split K: IQ4_XS 8192 x 8192 at 12
-// tokens 36 / 43, 14336 x 1024 at 9 tokens 20 / 19; Q2_K 4096 x 1024 at 10 tokens 12 / 14, 4096 x 4096 at 9 tokens 16 / 15;
-// unsplit: IQ4_XS 7168 x 748 at 32 tokens 34 / 58, 1024 x 4096 at 25 tokens 32 / 14), so both times are estimated, in us, with terms
-// fitted to 5000 measured products (to 12 and 7 per cent for nine in ten of them):
+// tokens 36 / 43, 1024 x 14336 at 9 tokens 20 / 19; Q2_K 1024 x 4096 at 10 tokens 12 / 14, 4096 x 4096 at 9 tokens 16 / 15;
+// unsplit: IQ4_XS 748 x 7168 at 32 tokens 34 / 58, 4096 x 1024 at 25 tokens 32 / 14), so both times are estimated, in us, with terms
+// fitted to 5000 measured products (to 13 and 9 per cent for nine in ten of them):
 //   GEMV   a launch per pass, then per token the rounds of 1024 rows (four a CU) and of 4096 values of a row
 //   GEMM   quantizer and launch (and slice sum), then the super-blocks a workgroup walks times the rounds of 256 workgroups; split K
 //          has most of the weights in flight at once and pays for their bytes too
@@ -1158,7 +1158,7 @@ static hipError_t launch_kq_type(const void *W, size_t nb01, int64_t K, int64_t 
 // runs one in eight of an expert's row tiles.  With ids drawn evenly n_as * (1 - e^(-pairs / n_as)) experts are picked.
 // (GEMV / GEMM, us: Q2_K 768 x 2048, 128 experts, 64 pairs 18 / 53, 1024 pairs 194 / 119; Q3_K 2048 x 768 at 256 pairs 171 / 87;
 // 14336 x 4096, 8 experts, 64 pairs 294 / 166.  Of 1500 drawn calls 12 took the
-// slower kernel by more than 5 %, one by more than 13 %.)
+// slower kernel by more than 5 %, the worst by 28 %: Q3_K 2048 x 768, 128 experts, 64 pairs 47 / 60.)
 bool gemm_kq_moe_ahead(int wtype, int64_t K, int64_t N, int64_t n_as, int64_t pairs) {
     if (wtype != T_Q3_K && wtype != T_Q2_K && wtype != T_IQ4_XS) return true;
     if (gemv_max_tokens(wtype, K, DeviceLimits{256, 160 * 1024}) < 1) return true;

@@ -134,7 +134,7 @@ CHIP_API int chip_convert_f32_to_f16(const float *x, int64_t ldx, int64_t n, int
  *               reference, sized by lm_ggml_graph_plan, ggml-cpu/ggml-cpu.c:2697-2704); holds the quantized
  *               activations in a kernel-private layout
  * n <= 4 runs the dot-product GEMV with the quantizer in its prologue; Q8_0 with n >= 5 the matrix-core GEMV
- * (16 tokens per pass over W); from 9 to 48 tokens on (by type and matrix size) the MFMA GEMM of the weight type;
+ * (16 tokens per pass over W); from 9 tokens on, where it is ahead for the type and the sizes, the MFMA GEMM of the weight type;
  * everything else the GEMV in token groups.
  * K must be a multiple of 256; for the types of 32-value blocks (Q4_0, Q8_0, Q5_0, IQ4_NL, Q4_1, Q5_1) a multiple of 64
  * is enough (hidden sizes such as 576, 896, 960: the GEMV and the GEMM).  W must be 16-byte aligned
