@@ -1,0 +1,711 @@
+// Prefill GEMM for gfx950 over K-quant weights (Q2_K .. Q6_K, IQ4_XS) and Q8_K activations: the batched form of
+// lm_ggml_vec_dot_q2_K_q8_K .. _q6_K_q8_K, _iq4_xs_q8_K (reference ggml-cpu/ggml-cpu-quants.c) as driven by
+// lm_ggml_compute_forward_mul_mat (ggml-cpu/ggml-cpu.c:1257-1449).
+//
+// Per 256-value super-block the reference forms two integers per (row, token), sumi = sum_j sc_j * dot(q_j, a_j) and (Q4_K, Q5_K,
+// Q2_K) summ = sum_j m_j * bsum_j, and applies d, dmin and the activation scale once.  As in gemm_kquant.hip the integer sub-block
+// scales ride in the int8 MFMA operand, as one or two digit planes whose products accumulate over the super-block in the MFMA's own int32
+// registers, and summ is one fp16 MFMA (mins times the 16 block sums, exact):
+//
+//   Q4_K           sc = 8*sh + sl (3-bit digits): planes q*sh and q*sl (<= 105), sumi = 8*P0 + P1
+//   Q5_K, Q6_K, IQ4_XS   the product v = q*sc, (q - 32)*sc, code*sc (16 bits) as 256*hi + lo with signed bytes, sumi = 256*P0 + P1
+//   Q3_K           (4 - q)*sc in -128..124: one plane, sumi = -P0
+//   Q2_K           q*sc <= 45: one plane, sumi = P0
+//
+// What is different is who expands.  There, staging waves write both planes of a 64 x 128 tile into LDS and every wave reads them back:
+// twice the packed bytes times four in LDS traffic, two barriers per super-block, one stage of loads in flight.  Here a wave owns 32 weight
+// rows and 64 tokens: it loads its rows' packed bytes in memory order, turns them round through a stretch of LDS of its own
+// (no barrier), reads its MFMA lanes' quants back and expands them in registers between its MFMAs.  Only the activations are shared by the
+// four waves of a k group (global_load_lds, double buffered), so a super-block needs one barrier and everything it waits for was
+// requested a whole super-block earlier.
+//
+// Bound: the vector instructions and MFMAs of a SIMD do not overlap (403 and 34 per super-block and wave for Q4_K; 62 % + 42 % of the cycles
+// by the counters, 16384 rows x 4096 values x 1024 tokens), LDS is 27 % busy without bank conflicts.  Reading operands a step ahead took
+// a quarter off the first form, in which every read was waited for at once (4096 x 4096 x 512 48 -> 36 us); widening d and dmin once instead
+// of in a half-rate v_fma_mix per output and full-rate v_bitop3 in place of v_and_or / v_bfi another 3 %.
+// Measured against the staging kernel (and, for Q4_K and Q5_K, the single-plane kernel) it replaced, us: Q4_K 512 x 4096 values x 4096
+// rows 40 -> 34, x 14336 rows 104 -> 94, 512 x 14336 x 4096 108 -> 94, 32 x 14336 x 4096 38 -> 22; Q2_K 512 x 4096 x 14336 84 -> 68; Q6_K
+// 1500 x 4096 x 14336 404 -> 316; Q5_K 512 x 14336 x 4096 139 -> 109.
+#include "dev_common.h"
+#include "act_layout.h"
+#include "kernels.h"
+#include <type_traits>
+
+namespace chip {
+
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+namespace {
+
+// two independent 16-bit products / multiply-adds per dword (v_pk_mul_lo_u16, v_pk_mad_u16)
+__device__ __forceinline__ uint32_t pk_mul16(uint32_t a, uint32_t b) {
+    return __builtin_bit_cast(uint32_t, (u16x2)(__builtin_bit_cast(u16x2, a) * __builtin_bit_cast(u16x2, b)));
+}
+__device__ __forceinline__ uint32_t pk_mad16(uint32_t a, uint32_t b, uint32_t c) {
+    return __builtin_bit_cast(uint32_t, (u16x2)(__builtin_bit_cast(u16x2, a) * __builtin_bit_cast(u16x2, b) + __builtin_bit_cast(u16x2, c)));
+}
+__device__ __forceinline__ uint32_t splat16(uint32_t v) { return (v & 0xffffu) | (v << 16); }
+
+// 6-bit scales and mins of sub-blocks 2jp and 2jp+1 (low byte, next byte) from the 12 packed bytes that follow
+// d and dmin (reference ggml-quants.c:625-632)
+__device__ __forceinline__ void scale_min_pair(const u32x4 &h, int jp, uint32_t &sc, uint32_t &mn) {
+    const int sh = 16 * (jp & 1);
+    const uint32_t a1 = h.y >> sh, a2 = h.z >> sh, a3 = h.w >> sh;
+    if (jp < 2) { sc = a1 & 0x3f3fu; mn = a2 & 0x3f3fu; }
+    else        { sc = (a3 & 0x0f0f0f0fu & 0xffffu) | ((a1 >> 2) & 0x3030u); mn = ((a3 >> 4) & 0x0f0fu) | ((a2 >> 2) & 0x3030u); }
+}
+// the same for four sub-blocks at once, one per byte: sub-blocks 0..3 (g = 0) or 4..7 (g = 1)
+__device__ __forceinline__ void scale_min_quad(const u32x4 &h, int g, uint32_t &sc, uint32_t &mn) {
+    const uint32_t sc0 = h.y & 0x3f3f3f3fu, mn0 = h.z & 0x3f3f3f3fu;
+    const uint32_t sc1 = (h.w & 0x0f0f0f0fu) | ((h.y >> 2) & 0x30303030u), mn1 = ((h.w >> 4) & 0x0f0f0f0fu) | ((h.z >> 2) & 0x30303030u);
+    sc = g ? sc1 : sc0;
+    mn = g ? mn1 : mn0;
+}
+// two small integers -> fp16 (exact)
+__device__ __forceinline__ uint32_t f16_pair(uint32_t a, uint32_t b) {
+    return (uint32_t)__half_as_ushort(__float2half_rn((float)a)) | ((uint32_t)__half_as_ushort(__float2half_rn((float)b)) << 16);
+}
+// four small integers (one per byte) -> the fp16 operand cell {b0, b0, b1, b1, b2, b2, b3, b3}: sub-block j stands
+// against the two 16-value bsums 2j and 2j+1
+__device__ __forceinline__ u32x4 bytes_to_f16_pairs(uint32_t v) {
+    u32x4 c;
+#pragma unroll
+    for (int i = 0; i < 4; i++) c[i] = f16_pair((v >> (8 * i)) & 0xffu, (v >> (8 * i)) & 0xffu);
+    return c;
+}
+// eight int16 -> eight fp16 (exact for |v| <= 2048)
+__device__ __forceinline__ u32x4 i16x8_to_f16(const u32x4 &v) {
+    u32x4 c;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const _Float16 lo = (_Float16)(int16_t)(v[i] & 0xffffu), hi = (_Float16)(int16_t)(v[i] >> 16);
+        c[i] = (uint32_t)__builtin_bit_cast(unsigned short, lo) | ((uint32_t)__builtin_bit_cast(unsigned short, hi) << 16);
+    }
+    return c;
+}
+// (a & m) | (b & ~m) as one full-rate instruction
+__device__ __forceinline__ uint32_t merge_bits(uint32_t m, uint32_t a, uint32_t b) { return __builtin_amdgcn_bitop3_b32(a, b, m, 0xe4); }
+// four 6- to 8-bit values (bytes of v, masked by m) times a signed scale: p = v * sc + bias - 128 = 256 * hi + lo with both
+// digits signed bytes.  mul = the scale, add = 128 plus the product's own bias, both in two 16-bit halves.
+__device__ __forceinline__ void byte_digits(uint32_t v, uint32_t m, uint32_t mul, uint32_t add, uint32_t &hi, uint32_t &lo) {
+    const uint32_t ue = pk_mad16(v & m, mul, add), uo = pk_mad16((v >> 8) & m, mul, add);
+    hi = __builtin_amdgcn_perm(uo, ue, 0x07030501u);
+    lo = __builtin_amdgcn_perm(uo, ue, 0x06020400u) ^ 0x80808080u;
+}
+
+// Per weight type.  A super-block is fetched as NCH 16-byte chunks (the last one ends with the super-block, so it may overlap the
+// one before) and kept in LDS as STRIDE cells of a row, STRIDE odd so that 16 rows' cells of one index fall into different banks.
+// Lane (row, hf) reads its share back: hdr() what all items need, load<Q>() the 16-value k-half hf of k-blocks KA(Q) and KB(Q), which
+// expand<Q>() turns into MFMA operand cells [k-block][plane].
+template <int WT> struct KR;
+
+template <> struct KR<T_Q4_K> {
+    static constexpr int BYTES = BYTES_Q4_K, NCH = 9, NPL = 2, NF16 = 1;
+    typedef u32x4 chunk_t;
+    struct Hdr { u32x4 h; };
+    __device__ static __forceinline__ Hdr hdr(const u32x4 *row, int) { return Hdr{row[0]}; }
+    static constexpr int KA(int q) { return 2 * q; }
+    static constexpr int KB(int q) { return 2 * q + 1; }
+    struct Raw { u32x4 q; };
+    template <int Q> __device__ static __forceinline__ Raw load(const u32x4 *row, int hf) { return Raw{row[1 + 2 * Q + hf]}; }
+    template <int Q> __device__ static __forceinline__ void expand(const Raw &r, const Hdr &h, int, u32x4 (&c)[2][2]) {
+        uint32_t sc, mn;
+        scale_min_pair(h.h, Q, sc, mn);
+        const uint32_t sh0 = (sc >> 3) & 7u, sl0 = sc & 7u, sh1 = sc >> 11, sl1 = (sc >> 8) & 7u;
+        const u32x4 q = r.q;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint32_t lo = q[i] & 0x0f0f0f0fu, hi = (q[i] >> 4) & 0x0f0f0f0fu;
+            c[0][0][i] = lo * sh0; c[0][1][i] = lo * sl0;                             // four byte products <= 105: no carries
+            c[1][0][i] = hi * sh1; c[1][1][i] = hi * sl1;
+        }
+    }
+    __device__ static __forceinline__ u32x4 f16_cell(const Hdr &h, int, int half) {
+        uint32_t sc, mn;
+        scale_min_quad(h.h, half, sc, mn);
+        return bytes_to_f16_pairs(mn);
+    }
+    __device__ static __forceinline__ uint32_t scales(const Hdr &h) { return h.h.x; }
+    __device__ static __forceinline__ float value(int p0, int p1, const float (&f)[2], float d, float dmin) {
+        return __builtin_fmaf(-dmin, f[0], d * (float)((p0 << 3) + p1));
+    }
+};
+
+template <> struct KR<T_Q5_K> {
+    static constexpr int BYTES = BYTES_Q5_K, NCH = 11, NPL = 2, NF16 = 1;
+    typedef u32x4 chunk_t;
+    struct Hdr { u32x4 h, qh; };
+    __device__ static __forceinline__ Hdr hdr(const u32x4 *row, int hf) { return Hdr{row[0], row[1 + hf]}; }
+    static constexpr int KA(int q) { return 2 * q; }
+    static constexpr int KB(int q) { return 2 * q + 1; }
+    struct Raw { u32x4 q; };
+    template <int Q> __device__ static __forceinline__ Raw load(const u32x4 *row, int hf) { return Raw{row[3 + 2 * Q + hf]}; }
+    template <int Q> __device__ static __forceinline__ void expand(const Raw &r, const Hdr &h, int, u32x4 (&c)[2][2]) {
+        uint32_t sc, mn;
+        scale_min_pair(h.h, Q, sc, mn);
+        const uint32_t m0 = splat16(sc & 0xffu), m1 = splat16(sc >> 8), add = splat16(128u);
+        const u32x4 q = r.q;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            // bit 2*jp of qh[l] is the fifth bit of element 64*jp + l, bit 2*jp + 1 that of 64*jp + 32 + l
+            // (reference ggml-quants.c:1460-1478); bits 5 to 7 are masked below
+            const uint32_t t0 = Q < 2 ? h.qh[i] << (4 - 2 * Q) : h.qh[i] >> (2 * Q - 4), t1 = Q < 2 ? h.qh[i] << (3 - 2 * Q) : h.qh[i] >> (2 * Q - 3);
+            uint32_t hi, lo;
+            byte_digits(merge_bits(0x0f0f0f0fu, q[i], t0), 0x001f001fu, m0, add, hi, lo);
+            c[0][0][i] = hi; c[0][1][i] = lo;
+            byte_digits(merge_bits(0x0f0f0f0fu, q[i] >> 4, t1), 0x001f001fu, m1, add, hi, lo);
+            c[1][0][i] = hi; c[1][1][i] = lo;
+        }
+    }
+    __device__ static __forceinline__ u32x4 f16_cell(const Hdr &h, int, int half) {
+        uint32_t sc, mn;
+        scale_min_quad(h.h, half, sc, mn);
+        return bytes_to_f16_pairs(mn);
+    }
+    __device__ static __forceinline__ uint32_t scales(const Hdr &h) { return h.h.x; }
+    __device__ static __forceinline__ float value(int p0, int p1, const float (&f)[2], float d, float dmin) {
+        return __builtin_fmaf(-dmin, f[0], d * (float)((p0 << 8) + p1));
+    }
+};
+
+template <> struct KR<T_Q6_K> {
+    static constexpr int BYTES = BYTES_Q6_K, NCH = 14, NPL = 2, NF16 = 0;
+    typedef u32x4_a2 chunk_t;
+    // ql[128] | qh[64] | scales[16] | d: cells 0..7, 8..11, 12, and d in the last two bytes of cell 13.
+    // Half h of a super-block holds, for l = 0..31, the elements 128h + 32b + l of k-blocks b = 0..3 as low / high nibble of
+    // ql[64h + l] (b = 0 / 2) and of ql[64h + 32 + l] (b = 1 / 3), two more bits from qh[32h + l] >> 2b, scale
+    // scales[8h + 2b + l/16]  (reference ggml-quants.c:1695-1711).  Item Q = 2h + p: k-blocks p and p + 2 of half h.
+    struct Hdr { u32x4 sc; uint32_t d; };
+    __device__ static __forceinline__ Hdr hdr(const u32x4 *row, int) { return Hdr{row[12], row[13].w >> 16}; }
+    static constexpr int KA(int q) { return 4 * (q >> 1) + (q & 1); }
+    static constexpr int KB(int q) { return KA(q) + 2; }
+    struct Raw { u32x4 ql, qh; };
+    template <int Q> __device__ static __forceinline__ Raw load(const u32x4 *row, int hf) {
+        return Raw{row[4 * (Q >> 1) + 2 * (Q & 1) + hf], row[8 + 2 * (Q >> 1) + hf]};
+    }
+    template <int Q> __device__ static __forceinline__ void expand(const Raw &r, const Hdr &h, int hf, u32x4 (&c)[2][2]) {
+        constexpr int H = Q >> 1, p = Q & 1;
+        // scales[8h + 2p + hf] and scales[8h + 2p + 4 + hf]: byte 2p + hf of dwords 2h and 2h + 1
+        const int s0 = (int8_t)(h.sc[2 * H] >> (16 * p + 8 * hf)), s1 = (int8_t)(h.sc[2 * H + 1] >> (16 * p + 8 * hf));
+        const uint32_t sa = splat16((uint32_t)s0), ba = splat16((uint32_t)(128 - 32 * s0));
+        const uint32_t sb = splat16((uint32_t)s1), bb = splat16((uint32_t)(128 - 32 * s1));
+        const u32x4 ql = r.ql, qh = r.qh;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint32_t t0 = qh[i] << (4 - 2 * p), t1 = qh[i] >> (2 * p);               // bits 4, 5 of every byte: the upper two bits
+            const uint32_t q0 = merge_bits(0x0f0f0f0fu, ql[i], t0);                        // bits 6, 7 are masked below
+            const uint32_t q1 = merge_bits(0x0f0f0f0fu, ql[i] >> 4, t1);
+            uint32_t hi, lo;
+            byte_digits(q0, 0x003f003fu, sa, ba, hi, lo);
+            c[0][0][i] = hi; c[0][1][i] = lo;
+            byte_digits(q1, 0x003f003fu, sb, bb, hi, lo);
+            c[1][0][i] = hi; c[1][1][i] = lo;
+        }
+    }
+    __device__ static __forceinline__ u32x4 f16_cell(const Hdr &, int, int) { return u32x4{0u, 0u, 0u, 0u}; }
+    __device__ static __forceinline__ uint32_t scales(const Hdr &h) { return h.d; }
+    __device__ static __forceinline__ float value(int p0, int p1, const float (&)[2], float d, float) { return d * (float)((p0 << 8) + p1); }
+};
+
+template <> struct KR<T_Q3_K> {
+    static constexpr int BYTES = BYTES_Q3_K, NCH = 7, NPL = 1, NF16 = 0;
+    typedef u32x4_a2 chunk_t;
+    // hmask[32] | qs[64] | scales[12] | d: cells 0, 1 and 2..5; cell 6 is bytes 94..109 (scales from its third byte, d at its end).
+    // Element 128h + 32v + l: bits 2v of qs[32h + l], bit 4h + v of hmask[l], scale 8h + 2v + l/16.  Item Q = 2h + p: v = p and p + 2.
+    struct Hdr { u32x4 hm; uint32_t s[3], d; };
+    __device__ static __forceinline__ Hdr hdr(const u32x4 *row, int hf) {
+        const u32x4 t = row[6];
+        Hdr h;
+        h.hm = row[hf];
+        h.s[0] = shr16(t.y, t.x); h.s[1] = shr16(t.z, t.y); h.s[2] = shr16(t.w, t.z);
+        h.d = t.w >> 16;
+        return h;
+    }
+    static constexpr int KA(int q) { return 4 * (q >> 1) + (q & 1); }
+    static constexpr int KB(int q) { return KA(q) + 2; }
+    struct Raw { u32x4 q; };
+    template <int Q> __device__ static __forceinline__ Raw load(const u32x4 *row, int hf) { return Raw{row[2 + 2 * (Q >> 1) + hf]}; }
+    template <int Q> __device__ static __forceinline__ void expand(const Raw &r, const Hdr &h, int hf, u32x4 (&c)[2][1]) {
+        constexpr int H = Q >> 1, p = Q & 1;
+        // 6-bit scale 4w + i is byte i of word w (reference ggml-quants.c:1062-1071): words 2h and 2h + 1 hold k-blocks 0, 1 and 2, 3
+        const uint32_t hi2 = h.s[2] >> (4 * H);
+        const uint32_t wa = ((h.s[0] >> (4 * H)) & 0x0f0f0f0fu) | ((hi2 & 0x03030303u) << 4);
+        const uint32_t wb = ((h.s[1] >> (4 * H)) & 0x0f0f0f0fu) | (((hi2 >> 2) & 0x03030303u) << 4);
+        const int b = 16 * p + 8 * hf;
+        const int sc[2] = {(int)((wa >> b) & 0xffu) - 32, (int)((wb >> b) & 0xffu) - 32};
+        const u32x4 q = r.q;
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            const int v = p + 2 * e;
+            // byte = 128 + (4 - q)*sc in 0..252: the two bytes of a 16-bit lane never carry into each other, whatever the sign of
+            // the multiplier (arithmetic modulo 2^16); flipping bit 7 gives the signed byte
+            const uint32_t mul = splat16((uint32_t)(-sc[e])), add = splat16((uint32_t)((128 + 4 * sc[e]) * 0x101));
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint32_t hb = 4 * H + v < 2 ? h.hm[i] << (2 - 4 * H - v) : h.hm[i] >> (4 * H + v - 2);
+                const uint32_t w = merge_bits(0x03030303u, q[i] >> (2 * v), hb) & 0x07070707u;
+                c[e][0][i] = pk_mad16(w, mul, add) ^ 0x80808080u;
+            }
+        }
+    }
+    __device__ static __forceinline__ u32x4 f16_cell(const Hdr &, int, int) { return u32x4{0u, 0u, 0u, 0u}; }
+    __device__ static __forceinline__ uint32_t scales(const Hdr &h) { return h.d; }
+    __device__ static __forceinline__ float value(int p0, int, const float (&)[2], float d, float) { return d * (float)-p0; }
+};
+
+template <> struct KR<T_Q2_K> {
+    static constexpr int BYTES = BYTES_Q2_K, NCH = 6, NPL = 1, NF16 = 1;      // fp16 product: sum_j m_j * bsum_j over the 16 sub-blocks
+    typedef u32x4_a4 chunk_t;
+    // scales[16] (low nibble scale, high nibble min) | qs[64] | d | dmin: cells 0, 1..4, and d | dmin in the last dword of cell 5
+    struct Hdr { u32x4 sc; uint32_t dd; };
+    __device__ static __forceinline__ Hdr hdr(const u32x4 *row, int) { return Hdr{row[0], row[5].w}; }
+    static constexpr int KA(int q) { return 4 * (q >> 1) + (q & 1); }
+    static constexpr int KB(int q) { return KA(q) + 2; }
+    struct Raw { u32x4 q; };
+    template <int Q> __device__ static __forceinline__ Raw load(const u32x4 *row, int hf) { return Raw{row[1 + 2 * (Q >> 1) + hf]}; }
+    template <int Q> __device__ static __forceinline__ void expand(const Raw &r, const Hdr &h, int hf, u32x4 (&c)[2][1]) {
+        constexpr int H = Q >> 1, p = Q & 1;
+        const int b = 16 * p + 8 * hf;
+        const uint32_t s0 = (h.sc[2 * H] >> b) & 15u, s1 = (h.sc[2 * H + 1] >> b) & 15u;
+        const u32x4 q = r.q;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            c[0][0][i] = ((q[i] >> (2 * p)) & 0x03030303u) * s0;                          // byte products <= 45
+            c[1][0][i] = ((q[i] >> (2 * p + 4)) & 0x03030303u) * s1;
+        }
+    }
+    // mins of sub-blocks 8 half .. 8 half + 7
+    __device__ static __forceinline__ u32x4 f16_cell(const Hdr &h, int, int half) {
+        const uint32_t a = half ? h.sc[2] : h.sc[0], b = half ? h.sc[3] : h.sc[1];
+        u32x4 c;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint32_t w = ((i < 2 ? a : b) >> (16 * (i & 1) + 4)) & 0x0f0fu;
+            c[i] = f16_pair(w & 0xffu, w >> 8);
+        }
+        return c;
+    }
+    __device__ static __forceinline__ uint32_t scales(const Hdr &h) { return h.dd; }
+    __device__ static __forceinline__ float value(int p0, int, const float (&f)[2], float d, float dmin) {
+        return __builtin_fmaf(-dmin, f[0], d * (float)p0);
+    }
+};
+
+template <> struct KR<T_IQ4_XS> {
+    static constexpr int BYTES = BYTES_IQ4_XS, NCH = 9, NPL = 2, NF16 = 0;
+    typedef u32x4_a4 chunk_t;
+    // d | u16 scales_h | scales_l[4] | qs[128]: sub-block ib is qs[16 ib ..], low nibbles elements 0..15, high nibbles 16..31.
+    // Cells 0..7 are bytes 0..127, cell 8 bytes 120..135 (sub-block 7).  Item Q: sub-blocks 2Q and 2Q + 1.
+    struct Hdr { u32x2 h; };
+    __device__ static __forceinline__ Hdr hdr(const u32x4 *row, int) { return Hdr{*reinterpret_cast<const u32x2 *>(row)}; }
+    static constexpr int KA(int q) { return 2 * q; }
+    static constexpr int KB(int q) { return 2 * q + 1; }
+    // four code indices (one per byte) -> code point + 128 of kvalues_iq4nl (reference ggml-common.h), 1..241
+    __device__ static __forceinline__ uint32_t lookup4(uint32_t idx) {
+        constexpr uint32_t F = 0x80808080u, T0 = 0xbfad9881u ^ F, T1 = 0xf6eaddcfu ^ F, T2 = 0x26190d01u ^ F, T3 = 0x71594535u ^ F;
+        const uint32_t sel = idx & 0x07070707u;
+        const uint32_t lo = __builtin_amdgcn_perm(T1, T0, sel), hi = __builtin_amdgcn_perm(T3, T2, sel);
+        const uint32_t m = ((idx >> 3) & 0x01010101u) * 0xffu;
+        return (lo & ~m) | (hi & m);
+    }
+    struct Raw { u32x2 q[4]; };
+    template <int Q> __device__ static __forceinline__ Raw load(const u32x4 *row, int) {
+        Raw r;
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            const u32x2 *qp = reinterpret_cast<const u32x2 *>(row) + (2 * Q + e < 7 ? 1 + 2 * (2 * Q + e) : 16);
+            r.q[2 * e] = qp[0];
+            r.q[2 * e + 1] = qp[1];
+        }
+        return r;
+    }
+    template <int Q> __device__ static __forceinline__ void expand(const Raw &r, const Hdr &h, int hf, u32x4 (&c)[2][2]) {
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            const int ib = 2 * Q + e;
+            const uint32_t nib = (h.h.y >> (4 * ib)) & 15u, top = (h.h.x >> (16 + 2 * ib)) & 3u;
+            const int ls = (int)(nib | (top << 4)) - 32;
+            const uint32_t mul = splat16((uint32_t)ls), add = splat16((uint32_t)(128 - 128 * ls));
+            const uint32_t w[4] = {r.q[2 * e].x, r.q[2 * e].y, r.q[2 * e + 1].x, r.q[2 * e + 1].y};
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                uint32_t hi, lo;
+                byte_digits(lookup4((w[i] >> (4 * hf)) & 0x0f0f0f0fu), 0x00ff00ffu, mul, add, hi, lo);
+                c[e][0][i] = hi; c[e][1][i] = lo;
+            }
+        }
+    }
+    __device__ static __forceinline__ u32x4 f16_cell(const Hdr &, int, int) { return u32x4{0u, 0u, 0u, 0u}; }
+    __device__ static __forceinline__ uint32_t scales(const Hdr &h) { return h.h.x & 0xffffu; }
+    __device__ static __forceinline__ float value(int p0, int p1, const float (&)[2], float d, float) { return d * (float)((p0 << 8) + p1); }
+};
+
+constexpr int KR_ROWS = 128;                  // weight rows per workgroup: four waves of 32
+
+template <int WT, int TN, int KS>
+struct KrCfg {
+    using T = KR<WT>;
+    static constexpr int NW = 4 * KS, NT = NW * 64;
+    static constexpr int BN = 32 * TN;                                    // tokens per workgroup
+    static constexpr int NLD = (32 * T::NCH + 63) / 64;                   // chunk loads of a lane per super-block
+    static constexpr int B_PER_W = BN / 16;                               // direct loads of a wave per super-block (four tokens each)
+    static constexpr size_t RAW = (size_t)NLD * 1024;                     // per wave: its 32 rows of one super-block, whole loads
+    static constexpr size_t OFF_B = RAW * NW;                             // [buffer][k group] activations, [token][16 cells] swizzled
+    static constexpr size_t B_BYTES = (size_t)BN * 256;
+    // What the fold reads has four buffers: a wave folds super-block j behind the barrier that follows its products, while a faster
+    // one already writes the values of super-block j + 2 in front of the next barrier.
+    static constexpr size_t OFF_FB = OFF_B + 2 * KS * B_BYTES;            // [j % 4][k group] fp16 cells [k-half][token]: the 16 bsums
+    static constexpr size_t FB_BYTES = T::NF16 > 0 ? (size_t)BN * 32 : 0;
+    static constexpr size_t OFF_SX = OFF_FB + 4 * KS * FB_BYTES;          // [j % 4][k group] f32 [token]: activation scale
+    static constexpr size_t OFF_ROW = OFF_SX + 4 * KS * (size_t)BN * 4;   // i32 [token]: output row (expert groups)
+    static constexpr size_t TOTAL0 = OFF_ROW + (size_t)BN * 4;
+    // the other k groups' partial outputs take the place of the operands at the end
+    static_assert((size_t)(KS - 1) * 4 * TN * 16 * 256 <= OFF_SX, "partial outputs lie in front of the output rows");
+    static constexpr size_t TOTAL = TOTAL0;
+};
+
+__device__ __forceinline__ void kr_load16_into_lds(const uint8_t *base, uint32_t off, uint32_t lds_addr) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_addr) : "memory");
+}
+__device__ __forceinline__ void kr_load16_into_lds(const uint8_t *src, uint32_t lds_addr) {
+    // M0 = LDS byte address of the wave's 1 KB destination; lane i's 16 bytes land at M0 + 16 i.  Inline assembly so that
+    // the compiler does not make every later LDS read wait for it; the kernel waits by hand in front of the barrier.
+    // Nothing else in the kernel may use M0 (no dynamic register indexing).
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_addr) : "memory");
+}
+
+template <int WT, int TN, int KS, int OCC, bool GATHER>
+__global__ __launch_bounds__(4 * KS * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
+void gemm_kr_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64_t N, const uint8_t *__restrict__ ws,
+                    size_t ws_stride, int64_t M, float *__restrict__ y, int64_t ldy, TileMap map, RowGather rg, int slice_sb) {
+    using T = KR<WT>;
+    using C = KrCfg<WT, TN, KS>;
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int grp = wave >> 2, wr = wave & 3;                            // k group, row tile
+    const int gt = tid & 255;                                            // thread of the k group
+    int sb0 = 0, nsb = (int)(K / QK_K);
+    if (!GATHER && slice_sb > 0) {
+        sb0 = (int)blockIdx.y * slice_sb;
+        nsb = min(slice_sb, nsb - sb0);
+        y += (size_t)blockIdx.y * (size_t)M * (size_t)ldy;
+    }
+    TileCoord tc;
+    int slot = 0;
+    if constexpr (GATHER) {
+        if (!gather_tile(rg, map, slot, tc.row_tile)) return;
+        tc.tok_tile = 0;
+    } else {
+        tc = xcd_tile(blockIdx.x, map);
+        if (tc.row_tile >= map.row_tiles || tc.tok_tile >= map.tok_tiles) return;        // padding of the tile map
+    }
+    size_t w_offset;
+    const GatherView gv = resolve_gather<GATHER>(rg, slot, w_offset, M);
+    W += w_offset;
+    const int64_t row_base = (int64_t)tc.row_tile * KR_ROWS + wr * 32;
+    const int64_t tok_base = (int64_t)(GATHER ? gv.tok_tile : tc.tok_tile) * C::BN;
+    if (tok_base >= M) return;
+    const int tokens = (int)min((int64_t)C::BN, M - tok_base);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
+    const size_t off_d = q8_K_off_d(K), off_bs = q8_K_off_bsums(K);
+    const int half = lane >> 5, l32 = lane & 31;
+
+    // ---- weights: the wave's own 32 rows, chunk by chunk in memory order, through registers into its own stretch of LDS ----
+    const int64_t row_c = min(row_base, N - 1);
+    const uint8_t *wbase = W + (size_t)row_c * nb01 + (size_t)sb0 * T::BYTES;
+    uint32_t woff[C::NLD];
+#pragma unroll
+    for (int t = 0; t < C::NLD; t++) {
+        const int i = min(lane + 64 * t, 32 * T::NCH - 1), r = i / T::NCH, c = i % T::NCH;
+        woff[t] = (uint32_t)(min(row_base + r, N - 1) - row_c) * (uint32_t)nb01 + (uint32_t)(c == T::NCH - 1 ? T::BYTES - 16 : 16 * c);
+    }
+    u32x4 *const raw_lds = reinterpret_cast<u32x4 *>(lds + C::RAW * wave);
+    u32x4 raw[C::NLD];
+    auto fetch_w = [&](int sb_wanted) {
+        const uint8_t *p = wbase + (size_t)min(sb_wanted, nsb - 1) * T::BYTES;
+#pragma unroll
+        for (int t = 0; t < C::NLD; t++) raw[t] = *reinterpret_cast<const typename T::chunk_t *>(p + woff[t]);
+    };
+    auto commit_w = [&]() {
+#pragma unroll
+        for (int t = 0; t < C::NLD; t++) raw_lds[lane + 64 * t] = raw[t];
+    };
+
+    // ---- activations: the k group's BN tokens of its super-block straight into LDS, 256-byte rows of 16 swizzled cells ----
+    // (a plain tile's tokens lie side by side: one scalar base and 32-bit offsets)
+    const uint8_t *const act0 = ws + (size_t)(GATHER ? 0 : tok_base) * ws_stride + (size_t)sb0 * QK_K;
+    const uint8_t *bsrc[GATHER ? C::B_PER_W : 1];
+    uint32_t boff[GATHER ? 1 : C::B_PER_W];
+#pragma unroll
+    for (int j = 0; j < C::B_PER_W; j++) {
+        const int t = (wr * C::B_PER_W + j) * 4 + (lane >> 4);
+        const uint32_t cell = 16u * (uint32_t)((lane & 15) ^ (t & 15));
+        if constexpr (GATHER) bsrc[j] = act0 + (size_t)gv.act_row(min(tok_base + t, M - 1)) * ws_stride + cell;
+        else boff[j] = (uint32_t)min(t, tokens - 1) * (uint32_t)ws_stride + cell;
+    }
+    auto issue_x = [&](int sb_wanted, int buf) {
+        const size_t o = (size_t)min(sb_wanted, nsb - 1) * QK_K;
+        const uint32_t dst = lds0 + (uint32_t)(C::OFF_B + (size_t)(buf * KS + grp) * C::B_BYTES) + (uint32_t)(wr * C::B_PER_W) * 1024u;
+#pragma unroll
+        for (int j = 0; j < C::B_PER_W; j++) {
+            const uint32_t d = __builtin_amdgcn_readfirstlane(dst + (uint32_t)j * 1024u);
+            if constexpr (GATHER) kr_load16_into_lds(bsrc[j] + o, d);
+            else kr_load16_into_lds(act0 + o, boff[j], d);
+        }
+    };
+    // activation scale: thread t < BN of the k group for token t; block sums: thread t < 2*BN for token t/2, k-half t&1
+    const uint8_t *ssrc = ws + (size_t)gv.act_row(min(tok_base + min(gt, C::BN - 1), M - 1)) * ws_stride + off_d + (size_t)sb0 * 4;
+    const uint8_t *bssrc = ws + (size_t)gv.act_row(min(tok_base + min(gt >> 1, C::BN - 1), M - 1)) * ws_stride + off_bs + 16 * (gt & 1) + (size_t)sb0 * 32;
+    float xs;
+    u32x4 bs;
+    auto fetch_s = [&](int sb_wanted) {
+        const int sb = min(sb_wanted, nsb - 1);
+        xs = reinterpret_cast<const float *>(ssrc)[sb];
+        if constexpr (T::NF16 > 0) bs = *reinterpret_cast<const u32x4 *>(bssrc + (size_t)sb * 32);
+    };
+    auto commit_s = [&](int it) {
+        const int q = (it & 3) * KS + grp;
+        if (gt < C::BN) reinterpret_cast<float *>(lds + C::OFF_SX)[q * C::BN + gt] = xs;
+        if constexpr (T::NF16 > 0)
+            if (gt < 2 * C::BN)
+                *reinterpret_cast<u32x4 *>(lds + C::OFF_FB + (size_t)q * C::FB_BYTES + (size_t)((gt & 1) * C::BN + (gt >> 1)) * 16) = i16x8_to_f16(bs);
+    };
+
+    float out[TN][16];
+#pragma unroll
+    for (int c = 0; c < TN; c++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) out[c][v] = 0.f;
+
+    // This wave's 32 rows against the first 32*NTL of the tile's tokens.  Activations are the MFMA's first operand: register v of tile c
+    // is token 32 c + 8 (v / 4) + 4 half + v % 4, the lane's l32 its row.
+    //
+    // Super-block it * KS + grp in iteration it, in four steps of two k-blocks.  Step Q multiplies what the step before it read and
+    // expanded, reads the operands of step Q + 1 and expands its weights between its own MFMAs.  The weights of the next iteration
+    // travel in registers and take the place of the current ones in LDS in step 3, when those have all been read; the next activations
+    // go straight into the other buffer.  Both were requested an iteration before the one barrier that makes them visible; behind it
+    // the fold runs together with the reads and the expansion of the next super-block's step 0.
+    constexpr int WAIT0 = 0x0F70;                                          // s_waitcnt vmcnt(0)
+    const int nit = (nsb + KS - 1) / KS;
+    const u32x4 *const row_lds = raw_lds + l32 * T::NCH;
+    const uint32_t b_lane = (uint32_t)l32 * 256u + 16u * (uint32_t)(half ^ (l32 & 15));
+    auto walk = [&](auto ntl_tag) {
+        constexpr int NTL = decltype(ntl_tag)::value;
+        typename T::Hdr h;
+        typename T::Raw r1;
+        u32x4 cc[2][T::NPL], cn[2][T::NPL], bc[2][NTL], bn[2][NTL];
+        i32x16 P[T::NPL][NTL];
+        auto load_b = [&](u32x4 (&b)[2][NTL], int buf, int ka, int kb) {
+            const uint8_t *p = lds + (C::OFF_B + (size_t)(buf * KS + grp) * C::B_BYTES);
+#pragma unroll
+            for (int e = 0; e < 2; e++)
+#pragma unroll
+                for (int c = 0; c < NTL; c++) b[e][c] = *reinterpret_cast<const u32x4 *>(p + (b_lane ^ (uint32_t)(32 * (e ? kb : ka))) + c * 8192);
+        };
+        auto multiply = [&](auto first_tag) {
+            constexpr bool first = decltype(first_tag)::value;
+            const i32x16 zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+            for (int e = 0; e < 2; e++)
+#pragma unroll
+                for (int c = 0; c < NTL; c++)
+#pragma unroll
+                    for (int pl = 0; pl < T::NPL; pl++)
+                        P[pl][c] = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, bc[e][c]), __builtin_bit_cast(i32x4, cc[e][pl]),
+                                                                         (first && e == 0) ? zero : P[pl][c], 0, 0, 0);
+        };
+        auto step = [&](auto q_tag, int buf) {
+            constexpr int Q = decltype(q_tag)::value;
+            typename T::Raw r2;
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (Q < 3) load_b(bn, buf, T::KA(Q + 1), T::KB(Q + 1));
+            if constexpr (Q < 2) r2 = T::template load<Q + 2>(row_lds, half);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (Q < 3) T::template expand<Q + 1>(r1, h, half, cn);
+            multiply(std::integral_constant<bool, Q == 0>{});
+            if constexpr (Q < 3) {
+                constexpr int MF = 2 * NTL * T::NPL;
+#pragma unroll
+                for (int i = 0; i < MF; i++) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, 96 / MF, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int e = 0; e < 2; e++) {
+#pragma unroll
+                    for (int pl = 0; pl < T::NPL; pl++) cc[e][pl] = cn[e][pl];
+#pragma unroll
+                    for (int c = 0; c < NTL; c++) bc[e][c] = bn[e][c];
+                }
+            }
+            if constexpr (Q < 2) r1 = r2;
+        };
+        // reads and expands step 0 of the super-block in `buf`
+        auto first_operands = [&](int buf) {
+            h = T::hdr(row_lds, half);
+            const typename T::Raw r0 = T::template load<0>(row_lds, half);
+            r1 = T::template load<1>(row_lds, half);
+            load_b(bc, buf, T::KA(0), T::KB(0));
+            T::template expand<0>(r0, h, half, cc);
+        };
+
+        issue_x(grp, 0);
+        fetch_w(grp);
+        fetch_s(grp);
+        if constexpr (GATHER)
+            if (tid < C::BN) reinterpret_cast<int32_t *>(lds + C::OFF_ROW)[tid] = gv.list[tok_base + min(tid, tokens - 1)];
+        commit_w();
+        commit_s(0);
+        __builtin_amdgcn_s_waitcnt(WAIT0);
+        __syncthreads();
+        if (nit > 1) {
+            fetch_w(grp + KS);
+            fetch_s(grp + KS);
+        }
+        first_operands(0);
+        for (int it = 0; it < nit; it++) {
+            const int buf = it & 1, sb = it * KS + grp, q4 = (it & 3) * KS + grp;
+            if (it + 1 < nit) issue_x(sb + KS, buf ^ 1);
+            step(std::integral_constant<int, 0>{}, buf);
+            step(std::integral_constant<int, 1>{}, buf);
+            step(std::integral_constant<int, 2>{}, buf);
+            step(std::integral_constant<int, 3>{}, buf);
+            float d = h2f(T::scales(h)), dmin = h2f(T::scales(h) >> 16);
+            asm volatile("" : "+v"(d), "+v"(dmin));                        // widened once: as halves they would make every multiply-add a half-rate mixed one
+            f16x8 fa[T::NF16 > 0 ? T::NF16 : 1];
+#pragma unroll
+            for (int f = 0; f < T::NF16; f++) fa[f] = __builtin_bit_cast(f16x8, T::f16_cell(h, f, half));
+            if (it + 1 < nit) {
+                commit_w();
+                commit_s(it + 1);
+                __builtin_amdgcn_s_waitcnt(WAIT0);
+                __syncthreads();
+                if (it + 2 < nit) {
+                    fetch_w(sb + 2 * KS);
+                    fetch_s(sb + 2 * KS);
+                }
+                first_operands(buf ^ 1);
+            }
+            // fold: out += dx * (d * float(sumi) - dmin * summ); the last iteration may lie past a k group's end
+#pragma unroll
+            for (int c = 0; c < NTL; c++) {
+                f32x16 F[T::NF16 > 0 ? T::NF16 : 1];
+                if constexpr (T::NF16 > 0) {
+                    const f16x8 fb = *reinterpret_cast<const f16x8 *>(lds + C::OFF_FB + (size_t)q4 * C::FB_BYTES + (size_t)(half * C::BN + c * 32 + l32) * 16);
+                    const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int f = 0; f < T::NF16; f++) F[f] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb, fa[f], zero, 0, 0, 0);
+                }
+                const float *sx = reinterpret_cast<const float *>(lds + C::OFF_SX) + q4 * C::BN + c * 32 + 4 * half;
+                float dxv[16];
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const float4 dx = *reinterpret_cast<const float4 *>(sx + 8 * g);
+                    dxv[4 * g] = dx.x; dxv[4 * g + 1] = dx.y; dxv[4 * g + 2] = dx.z; dxv[4 * g + 3] = dx.w;
+                }
+                if (KS == 1 || sb < nsb) {
+#pragma unroll
+                for (int v = 0; v < 16; v++) {
+                    float f[2] = {0.f, 0.f};
+#pragma unroll
+                    for (int j = 0; j < T::NF16; j++) f[j] = F[j][v];
+                    out[c][v] = __builtin_fmaf(T::value(P[0][c][v], P[T::NPL - 1][c][v], f, d, dmin), dxv[v], out[c][v]);
+                }
+                }
+            }
+        }
+        __syncthreads();
+    };
+    if (TN > 1 && tokens <= 32) walk(std::integral_constant<int, 1>{});
+    else walk(std::integral_constant<int, TN>{});
+
+    // the k groups' partial sums meet in LDS and are added in order
+    if constexpr (KS > 1) {
+        float *part = reinterpret_cast<float *>(lds);
+        if (grp > 0) {
+#pragma unroll
+            for (int c = 0; c < TN; c++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) part[(((grp - 1) * 4 + wr) * TN * 16 + c * 16 + v) * 64 + lane] = out[c][v];
+        }
+        __syncthreads();
+        if (grp > 0) return;
+#pragma unroll
+        for (int g = 1; g < KS; g++)
+#pragma unroll
+            for (int c = 0; c < TN; c++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) out[c][v] += part[(((g - 1) * 4 + wr) * TN * 16 + c * 16 + v) * 64 + lane];
+    }
+    const int64_t row = row_base + l32;
+    if (row >= N) return;
+#pragma unroll
+    for (int c = 0; c < TN; c++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const int t0 = c * 32 + 8 * g + 4 * half;
+            int32_t orow[4];
+            if constexpr (GATHER) *reinterpret_cast<u32x4 *>(orow) = *reinterpret_cast<const u32x4 *>(lds + C::OFF_ROW + t0 * 4);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (t0 + e < tokens) y[(size_t)(GATHER ? orow[e] : tok_base + t0 + e) * ldy + row] = out[c][4 * g + e];
+        }
+}
+
+template <int WT, int TN, int KS, int OCC, bool GATHER>
+hipError_t launch_kr(const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, int64_t M, float *y, int64_t ldy,
+                     const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t slots, int slices, float *part) {
+    using C = KrCfg<WT, TN, KS>;
+    if ((int64_t)C::TOTAL > lim.max_lds_per_block) return hipErrorInvalidValue;
+    auto kfn = gemm_kr_kernel<WT, TN, KS, OCC, GATHER>;
+    static LdsGrant grant;                                               // one per kernel instantiation
+    if (hipError_t e = grant_dynamic_lds(kfn, C::TOTAL, lim, grant); e != hipSuccess) return e;
+    const int per_cu = (int)(160 * 1024 / C::TOTAL) > 0 ? (int)(160 * 1024 / C::TOTAL) : 1;
+    if constexpr (GATHER) {
+        TileMap map = make_tile_map(ceil_div(N, KR_ROWS), 1, 32 * per_cu);
+        const dim3 grid = gather_grid(map, slots, C::NT);
+        hipLaunchKernelGGL(kfn, grid, dim3(C::NT), C::TOTAL, st, (const uint8_t *)W, nb01, K, N, (const uint8_t *)ws, ws_stride, M, y, ldy, map, rg, 0);
+        return hipGetLastError();
+    } else {
+        const TileMap map = make_tile_map(ceil_div(N, KR_ROWS), ceil_div(M, C::BN), 32 * per_cu);
+        const int slice_sb = slices > 1 ? (int)ceil_div(K / QK_K, (int64_t)slices) : 0;
+        hipLaunchKernelGGL(kfn, dim3(map.grid, (unsigned)slices), dim3(C::NT), C::TOTAL, st, (const uint8_t *)W, nb01, K, N,
+                           (const uint8_t *)ws, ws_stride, M, slices > 1 ? part : y, slices > 1 ? N : ldy, map, rg, slice_sb);
+        if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+        return slices > 1 ? launch_sum_slices(part, slices, M, N, y, ldy, st) : hipSuccess;
+    }
+}
+
+template <int WT>
+hipError_t launch_kr_groups(int groups, const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, int64_t M, float *y, int64_t ldy,
+                         const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t slots, int slices, float *part) {
+    if (rg.perm) {
+        if (groups == 2) return launch_kr<WT, 2, 2, 2, true>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, 1, nullptr);
+        return launch_kr<WT, 2, 1, 2, true>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, 1, nullptr);
+    }
+    if (groups == 2) return launch_kr<WT, 2, 2, 2, false>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, slices, part);
+    return launch_kr<WT, 2, 1, 2, false>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, slices, part);
+}
+
+}  // namespace
+
+hipError_t launch_gemm_kr(int groups, int wtype, const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, int64_t M,
+                          float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t slots, int slices, float *part) {
+    switch (wtype) {
+        case T_Q4_K: return launch_kr_groups<T_Q4_K>(groups, W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, slices, part);
+        case T_Q5_K: return launch_kr_groups<T_Q5_K>(groups, W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, slices, part);
+        case T_Q6_K: return launch_kr_groups<T_Q6_K>(groups, W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, slices, part);
+        case T_Q3_K: return launch_kr_groups<T_Q3_K>(groups, W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, slices, part);
+        case T_Q2_K: return launch_kr_groups<T_Q2_K>(groups, W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, slices, part);
+        case T_IQ4_XS: return launch_kr_groups<T_IQ4_XS>(groups, W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, slices, part);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace chip

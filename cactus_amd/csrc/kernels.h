@@ -114,12 +114,12 @@ struct GatherView {                // resolved once per workgroup
 // Sets the token count M and the byte offset of the weight matrix to the expert's and returns its view.  GATHER is a
 // template argument of the kernels so that the plain MUL_MAT instantiations carry none of this.
 template <bool GATHER>
-__device__ __forceinline__ GatherView resolve_gather(const RowGather &rg, size_t &w_offset, int64_t &M) {
+__device__ __forceinline__ GatherView resolve_gather(const RowGather &rg, int slot, size_t &w_offset, int64_t &M) {
     GatherView v{nullptr, rg.n_used, rg.ne11, 0};
     w_offset = 0;
     if constexpr (GATHER) {
-        if ((int)blockIdx.y >= rg.tiles[0]) { v.tok_tile = -1; return v; }
-        const int32_t d = rg.tiles[1 + blockIdx.y];
+        if (slot >= rg.tiles[0]) { v.tok_tile = -1; return v; }
+        const int32_t d = rg.tiles[1 + slot];
         const int e = d & ((1 << MOE_EXPERT_BITS) - 1);
         const int32_t off = rg.offsets[e];
         M = rg.offsets[e + 1] - off;
@@ -128,6 +128,27 @@ __device__ __forceinline__ GatherView resolve_gather(const RowGather &rg, size_t
         w_offset = (size_t)e * rg.nb02;
     }
     return v;
+}
+template <bool GATHER>
+__device__ __forceinline__ GatherView resolve_gather(const RowGather &rg, size_t &w_offset, int64_t &M) {
+    return resolve_gather<GATHER>(rg, (int)blockIdx.y, w_offset, M);
+}
+// Expert groups over a grid of one dimension (cut into two only where HIP's limit asks for it): the (entry, row tile) pairs of the
+// list, an entry's row tiles side by side, are cut into 8 equal stretches, one per XCD.  The length of the list is known on the
+// device only, so the grid provides for `slots` entries and the workgroups past the end exit at once.
+__device__ __forceinline__ bool gather_tile(const RowGather &rg, const TileMap &m, int &slot, int &row_tile) {
+    const unsigned wg = blockIdx.x + gridDim.x * blockIdx.y;
+    const unsigned total = (unsigned)rg.tiles[0] * (unsigned)m.row_tiles, per = (total + XCDS - 1) / XCDS;
+    const unsigned idx = (wg % XCDS) * per + wg / XCDS;
+    if (wg / XCDS >= per || idx >= total) return false;
+    slot = (int)(idx / (unsigned)m.row_tiles);
+    row_tile = (int)(idx % (unsigned)m.row_tiles);
+    return true;
+}
+inline dim3 gather_grid(const TileMap &m, int64_t slots, int threads) {
+    const int64_t wgs = ceil_div(slots * m.row_tiles, XCDS), x_max = ((int64_t)1 << 31) / threads / XCDS;
+    const int64_t rows = ceil_div(wgs, x_max);
+    return dim3((unsigned)(ceil_div(wgs, rows) * XCDS), (unsigned)rows);
 }
 
 // quantize.hip
@@ -255,6 +276,10 @@ bool       gemm_kq_supported(int wtype, int64_t K, int64_t N, int64_t n, bool ca
 hipError_t launch_gemm_kq(int wtype, const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride,
                           int64_t n, float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st, const RowGather *rg = nullptr,
                           int64_t n_as = 1, SplitK split = SplitK{nullptr, 0});
+// gemm_kquant_rows.hip: the same product by waves that expand their own rows; groups: 1 or 2 k groups a workgroup, slices: parts of K
+hipError_t launch_gemm_kr(int groups, int wtype, const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride,
+                          int64_t n, float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t slots,
+                          int slices, float *part);
 // In the three GEMM launchers: with rg, n_as is the number of token-tile slots the grid provides in y (an upper bound
 // of the tile list's length) and n is ignored; gemm_*_moe_tile_tokens gives the tile height the list must be built for.
 

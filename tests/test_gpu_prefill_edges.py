@@ -76,6 +76,31 @@ def test_low_bit_kquant_gemm(dev, orc, wt, K, N, n):
     check(y[np.ix_(toks, rows)], ref, "low-bit k-quant gemm")
 
 
+# The GEMM whose waves expand their own rows, (K, N, n): two workgroups a CU, ragged rows and tokens; two k groups over an odd number
+# of super-blocks; uneven slices and a last tile of one token; two k groups in two slices of different length
+@pytest.mark.parametrize("wt", (O.Q4_K, O.Q5_K, O.Q6_K) + LOW_BIT, ids=lambda t: O.TYPE_NAMES[t])
+@pytest.mark.parametrize("K,N,n", [(512, 4200, 1100), (1280, 4100, 260), (2816, 131, 33), (8448, 4100, 130)])
+def test_kquant_row_gemm(dev, orc, wt, K, N, n):
+    rng = np.random.default_rng(K + N + wt)
+    w = rng.integers(0, 256, (N, K // 256, O.BLOCK_BYTES[wt]), dtype=np.uint8)
+    for r, fill in enumerate((0xFF, 0x00, 0x80, 0x7F)):
+        w[r] = fill
+    half = np.array([1.0], np.float16).view(np.uint8)
+    for at in {O.Q4_K: (0, 2), O.Q5_K: (0, 2), O.Q6_K: (208,), O.Q3_K: (108,), O.Q2_K: (80, 82), O.IQ4_XS: (0,)}[wt]:
+        w[..., at:at + 2] = half
+    w = w.reshape(N, -1)
+    x = common.activations_f32(K + n, n, K)
+    x[3] = 0
+    x[4] = 127.0
+    x[5] = -127.0
+    y = dev.mul_mat(wt, w, x)
+    rows = np.unique(np.concatenate([[0, 1, 2, 3, N - 1], rng.choice(N, min(N, 150), replace=False)]))
+    toks = np.unique(np.concatenate([[0, 3, 4, 5, n - 1], rng.choice(n, min(n, 48), replace=False)]))
+    ref = orc.mul_mat(wt, w[rows], x[toks], nthreads=8, want=("sum_abs",))
+    check(y[np.ix_(toks, rows)], ref, "k-quant row gemm")
+    assert np.isfinite(y).all()
+
+
 @pytest.mark.parametrize("wt", LOW_BIT, ids=lambda t: O.TYPE_NAMES[t])
 def test_low_bit_kquant_integer_sums_bit_exact(dev, orc, wt):
     """d = dmin = 1 and activation scale 1: the output of one super-block is the integer sumi - summ itself (below 2^24)."""
