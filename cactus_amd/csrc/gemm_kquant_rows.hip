@@ -29,26 +29,15 @@
 #include "dev_common.h"
 #include "act_layout.h"
 #include "kernels.h"
+#include "kquant_dev.h"
 #include <type_traits>
 
 namespace chip {
 
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-typedef int i32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
 namespace {
-
-// two independent 16-bit products / multiply-adds per dword (v_pk_mul_lo_u16, v_pk_mad_u16)
-__device__ __forceinline__ uint32_t pk_mul16(uint32_t a, uint32_t b) {
-    return __builtin_bit_cast(uint32_t, (u16x2)(__builtin_bit_cast(u16x2, a) * __builtin_bit_cast(u16x2, b)));
-}
-__device__ __forceinline__ uint32_t pk_mad16(uint32_t a, uint32_t b, uint32_t c) {
-    return __builtin_bit_cast(uint32_t, (u16x2)(__builtin_bit_cast(u16x2, a) * __builtin_bit_cast(u16x2, b) + __builtin_bit_cast(u16x2, c)));
-}
-__device__ __forceinline__ uint32_t splat16(uint32_t v) { return (v & 0xffffu) | (v << 16); }
 
 // 6-bit scales and mins of sub-blocks 2jp and 2jp+1 (low byte, next byte) from the 12 packed bytes that follow
 // d and dmin (reference ggml-quants.c:625-632)
@@ -87,16 +76,6 @@ __device__ __forceinline__ u32x4 i16x8_to_f16(const u32x4 &v) {
     }
     return c;
 }
-// (a & m) | (b & ~m) as one full-rate instruction
-__device__ __forceinline__ uint32_t merge_bits(uint32_t m, uint32_t a, uint32_t b) { return __builtin_amdgcn_bitop3_b32(a, b, m, 0xe4); }
-// four 6- to 8-bit values (bytes of v, masked by m) times a signed scale: p = v * sc + bias - 128 = 256 * hi + lo with both
-// digits signed bytes.  mul = the scale, add = 128 plus the product's own bias, both in two 16-bit halves.
-__device__ __forceinline__ void byte_digits(uint32_t v, uint32_t m, uint32_t mul, uint32_t add, uint32_t &hi, uint32_t &lo) {
-    const uint32_t ue = pk_mad16(v & m, mul, add), uo = pk_mad16((v >> 8) & m, mul, add);
-    hi = __builtin_amdgcn_perm(uo, ue, 0x07030501u);
-    lo = __builtin_amdgcn_perm(uo, ue, 0x06020400u) ^ 0x80808080u;
-}
-
 // Per weight type.  A super-block is fetched as NCH 16-byte chunks (the last one ends with the super-block, so it may overlap the
 // one before) and kept in LDS as STRIDE cells of a row, STRIDE odd so that 16 rows' cells of one index fall into different banks.
 // Lane (row, hf) reads its share back: hdr() what all items need, load<Q>() the 16-value k-half hf of k-blocks KA(Q) and KB(Q), which
@@ -685,15 +664,14 @@ hipError_t launch_kr(const void *W, size_t nb01, int64_t K, int64_t N, const voi
 template <int WT>
 hipError_t launch_kr_groups(int groups, const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, int64_t M, float *y, int64_t ldy,
                          const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t slots, int slices, float *part) {
-    if (rg.perm) {
-        if (groups == 2) return launch_kr<WT, 2, 2, 2, true>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, 1, nullptr);
-        return launch_kr<WT, 2, 1, 2, true>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, 1, nullptr);
-    }
+    if (rg.perm) return launch_kr<WT, 2, 1, 2, true>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, 1, nullptr);   // expert groups
     if (groups == 2) return launch_kr<WT, 2, 2, 2, false>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, slices, part);
     return launch_kr<WT, 2, 1, 2, false>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, slices, part);
 }
 
 }  // namespace
+
+int gemm_kr_tile_tokens() { return KrCfg<T_Q4_K, 2, 1>::BN; }
 
 hipError_t launch_gemm_kr(int groups, int wtype, const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, int64_t M,
                           float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t slots, int slices, float *part) {

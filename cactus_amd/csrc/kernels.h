@@ -280,6 +280,7 @@ hipError_t launch_gemm_kq(int wtype, const void *W, size_t nb01, int64_t K, int6
 hipError_t launch_gemm_kr(int groups, int wtype, const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride,
                           int64_t n, float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t slots,
                           int slices, float *part);
+int        gemm_kr_tile_tokens();
 // In the three GEMM launchers: with rg, n_as is the number of token-tile slots the grid provides in y (an upper bound
 // of the tile list's length) and n is ignored; gemm_*_moe_tile_tokens gives the tile height the list must be built for.
 
