@@ -227,11 +227,18 @@ void gemm_blk32_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, in
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = wave / WC, wc = wave % WC;
     const int half = lane >> 5, l32 = lane & 31;
-    const TileCoord tc = xcd_tile(blockIdx.x, map);
-    if (tc.row_tile >= map.row_tiles || tc.tok_tile >= map.tok_tiles) return;
+    TileCoord tc;
+    int slot = 0;
+    if constexpr (GATHER) {
+        if (!gather_tile(rg, map, slot, tc.row_tile)) return;
+        tc.tok_tile = 0;
+    } else {
+        tc = xcd_tile(blockIdx.x, map);
+        if (tc.row_tile >= map.row_tiles || tc.tok_tile >= map.tok_tiles) return;
+    }
     const int64_t row_base = (int64_t)tc.row_tile * C::BM;
     size_t w_offset;
-    const GatherView gv = resolve_gather<GATHER>(rg, w_offset, M);
+    const GatherView gv = resolve_gather<GATHER>(rg, slot, w_offset, M);
     W += w_offset;
     if (gv.tok_tile < 0) return;
     const int64_t tok_base = (int64_t)(GATHER ? gv.tok_tile : tc.tok_tile) * C::BN;
@@ -637,7 +644,8 @@ static hipError_t launch_direct(const void *W, size_t nb01, int64_t K, int64_t N
         if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
         return launch_sum_slices(part, slices, M, N, y, ldy, st);
     }
-    hipLaunchKernelGGL(kfn, dim3(map.grid, (unsigned)n_as), dim3(C::NT), lds_bytes, st, (const uint8_t *)W, nb01, K, N,
+    const dim3 grid = GATHER ? gather_grid(map, n_as, C::NT) : dim3(map.grid);
+    hipLaunchKernelGGL(kfn, grid, dim3(C::NT), lds_bytes, st, (const uint8_t *)W, nb01, K, N,
                        (const uint8_t *)ws, ws_stride, M, y, ldy, map, rg, 0);
     return hipGetLastError();
 }
