@@ -217,9 +217,8 @@ __device__ __forceinline__ void load16_into_lds(const uint8_t *src, uint32_t lds
 // of 6 - 8 us, 110 - 140 us a matrix; one launch of 8 - 12 us with this kernel; an 8-layer step 5818 -> 995 us).
 template <int WT, int TM, int TN, int WR, int WC, int OCC, bool GATHER, bool TAIL>
 __global__ __launch_bounds__(WR *WC * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
-void gemm_blk32_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64_t N, const uint8_t *__restrict__ ws,
-                              size_t ws_stride, int64_t M, float *__restrict__ y, int64_t ldy, TileMap map, RowGather rg,
-                              int slice_stages) {
+void gemm_blk32_kernel(GemmMats mats, int64_t K, const uint8_t *__restrict__ ws, size_t ws_stride, int64_t M, TileMap map, RowGather rg,
+                       int slice_stages) {
     using T = Blk32<WT>;
     using C = DirectCfg<TM, TN, WR, WC, T::HAS_MIN>;
     extern __shared__ __align__(16) uint8_t lds[];
@@ -236,10 +235,14 @@ void gemm_blk32_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, in
         tc = xcd_tile(blockIdx.x, map);
         if (tc.row_tile >= map.row_tiles || tc.tok_tile >= map.tok_tiles) return;
     }
+    const GemmMat mat = GATHER ? mats.m[0] : pick_gemm_mat(mats, tc.row_tile);
+    const int64_t N = mat.N, ldy = mat.ldy;
+    const size_t nb01 = mat.nb01;
+    float *__restrict__ y = mat.y;
     const int64_t row_base = (int64_t)tc.row_tile * C::BM;
     size_t w_offset;
     const GatherView gv = resolve_gather<GATHER>(rg, slot, w_offset, M);
-    W += w_offset;
+    const uint8_t *__restrict__ W = mat.W + w_offset;
     if (gv.tok_tile < 0) return;
     const int64_t tok_base = (int64_t)(GATHER ? gv.tok_tile : tc.tok_tile) * C::BN;
     if (tok_base >= M) return;
@@ -622,12 +625,11 @@ static int blk32_slices_for(int64_t K, int64_t N, int64_t M, int64_t cus) {
 }
 
 template <int WT, int TM, int TN, int WR, int WC, int OCC, bool GATHER, bool TAIL = false>
-static hipError_t launch_direct(const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, int64_t M,
-                                float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t n_as,
-                                int slices = 1, float *part = nullptr) {
+static hipError_t launch_direct(GemmMats mats, int64_t K, const void *ws, size_t ws_stride, int64_t M, const DeviceLimits &lim, hipStream_t st,
+                                const RowGather &rg, int64_t n_as, int slices = 1, float *part = nullptr) {
     if constexpr (!GATHER && !TAIL) {
         if (K % (32 * GEMM_KB) != 0)
-            return launch_direct<WT, TM, TN, WR, WC, OCC, GATHER, true>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as, slices, part);
+            return launch_direct<WT, TM, TN, WR, WC, OCC, GATHER, true>(mats, K, ws, ws_stride, M, lim, st, rg, n_as, slices, part);
     }
     using C = DirectCfg<TM, TN, WR, WC, Blk32<WT>::HAS_MIN>;
     const size_t lds_bytes = 2 * C::STAGE;
@@ -636,47 +638,43 @@ static hipError_t launch_direct(const void *W, size_t nb01, int64_t K, int64_t N
     static LdsGrant grant;
     if (hipError_t e = grant_dynamic_lds(kfn, lds_bytes, lim, grant); e != hipSuccess) return e;
     const int per_cu = (int)(lds_bytes > 80 * 1024 ? 1 : (4 * OCC / C::NW > 0 ? 4 * OCC / C::NW : 1));
-    const TileMap map = make_tile_map(ceil_div(N, C::BM), GATHER ? 1 : ceil_div(M, C::BN), 32 * per_cu);
-    if (!GATHER && slices > 1) {
-        const int slice_stages = (int)ceil_div(ceil_div(K, (int64_t)(32 * GEMM_KB)), (int64_t)slices);
-        hipLaunchKernelGGL(kfn, dim3(map.grid, (unsigned)slices), dim3(C::NT), lds_bytes, st, (const uint8_t *)W, nb01, K, N,
-                           (const uint8_t *)ws, ws_stride, M, part, N, map, rg, slice_stages);
-        if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-        return launch_sum_slices(part, slices, M, N, y, ldy, st);
-    }
-    const dim3 grid = GATHER ? gather_grid(map, n_as, C::NT) : dim3(map.grid);
-    hipLaunchKernelGGL(kfn, grid, dim3(C::NT), lds_bytes, st, (const uint8_t *)W, nb01, K, N,
-                       (const uint8_t *)ws, ws_stride, M, y, ldy, map, rg, 0);
-    return hipGetLastError();
+    const TileMap map = make_tile_map(number_row_tiles(mats, C::BM), GATHER ? 1 : ceil_div(M, C::BN), 32 * per_cu);
+    const GemmMat out = mats.m[0];
+    const bool split = !GATHER && slices > 1;                                     // (one matrix)
+    if (split) { mats.m[0].y = part; mats.m[0].ldy = out.N; }
+    const dim3 grid = GATHER ? gather_grid(map, n_as, C::NT) : dim3(map.grid, (unsigned)slices);
+    hipLaunchKernelGGL(kfn, grid, dim3(C::NT), lds_bytes, st, mats, K, (const uint8_t *)ws, ws_stride, M, map, rg,
+                       split ? (int)ceil_div(ceil_div(K, (int64_t)(32 * GEMM_KB)), (int64_t)slices) : 0);
+    if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    return split ? launch_sum_slices(part, slices, M, out.N, out.y, out.ldy, st) : hipSuccess;
 }
 
 template <int WT>
-static hipError_t launch_type(const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, int64_t M,
-                              float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t n_as,
-                              SplitK split) {
+static hipError_t launch_type(const GemmMats &mats, int64_t K, const void *ws, size_t ws_stride, int64_t M, const DeviceLimits &lim, hipStream_t st,
+                              const RowGather &rg, int64_t n_as, SplitK split) {
     const int64_t cus = lim.compute_units > 0 ? lim.compute_units : 256;
     if (!rg.perm && split.part) {
+        const int64_t N = mats.m[0].N;
         const int slices = blk32_slices_for(K, N, M, cus);
         if (slices > 1 && split.bytes >= (size_t)slices * (size_t)M * (size_t)N * sizeof(float) && (((uintptr_t)split.part) & 15) == 0) {
-            return launch_direct<WT, 1, 1, 2, 2, 3, false>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as, slices, split.part);
+            return launch_direct<WT, 1, 1, 2, 2, 3, false>(mats, K, ws, ws_stride, M, lim, st, rg, n_as, slices, split.part);
         }
     }
-    if (rg.perm) {                                                                   // expert groups: 64 x 64 tiles
-        return launch_direct<WT, 1, 1, 2, 2, 3, true>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
-    }
+    if (rg.perm) return launch_direct<WT, 1, 1, 2, 2, 3, true>(mats, K, ws, ws_stride, M, lim, st, rg, n_as);      // expert groups: 64 x 64 tiles
     // Two 4-wave workgroups of 128 x 128 per CU when that fills the device, else 64 x 128, else 64 x 64 (three workgroups
     // per CU).  Measured on Q4_0 with K = 4096 (us; 128 x 128 / 64 x 128 / 64 x 64 / 128 x 256 with 8 waves): 14336 x 2048
     // tokens 375 / 413 / 468 / 415, 4096 x 2048 106 / 115 / 130 / 106, 14336 x 512 103 / 110 / 114 / 102, 4096 x 512
     // 63 / 38 / 38 / 81.
-    const int64_t g128 = ceil_div(N, 128) * ceil_div(M, 128), g64x128 = ceil_div(N, 64) * ceil_div(M, 128);
+    int64_t rows128 = 0, rows64 = 0;
+    for (int i = 0; i < mats.count; i++) { rows128 += ceil_div(mats.m[i].N, 128); rows64 += ceil_div(mats.m[i].N, 64); }
+    const int64_t g128 = rows128 * ceil_div(M, 128), g64x128 = rows64 * ceil_div(M, 128);
     const int cfg = (int)tune("CHIP_GEMM_CFG", 2 * g128 >= 3 * cus ? 3 : 2 * g64x128 >= 3 * cus ? 6 : 4);
     switch (cfg) {
-        case 3: return launch_direct<WT, 2, 2, 2, 2, 2, false>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);   // 128 x 128, 4 waves
-        case 4: return launch_direct<WT, 1, 1, 2, 2, 3, false>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);   // 64 x 64, 4 waves
-        case 6: return launch_direct<WT, 1, 2, 2, 2, 2, false>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);   // 64 x 128, 4 waves
+        case 3: return launch_direct<WT, 2, 2, 2, 2, 2, false>(mats, K, ws, ws_stride, M, lim, st, rg, n_as);   // 128 x 128, 4 waves
+        case 4: return launch_direct<WT, 1, 1, 2, 2, 3, false>(mats, K, ws, ws_stride, M, lim, st, rg, n_as);   // 64 x 64, 4 waves
+        case 6: return launch_direct<WT, 1, 2, 2, 2, 2, false>(mats, K, ws, ws_stride, M, lim, st, rg, n_as);   // 64 x 128, 4 waves
         default: return hipErrorInvalidValue;
     }
-    return hipErrorInvalidValue;
 }
 
 int gemm_blk32_slices(int wtype, int64_t K, int64_t N, int64_t n, int compute_units) {
@@ -686,20 +684,37 @@ int gemm_blk32_slices(int wtype, int64_t K, int64_t N, int64_t n, int compute_un
 
 int gemm_blk32_moe_tile_tokens() { return DirectCfg<1, 1, 2, 2, false>::BN; }   // the 64 x 64 shape serves the expert groups
 
+static hipError_t launch_blk32_mats(int wtype, const GemmMats &mats, int64_t K, const void *ws, size_t ws_stride, int64_t M,
+                                    const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t n_as, SplitK split) {
+    switch (wtype) {
+        case T_Q4_0:   return launch_type<T_Q4_0>(mats, K, ws, ws_stride, M, lim, st, rg, n_as, split);
+        case T_Q8_0:   return launch_type<T_Q8_0>(mats, K, ws, ws_stride, M, lim, st, rg, n_as, split);
+        case T_Q5_0:   return launch_type<T_Q5_0>(mats, K, ws, ws_stride, M, lim, st, rg, n_as, split);
+        case T_IQ4_NL: return launch_type<T_IQ4_NL>(mats, K, ws, ws_stride, M, lim, st, rg, n_as, split);
+        case T_Q4_1:   return launch_type<T_Q4_1>(mats, K, ws, ws_stride, M, lim, st, rg, n_as, split);
+        case T_Q5_1:   return launch_type<T_Q5_1>(mats, K, ws, ws_stride, M, lim, st, rg, n_as, split);
+        default: return hipErrorInvalidValue;
+    }
+}
 hipError_t launch_gemm_blk32(int wtype, const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride,
                              int64_t M, float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st, const RowGather *rgp,
                              int64_t n_as, SplitK split) {
     if (M <= 0 || N <= 0 || n_as <= 0) return hipSuccess;
-    const RowGather rg = rgp ? *rgp : RowGather{nullptr, nullptr, nullptr, 1, 1, 0};
-    switch (wtype) {
-        case T_Q4_0:   return launch_type<T_Q4_0>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as, split);
-        case T_Q8_0:   return launch_type<T_Q8_0>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as, split);
-        case T_Q5_0:   return launch_type<T_Q5_0>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as, split);
-        case T_IQ4_NL: return launch_type<T_IQ4_NL>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as, split);
-        case T_Q4_1:   return launch_type<T_Q4_1>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as, split);
-        case T_Q5_1:   return launch_type<T_Q5_1>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as, split);
-        default: return hipErrorInvalidValue;
-    }
+    return launch_blk32_mats(wtype, one_gemm_mat(W, nb01, N, y, ldy), K, ws, ws_stride, M, lim, st,
+                             rgp ? *rgp : RowGather{nullptr, nullptr, nullptr, 1, 1, 0}, n_as, split);
+}
+
+// Members that run unsplit by themselves: the same bits, fewer launches (us, Q4_0 at 133 tokens x 960 values: wq + wk + wv of 960 + 320 +
+// 320 rows 31 -> 13, ffn_gate + ffn_up of 2560 rows 23 -> 14; 512 tokens x 4096 values x 14336 rows twice 195 -> 185).
+bool gemm_blk32_group_applicable(int wtype, int64_t K, const GemmMats &mats, int64_t n, int compute_units) {
+    if (mats.count < 2) return false;
+    for (int i = 0; i < mats.count; i++)
+        if (!gemm_blk32_supported(wtype, K, mats.m[i].N, n, false) || gemm_blk32_slices(wtype, K, mats.m[i].N, n, compute_units) != 1) return false;
+    return true;
+}
+hipError_t launch_gemm_blk32_group(int wtype, const GemmMats &mats, int64_t K, const void *ws, size_t ws_stride, int64_t n, const DeviceLimits &lim,
+                                   hipStream_t st) {
+    return launch_blk32_mats(wtype, mats, K, ws, ws_stride, n, lim, st, RowGather{nullptr, nullptr, nullptr, 1, 1, 0}, 1, SplitK{nullptr, 0});
 }
 
 }  // namespace chip

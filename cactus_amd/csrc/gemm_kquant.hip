@@ -2,15 +2,15 @@
 // lm_ggml_vec_dot_q2_K_q8_K .. _q6_K_q8_K, _iq4_xs_q8_K (reference ggml-cpu/ggml-cpu-quants.c) as driven by
 // lm_ggml_compute_forward_mul_mat (ggml-cpu/ggml-cpu.c:1257-1449).
 //
-// This file holds the choice of the kernel and the staging kernel, which runs Q6_K where there is a tile for at most every CU;
+// This file holds the choice of the kernel and the staging kernel, which runs Q6_K and Q3_K where there is a tile for at most every CU;
 // gemm_kr_kernel (gemm_kquant_rows.hip) runs everything else.
 //
-// Per 256-value super-block the reference forms sumi = sum_j sc_j * dot(q_j, a_j) with 8-bit signed scales per 16 values, and applies d
-// and the activation scale once.  The integer scales are folded into the int8 MFMA operand, as the two signed bytes of (q - 32)*sc =
-// 256*hi + lo, so both planes accumulate in the MFMA's own int32 accumulator over the 8 k-blocks of a super-block, sumi = 256*P0 + P1
-// is exact, and the vector unit works once per super-block and output.
+// Per 256-value super-block the reference forms sumi = sum_j sc_j * dot(q_j, a_j) with signed scales per 16 values, and applies d
+// and the activation scale once.  The integer scales are folded into the int8 MFMA operand: Q6_K as the two signed bytes of (q - 32)*sc =
+// 256*hi + lo, sumi = 256*P0 + P1; Q3_K as one plane (4 - q)*sc in -128..124, sumi = -P0.  The planes accumulate in the MFMA's own int32
+// accumulator over the 8 k-blocks of a super-block, all sums are exact, and the vector unit works once per super-block and output.
 //
-// Measured with these digits against base-64 digits of the product plus 4064 (16 instead of 10 vector instructions per four weights, and a
+// Measured for Q6_K with these digits against base-64 digits of the product plus 4064 (16 instead of 10 vector instructions per four weights, and a
 // correction by the block sums), us: 14336 values x 4096 rows at 512 tokens 129 -> 113, 4096 x 4096 at 512 tokens 43 -> 38.6.
 //
 // Structure: a workgroup of WR x WC waves owns 32*WR rows x 64*WC tokens; each wave owns one 32-row tile by two
@@ -30,52 +30,96 @@ namespace chip {
 constexpr int KQ_KB = 4;                      // 32-value k-blocks per LDS stage
 constexpr int KQ_TN = 2;                      // 32-token tiles per wave
 
-// Half h of a super-block holds, for l = 0..31, the elements 128h + 32b + l of k-blocks b = 0..3 as
-//   low / high nibble of ql[64h + l] (b = 0 / 2) and of ql[64h + 32 + l] (b = 1 / 3), two more bits from
-//   qh[32h + l] >> 2b, scale scales[8h + 2b + l/16]                       (reference ggml-quants.c:1695-1711)
-// One staging item = (row, x) of a stage h: p = x / 2 picks the ql half (k-blocks p and p + 2), hf = x & 1 the 16 values
-// l = 16*hf + [0,16) of both, which expand into one operand cell per digit plane and k-block.
-struct Q6Item { u32x4 ql[2], qh[2], sc; uint32_t d; };
-__device__ __forceinline__ void q6_fetch(Q6Item &r, const uint8_t *blk, int x) {
-    const int p = x >> 1, hf = x & 1;
+// One staging item = (row, x) of a stage h (half of a super-block): p = x / 2, the 16 values hf = x & 1 of k-blocks p and p + 2 of that
+// half, which expand into one operand cell per digit plane and k-block.
+template <int WT> struct KQ;
+
+template <> struct KQ<T_Q6_K> {
+    static constexpr int BYTES = BYTES_Q6_K, NPL = 2;              // int8 digit planes
+    // Half h of a super-block holds, for l = 0..31, the elements 128h + 32b + l of k-blocks b = 0..3 as
+    //   low / high nibble of ql[64h + l] (b = 0 / 2) and of ql[64h + 32 + l] (b = 1 / 3), two more bits from
+    //   qh[32h + l] >> 2b, scale scales[8h + 2b + l/16]                       (reference ggml-quants.c:1695-1711)
+    struct Raw { u32x4 ql[2], qh[2], sc; uint32_t d; };
+    __device__ static __forceinline__ void fetch(Raw &r, const uint8_t *blk, int x) {
+        const int p = x >> 1, hf = x & 1;
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-        r.ql[h] = *reinterpret_cast<const u32x4_a2 *>(blk + 64 * h + 32 * p + 16 * hf);
-        r.qh[h] = *reinterpret_cast<const u32x4_a2 *>(blk + 128 + 32 * h + 16 * hf);
+        for (int h = 0; h < 2; h++) {
+            r.ql[h] = *reinterpret_cast<const u32x4_a2 *>(blk + 64 * h + 32 * p + 16 * hf);
+            r.qh[h] = *reinterpret_cast<const u32x4_a2 *>(blk + 128 + 32 * h + 16 * hf);
+        }
+        r.sc = *reinterpret_cast<const u32x4_a2 *>(blk + 192);
+        r.d = *reinterpret_cast<const unsigned short *>(blk + 208);
     }
-    r.sc = *reinterpret_cast<const u32x4_a2 *>(blk + 192);
-    r.d = *reinterpret_cast<const unsigned short *>(blk + 208);
-}
-// cell[plane][0: k-block p, 1: k-block p + 2]
-__device__ __forceinline__ void q6_expand(u32x4 (&cell)[2][2], const Q6Item &r, int h, int x) {
-    const int p = x >> 1, hf = x & 1;
-    // scales[8h + 2p + hf] and scales[8h + 2p + 4 + hf]: byte 2p + hf of dwords 2h and 2h + 1
-    const int s0 = __builtin_amdgcn_sbfe((int)r.sc[2 * h], 8 * (2 * p + hf), 8);
-    const int s1 = __builtin_amdgcn_sbfe((int)r.sc[2 * h + 1], 8 * (2 * p + hf), 8);
-    const uint32_t sa = splat16((uint32_t)s0), ba = splat16((uint32_t)(128 - 32 * s0));
-    const uint32_t sb = splat16((uint32_t)s1), bb = splat16((uint32_t)(128 - 32 * s1));
-    const u32x4 ql = r.ql[h], qh = r.qh[h];
+    __device__ static __forceinline__ void expand(u32x4 (&cell)[NPL][2], const Raw &r, int h, int x) {
+        const int p = x >> 1, hf = x & 1;
+        // scales[8h + 2p + hf] and scales[8h + 2p + 4 + hf]: byte 2p + hf of dwords 2h and 2h + 1
+        const int s0 = __builtin_amdgcn_sbfe((int)r.sc[2 * h], 8 * (2 * p + hf), 8);
+        const int s1 = __builtin_amdgcn_sbfe((int)r.sc[2 * h + 1], 8 * (2 * p + hf), 8);
+        const uint32_t sa = splat16((uint32_t)s0), ba = splat16((uint32_t)(128 - 32 * s0));
+        const uint32_t sb = splat16((uint32_t)s1), bb = splat16((uint32_t)(128 - 32 * s1));
+        const u32x4 ql = r.ql[h], qh = r.qh[h];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const uint32_t hb = qh[i] >> (2 * p);                                               // bits 0, 1 / 4, 5: the upper two bits
-        uint32_t hi, lo;
-        byte_digits(merge_bits(0x0f0f0f0fu, ql[i], hb << 4), 0x003f003fu, sa, ba, hi, lo);  // k-block p
-        cell[0][0][i] = hi; cell[1][0][i] = lo;
-        byte_digits(merge_bits(0x0f0f0f0fu, ql[i] >> 4, hb), 0x003f003fu, sb, bb, hi, lo);  // k-block p + 2
-        cell[0][1][i] = hi; cell[1][1][i] = lo;
+        for (int i = 0; i < 4; i++) {
+            const uint32_t hb = qh[i] >> (2 * p);                                               // bits 0, 1 / 4, 5: the upper two bits
+            uint32_t hi, lo;
+            byte_digits(merge_bits(0x0f0f0f0fu, ql[i], hb << 4), 0x003f003fu, sa, ba, hi, lo);  // k-block p
+            cell[0][0][i] = hi; cell[1][0][i] = lo;
+            byte_digits(merge_bits(0x0f0f0f0fu, ql[i] >> 4, hb), 0x003f003fu, sb, bb, hi, lo);  // k-block p + 2
+            cell[0][1][i] = hi; cell[1][1][i] = lo;
+        }
     }
-}
+    __device__ static __forceinline__ int sumi(int p0, int p1) { return (p0 << 8) + p1; }
+};
+
+template <> struct KQ<T_Q3_K> {
+    static constexpr int BYTES = BYTES_Q3_K, NPL = 1;
+    // hmask[32] | qs[64] | scales[12] | d.  Element 128h + 32v + l: bits 2v of qs[32h + l], bit 4h + v of hmask[l], scale 8h + 2v + l/16.
+    // The two items of a k-half read the same bytes.
+    struct Raw { u32x4 hm, q[2]; uint32_t s[3], d; };
+    __device__ static __forceinline__ void fetch(Raw &r, const uint8_t *blk, int x) {
+        const int hf = x & 1;
+        r.hm = *reinterpret_cast<const u32x4_a2 *>(blk + 16 * hf);
+        r.q[0] = *reinterpret_cast<const u32x4_a2 *>(blk + 32 + 16 * hf);
+        r.q[1] = *reinterpret_cast<const u32x4_a2 *>(blk + 64 + 16 * hf);
+#pragma unroll
+        for (int i = 0; i < 3; i++) r.s[i] = *reinterpret_cast<const u32_a2 *>(blk + 96 + 4 * i);
+        r.d = *reinterpret_cast<const unsigned short *>(blk + 108);
+    }
+    __device__ static __forceinline__ void expand(u32x4 (&cell)[NPL][2], const Raw &r, int h, int x) {
+        const int p = x >> 1, hf = x & 1;
+        // 6-bit scale 4w + i is byte i of word w (reference ggml-quants.c:1062-1071): words 2h and 2h + 1 hold k-blocks 0, 1 and 2, 3
+        const uint32_t hi2 = r.s[2] >> (4 * h);
+        const uint32_t wa = ((r.s[0] >> (4 * h)) & 0x0f0f0f0fu) | ((hi2 & 0x03030303u) << 4);
+        const uint32_t wb = ((r.s[1] >> (4 * h)) & 0x0f0f0f0fu) | (((hi2 >> 2) & 0x03030303u) << 4);
+        const int b = 8 * (2 * p + hf);
+        const int sc[2] = {(int)((wa >> b) & 0xffu) - 32, (int)((wb >> b) & 0xffu) - 32};
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const int v = p + 2 * c;
+            // byte = 128 + (4 - q)*sc in 0..252: the two bytes of a 16-bit lane never carry into each other, whatever the sign of
+            // the multiplier (arithmetic modulo 2^16); flipping bit 7 gives the signed byte
+            const uint32_t mul = splat16((uint32_t)(-sc[c])), add = splat16((uint32_t)((128 + 4 * sc[c]) * 0x101));
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint32_t q = merge_bits(0x03030303u, r.q[h][i] >> (2 * v), (r.hm[i] >> (4 * h + v)) << 2) & 0x07070707u;
+                cell[0][c][i] = pk_mad16(q, mul, add) ^ 0x80808080u;
+            }
+        }
+    }
+    __device__ static __forceinline__ int sumi(int p0, int) { return -p0; }
+};
 
 constexpr int KQ_PRODUCERS = 4;               // staging waves per workgroup, one per SIMD
 
-template <int WR, int WC>
+template <int WT, int WR, int WC>
 struct KqCfg {
+    using T = KQ<WT>;
     static constexpr int NC = WR * WC;                             // MFMA waves
     static constexpr int NW = NC + KQ_PRODUCERS, NT = NW * 64;
     static constexpr int NPT = KQ_PRODUCERS * 64;                  // staging threads
     static constexpr int BM = 32 * WR;                             // weight rows per workgroup
     static constexpr int BN = 32 * KQ_TN * WC;                     // tokens per workgroup
-    static constexpr int NPL = 2;                                  // int8 digit planes
+    static constexpr int NPL = T::NPL;
     // plane stride 2 mod 16 cells: the staging threads of one wave spread over the bank groups
     static constexpr int A_PLANE = BM + 2, B_PLANE = BN + 2;
     static constexpr int A_CELLS = NPL * KQ_KB * 2 * A_PLANE;   // 16-byte cells
@@ -110,11 +154,12 @@ struct KqCfg {
 // The two kinds of wave run side by side on every SIMD, so operand expansion (vector pipe, LDS writes, memory
 // latency) overlaps the matrix pipe by construction instead of by instruction scheduling.  Nothing in the loops is
 // conditional: loads past the last stage repeat it, and stores that do not apply go to a per-thread dump slot.
-template <int WR, int WC, int OCC>
+template <int WT, int WR, int WC, int OCC>
 __global__ __launch_bounds__((WR * WC + KQ_PRODUCERS) * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 void gemm_kq_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64_t N, const uint8_t *__restrict__ ws,
                     size_t ws_stride, int64_t M, float *__restrict__ y, int64_t ldy, TileMap map, int slice_sb) {
-    using C = KqCfg<WR, WC>;
+    using T = KQ<WT>;
+    using C = KqCfg<WT, WR, WC>;
     constexpr int TN = KQ_TN;
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -142,7 +187,7 @@ void gemm_kq_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64
             u32x4 x[C::X_PER_T];
             float xs;
         };
-        struct Wts { Q6Item w[C::W_PER_T]; };
+        struct Wts { typename T::Raw w[C::W_PER_T]; };
         Acts E, O;             // activations of an even / odd stage
         Wts W0, W1;            // weights of an even / odd super-block (both halves: every cache line is fetched once)
         // per-thread source addresses of stage 0 (they advance by a constant per stage / super-block)
@@ -159,7 +204,7 @@ void gemm_kq_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64
         auto fetch_w = [&](Wts &R, int sb_wanted) {
             const int sb = min(sb_wanted, nsb - 1);
 #pragma unroll
-            for (int i = 0; i < C::W_PER_T; i++) q6_fetch(R.w[i], wsrc[i] + (size_t)(sb0 + sb) * BYTES_Q6_K, (pt + i * C::NPT) & 3);
+            for (int i = 0; i < C::W_PER_T; i++) T::fetch(R.w[i], wsrc[i] + (size_t)(sb0 + sb) * T::BYTES, (pt + i * C::NPT) & 3);
         };
         auto fetch_x = [&](Acts &R, int stage_wanted, auto even_tag) {
             constexpr bool even = decltype(even_tag)::value;
@@ -184,8 +229,8 @@ void gemm_kq_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64
             for (int i = 0; i < C::W_PER_T; i++) {
                 const int item = pt + i * C::NPT;
                 const int r = item >> 2, x = item & 3;
-                u32x4 cell[2][2];
-                q6_expand(cell, RW.w[i], h, x);
+                u32x4 cell[C::NPL][2];
+                T::expand(cell, RW.w[i], h, x);
                 const int c0 = (x >> 1) * 2 + (x & 1), c1 = c0 + 4;       // [k-block][k-half]
 #pragma unroll
                 for (int pl = 0; pl < C::NPL; pl++) {
@@ -282,7 +327,7 @@ void gemm_kq_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64
         }
     };
 
-    // once per super-block: fold the planes, out += d * float(256 * P0 + P1) * dx
+    // once per super-block: fold the planes, out += d * float(sumi) * dx
     auto fold = [&](int sbp) {
         const uint8_t *sblk = lds + C::OFF_SBLK + (size_t)sbp * C::SBLK;
         const u32x4 *sp = reinterpret_cast<const u32x4 *>(sblk + C::OFF_SD) + (r0 + half * 16) / 4;
@@ -292,7 +337,7 @@ void gemm_kq_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64
         for (int c = 0; c < TN; c++) {
             const float dx = reinterpret_cast<const float *>(sblk + C::OFF_SX)[n0 + c * 32 + l32];
 #pragma unroll
-            for (int v = 0; v < 16; v++) out[c][v] = __builtin_fmaf(h2f(sd[v]) * (float)((P[0][c][v] << 8) + P[1][c][v]), dx, out[c][v]);
+            for (int v = 0; v < 16; v++) out[c][v] = __builtin_fmaf(h2f(sd[v]) * (float)T::sumi(P[0][c][v], P[C::NPL - 1][c][v]), dx, out[c][v]);
         }
     };
 
@@ -326,21 +371,40 @@ void gemm_kq_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64
 }
 
 static bool kq_splittable(int64_t N) { return ceil_div(N, (int64_t)64) <= 128; }
-// How gemm_kr_kernel covers a product with `tiles` of 128 rows x 64 tokens: k groups of a workgroup (1: four waves, two workgroups
-// a CU; 2: eight waves, one workgroup a CU) and slices of K over the grid's second dimension.
-//   more tiles than CUs     one group: two independent workgroups a CU (us, 512 tokens x 4096 values, one / two groups: Q4_K 4608 rows
-//                           48 / 55, 14336 rows 93 / 112; Q6_K 62 / 76, 120 / 142)
-//   above half as many      two groups walk the super-blocks in turn, so that every SIMD has two waves (4096 rows: Q4_K 37.5 / 33.7,
-//                           Q5_K 40 / 38.5, Q2_K 29 / 27; Q3_K 31.8 / 30.5); so too with 2 slices of rows above 8192 values
-//                           (14336 values x 4096 rows at 201 tokens: Q4_K 59 / 54, Q3_K 53 / 48)
+// Slices of K over the grid's second dimension, each a serial walk whose partial outputs are added in order: for 64 rows x 128 tokens up to
+// two workgroups per CU with one token tile, one per CU with more (the partial outputs grow with the token count), at least four
+// super-blocks each.  The same for both kernels, so that the bits of a product do not depend on which one runs it.
+static int kq_slices_for(int64_t K, int64_t N, int64_t M, int64_t cus) {
+    const int64_t units = K / QK_K, tiles = ceil_div(N, (int64_t)64) * ceil_div(M, (int64_t)128);
+    if (units < 8 || (M <= 128 && !kq_splittable(N))) return 1;
+    const int64_t s = std::min({(M <= 128 ? 2 : 1) * cus / tiles, units / 4, (int64_t)16});
+    if (s < 2) return 1;
+    const int64_t per = ceil_div(units, s);
+    return (int)ceil_div(units, per);                                   // no empty slice
+}
+// Q6_K and Q3_K with at most a 128 x 64 tile for every CU: gemm_kq_kernel, whose staging waves expand a weight once for 128 tokens (us,
+// staged / gemm_kr_kernel: Q6_K 14336 values x 4096 rows at 512 tokens 113 / 128, 201 tokens 66 / 74, 4096 x 4096 at 512 tokens 38.6 / 44; Q3_K
+// 14336 x 4096 at 201 tokens 49 / 53) - unless half of its 128-token tile would be empty and the slices give gemm_kr_kernel a workgroup for
+// every CU (32 tokens: Q6_K 41 / 27, Q3_K 30 / 20).
+static bool kq_staged(int wtype, int64_t K, int64_t N, int64_t M, int64_t cus) {
+    const int64_t tiles = ceil_div(N, (int64_t)128) * ceil_div(M, (int64_t)64);
+    if ((wtype != T_Q6_K && wtype != T_Q3_K) || tiles > cus) return false;
+    return M > 64 || tiles * kq_slices_for(K, N, M, cus) < cus;
+}
+// How gemm_kr_kernel covers a product: k groups of a workgroup (1: four waves that walk the super-blocks in order, two workgroups a CU; 2: eight
+// waves, four on the even and four on the odd super-blocks, one workgroup a CU) and slices of K.  Q3_K .. Q6_K run in one group and the
+// slices above.  Q2_K and IQ4_XS by their number of 128 x 64 tiles:
+//   more tiles than CUs     one group (us, 512 tokens x 4096 values x 4608 rows, one / two groups: Q2_K 36 / 44, IQ4_XS 66 / 72)
+//   above half as many      two groups, so that every SIMD has two waves (4096 rows: Q2_K 29 / 27, IQ4_XS 45 / 42); so too with 2 slices of
+//                           rows above 8192 values (14336 values x 4096 rows at 201 tokens: Q2_K 47 / 42, IQ4_XS 75 / 68)
 //   fewer                   as many slices as give every CU a workgroup, at most 8, or 16 of four super-blocks (a slice more costs its
-//                           partial outputs: Q4_K 14336 values x 4096 rows at 64 tokens 88, 53, 34, 27, 30 us in 1, 2, 4, 8, 12; 1024
-//                           rows at 17 tokens 18.0 / 16.6 in 8 / 12).  Not rounded up: 96 tiles in 3 slices leave 32 workgroups for a
-//                           second turn (Q6_K 4096 x 4096 at 130 tokens 29 / 31 us in 2 / 3).  The slice sum pays for at most
-//                           150000 partial outputs a super-block of a row (1024 values x 4096 rows whole / in 4: Q4_K 17 tokens 12.5 /
-//                           11.6, Q3_K 64 tokens 12.8 / 13.3; 1792 x 4096 at 64 tokens 19 / 16), not for rows of three or less or for two slices of less than 8.
+//                           partial outputs: Q2_K 14336 values x 4096 rows at 64 tokens 68, 42, 29, 23, 26 us in 1, 2, 4, 8, 12).  Not
+//                           rounded up: 96 tiles in 3 slices leave 32 workgroups for a second turn (IQ4_XS 4096 x 4096 at 130 tokens 29 / 31 us
+//                           in 2 / 3).  The slice sum pays for at most 150000 partial outputs a super-block of a row (IQ4_XS 1792 values x
+//                           4096 rows at 64 tokens 21.7 / 16.4 whole / in 4), not for rows of three or less or for two slices of less than 8.
 struct KrPlan { int groups, slices; };
-static KrPlan kr_plan(int64_t K, int64_t N, int64_t M, int64_t cus) {
+static KrPlan kr_plan(int wtype, int64_t K, int64_t N, int64_t M, int64_t cus) {
+    if (wtype != T_Q2_K && wtype != T_IQ4_XS) return KrPlan{1, kq_slices_for(K, N, M, cus)};
     const int64_t tiles = ceil_div(N, (int64_t)128) * ceil_div(M, (int64_t)64), units = K / QK_K;
     if (tiles > cus || units == 1) return KrPlan{1, 1};
     const int64_t most = std::max<int64_t>(8, std::min<int64_t>(16, units / 4));
@@ -350,36 +414,19 @@ static KrPlan kr_plan(int64_t K, int64_t N, int64_t M, int64_t cus) {
     s = ceil_div(units, per);                                           // no empty slice
     return KrPlan{s == 2 && units > 32 ? 2 : 1, (int)s};
 }
-// Q6_K with a tile for at most every CU and more than a third as many, or on rows of fewer than 8 super-blocks: gemm_kq_kernel, whose
-// staging waves expand a weight once for 128 tokens, in slices of its own (us, staged / gemm_kr_kernel: 14336 values x 4096 rows at 512 tokens
-// 113 / 121, 201 tokens 66 / 73; 4096 x 4096 at 512 tokens 38.6 / 41.7; 1024 values x 4096 rows at 64 tokens 14.7 / 15.9).
-static bool kq_staged(int wtype, int64_t K, int64_t N, int64_t M, int64_t cus) {
-    const int64_t tiles = ceil_div(N, (int64_t)128) * ceil_div(M, (int64_t)64);
-    if (wtype != T_Q6_K || tiles > cus) return false;
-    return K < 8 * QK_K || (3 * tiles > cus && (M > 128 || kq_splittable(N)));
-}
-// Its slices of K for 64 x 128 tiles: up to two workgroups per CU with one token tile, one per CU with more, at least four super-blocks
-// each.  low_bit_gemm_ahead below was fitted to times of that kernel and asks for them too.
-static int kq_staged_slices(int64_t K, int64_t N, int64_t M, int64_t cus) {
-    const int64_t units = K / QK_K, tiles = ceil_div(N, (int64_t)64) * ceil_div(M, (int64_t)128);
-    if (units < 8 || (M <= 128 && !kq_splittable(N))) return 1;
-    const int64_t s = std::min({(M <= 128 ? 2 : 1) * cus / tiles, units / 4, (int64_t)16});
-    if (s < 2) return 1;
-    const int64_t per = ceil_div(units, s);
-    return (int)ceil_div(units, per);
-}
-static int planned_slices(int wtype, int64_t K, int64_t N, int64_t n, int64_t cus) {
-    return kq_staged(wtype, K, N, n, cus) ? kq_staged_slices(K, N, n, cus) : kr_plan(K, N, n, cus).slices;
-}
+
 // With few tokens the GEMM's time is its walk over K, whatever the token count, while the GEMV forms pass over the weights once
-// per 8 (Q6_K) or 16 tokens (Q4_K, Q5_K) at memory speed.  The GEMM as planned above is ahead from the first token of a second pass on
-// (us, GEMV passes / GEMM: Q4_K at 17 tokens 4096 x 4096 17.4 / 14.3, 1024 values x 2048 rows 17.9 / 11.0, 4096 values x 16640 rows at 20 tokens
-// 35 / 27; Q6_K at 17 tokens 1280 x 8192 34 / 16).  Where it wants slices and the caller's workspace has no room for their partial
-// outputs, the unsplit walk pays later.
-static int64_t gemm_kq_min_tokens(int wtype, int64_t K, int64_t N, int64_t n, bool can_split) {
-    if (can_split || planned_slices(wtype, K, N, n, 256) == 1) return wtype == T_Q6_K ? 9 : 17;
-    const bool long_rows = K > 8192;
-    return wtype == T_Q6_K ? (long_rows ? 41 : 25) : (long_rows ? 33 : 49);
+// per 8 (Q6_K) or 16 tokens (Q4_K, Q5_K) at memory speed.  With K in slices, or on rows too short for them, the GEMM is ahead from the first
+// token of a second pass on (us, GEMV passes / GEMM: Q4_K at 17 tokens 4096 x 4096 17.4 / 15.1, at 33 tokens 1536 values x 2048 rows 31 / 15,
+// at 18 tokens 512 x 4096 12 / 9.5; Q6_K at 17 tokens 1280 x 8192 34 / 16).  On matrices with too many rows to split Q4_K and Q5_K stay with a
+// second pass (14336 rows x 4096 values at 24 tokens 27.7 / 27.5), and where the caller's workspace has no room for the partial outputs
+// the unsplit walk pays later.
+static int64_t gemm_kq_min_tokens(int wtype, int64_t K, int64_t N, bool can_split) {
+    const bool q6 = wtype == T_Q6_K, long_rows = K > 8192;
+    if (can_split) return q6 ? 9 : 17;
+    if (!kq_splittable(N)) return q6 ? 9 : 33;
+    if (K < 8 * QK_K) return q6 ? 9 : 17;
+    return q6 ? (long_rows ? 41 : 25) : (long_rows ? 33 : 49);
 }
 
 // Q3_K, Q2_K and IQ4_XS: the dot-product GEMV passes of 8 tokens, whose time grows with the tokens, against the GEMM, whose time
@@ -410,21 +457,22 @@ bool gemm_kq_supported(int wtype, int64_t K, int64_t N, int64_t n, bool can_spli
     const int64_t forced = tune("CHIP_GEMM_MIN_TOKENS", 0);
     if (forced > 0) return n >= forced;
     if (wtype == T_Q3_K || wtype == T_Q2_K || wtype == T_IQ4_XS)
-        return low_bit_gemm_ahead(wtype, K, N, n, can_split ? kq_staged_slices(K, N, n, 256) : 1);
-    return n >= gemm_kq_min_tokens(wtype, K, N, n, can_split);
+        return low_bit_gemm_ahead(wtype, K, N, n, can_split ? kq_slices_for(K, N, n, 256) : 1);
+    return n >= gemm_kq_min_tokens(wtype, K, N, can_split);
 }
 int gemm_kq_slices(int wtype, int64_t K, int64_t N, int64_t n, int compute_units) {
     const int64_t cus = compute_units > 0 ? compute_units : 256;
     if (!gemm_kq_supported(wtype, K, N, n, true)) return 1;
-    return planned_slices(wtype, K, N, n, cus);
+    return kr_plan(wtype, K, N, n, cus).slices;
 }
 
+template <int WT>
 static hipError_t launch_kq(const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, int64_t M,
                             float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st, int slices, float *part) {
-    using C = KqCfg<2, 2>;                                               // 64 x 128, 4 + 4 waves
+    using C = KqCfg<WT, 2, 2>;                                               // 64 x 128, 4 + 4 waves
     const size_t lds_bytes = C::TOTAL;
     if ((int64_t)lds_bytes > lim.max_lds_per_block) return hipErrorInvalidValue;
-    auto kfn = gemm_kq_kernel<2, 2, 2>;
+    auto kfn = gemm_kq_kernel<WT, 2, 2, 2>;
     static LdsGrant grant;
     if (hipError_t e = grant_dynamic_lds(kfn, lds_bytes, lim, grant); e != hipSuccess) return e;
     const TileMap map = make_tile_map(ceil_div(N, C::BM), ceil_div(M, C::BN), 32);      // 32 workgroups run on an XCD at a time
@@ -460,19 +508,36 @@ hipError_t launch_gemm_kq(int wtype, const void *W, size_t nb01, int64_t K, int6
     if (M <= 0 || N <= 0 || n_as <= 0) return hipSuccess;
     if (!gemm_kq_type(wtype)) return hipErrorInvalidValue;
     const RowGather rg = rgp ? *rgp : RowGather{nullptr, nullptr, nullptr, 1, 1, 0};
-    if (rg.perm) return launch_gemm_kr(1, wtype, W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as, 1, nullptr);
+    const GemmMats mats = one_gemm_mat(W, nb01, N, y, ldy);
+    if (rg.perm) return launch_gemm_kr(1, wtype, mats, K, ws, ws_stride, M, lim, st, rg, n_as, 1, nullptr);
     const int64_t cus = lim.compute_units > 0 ? lim.compute_units : 256;
     auto room = [&](int slices) {
         return slices <= 1 || (split.part && split.bytes >= (size_t)slices * (size_t)M * (size_t)N * sizeof(float) && (((uintptr_t)split.part) & 15) == 0);
     };
-    KrPlan p = kr_plan(K, N, M, cus);
-    const bool staged = kq_staged(wtype, K, N, M, cus);
-    if (wtype == T_Q6_K && (staged || !room(p.slices))) {                            // (the unsplit walk of few tiles: staged too)
-        const int slices = staged ? kq_staged_slices(K, N, M, cus) : 1;
-        return launch_kq(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, room(slices) ? slices : 1, split.part);
-    }
+    KrPlan p = kr_plan(wtype, K, N, M, cus);
     if (!room(p.slices)) p = KrPlan{2, 1};
-    return launch_gemm_kr(p.groups, wtype, W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as, p.slices, split.part);
+    if (kq_staged(wtype, K, N, M, cus))
+        return wtype == T_Q6_K ? launch_kq<T_Q6_K>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, p.slices, split.part)
+                               : launch_kq<T_Q3_K>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, p.slices, split.part);
+    return launch_gemm_kr(p.groups, wtype, mats, K, ws, ws_stride, M, lim, st, rg, n_as, p.slices, split.part);
+}
+
+// Members that run unsplit by themselves: the same bits, fewer launches and one set of tiles (us, ffn_gate + ffn_up, Q4_K
+// of 4096 values x 14336 rows at 512 tokens, whose 896 tiles each leave a quarter of the second turn idle: 2 x 93.5 -> 164; wq + wk + wv of 1024
+// values x 1024 + 256 + 256 rows at 128 tokens 36 -> 13).
+bool gemm_kq_group_applicable(int wtype, int64_t K, const GemmMats &mats, int64_t n, int compute_units) {
+    const int64_t cus = compute_units > 0 ? compute_units : 256;
+    if (mats.count < 2 || !gemm_kq_type(wtype)) return false;
+    for (int i = 0; i < mats.count; i++) {
+        const int64_t N = mats.m[i].N;
+        const KrPlan p = kr_plan(wtype, K, N, n, cus);
+        if (!gemm_kq_supported(wtype, K, N, n, false) || p.slices != 1 || p.groups != 1 || kq_staged(wtype, K, N, n, cus)) return false;
+    }
+    return true;
+}
+hipError_t launch_gemm_kq_group(int wtype, const GemmMats &mats, int64_t K, const void *ws, size_t ws_stride, int64_t n, const DeviceLimits &lim,
+                                hipStream_t st) {
+    return launch_gemm_kr(1, wtype, mats, K, ws, ws_stride, n, lim, st, RowGather{nullptr, nullptr, nullptr, 1, 1, 0}, 1, 1, nullptr);
 }
 
 }  // namespace chip

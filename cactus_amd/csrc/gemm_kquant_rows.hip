@@ -21,11 +21,11 @@
 //
 // Bound: the vector instructions and MFMAs of a SIMD do not overlap (403 and 34 per super-block and wave for Q4_K; 62 % + 42 % of the cycles
 // by the counters, 16384 rows x 4096 values x 1024 tokens), LDS is 27 % busy without bank conflicts.  Reading operands a step ahead took
-// a quarter off the first form, in which every read was waited for at once (4096 x 4096 x 512 48 -> 36 us); widening d and dmin once instead
+// a quarter off the first form, in which every read was waited for at once; widening d and dmin once instead
 // of in a half-rate v_fma_mix per output and full-rate v_bitop3 in place of v_and_or / v_bfi another 3 %.
-// Measured against the staging kernel (and, for Q4_K and Q5_K, the single-plane kernel) it replaced, us: Q4_K 512 x 4096 values x 4096
-// rows 40 -> 34, x 14336 rows 104 -> 94, 512 x 14336 x 4096 108 -> 94, 32 x 14336 x 4096 38 -> 22; Q2_K 512 x 4096 x 14336 84 -> 68; Q6_K
-// 1500 x 4096 x 14336 404 -> 316; Q5_K 512 x 14336 x 4096 139 -> 109.
+// Measured against the staging kernel (Q4_K, Q5_K: the single-plane kernel) that ran these before, us for values x rows: Q4_K 512 tokens
+// 4096 x 4096 40 -> 36.7, x 14336 105 -> 93.5, 14336 x 4096 110 -> 102, 32 tokens 14336 x 4096 38 -> 23; Q2_K 512 tokens 4096 x 14336
+// 84 -> 68; Q5_K 512 tokens 14336 x 4096 139 -> 120; Q6_K 4096 x 14336 143 -> 121 at 512 tokens, 404 -> 316 at 1500.
 #include "dev_common.h"
 #include "act_layout.h"
 #include "kernels.h"
@@ -359,8 +359,8 @@ __device__ __forceinline__ void kr_load16_into_lds(const uint8_t *src, uint32_t 
 
 template <int WT, int TN, int KS, int OCC, bool GATHER>
 __global__ __launch_bounds__(4 * KS * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
-void gemm_kr_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64_t N, const uint8_t *__restrict__ ws,
-                    size_t ws_stride, int64_t M, float *__restrict__ y, int64_t ldy, TileMap map, RowGather rg, int slice_sb) {
+void gemm_kr_kernel(GemmMats mats, int64_t K, const uint8_t *__restrict__ ws, size_t ws_stride, int64_t M, TileMap map, RowGather rg,
+                    int slice_sb) {
     using T = KR<WT>;
     using C = KrCfg<WT, TN, KS>;
     extern __shared__ __align__(16) uint8_t lds[];
@@ -372,7 +372,6 @@ void gemm_kr_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64
     if (!GATHER && slice_sb > 0) {
         sb0 = (int)blockIdx.y * slice_sb;
         nsb = min(slice_sb, nsb - sb0);
-        y += (size_t)blockIdx.y * (size_t)M * (size_t)ldy;
     }
     TileCoord tc;
     int slot = 0;
@@ -383,9 +382,14 @@ void gemm_kr_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64
         tc = xcd_tile(blockIdx.x, map);
         if (tc.row_tile >= map.row_tiles || tc.tok_tile >= map.tok_tiles) return;        // padding of the tile map
     }
+    const GemmMat mat = GATHER ? mats.m[0] : pick_gemm_mat(mats, tc.row_tile);
+    const int64_t N = mat.N, ldy = mat.ldy;
+    const size_t nb01 = mat.nb01;
+    float *__restrict__ y = mat.y;
+    if (!GATHER && slice_sb > 0) y += (size_t)blockIdx.y * (size_t)M * (size_t)ldy;
     size_t w_offset;
     const GatherView gv = resolve_gather<GATHER>(rg, slot, w_offset, M);
-    W += w_offset;
+    const uint8_t *__restrict__ W = mat.W + w_offset;
     const int64_t row_base = (int64_t)tc.row_tile * KR_ROWS + wr * 32;
     const int64_t tok_base = (int64_t)(GATHER ? gv.tok_tile : tc.tok_tile) * C::BN;
     if (tok_base >= M) return;
@@ -525,13 +529,13 @@ void gemm_kr_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64
             }
             if constexpr (Q < 2) r1 = r2;
         };
-        // reads and expands step 0 of the super-block in `buf`
+        // reads step 0 of the super-block in `buf`; its weights are expanded behind the fold, whose registers are free then
+        typename T::Raw r0;
         auto first_operands = [&](int buf) {
             h = T::hdr(row_lds, half);
-            const typename T::Raw r0 = T::template load<0>(row_lds, half);
+            r0 = T::template load<0>(row_lds, half);
             r1 = T::template load<1>(row_lds, half);
             load_b(bc, buf, T::KA(0), T::KB(0));
-            T::template expand<0>(r0, h, half, cc);
         };
 
         issue_x(grp, 0);
@@ -543,14 +547,14 @@ void gemm_kr_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64
         commit_s(0);
         __builtin_amdgcn_s_waitcnt(WAIT0);
         __syncthreads();
-        if (nit > 1) {
-            fetch_w(grp + KS);
-            fetch_s(grp + KS);
-        }
+        fetch_w(grp + KS);
+        fetch_s(grp + KS);
         first_operands(0);
-        for (int it = 0; it < nit; it++) {
+        T::template expand<0>(r0, h, half, cc);
+        auto iteration = [&](int it, auto last_tag) {
+            constexpr bool last = decltype(last_tag)::value;                  // nothing left to request
             const int buf = it & 1, sb = it * KS + grp, q4 = (it & 3) * KS + grp;
-            if (it + 1 < nit) issue_x(sb + KS, buf ^ 1);
+            if constexpr (!last) issue_x(sb + KS, buf ^ 1);
             step(std::integral_constant<int, 0>{}, buf);
             step(std::integral_constant<int, 1>{}, buf);
             step(std::integral_constant<int, 2>{}, buf);
@@ -560,15 +564,13 @@ void gemm_kr_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64
             f16x8 fa[T::NF16 > 0 ? T::NF16 : 1];
 #pragma unroll
             for (int f = 0; f < T::NF16; f++) fa[f] = __builtin_bit_cast(f16x8, T::f16_cell(h, f, half));
-            if (it + 1 < nit) {
+            if constexpr (!last) {
                 commit_w();
                 commit_s(it + 1);
                 __builtin_amdgcn_s_waitcnt(WAIT0);
                 __syncthreads();
-                if (it + 2 < nit) {
-                    fetch_w(sb + 2 * KS);
-                    fetch_s(sb + 2 * KS);
-                }
+                fetch_w(sb + 2 * KS);
+                fetch_s(sb + 2 * KS);
                 first_operands(buf ^ 1);
             }
             // fold: out += dx * (d * float(sumi) - dmin * summ); the last iteration may lie past a k group's end
@@ -598,7 +600,11 @@ void gemm_kr_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64
                 }
                 }
             }
-        }
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (!last) T::template expand<0>(r0, h, half, cc);
+        };
+        for (int it = 0; it + 1 < nit; it++) iteration(it, std::false_type{});
+        iteration(nit - 1, std::true_type{});
         __syncthreads();
     };
     if (TN > 1 && tokens <= 32) walk(std::integral_constant<int, 1>{});
@@ -638,50 +644,52 @@ void gemm_kr_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64
 }
 
 template <int WT, int TN, int KS, int OCC, bool GATHER>
-hipError_t launch_kr(const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, int64_t M, float *y, int64_t ldy,
-                     const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t slots, int slices, float *part) {
+hipError_t launch_kr(GemmMats mats, int64_t K, const void *ws, size_t ws_stride, int64_t M, const DeviceLimits &lim, hipStream_t st,
+                     const RowGather &rg, int64_t slots, int slices, float *part) {
     using C = KrCfg<WT, TN, KS>;
     if ((int64_t)C::TOTAL > lim.max_lds_per_block) return hipErrorInvalidValue;
     auto kfn = gemm_kr_kernel<WT, TN, KS, OCC, GATHER>;
     static LdsGrant grant;                                               // one per kernel instantiation
     if (hipError_t e = grant_dynamic_lds(kfn, C::TOTAL, lim, grant); e != hipSuccess) return e;
     const int per_cu = (int)(160 * 1024 / C::TOTAL) > 0 ? (int)(160 * 1024 / C::TOTAL) : 1;
+    const int64_t row_tiles = number_row_tiles(mats, KR_ROWS);
     if constexpr (GATHER) {
-        TileMap map = make_tile_map(ceil_div(N, KR_ROWS), 1, 32 * per_cu);
-        const dim3 grid = gather_grid(map, slots, C::NT);
-        hipLaunchKernelGGL(kfn, grid, dim3(C::NT), C::TOTAL, st, (const uint8_t *)W, nb01, K, N, (const uint8_t *)ws, ws_stride, M, y, ldy, map, rg, 0);
+        const TileMap map = make_tile_map(row_tiles, 1, 32 * per_cu);
+        hipLaunchKernelGGL(kfn, gather_grid(map, slots, C::NT), dim3(C::NT), C::TOTAL, st, mats, K, (const uint8_t *)ws, ws_stride, M, map, rg, 0);
         return hipGetLastError();
     } else {
-        const TileMap map = make_tile_map(ceil_div(N, KR_ROWS), ceil_div(M, C::BN), 32 * per_cu);
+        const TileMap map = make_tile_map(row_tiles, ceil_div(M, C::BN), 32 * per_cu);
+        const GemmMat out = mats.m[0];
         const int slice_sb = slices > 1 ? (int)ceil_div(K / QK_K, (int64_t)slices) : 0;
-        hipLaunchKernelGGL(kfn, dim3(map.grid, (unsigned)slices), dim3(C::NT), C::TOTAL, st, (const uint8_t *)W, nb01, K, N,
-                           (const uint8_t *)ws, ws_stride, M, slices > 1 ? part : y, slices > 1 ? N : ldy, map, rg, slice_sb);
+        if (slices > 1) { mats.m[0].y = part; mats.m[0].ldy = out.N; }                  // (one matrix)
+        hipLaunchKernelGGL(kfn, dim3(map.grid, (unsigned)slices), dim3(C::NT), C::TOTAL, st, mats, K, (const uint8_t *)ws, ws_stride, M, map, rg, slice_sb);
         if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-        return slices > 1 ? launch_sum_slices(part, slices, M, N, y, ldy, st) : hipSuccess;
+        return slices > 1 ? launch_sum_slices(part, slices, M, out.N, out.y, out.ldy, st) : hipSuccess;
     }
 }
 
 template <int WT>
-hipError_t launch_kr_groups(int groups, const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, int64_t M, float *y, int64_t ldy,
-                         const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t slots, int slices, float *part) {
-    if (rg.perm) return launch_kr<WT, 2, 1, 2, true>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, 1, nullptr);   // expert groups
-    if (groups == 2) return launch_kr<WT, 2, 2, 2, false>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, slices, part);
-    return launch_kr<WT, 2, 1, 2, false>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, slices, part);
+hipError_t launch_kr_groups(int groups, const GemmMats &mats, int64_t K, const void *ws, size_t ws_stride, int64_t M, const DeviceLimits &lim,
+                            hipStream_t st, const RowGather &rg, int64_t slots, int slices, float *part) {
+    if (rg.perm) return launch_kr<WT, 2, 1, 2, true>(mats, K, ws, ws_stride, M, lim, st, rg, slots, 1, nullptr);   // expert groups
+    if constexpr (WT == T_Q2_K || WT == T_IQ4_XS)
+        if (groups == 2) return launch_kr<WT, 2, 2, 2, false>(mats, K, ws, ws_stride, M, lim, st, rg, slots, slices, part);
+    return launch_kr<WT, 2, 1, 2, false>(mats, K, ws, ws_stride, M, lim, st, rg, slots, slices, part);
 }
 
 }  // namespace
 
 int gemm_kr_tile_tokens() { return KrCfg<T_Q4_K, 2, 1>::BN; }
 
-hipError_t launch_gemm_kr(int groups, int wtype, const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, int64_t M,
-                          float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t slots, int slices, float *part) {
+hipError_t launch_gemm_kr(int groups, int wtype, const GemmMats &mats, int64_t K, const void *ws, size_t ws_stride, int64_t M,
+                          const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t slots, int slices, float *part) {
     switch (wtype) {
-        case T_Q4_K: return launch_kr_groups<T_Q4_K>(groups, W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, slices, part);
-        case T_Q5_K: return launch_kr_groups<T_Q5_K>(groups, W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, slices, part);
-        case T_Q6_K: return launch_kr_groups<T_Q6_K>(groups, W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, slices, part);
-        case T_Q3_K: return launch_kr_groups<T_Q3_K>(groups, W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, slices, part);
-        case T_Q2_K: return launch_kr_groups<T_Q2_K>(groups, W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, slices, part);
-        case T_IQ4_XS: return launch_kr_groups<T_IQ4_XS>(groups, W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, slices, part);
+        case T_Q4_K: return launch_kr_groups<T_Q4_K>(groups, mats, K, ws, ws_stride, M, lim, st, rg, slots, slices, part);
+        case T_Q5_K: return launch_kr_groups<T_Q5_K>(groups, mats, K, ws, ws_stride, M, lim, st, rg, slots, slices, part);
+        case T_Q6_K: return launch_kr_groups<T_Q6_K>(groups, mats, K, ws, ws_stride, M, lim, st, rg, slots, slices, part);
+        case T_Q3_K: return launch_kr_groups<T_Q3_K>(groups, mats, K, ws, ws_stride, M, lim, st, rg, slots, slices, part);
+        case T_Q2_K: return launch_kr_groups<T_Q2_K>(groups, mats, K, ws, ws_stride, M, lim, st, rg, slots, slices, part);
+        case T_IQ4_XS: return launch_kr_groups<T_IQ4_XS>(groups, mats, K, ws, ws_stride, M, lim, st, rg, slots, slices, part);
         default: return hipErrorInvalidValue;
     }
 }

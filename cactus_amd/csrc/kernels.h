@@ -88,6 +88,37 @@ __host__ __device__ __forceinline__ TileCoord xcd_tile(unsigned wg, const TileMa
     return t;
 }
 
+// Up to four matrices of one type over the same activation rows in one GEMM launch: their row tiles are numbered one matrix after the
+// other, first[i] is the number of matrix i's first one.  A plain product is a table of one.
+constexpr int GEMM_MATS_MAX = 4;
+struct GemmMat { const uint8_t *W; size_t nb01; int64_t N; float *y; int64_t ldy; };
+struct GemmMats { GemmMat m[GEMM_MATS_MAX]; int first[GEMM_MATS_MAX]; int count; };
+inline GemmMats one_gemm_mat(const void *W, size_t nb01, int64_t N, float *y, int64_t ldy) {
+    GemmMats t{};
+    t.m[0] = GemmMat{(const uint8_t *)W, nb01, N, y, ldy};
+    t.count = 1;
+    return t;
+}
+// numbers the row tiles of `rows` rows; returns how many there are
+inline int64_t number_row_tiles(GemmMats &t, int64_t rows) {
+    int64_t n = 0;
+    for (int i = 0; i < t.count; i++) {
+        t.first[i] = (int)n;
+        n += ceil_div(t.m[i].N, rows);
+    }
+    return n;
+}
+// the matrix of a row tile (uniform per workgroup; constant indexes, so the table stays in scalar registers); row_tile becomes its own
+__device__ __forceinline__ GemmMat pick_gemm_mat(const GemmMats &t, int &row_tile) {
+    GemmMat m = t.m[0];
+    int first = 0;
+#pragma unroll
+    for (int i = 1; i < GEMM_MATS_MAX; i++)
+        if (i < t.count && row_tile >= t.first[i]) { m = t.m[i]; first = t.first[i]; }
+    row_tile -= first;
+    return m;
+}
+
 // Row gather of LM_GGML_OP_MUL_MAT_ID for the GEMM kernels (reference ggml-cpu/ggml-cpu.c:1460-1710 groups the (token,
 // slot) pairs by expert the same way: matrix_rows / matrix_row_counts).  With perm set, blockIdx.y walks a list of
 // token tiles built on the device: entry i = expert | tile << 12 says "pairs perm[offsets[e] + tile * BN ...] of expert
@@ -277,10 +308,17 @@ hipError_t launch_gemm_kq(int wtype, const void *W, size_t nb01, int64_t K, int6
                           int64_t n, float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st, const RowGather *rg = nullptr,
                           int64_t n_as = 1, SplitK split = SplitK{nullptr, 0});
 // gemm_kquant_rows.hip: the same product by waves that expand their own rows; groups: 1 or 2 k groups a workgroup, slices: parts of K
-hipError_t launch_gemm_kr(int groups, int wtype, const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride,
-                          int64_t n, float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t slots,
-                          int slices, float *part);
+hipError_t launch_gemm_kr(int groups, int wtype, const GemmMats &mats, int64_t K, const void *ws, size_t ws_stride, int64_t n,
+                          const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t slots, int slices, float *part);
 int        gemm_kr_tile_tokens();
+// Several matrices of one type on the same rows in one launch.  _applicable: every member alone would take the GEMM, unsplit; its
+// outputs have the same bits.
+bool       gemm_blk32_group_applicable(int wtype, int64_t K, const GemmMats &mats, int64_t n, int compute_units);
+hipError_t launch_gemm_blk32_group(int wtype, const GemmMats &mats, int64_t K, const void *ws, size_t ws_stride, int64_t n, const DeviceLimits &lim,
+                                   hipStream_t st);
+bool       gemm_kq_group_applicable(int wtype, int64_t K, const GemmMats &mats, int64_t n, int compute_units);
+hipError_t launch_gemm_kq_group(int wtype, const GemmMats &mats, int64_t K, const void *ws, size_t ws_stride, int64_t n, const DeviceLimits &lim,
+                                hipStream_t st);
 // In the three GEMM launchers: with rg, n_as is the number of token-tile slots the grid provides in y (an upper bound
 // of the tile list's length) and n is ignored; gemm_*_moe_tile_tokens gives the tile height the list must be built for.
 
