@@ -497,6 +497,33 @@ int chip_mul_mat_noalloc(int type, const void *W, size_t nb01, int64_t K, int64_
     return chip_mul_mat(type, W, nb01, K, N, x, ldx, n, y, ldy, sp, NOALLOC_SCRATCH_BYTES, stream);
 }
 
+// The members [0, live) of a group over prepared rows, each as chip_mul_mat_run would; those of one type that the GEMM takes, and whose
+// tiles it runs faster together, in one launch.
+static int run_members(const GroupMat *gm, int live, int64_t K, int64_t n, void *workspace, size_t workspace_bytes, const DeviceLimits &lim, void *stream) {
+    unsigned done = 0;
+    for (int i = 0; i < live; i++) {
+        if (done >> i & 1) continue;
+        const int type = gm[i].wtype;
+        GemmMats mats{};
+        unsigned set = 0;
+        for (int j = i; j < live; j++)
+            if (gm[j].wtype == type && mats.count < GEMM_MATS_MAX) {
+                mats.m[mats.count++] = GemmMat{(const uint8_t *)gm[j].W, gm[j].nb01, gm[j].N, gm[j].y, gm[j].ldy};
+                set |= 1u << j;
+            }
+        const size_t stride = act_stride(chip_vec_dot_type(type), K);
+        hipError_t e = hipErrorNotSupported;
+        if (mats.count > 1 && gemm_blk32_group_applicable(type, K, mats, n, lim.compute_units))
+            e = launch_gemm_blk32_group(type, mats, K, workspace, stride, n, lim, (hipStream_t)stream);
+        else if (mats.count > 1 && gemm_kq_group_applicable(type, K, mats, n, lim.compute_units))
+            e = launch_gemm_kq_group(type, mats, K, workspace, stride, n, lim, (hipStream_t)stream);
+        if (e == hipSuccess) { done |= set; continue; }
+        if (e != hipErrorNotSupported) return (int)e;
+        if (int rc = mul_mat_run(type, gm[i].W, gm[i].nb01, K, gm[i].N, n, workspace, workspace_bytes, gm[i].y, gm[i].ldy, stream); rc) return rc;
+    }
+    return CHIP_OK;
+}
+
 // Two matmuls on one activation (ffn_gate / ffn_up).  Up to 4 tokens: one launch of the prologue-quantizing GEMV over
 // both matrices; more tokens: one quantizer, then each matrix on its own path.
 int chip_mul_mat_pair(int type, const void *W1, const void *W2, size_t nb01, int64_t K, int64_t N, const float *x, int64_t ldx,
@@ -517,8 +544,8 @@ int chip_mul_mat_pair(int type, const void *W1, const void *W2, size_t nb01, int
     if (mmv_pair_applicable(type, K, N, n, lim))
         return hip_rc(launch_mmv_q4k(type, W1, nb01, K, N, workspace, act_stride(chip_vec_dot_type(type), K), (int)n, y1, ldy, lim,
                                      (hipStream_t)stream, W2, y2));
-    if (int rc = mul_mat_run(type, W1, nb01, K, N, n, workspace, workspace_bytes, y1, ldy, stream); rc) return rc;
-    return mul_mat_run(type, W2, nb01, K, N, n, workspace, workspace_bytes, y2, ldy, stream);
+    const GroupMat gm[2] = {{type, W1, nb01, N, y1, ldy, nullptr, 0}, {type, W2, nb01, N, y2, ldy, nullptr, 0}};
+    return run_members(gm, 2, K, n, workspace, workspace_bytes, lim, stream);
 }
 
 // MUL(SILU(MUL_MAT(W1, x)), MUL_MAT(W2, x)) in one launch, where chip_mul_mat_pair runs its one-launch GEMV
@@ -700,9 +727,9 @@ static int mul_mat_group(const chip_mat *mats, int count, int64_t K, const float
         if (twins && mmv_pair_applicable(a.wtype, K, a.N, n, lim))
             return hip_rc(launch_mmv_q4k(a.wtype, a.W, a.nb01, K, a.N, workspace, stride, (int)n, a.y, a.ldy, lim, st, b.W, b.y));
     }
+    if (int rc = run_members(gm, live, K, n, workspace, workspace_bytes, lim, stream); rc) return rc;
     for (int i = 0; i < live; i++) {
         const GroupMat &m = gm[i];
-        if (int rc = mul_mat_run(m.wtype, m.W, m.nb01, K, m.N, n, workspace, workspace_bytes, m.y, m.ldy, stream); rc) return rc;
         if (m.t16) {
             const int64_t ne[4] = {n, m.N, 1, 1};
             const int64_t nbs[4] = {m.ldy * 4, 4, m.N * 4, m.N * 4}, nbd[4] = {2, m.t16_ld * 2, m.N * m.t16_ld * 2, m.N * m.t16_ld * 2};

@@ -167,3 +167,48 @@ def test_f16_gemm_stage_counts(dev, orc, K, N, n):
     toks = np.unique(np.concatenate([[0, n - 1], rng.choice(n, min(n, 64), replace=False)]))
     ref = orc.mul_mat(O.F16, w[rows], x[toks], nthreads=8, want=("sum_abs",))
     check(y[np.ix_(toks, rows)], ref, "F16 gemm, %d stages" % (K // 64))
+
+
+# ---- matrices on one activation whose tiles share a launch: the bits of each by itself ----
+# (type, K, rows of each, n): one row tile and a ragged one, 64 x 64 tiles; more row tiles than CUs; a first member of one row; two
+# super-blocks and one of another type between; a K that is no multiple of a stage
+@pytest.mark.parametrize("wt,K,rows,n", [(O.Q4_0, 960, (960, 320, 320), 133), (O.Q8_0, 192, (1, 65, 130, 64), 70), (O.Q5_1, 256, (8200, 8190), 130),
+                                         (O.Q4_K, 1024, (129, 128, 1), 140), (O.Q5_K, 512, (4100, 4100), 260), (O.Q6_K, 256, (300, 70), 65),
+                                         (O.Q3_K, 512, (200, 1030), 129), (O.Q2_K, 768, (33, 500), 200)],
+                         ids=lambda v: O.TYPE_NAMES[v] if isinstance(v, int) and v in O.TYPE_NAMES else None)
+def test_grouped_gemms_equal_single_calls(dev, orc, wt, K, rows, n):
+    rng = np.random.default_rng(K + n)
+    other = O.Q4_K if wt in (O.Q5_K, O.Q6_K, O.Q3_K, O.Q2_K) else None
+    types = [wt] * len(rows)
+    if other is not None and len(rows) == 2:
+        types.insert(1, other)
+        rows = (rows[0], 64, rows[1])
+    ws = [(t, orc.quantize_weights(t, common.weights_f32(K + N + i, N, K))) for i, (t, N) in enumerate(zip(types, rows))]
+    x = common.activations_f32(K + n, n, K)
+    ys = dev.mul_mat_group(ws, x)
+    for i, ((t, W), y) in enumerate(zip(ws, ys)):
+        assert y.tobytes() == dev.mul_mat(t, W, x).tobytes(), i
+    if len(rows) == 2 or other is not None:
+        a, b = ws[0], ws[-1]
+        N = min(a[1].shape[0], b[1].shape[0])
+        y1, y2 = dev.mul_mat_pair(wt, a[1][:N], b[1][:N], x)
+        assert y1.tobytes() == dev.mul_mat(wt, a[1][:N], x).tobytes() and y2.tobytes() == dev.mul_mat(wt, b[1][:N], x).tobytes()
+    toks = np.unique(np.concatenate([[0, n - 1], rng.choice(n, 40, replace=False)]))
+    W = ws[-1][1]
+    pick = np.unique(np.concatenate([[0, W.shape[0] - 1], rng.choice(W.shape[0], min(W.shape[0], 100), replace=False)]))
+    ref = orc.mul_mat(ws[-1][0], W[pick], x[toks], nthreads=8, want=("sum_abs",))
+    check(ys[-1][np.ix_(toks, pick)], ref, "last member")
+
+
+# ---- expert groups: pairs of each expert around a tile of 64, more experts than a turn of the scan takes, more pairs than are kept in registers ----
+@pytest.mark.parametrize("counts,n_used", [((0, 1, 31, 33, 64, 65, 129), 1), ((3, 0) * 160, 1), ((2100, 2101, 0, 2200, 1999), 2)],
+                         ids=("tile edges", "320 experts", "8400 pairs"))
+@pytest.mark.parametrize("wt", (O.Q4_K, O.Q6_K, O.Q4_0, O.F16), ids=lambda t: O.TYPE_NAMES[t])
+def test_expert_groups(dev, orc, wt, counts, n_used):
+    K, N = 256, 70
+    rng = np.random.default_rng(wt + len(counts))
+    ids = rng.permutation(np.repeat(np.arange(len(counts)), counts)).astype(np.int32).reshape(-1, n_used)
+    n_tokens = ids.shape[0]
+    experts = np.stack([orc.quantize_weights(wt, common.weights_f32(wt + e, N, K)) for e in range(len(counts))])
+    x = common.activations_f32(wt, n_tokens, K).reshape(n_tokens, 1, K)
+    check(dev.mul_mat_id(wt, experts, x, ids), orc.mul_mat_id(wt, experts, x, ids, want=("sum_abs",)), "expert groups")
