@@ -543,6 +543,10 @@ static int64_t gemm_blk32_min_tokens(int wtype, int64_t K, int64_t N, bool can_s
         if (K % (32 * GEMM_KB) != 0 && K <= 4096 && N <= 1024 && (wtype == T_Q5_0 || wtype == T_Q4_1 || wtype == T_Q5_1)) return 19;
         return (wtype == T_Q8_0 && long_rows) ? 9 : 17;
     }
+    // Rows too short to be split (less than 16 stages): the walk ends before a third GEMV pass does (us, passes / GEMM, 960 x 960 at 17 tokens
+    // Q4_0 16.8 / 11.2, Q8_0 14.7 / 11.4, Q5_0 14.9 / 12.9, Q4_1 14.6 / 12.5, 1024 x 14336 Q4_0 15.3 / 12.2, Q5_0 43 / 14; 960 x 2560 at 32
+    // tokens Q4_0 34 / 11.5, Q5_0 31 / 13), from 12 stages on with few rows a fourth (1920 x 576 at 17 tokens Q8_0 14.9 / 15.5, Q5_0 14.9 / 18.7)
+    if (const int64_t stages = ceil_div(K, (int64_t)(32 * GEMM_KB)); stages < 16) return stages >= 12 && N <= 2048 ? 25 : 17;
     // too many row tiles to split, or no room for the partial outputs in the caller's workspace: the unsplit walk
     // (long rows with a short last stage, few of them: the walk is slower than the passes up to some 60 tokens - us, passes / GEMM,
     // 320 x 12352: Q5_0 48 tokens 67 / 97, 65 tokens 93 / 97, Q4_1 64 tokens 85 / 93, IQ4_NL 48 tokens 69 / 77, 56 tokens 78 / 77, Q8_0
