@@ -790,10 +790,6 @@ size_t chip_mul_mat_id_workspace_size(int type, int64_t K, int64_t n_as, int64_t
            align16(4 * (pairs / 64 + (size_t)n_as + 2));                // pair list, then the tile list (tiles of >= 64 pairs)
 }
 
-// from this many (token, slot) pairs on, the pairs are grouped by expert and run through the GEMM of the weight type
-// (one-token GEMVs re-read an expert's matrix for every pair)
-constexpr int64_t MOE_GEMM_MIN_PAIRS = 64;
-
 int chip_mul_mat_id(int type, const void *W, size_t nb01, size_t nb02, int64_t K, int64_t N, int64_t n_as, const float *x,
                     int64_t ldx, int64_t ne11, const int32_t *ids, int64_t ids_stride, int64_t n_used, int64_t n_tokens,
                     float *y, int64_t ldy, void *workspace, size_t workspace_bytes, void *stream) {
@@ -816,7 +812,7 @@ int chip_mul_mat_id(int type, const void *W, size_t nb01, size_t nb02, int64_t K
     hipStream_t st = (hipStream_t)stream;
 
     const bool kq = gemm_kq_type(type);
-    if (pairs >= tune("CHIP_MOE_MIN", MOE_GEMM_MIN_PAIRS) && moe_group_supported(n_as, pairs) && (!kq || gemm_kq_moe_ahead(type, K, N, n_as, pairs))) {
+    if (moe_group_supported(n_as, pairs) && moe_gemm_ahead(type, K, N, n_as, pairs)) {
         rc = chip_mul_mat_prepare(type, K, x, ldx, rows, workspace, workspace_bytes, stream);
         if (rc) return rc;
         int32_t *offsets = reinterpret_cast<int32_t *>((uint8_t *)workspace + moe_rows_bytes(type, K, rows));

@@ -21,7 +21,6 @@
 #include "kernels.h"
 #include "kquant_dev.h"
 #include <algorithm>
-#include <cmath>
 #include <cstdlib>
 #include <type_traits>
 
@@ -483,23 +482,6 @@ static hipError_t launch_kq(const void *W, size_t nb01, int64_t K, int64_t N, co
     return slices > 1 ? launch_sum_slices(part, slices, M, N, y, ldy, st) : hipSuccess;
 }
 
-// MUL_MAT_ID of Q3_K, Q2_K and IQ4_XS, both times estimated in us as above.  A GEMV per (token, expert) pair costs its rows by
-// the 4096 values; the GEMM walks a whole 64 x 128 tile per row tile of a picked expert, for a single pair too, and an XCD (32 CUs)
-// runs one in eight of an expert's row tiles.  With ids drawn evenly n_as * (1 - e^(-pairs / n_as)) experts are picked.
-// (GEMV / GEMM, us: Q2_K 768 x 2048, 128 experts, 64 pairs 18 / 53, 1024 pairs 194 / 119; Q3_K 2048 x 768 at 256 pairs 171 / 87;
-// 14336 x 4096, 8 experts, 64 pairs 294 / 166.  Of 1500 drawn calls 12 took the
-// slower kernel by more than 5 %, the worst by 28 %: Q3_K 2048 x 768, 128 experts, 64 pairs 47 / 60.)
-bool gemm_kq_moe_ahead(int wtype, int64_t K, int64_t N, int64_t n_as, int64_t pairs) {
-    if (wtype != T_Q3_K && wtype != T_Q2_K && wtype != T_IQ4_XS) return true;
-    if (gemv_max_tokens(wtype, K, DeviceLimits{256, 160 * 1024}) < 1) return true;
-    const float n_pairs = (float)pairs, experts = (float)n_as;
-    const float gemv = 7.5f + (wtype == T_Q3_K ? 0.34f : wtype == T_Q2_K ? 0.238f : 0.382f) * n_pairs * (float)N / 1024.f * (float)ceil_div(K, (int64_t)4096);
-    const float per_sb = wtype == T_Q3_K ? 0.95f : wtype == T_Q2_K ? 1.05f : 1.6f;
-    const float tiles = experts * (1.f - std::exp(-n_pairs / experts)) + n_pairs / 128.f;
-    const float rounds = (float)ceil_div(ceil_div(N, (int64_t)64), (int64_t)8) * tiles / 32.f + 0.3f;
-    const float gemm = 12.f + (rounds > 1.f ? rounds : 1.f) * (per_sb * (float)(K / QK_K) + 2.2f);
-    return gemm < gemv;
-}
 int gemm_kq_moe_tile_tokens() { return gemm_kr_tile_tokens(); }
 
 hipError_t launch_gemm_kq(int wtype, const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride,

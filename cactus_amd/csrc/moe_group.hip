@@ -4,6 +4,7 @@
 // (atomic cursors); no output depends on it, since every output row is computed on its own.
 #include "dev_common.h"
 #include "kernels.h"
+#include <cmath>
 
 namespace chip {
 
@@ -107,6 +108,42 @@ hipError_t launch_moe_group(const int32_t *ids, int64_t ids_stride, int64_t n_us
     hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(MOE_GROUP_THREADS), 0, st, ids, ids_stride, (unsigned)n_used, (unsigned)pairs, (int)n_as,
                        tile_tokens, offsets, perm, tiles);
     return hipGetLastError();
+}
+
+// MUL_MAT_ID: the pairs grouped by expert and run through the GEMM of the weight type, or a GEMV per pair?  Both times estimated in us, with
+// terms fitted to 40 measured products of each type (6 to 520 pairs, 8 to 128 experts, 512 to 14336 values, at most 0.5 GB of experts; one in ten
+// off by more than 10 to 20 per cent):
+//   GEMV   a pair costs its rows by the 4096 values of one of them; that pairs share an expert buys nothing
+//   GEMM   quantizer, grouping and launch, a walk over K, and the tiles by the 512 that the chip runs at a time.  With ids drawn evenly
+//          n_as * (1 - e^(-pairs / n_as)) experts are picked, and a single pair has its row tiles walked whole
+// (us, GEMV / GEMM: Q4_K 2048 values x 768 rows, 128 experts, 64 pairs 17 / 26, 128 pairs 28.5 / 28.2; 768 x 2048 64 pairs 34 / 24; 4096 x
+// 14336, 8 experts, 16 pairs 63 / 70, 32 pairs 105 / 69; Q8_0 2048 x 768, 128 experts, 256 pairs 46 / 54; 14336 x 4096, 8 experts, 32 pairs
+// 198 / 135.  A limit of 64 pairs for all was 18 per cent above the better of the two on average for Q4_K, this is 0.4; the worst of all
+// 500 products 34 per cent.)  F16 stays with the limit: its GEMV's time is that of the experts' bytes, which the terms do not hold.
+bool moe_gemm_ahead(int wtype, int64_t K, int64_t N, int64_t n_as, int64_t pairs) {
+    const int64_t forced = tune("CHIP_MOE_MIN", 0);
+    if (forced > 0) return pairs >= forced;
+    if (wtype == T_F16 || gemv_max_tokens(wtype, K, DeviceLimits{256, 160 * 1024}) < 1) return pairs >= 64;
+    if (pairs < 16 || pairs >= 4096) return pairs >= 16;
+    struct { float pair, walk, turn, ends; } c;                         // pair: per 1024 rows x 4096 values; the others per super-block, per tile
+    switch (wtype) {
+        case T_Q4_K:   c = {0.235f, 0.92f, 1.25f, 3.5f}; break;
+        case T_Q5_K:   c = {0.365f, 1.10f, 1.50f, 4.0f}; break;
+        case T_Q6_K:   c = {0.390f, 1.50f, 1.55f, 5.0f}; break;
+        case T_Q3_K:   c = {0.355f, 0.90f, 1.30f, 3.5f}; break;
+        case T_Q2_K:   c = {0.255f, 0.80f, 1.20f, 3.5f}; break;
+        case T_IQ4_XS: c = {0.390f, 1.30f, 1.80f, 3.5f}; break;
+        case T_Q8_0:   c = {0.230f, 1.00f, 1.60f, 2.0f}; break;
+        case T_Q4_0:   c = {0.170f, 1.00f, 0.95f, 2.2f}; break;
+        case T_Q5_0:   c = {0.300f, 1.60f, 1.00f, 3.0f}; break;
+        case T_Q4_1:   c = {0.200f, 1.30f, 1.00f, 2.0f}; break;
+        case T_Q5_1:   c = {0.300f, 1.45f, 1.00f, 2.4f}; break;
+        default:       c = {0.380f, 1.07f, 1.05f, 2.1f};                // IQ4_NL
+    }
+    const float n_pairs = (float)pairs, experts = (float)n_as, units = (float)K / 256.f;
+    const float gemv = 6.5f + c.pair * n_pairs * (float)N / 1024.f * (float)ceil_div(K, (int64_t)4096);
+    const float tiles = (experts * (1.f - std::exp(-n_pairs / experts)) + n_pairs / 64.f) * (float)ceil_div(N, (int64_t)(gemm_kq_type(wtype) ? 128 : 64));
+    return 10.f + c.walk * units + tiles / 512.f * (c.turn * units + c.ends) < gemv;
 }
 
 }  // namespace chip
