@@ -212,3 +212,23 @@ def test_expert_groups(dev, orc, wt, counts, n_used):
     experts = np.stack([orc.quantize_weights(wt, common.weights_f32(wt + e, N, K)) for e in range(len(counts))])
     x = common.activations_f32(wt, n_tokens, K).reshape(n_tokens, 1, K)
     check(dev.mul_mat_id(wt, experts, x, ids), orc.mul_mat_id(wt, experts, x, ids, want=("sum_abs",)), "expert groups")
+
+
+# ---- rows too short to be split: the GEMM from 17 tokens on, from 25 with few rows of 1536 values and more; the token in front of each line ----
+@pytest.mark.parametrize("K,N,n", [(256, 33, 17), (960, 130, 16), (960, 130, 17), (1472, 70, 31), (1536, 130, 24), (1536, 130, 25), (1920, 2049, 17)])
+@pytest.mark.parametrize("wt", (O.Q4_0, O.Q8_0, O.Q5_1, O.IQ4_NL), ids=lambda t: O.TYPE_NAMES[t])
+def test_block32_short_rows_of_few_tokens(dev, orc, wt, K, N, n):
+    w = orc.quantize_weights(wt, common.weights_f32(K + N, N, K))
+    x = common.activations_f32(K + n, n, K)
+    check(dev.mul_mat(wt, w, x), orc.mul_mat(wt, w, x, nthreads=8, want=("sum_abs",)), "%d tokens" % n)
+
+
+# ---- 15 pairs (a GEMV each), 16 pairs of long rows on few experts (grouped), 130 pairs on many experts with few rows (a GEMV each) ----
+@pytest.mark.parametrize("n_tokens,n_used,n_as,K,N", [(15, 1, 2, 4096, 2000), (8, 2, 2, 4096, 2000), (65, 2, 64, 512, 24)])
+@pytest.mark.parametrize("wt", (O.Q4_K, O.Q3_K, O.Q4_0), ids=lambda t: O.TYPE_NAMES[t])
+def test_expert_matmul_of_few_pairs(dev, orc, wt, n_tokens, n_used, n_as, K, N):
+    rng = np.random.default_rng(n_tokens + wt)
+    experts = np.stack([orc.quantize_weights(wt, common.weights_f32(wt + e, N, K)) for e in range(n_as)])
+    x = common.activations_f32(wt, n_tokens, K).reshape(n_tokens, 1, K)
+    ids = np.stack([rng.permutation(n_as)[:n_used] for _ in range(n_tokens)]).astype(np.int32)
+    check(dev.mul_mat_id(wt, experts, x, ids), orc.mul_mat_id(wt, experts, x, ids, want=("sum_abs",)), "few pairs")
