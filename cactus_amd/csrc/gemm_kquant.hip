@@ -514,6 +514,7 @@ bool gemm_kq_group_applicable(int wtype, int64_t K, const GemmMats &mats, int64_
         const int64_t N = mats.m[i].N;
         const KrPlan p = kr_plan(wtype, K, N, n, cus);
         if (!gemm_kq_supported(wtype, K, N, n, false) || p.slices != 1 || p.groups != 1 || kq_staged(wtype, K, N, n, cus)) return false;
+        if (gemm_kr_rows_in_reach(mats.m[i].nb01) < 32) return false;
     }
     return true;
 }

@@ -681,8 +681,25 @@ hipError_t launch_kr_groups(int groups, const GemmMats &mats, int64_t K, const v
 
 int gemm_kr_tile_tokens() { return KrCfg<T_Q4_K, 2, 1>::BN; }
 
+// A lane reaches its rows by 32-bit offsets from the first of the wave's 32: how many rows of this stride they cover (32: any tile).
+int64_t gemm_kr_rows_in_reach(size_t nb01) {
+    const size_t more = (size_t)(0xffffffffu - BYTES_Q6_K) / nb01;
+    return more < 31 ? (int64_t)more + 1 : 32;
+}
+
 hipError_t launch_gemm_kr(int groups, int wtype, const GemmMats &mats, int64_t K, const void *ws, size_t ws_stride, int64_t M,
                           const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t slots, int slices, float *part) {
+    // rows more than 138 MB apart (a view of every n-th row, say): a launch for every stretch within reach
+    if (const int64_t reach = gemm_kr_rows_in_reach(mats.m[0].nb01), N = mats.m[0].N; reach < 32 && reach < N) {
+        for (int64_t r = 0; r < N; r += reach) {
+            GemmMats t = mats;                                           // (one matrix: gemm_kq_group_applicable)
+            t.m[0].W += (size_t)r * t.m[0].nb01;
+            t.m[0].y += r;
+            t.m[0].N = reach < N - r ? reach : N - r;
+            if (hipError_t e = launch_gemm_kr(groups, wtype, t, K, ws, ws_stride, M, lim, st, rg, slots, slices, part); e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
     switch (wtype) {
         case T_Q4_K: return launch_kr_groups<T_Q4_K>(groups, mats, K, ws, ws_stride, M, lim, st, rg, slots, slices, part);
         case T_Q5_K: return launch_kr_groups<T_Q5_K>(groups, mats, K, ws, ws_stride, M, lim, st, rg, slots, slices, part);

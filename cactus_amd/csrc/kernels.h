@@ -311,6 +311,7 @@ hipError_t launch_gemm_kq(int wtype, const void *W, size_t nb01, int64_t K, int6
 hipError_t launch_gemm_kr(int groups, int wtype, const GemmMats &mats, int64_t K, const void *ws, size_t ws_stride, int64_t n,
                           const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t slots, int slices, float *part);
 int        gemm_kr_tile_tokens();
+int64_t    gemm_kr_rows_in_reach(size_t nb01);
 // Several matrices of one type on the same rows in one launch.  _applicable: every member alone would take the GEMM, unsplit; its
 // outputs have the same bits.
 bool       gemm_blk32_group_applicable(int wtype, int64_t K, const GemmMats &mats, int64_t n, int compute_units);

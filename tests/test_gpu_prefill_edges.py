@@ -101,6 +101,33 @@ def test_kquant_row_gemm(dev, orc, wt, K, N, n):
     assert np.isfinite(y).all()
 
 
+# Rows so far apart that a tile spans more than 2^32 bytes, and more than 2^32 bytes apart each: (type, stride, rows, tokens).  One whole tile
+# and a ragged one; K split (3584 values at 20 tokens); rows that lie alone
+@pytest.mark.parametrize("wt,K,stride,N,n", [(O.Q4_K, 512, 140 << 20, 40, 70), (O.Q2_K, 3584, 150 << 20, 33, 20), (O.IQ4_XS, 256, (4 << 30) + 64, 3, 60),
+                                             (O.Q5_K, 3584, (2 << 30) + 16, 5, 80)],
+                         ids=lambda v: O.TYPE_NAMES[v] if isinstance(v, int) and v in O.TYPE_NAMES else None)
+def test_kquant_rows_far_apart(dev, orc, wt, K, stride, N, n):
+    L = dev.lib
+    w = orc.quantize_weights(wt, common.weights_f32(K + N, N, K))
+    x = common.activations_f32(K + n, n, K)
+    dW, dx, dy = dev.alloc((N - 1) * stride + w.shape[1]), dev.to_device(x), dev.alloc(2 * n * N * 4)
+    for r in range(N):
+        dW.upload(w[r], r * stride)
+    wsz = max(L.chip_mul_mat_workspace_size_n(wt, K, N, n), L.chip_mul_mat_id_workspace_size(wt, K, 1, 1, n, 1))
+    ws, ids = dev.alloc(wsz), dev.to_device(np.zeros(n, np.int32))
+    ref = orc.mul_mat(wt, w, x, nthreads=8, want=("sum_abs",))
+    y2 = dy.ptr + n * N * 4
+    for call in (lambda: L.chip_mul_mat(wt, dW.ptr, stride, K, N, dx.ptr, K, n, dy.ptr, N, ws.ptr, wsz, None),
+                 lambda: L.chip_mul_mat_pair(wt, dW.ptr, dW.ptr, stride, K, N, dx.ptr, K, n, dy.ptr, y2, N, ws.ptr, wsz, None),
+                 lambda: L.chip_mul_mat_id(wt, dW.ptr, stride, N * stride, K, N, 1, dx.ptr, K, 1, ids.ptr, 1, 1, n, dy.ptr, N, ws.ptr, wsz, None)):
+        dev.check(L.chip_memset(dy.ptr, 0xFF, 2 * n * N * 4, None))
+        dev.check(call())
+        dev.sync()
+        y = dy.download(np.float32, 2 * n * N).reshape(2, n, N)
+        check(y[0], ref, "rows far apart")
+        assert np.isnan(y[1]).all() or y[1].tobytes() == y[0].tobytes()
+
+
 @pytest.mark.parametrize("wt", LOW_BIT, ids=lambda t: O.TYPE_NAMES[t])
 def test_low_bit_kquant_integer_sums_bit_exact(dev, orc, wt):
     """d = dmin = 1 and activation scale 1: the output of one super-block is the integer sumi - summ itself (below 2^24)."""
