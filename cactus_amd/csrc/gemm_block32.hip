@@ -215,7 +215,12 @@ __device__ __forceinline__ void load16_into_lds(const uint8_t *src, uint32_t lds
 // because the selects that zero the activation scales would sit in every stage of the K % 128 == 0 shapes too.  Before this form
 // such rows ran through the dot-product GEMV, a pass per 8 tokens (Q4_0, 133 tokens, 960 and 2560 rows of 960 values: 17 passes
 // of 6 - 8 us, 110 - 140 us a matrix; one launch of 8 - 12 us with this kernel; an 8-layer step 5818 -> 995 us).
-template <int WT, int TM, int TN, int WR, int WC, int OCC, bool GATHER, bool TAIL>
+// NEAR: a stage's four products are summed by themselves, and what rounding takes from the sum of the stages is kept and added at the
+// end.  One chain of K / 32 additions is up to 4.5 times as far from the 64-bit sum as the lanes of a GEMV (relative 2-norm, Q4_0, chain / GEMV:
+// 960 values 1.0e-7 / 6.3e-8, 14336 values 3.8e-7 / 8.4e-8); this stays at 4.9e-8 whatever the length.  It costs a tenth of the walk (us, chain
+// / NEAR: Q4_0 1345 rows x 1024 values at 19 tokens 11.3 / 12.3, IQ4_NL 3538 x 960 at 41 12.7 / 13.7).  Not for the types with a minimum, whose fp16 product of minima and block sums already rounds once per stage (Q4_1 960
+// values: GEMV 8.8e-8, NEAR 1.09e-7).
+template <int WT, int TM, int TN, int WR, int WC, int OCC, bool GATHER, bool TAIL, bool NEAR>
 __global__ __launch_bounds__(WR *WC * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 void gemm_blk32_kernel(GemmMats mats, int64_t K, const uint8_t *__restrict__ ws, size_t ws_stride, int64_t M, TileMap map, RowGather rg,
                        int slice_stages) {
@@ -352,6 +357,7 @@ void gemm_blk32_kernel(GemmMats mats, int64_t K, const uint8_t *__restrict__ ws,
         for (int c = 0; c < TN; c++)
 #pragma unroll
             for (int v = 0; v < 16; v++) acc[a][c][v] = 0.f;
+    float sum[NEAR ? TM : 1][NEAR ? TN : 1][16] = {}, off[NEAR ? TM : 1][NEAR ? TN : 1][16] = {};
     i32x16 magic;
 #pragma unroll
     for (int v = 0; v < 16; v++) {
@@ -463,6 +469,19 @@ void gemm_blk32_kernel(GemmMats mats, int64_t K, const uint8_t *__restrict__ ws,
                 }
             }
         }
+        if constexpr (NEAR) {
+#pragma unroll
+            for (int a = 0; a < TM; a++)
+#pragma unroll
+                for (int c = 0; c < TN; c++)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) {
+                        const float t = sum[a][c][v] + acc[a][c][v];
+                        off[a][c][v] += acc[a][c][v] - (t - sum[a][c][v]);
+                        sum[a][c][v] = t;
+                        acc[a][c][v] = 0.f;
+                    }
+        }
     };
 
     // Every load gets a whole stage to arrive.  A stage begins by expanding the weights fetched during the previous stage
@@ -500,6 +519,15 @@ void gemm_blk32_kernel(GemmMats mats, int64_t K, const uint8_t *__restrict__ ws,
         }
     }
     __builtin_amdgcn_s_waitcnt(wait_vm0());
+    if constexpr (NEAR) {
+#pragma unroll
+        for (int a = 0; a < TM; a++)
+#pragma unroll
+            for (int c = 0; c < TN; c++)
+#pragma unroll
+                for (int v = 0; v < 16; v++)                                        // (an infinite sum leaves NaN in off)
+                    acc[a][c][v] = off[a][c][v] == off[a][c][v] ? sum[a][c][v] + off[a][c][v] : sum[a][c][v];
+    }
 
     // ---- epilogue: register v of tile (a, c) is row 8*(v/4) + 4*half + v%4, token l32 ----
     constexpr float POST = T::HAS_MIN ? 1.f : T::INV_MULT;
@@ -534,6 +562,13 @@ void gemm_blk32_kernel(GemmMats mats, int64_t K, const uint8_t *__restrict__ ws,
 // ahead, measured on 4096 x 4096, 14336 x 4096 and 4096 x 14336 (Q8_0 and Q4_0 have the matrix-core GEMV of 16 tokens
 // a pass, 8 on very long rows; the other types pass once per 8 tokens or fewer):
 static bool blk32_splittable(int64_t N) { return ceil_div(N, (int64_t)64) <= 384; }
+// Rows too short to be split (256 to 1920 values, less than 16 stages): with the NEAR sums the walk ends before a third GEMV pass does (us,
+// passes / GEMM, rows x values: Q8_0 1004 x 960 at 17 tokens 14.6 / 11.9, Q4_0 939 x 1088 at 17 16.7 / 13.5, IQ4_NL 975 x 1152 at 22 17.3 / 14.0, Q4_0
+// 10594 x 960 at 31 54 / 13.8), on longer ones of them with few rows a fourth (Q5_0 949 x 1216 at 17 14.9 / 16.2; Q4_0 2222 x 1600 at 22 25.5 / 17.1)
+static int64_t blk32_near_tokens(int wtype, int64_t K, int64_t N) {
+    if (wtype == T_Q4_1 || wtype == T_Q5_1 || K < 256 || K > 15 * 32 * GEMM_KB) return INT64_MAX;
+    return K > (wtype == T_Q5_0 ? 9 : 11) * 32 * GEMM_KB && N <= 2048 ? 25 : 17;
+}
 static int64_t gemm_blk32_min_tokens(int wtype, int64_t K, int64_t N, bool can_split) {
     const bool long_rows = K > 8192, big = N * K >= ((int64_t)48 << 20);
     if (can_split && blk32_splittable(N)) {
@@ -543,10 +578,6 @@ static int64_t gemm_blk32_min_tokens(int wtype, int64_t K, int64_t N, bool can_s
         if (K % (32 * GEMM_KB) != 0 && K <= 4096 && N <= 1024 && (wtype == T_Q5_0 || wtype == T_Q4_1 || wtype == T_Q5_1)) return 19;
         return (wtype == T_Q8_0 && long_rows) ? 9 : 17;
     }
-    // Rows too short to be split (less than 16 stages): the walk ends before a third GEMV pass does (us, passes / GEMM, 960 x 960 at 17 tokens
-    // Q4_0 16.8 / 11.2, Q8_0 14.7 / 11.4, Q5_0 14.9 / 12.9, Q4_1 14.6 / 12.5, 1024 x 14336 Q4_0 15.3 / 12.2, Q5_0 43 / 14; 960 x 2560 at 32
-    // tokens Q4_0 34 / 11.5, Q5_0 31 / 13), from 12 stages on with few rows a fourth (1920 x 576 at 17 tokens Q8_0 14.9 / 15.5, Q5_0 14.9 / 18.7)
-    if (const int64_t stages = ceil_div(K, (int64_t)(32 * GEMM_KB)); stages < 16) return stages >= 12 && N <= 2048 ? 25 : 17;
     // too many row tiles to split, or no room for the partial outputs in the caller's workspace: the unsplit walk
     // (long rows with a short last stage, few of them: the walk is slower than the passes up to some 60 tokens - us, passes / GEMM,
     // 320 x 12352: Q5_0 48 tokens 67 / 97, 65 tokens 93 / 97, Q4_1 64 tokens 85 / 93, IQ4_NL 48 tokens 69 / 77, 56 tokens 78 / 77, Q8_0
@@ -558,12 +589,16 @@ static int64_t gemm_blk32_min_tokens(int wtype, int64_t K, int64_t N, bool can_s
         default:     return big ? 32 : 48;
     }
 }
+// few tokens that the GEMM takes by itself for its NEAR sums only
+static bool blk32_near(int wtype, int64_t K, int64_t N, int64_t n) {
+    return n >= blk32_near_tokens(wtype, K, N) && n < gemm_blk32_min_tokens(wtype, K, N, false);
+}
 bool gemm_blk32_supported(int wtype, int64_t K, int64_t N, int64_t n, bool can_split) {
     if (!(wtype == T_Q4_0 || wtype == T_Q8_0 || wtype == T_Q5_0 || wtype == T_IQ4_NL || wtype == T_Q4_1 || wtype == T_Q5_1)) return false;
     if (K < 64 || K % 64 != 0 || N < 1) return false;
     const int64_t forced = tune("CHIP_GEMM_MIN_TOKENS", 0);
     if (forced > 0) return n >= forced;
-    return n >= gemm_blk32_min_tokens(wtype, K, N, can_split);
+    return n >= gemm_blk32_min_tokens(wtype, K, N, can_split) || blk32_near(wtype, K, N, n);
 }
 
 // ---- split K: the partial outputs [slice][token][row] added in slice order ----
@@ -628,17 +663,17 @@ static int blk32_slices_for(int64_t K, int64_t N, int64_t M, int64_t cus) {
     return (int)ceil_div(units, per);                                   // no empty slice
 }
 
-template <int WT, int TM, int TN, int WR, int WC, int OCC, bool GATHER, bool TAIL = false>
+template <int WT, int TM, int TN, int WR, int WC, int OCC, bool GATHER, bool NEAR = false, bool TAIL = false>
 static hipError_t launch_direct(GemmMats mats, int64_t K, const void *ws, size_t ws_stride, int64_t M, const DeviceLimits &lim, hipStream_t st,
                                 const RowGather &rg, int64_t n_as, int slices = 1, float *part = nullptr) {
     if constexpr (!GATHER && !TAIL) {
         if (K % (32 * GEMM_KB) != 0)
-            return launch_direct<WT, TM, TN, WR, WC, OCC, GATHER, true>(mats, K, ws, ws_stride, M, lim, st, rg, n_as, slices, part);
+            return launch_direct<WT, TM, TN, WR, WC, OCC, GATHER, NEAR, true>(mats, K, ws, ws_stride, M, lim, st, rg, n_as, slices, part);
     }
     using C = DirectCfg<TM, TN, WR, WC, Blk32<WT>::HAS_MIN>;
     const size_t lds_bytes = 2 * C::STAGE;
     if ((int64_t)lds_bytes > lim.max_lds_per_block) return hipErrorInvalidValue;
-    auto kfn = gemm_blk32_kernel<WT, TM, TN, WR, WC, OCC, GATHER, TAIL>;
+    auto kfn = gemm_blk32_kernel<WT, TM, TN, WR, WC, OCC, GATHER, TAIL, NEAR>;
     static LdsGrant grant;
     if (hipError_t e = grant_dynamic_lds(kfn, lds_bytes, lim, grant); e != hipSuccess) return e;
     const int per_cu = (int)(lds_bytes > 80 * 1024 ? 1 : (4 * OCC / C::NW > 0 ? 4 * OCC / C::NW : 1));
@@ -663,6 +698,12 @@ static hipError_t launch_type(const GemmMats &mats, int64_t K, const void *ws, s
         if (slices > 1 && split.bytes >= (size_t)slices * (size_t)M * (size_t)N * sizeof(float) && (((uintptr_t)split.part) & 15) == 0) {
             return launch_direct<WT, 1, 1, 2, 2, 3, false>(mats, K, ws, ws_stride, M, lim, st, rg, n_as, slices, split.part);
         }
+    }
+    // What would be GEMV passes but for the NEAR sums.  Three waves a SIMD for expert groups, whose tiles are often more than 512 (iq4_nl, 16
+    // pairs over 10672 rows of 512 values 43 -> 38 us), two for the few tiles of a plain product (no spills: 5 - 10 per cent ahead).
+    if constexpr (!Blk32<WT>::HAS_MIN) {
+        if (rg.perm && M < MOE_FEW_PAIRS) return launch_direct<WT, 1, 1, 2, 2, 3, true, true>(mats, K, ws, ws_stride, M, lim, st, rg, n_as);
+        if (!rg.perm && blk32_near(WT, K, mats.m[0].N, M)) return launch_direct<WT, 1, 1, 2, 2, 2, false, true>(mats, K, ws, ws_stride, M, lim, st, rg, n_as);
     }
     if (rg.perm) return launch_direct<WT, 1, 1, 2, 2, 3, true>(mats, K, ws, ws_stride, M, lim, st, rg, n_as);      // expert groups: 64 x 64 tiles
     // Two 4-wave workgroups of 128 x 128 per CU when that fills the device, else 64 x 128, else 64 x 64 (three workgroups
@@ -713,7 +754,9 @@ hipError_t launch_gemm_blk32(int wtype, const void *W, size_t nb01, int64_t K, i
 bool gemm_blk32_group_applicable(int wtype, int64_t K, const GemmMats &mats, int64_t n, int compute_units) {
     if (mats.count < 2) return false;
     for (int i = 0; i < mats.count; i++)
-        if (!gemm_blk32_supported(wtype, K, mats.m[i].N, n, false) || gemm_blk32_slices(wtype, K, mats.m[i].N, n, compute_units) != 1) return false;
+        if (!gemm_blk32_supported(wtype, K, mats.m[i].N, n, false) || gemm_blk32_slices(wtype, K, mats.m[i].N, n, compute_units) != 1 ||
+            blk32_near(wtype, K, mats.m[i].N, n) != blk32_near(wtype, K, mats.m[0].N, n))
+            return false;
     return true;
 }
 hipError_t launch_gemm_blk32_group(int wtype, const GemmMats &mats, int64_t K, const void *ws, size_t ws_stride, int64_t n, const DeviceLimits &lim,

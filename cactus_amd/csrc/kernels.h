@@ -320,8 +320,10 @@ hipError_t launch_gemm_blk32_group(int wtype, const GemmMats &mats, int64_t K, c
 bool       gemm_kq_group_applicable(int wtype, int64_t K, const GemmMats &mats, int64_t n, int compute_units);
 hipError_t launch_gemm_kq_group(int wtype, const GemmMats &mats, int64_t K, const void *ws, size_t ws_stride, int64_t n, const DeviceLimits &lim,
                                 hipStream_t st);
+// Expert matmuls of fewer pairs than this are a GEMV per pair, unless the grouped GEMM is both ahead and as near to the 64-bit sums
+constexpr int64_t MOE_FEW_PAIRS = 64;
 // In the three GEMM launchers: with rg, n_as is the number of token-tile slots the grid provides in y (an upper bound
-// of the tile list's length) and n is ignored; gemm_*_moe_tile_tokens gives the tile height the list must be built for.
+// of the tile list's length) and n is the number of pairs; gemm_*_moe_tile_tokens gives the tile height the list must be built for.
 
 // ops.hip: RMS_NORM, ADD, MUL, SILU over F32 rows (ldb = 0 broadcasts one row of b over all rows of a).
 // LM_GGML_OP_MUL_MAT with a batched, strided F16 src0 (the attention matmuls over the KV cache):

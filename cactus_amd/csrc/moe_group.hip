@@ -123,8 +123,9 @@ hipError_t launch_moe_group(const int32_t *ids, int64_t ids_stride, int64_t n_us
 bool moe_gemm_ahead(int wtype, int64_t K, int64_t N, int64_t n_as, int64_t pairs) {
     const int64_t forced = tune("CHIP_MOE_MIN", 0);
     if (forced > 0) return pairs >= forced;
-    if (wtype == T_F16 || gemv_max_tokens(wtype, K, DeviceLimits{256, 160 * 1024}) < 1) return pairs >= 64;
+    if (wtype == T_F16 || gemv_max_tokens(wtype, K, DeviceLimits{256, 160 * 1024}) < 1) return pairs >= MOE_FEW_PAIRS;
     if (pairs < 16 || pairs >= 4096) return pairs >= 16;
+    if (pairs < MOE_FEW_PAIRS && (wtype == T_Q4_1 || wtype == T_Q5_1)) return false;    // one chain of additions, twice as far off as the GEMV's lanes
     struct { float pair, walk, turn, ends; } c;                         // pair: per 1024 rows x 4096 values; the others per super-block, per tile
     switch (wtype) {
         case T_Q4_K:   c = {0.235f, 0.92f, 1.25f, 3.5f}; break;

@@ -241,7 +241,57 @@ def test_expert_groups(dev, orc, wt, counts, n_used):
     check(dev.mul_mat_id(wt, experts, x, ids), orc.mul_mat_id(wt, experts, x, ids, want=("sum_abs",)), "expert groups")
 
 
-# ---- rows too short to be split: the GEMM from 17 tokens on, from 25 with few rows of 1536 values and more; the token in front of each line ----
+# ---- rows too short to be split: few tokens and expert pairs as near to the 64-bit sums as the GEMV's 8 tokens are ----
+def distance(orc, wt, K, w, x, y):
+    """2-norm of y - sum in 64 bits over that of the sum, of the same quantized operands"""
+    aq = orc.quantize_activation(O.VEC_DOT_TYPE[wt], x)
+    ref = np.array([[orc.vec_dot_exact(wt, K, r, a)[0] for r in w] for a in aq])
+    return np.linalg.norm(y - ref) / np.linalg.norm(ref)
+
+
+# 1600 outputs pin a rounding error's 2-norm to 2 per cent, so a tenth more is a larger error (one chain of additions: 1.3 to 2 times)
+@pytest.mark.parametrize("K,n", [(512, 17), (960, 17), (1024, 47), (1920, 32)])
+@pytest.mark.parametrize("wt", (O.Q4_0, O.Q8_0, O.Q5_0, O.IQ4_NL, O.Q4_1, O.Q5_1), ids=lambda t: O.TYPE_NAMES[t])
+def test_block32_few_tokens_as_near_as_the_gemv(dev, orc, wt, K, n):
+    N = 100
+    w = orc.quantize_weights(wt, common.weights_f32(K + N, N, K))
+    x = common.activations_f32(K + n, n, K)
+    gemv = np.concatenate([dev.mul_mat(wt, w, x[i:i + 4]) for i in range(0, n, 4)])
+    y = dev.mul_mat(wt, w, x)
+    check(y, orc.mul_mat(wt, w, x, nthreads=8, want=("sum_abs",)), "few tokens")
+    assert distance(orc, wt, K, w, x, y) <= 1.1 * distance(orc, wt, K, w, x, gemv)
+
+
+# 60 pairs of 4 experts (grouped, but for the types with a minimum) against the same tokens three at a time (a GEMV per pair)
+@pytest.mark.parametrize("K", (512, 4096))
+@pytest.mark.parametrize("wt", (O.Q4_0, O.Q8_0, O.Q5_0, O.IQ4_NL, O.Q4_1, O.Q5_1), ids=lambda t: O.TYPE_NAMES[t])
+def test_block32_few_expert_pairs_as_near_as_the_gemv(dev, orc, wt, K):
+    N, n_as, n_used, n = 5000, 4, 4, 15
+    w = np.tile(orc.quantize_weights(wt, common.weights_f32(K, 250, K)), (n_as * N // 250, 1)).reshape(n_as, N, -1)
+    x = common.activations_f32(K, n, K).reshape(n, 1, K)
+    ids = np.tile(np.arange(4, dtype=np.int32), (n, 1))
+    y = dev.mul_mat_id(wt, w, x, ids)[:, :, :100].reshape(n, -1)
+    gemv = np.concatenate([dev.mul_mat_id(wt, w, x[i:i + 3], ids[i:i + 3]) for i in range(0, n, 3)])[:, :, :100].reshape(n, -1)
+    rows = w[:, :100].reshape(400, -1)
+    assert distance(orc, wt, K, rows, x[:, 0], y) <= 1.1 * distance(orc, wt, K, rows, x[:, 0], gemv)
+
+
+# an infinite weight scale gives infinities, not NaN, also where the roundings of the sum are kept
+@pytest.mark.parametrize("wt", (O.Q4_0, O.Q8_0, O.Q5_0, O.IQ4_NL), ids=lambda t: O.TYPE_NAMES[t])
+def test_block32_few_tokens_with_an_infinite_scale(dev, orc, wt):
+    K, N, n = 768, 70, 20
+    w = orc.quantize_weights(wt, common.weights_f32(K + N, N, K))
+    w[5, :2] = np.array([np.inf], np.float16).view(np.uint8)
+    w[7, 10 * (w.shape[1] // 24):][:2] = np.array([-np.inf], np.float16).view(np.uint8)
+    x = common.activations_f32(K + n, n, K)
+    aq = orc.quantize_activation(O.VEC_DOT_TYPE[wt], x)
+    ref = np.array([[orc.vec_dot_exact(wt, K, w[r], a)[0] for r in (5, 7)] for a in aq])
+    y = dev.mul_mat(wt, w, x)
+    assert np.isinf(ref).sum() > n and np.array_equal(y[:, (5, 7)], ref, equal_nan=True)
+    assert np.isfinite(np.delete(y, (5, 7), axis=1)).all()
+
+
+# ---- the GEMM from 17 tokens on, from 25 with few rows of 1536 values and more; the token in front of each line; a type with a minimum: GEMV passes ----
 @pytest.mark.parametrize("K,N,n", [(256, 33, 17), (960, 130, 16), (960, 130, 17), (1472, 70, 31), (1536, 130, 24), (1536, 130, 25), (1920, 2049, 17)])
 @pytest.mark.parametrize("wt", (O.Q4_0, O.Q8_0, O.Q5_1, O.IQ4_NL), ids=lambda t: O.TYPE_NAMES[t])
 def test_block32_short_rows_of_few_tokens(dev, orc, wt, K, N, n):
