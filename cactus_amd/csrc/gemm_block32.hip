@@ -607,6 +607,9 @@ bool gemm_blk32_supported(int wtype, int64_t K, int64_t N, int64_t n, bool can_s
 // at N - 4 and stores only the rows that the group before it has not, so that every load is a whole one.  One launch for every N: such
 // an N used to take a launch per token (us of the whole product, before -> now: Q3_K 694 x 4352 at 363 tokens 909 -> 22, Q2_K 1159 x 13056
 // at 69 tokens 331 -> 27, Q8_0 670 x 5312 at 1107 tokens 2403 -> 42).
+// S: float, or double where K is cut into slices of one to three super-blocks (Q2_K, IQ4_XS): up to eight roundings of the whole sum would
+// otherwise be most of the error (relative 2-norm, IQ4_XS 4096 values at 64 tokens 7.7e-8 with float sums, 5.8e-8 with double; the same time).
+template <typename S>
 __global__ __launch_bounds__(256) void sum_slices_kernel(const float *__restrict__ part, int slices, int64_t n, int64_t N,
                                                          float *__restrict__ y, int64_t ldy) {
     typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
@@ -615,15 +618,15 @@ __global__ __launch_bounds__(256) void sum_slices_kernel(const float *__restrict
     const int64_t t = g / groups, r = (g - t * groups) * 4, per_slice = n * N;
     if (N < 4) {                                                                     // one group of one to three rows
         for (int64_t k = 0; k < N; k++) {
-            float v = 0.f;
-            for (int s = 0; s < slices; s++) v += part[(size_t)s * per_slice + t * N + k];
-            y[(size_t)t * ldy + k] = v;
+            S v = 0;
+            for (int s = 0; s < slices; s++) v += (S)part[(size_t)s * per_slice + t * N + k];
+            y[(size_t)t * ldy + k] = (float)v;
         }
         return;
     }
     const int64_t first = r < N - 4 ? r : N - 4;
     const float *src = part + t * N + first;
-    f32x4_a4 v = {0.f, 0.f, 0.f, 0.f};
+    S v[4] = {0, 0, 0, 0};
     for (int s0 = 0; s0 < slices; s0 += 8) {
         f32x4_a4 p[8];
 #pragma unroll
@@ -631,16 +634,18 @@ __global__ __launch_bounds__(256) void sum_slices_kernel(const float *__restrict
             if (s0 + j < slices) p[j] = *reinterpret_cast<const f32x4_a4 *>(src + (size_t)(s0 + j) * per_slice);
 #pragma unroll
         for (int j = 0; j < 8; j++)
-            if (s0 + j < slices) v += p[j];
+            if (s0 + j < slices)
+#pragma unroll
+                for (int k = 0; k < 4; k++) v[k] += (S)p[j][k];
     }
     float *dst = y + (size_t)t * ldy + first;
 #pragma unroll
     for (int k = 0; k < 4; k++)
-        if (first + k >= r) dst[k] = v[k];
+        if (first + k >= r) dst[k] = (float)v[k];
 }
-hipError_t launch_sum_slices(const float *part, int slices, int64_t n, int64_t N, float *y, int64_t ldy, hipStream_t st) {
+hipError_t launch_sum_slices(const float *part, int slices, int64_t n, int64_t N, float *y, int64_t ldy, hipStream_t st, bool in_double) {
     if (n <= 0 || N <= 0 || slices <= 0) return hipSuccess;
-    hipLaunchKernelGGL(sum_slices_kernel, dim3((unsigned)ceil_div(n * ceil_div(N, (int64_t)4), (int64_t)256)), dim3(256), 0, st, part, slices,
+    hipLaunchKernelGGL(in_double ? sum_slices_kernel<double> : sum_slices_kernel<float>, dim3((unsigned)ceil_div(n * ceil_div(N, (int64_t)4), (int64_t)256)), dim3(256), 0, st, part, slices,
                        n, N, y, ldy);
     return hipGetLastError();
 }

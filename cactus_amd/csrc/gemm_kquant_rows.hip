@@ -664,7 +664,7 @@ hipError_t launch_kr(GemmMats mats, int64_t K, const void *ws, size_t ws_stride,
         if (slices > 1) { mats.m[0].y = part; mats.m[0].ldy = out.N; }                  // (one matrix)
         hipLaunchKernelGGL(kfn, dim3(map.grid, (unsigned)slices), dim3(C::NT), C::TOTAL, st, mats, K, (const uint8_t *)ws, ws_stride, M, map, rg, slice_sb);
         if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-        return slices > 1 ? launch_sum_slices(part, slices, M, out.N, out.y, out.ldy, st) : hipSuccess;
+        return slices > 1 ? launch_sum_slices(part, slices, M, out.N, out.y, out.ldy, st, WT == T_Q2_K || WT == T_IQ4_XS) : hipSuccess;
     }
 }
 

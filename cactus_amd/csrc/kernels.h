@@ -280,7 +280,7 @@ hipError_t launch_mmv(int wtype, const void *W, size_t nb01, int64_t K, int64_t 
 struct SplitK { float *part; size_t bytes; };
 int        gemm_blk32_slices(int wtype, int64_t K, int64_t N, int64_t n, int compute_units);
 int        gemm_kq_slices(int wtype, int64_t K, int64_t N, int64_t n, int compute_units);
-hipError_t launch_sum_slices(const float *part, int slices, int64_t n, int64_t N, float *y, int64_t ldy, hipStream_t st);
+hipError_t launch_sum_slices(const float *part, int slices, int64_t n, int64_t N, float *y, int64_t ldy, hipStream_t st, bool in_double = false);
 bool       gemm_blk32_supported(int wtype, int64_t K, int64_t N, int64_t n, bool can_split = false);
 hipError_t launch_gemm_blk32(int wtype, const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride,
                              int64_t n, float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st,

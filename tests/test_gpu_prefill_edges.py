@@ -276,6 +276,17 @@ def test_block32_few_expert_pairs_as_near_as_the_gemv(dev, orc, wt, K):
     assert distance(orc, wt, K, rows, x[:, 0], y) <= 1.1 * distance(orc, wt, K, rows, x[:, 0], gemv)
 
 
+# K in eight slices of one super-block (Q2_K, IQ4_XS) and in two of four: no further off than rows walked whole (8192 outputs: within 1 per cent)
+@pytest.mark.parametrize("wt", LOW_BIT, ids=lambda t: O.TYPE_NAMES[t])
+def test_slices_of_k_as_near_as_whole_rows(dev, orc, wt):
+    K, N, n = 2048, 128, 64
+    w = orc.quantize_weights(wt, common.weights_f32(K + N, N, K))
+    x = common.activations_f32(K + n, n, K)
+    whole, slices = dev.mul_mat(wt, w, x, split_k=False), dev.mul_mat(wt, w, x)
+    assert slices.tobytes() != whole.tobytes()
+    assert distance(orc, wt, K, w, x, slices) <= 1.03 * distance(orc, wt, K, w, x, whole)
+
+
 # an infinite weight scale gives infinities, not NaN, also where the roundings of the sum are kept
 @pytest.mark.parametrize("wt", (O.Q4_0, O.Q8_0, O.Q5_0, O.IQ4_NL), ids=lambda t: O.TYPE_NAMES[t])
 def test_block32_few_tokens_with_an_infinite_scale(dev, orc, wt):
