@@ -232,9 +232,9 @@ void gemm_blk32_kernel(GemmMats mats, int64_t K, const uint8_t *__restrict__ ws,
     const int wr = wave / WC, wc = wave % WC;
     const int half = lane >> 5, l32 = lane & 31;
     TileCoord tc;
-    int slot = 0;
+    int32_t entry = 0;
     if constexpr (GATHER) {
-        if (!gather_tile(rg, map, slot, tc.row_tile)) return;
+        if (!gather_tile<C::BN>(rg, map, entry, tc.row_tile)) return;
         tc.tok_tile = 0;
     } else {
         tc = xcd_tile(blockIdx.x, map);
@@ -246,9 +246,8 @@ void gemm_blk32_kernel(GemmMats mats, int64_t K, const uint8_t *__restrict__ ws,
     float *__restrict__ y = mat.y;
     const int64_t row_base = (int64_t)tc.row_tile * C::BM;
     size_t w_offset;
-    const GatherView gv = resolve_gather<GATHER>(rg, slot, w_offset, M);
+    const GatherView gv = resolve_gather<GATHER>(rg, entry, w_offset, M);
     const uint8_t *__restrict__ W = mat.W + w_offset;
-    if (gv.tok_tile < 0) return;
     const int64_t tok_base = (int64_t)(GATHER ? gv.tok_tile : tc.tok_tile) * C::BN;
     if (tok_base >= M) return;
     static_assert(!(GATHER && TAIL), "expert rows are whole stages");

@@ -374,9 +374,9 @@ void gemm_kr_kernel(GemmMats mats, int64_t K, const uint8_t *__restrict__ ws, si
         nsb = min(slice_sb, nsb - sb0);
     }
     TileCoord tc;
-    int slot = 0;
+    int32_t entry = 0;
     if constexpr (GATHER) {
-        if (!gather_tile(rg, map, slot, tc.row_tile)) return;
+        if (!gather_tile<C::BN>(rg, map, entry, tc.row_tile)) return;
         tc.tok_tile = 0;
     } else {
         tc = xcd_tile(blockIdx.x, map);
@@ -388,7 +388,7 @@ void gemm_kr_kernel(GemmMats mats, int64_t K, const uint8_t *__restrict__ ws, si
     float *__restrict__ y = mat.y;
     if (!GATHER && slice_sb > 0) y += (size_t)blockIdx.y * (size_t)M * (size_t)ldy;
     size_t w_offset;
-    const GatherView gv = resolve_gather<GATHER>(rg, slot, w_offset, M);
+    const GatherView gv = resolve_gather<GATHER>(rg, entry, w_offset, M);
     const uint8_t *__restrict__ W = mat.W + w_offset;
     const int64_t row_base = (int64_t)tc.row_tile * KR_ROWS + wr * 32;
     const int64_t tok_base = (int64_t)(GATHER ? gv.tok_tile : tc.tok_tile) * C::BN;

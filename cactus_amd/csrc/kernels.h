@@ -130,6 +130,7 @@ struct RowGather {
     const int32_t *perm, *offsets, *tiles;     // tiles[0] = number of entries, entries from tiles[1]
     int32_t n_used, ne11;
     size_t nb02;
+    bool columns;                              // an expert's token tiles in columns (gather_tile)
 };
 struct GatherView {                // resolved once per workgroup
     const int32_t *list;           // this expert's pairs, or nullptr
@@ -142,38 +143,60 @@ struct GatherView {                // resolved once per workgroup
     }
     __device__ __forceinline__ int64_t out_row(int64_t tok) const { return list ? (int64_t)list[tok] : tok; }
 };
-// Sets the token count M and the byte offset of the weight matrix to the expert's and returns its view.  GATHER is a
+// Sets the token count M and the byte offset of the weight matrix to those of a list entry's expert and returns its view.  GATHER is a
 // template argument of the kernels so that the plain MUL_MAT instantiations carry none of this.
 template <bool GATHER>
-__device__ __forceinline__ GatherView resolve_gather(const RowGather &rg, int slot, size_t &w_offset, int64_t &M) {
+__device__ __forceinline__ GatherView resolve_gather(const RowGather &rg, int32_t entry, size_t &w_offset, int64_t &M) {
     GatherView v{nullptr, rg.n_used, rg.ne11, 0};
     w_offset = 0;
     if constexpr (GATHER) {
-        if (slot >= rg.tiles[0]) { v.tok_tile = -1; return v; }
-        const int32_t d = rg.tiles[1 + slot];
-        const int e = d & ((1 << MOE_EXPERT_BITS) - 1);
+        const int e = entry & ((1 << MOE_EXPERT_BITS) - 1);
         const int32_t off = rg.offsets[e];
         M = rg.offsets[e + 1] - off;
         v.list = rg.perm + off;
-        v.tok_tile = d >> MOE_EXPERT_BITS;
+        v.tok_tile = entry >> MOE_EXPERT_BITS;
         w_offset = (size_t)e * rg.nb02;
     }
     return v;
 }
+// the entry that blockIdx.y walks (the F16 kernel)
 template <bool GATHER>
 __device__ __forceinline__ GatherView resolve_gather(const RowGather &rg, size_t &w_offset, int64_t &M) {
-    return resolve_gather<GATHER>(rg, (int)blockIdx.y, w_offset, M);
+    if (GATHER && (int)blockIdx.y >= rg.tiles[0]) return GatherView{nullptr, rg.n_used, rg.ne11, -1};
+    return resolve_gather<GATHER>(rg, GATHER ? rg.tiles[1 + blockIdx.y] : 0, w_offset, M);
 }
 // Expert groups over a grid of one dimension (cut into two only where HIP's limit asks for it): the (entry, row tile) pairs of the
-// list, an entry's row tiles side by side, are cut into 8 equal stretches, one per XCD.  The length of the list is known on the
+// list, an expert's side by side, are cut into 8 equal stretches, one per XCD.  The length of the list is known on the
 // device only, so the grid provides for `slots` entries and the workgroups past the end exit at once.
-__device__ __forceinline__ bool gather_tile(const RowGather &rg, const TileMap &m, int &slot, int &row_tile) {
+// An expert whose matrix fits the 4 MB of an XCD's L2 has its row tiles innermost.  Of a larger one (columns) the token tiles are taken 8 at a time and
+// those innermost: the 64 to 96 tiles that an XCD works on then share some ten row tiles of weights and 8 of activations.  With its row tiles
+// innermost its weights went through the L2 once per token tile, and eight XCDs on as many experts had more of them in flight than the
+// memory-side cache holds (us, before -> now: Q8_0 3328 values x 13688 rows, 64 experts, 6664 pairs 2179 -> 1779; Q5_1 4096 x 11080, 16 experts,
+// 11272 pairs 2473 -> 2075; Q4_K 4864 x 16312, 16 experts, 7384 pairs 1923 -> 1669.  On small matrices, where full and nearly empty token tiles would
+// alternate: Q4_K 1792 x 3096, 8 experts, 744 pairs 29 with row tiles innermost, 32 in columns).
+constexpr unsigned GATHER_COLUMN = 8;
+__host__ __device__ __forceinline__ void gather_order(unsigned i, unsigned row_tiles, unsigned tok_tiles, int &row_tile, int &tok_tile) {
+    const unsigned first = i / (GATHER_COLUMN * row_tiles) * GATHER_COLUMN, left = tok_tiles - first, width = left < GATHER_COLUMN ? left : GATHER_COLUMN;
+    i -= first * row_tiles;
+    row_tile = (int)(i / width);
+    tok_tile = (int)(first + i % width);
+}
+template <int BN>
+__device__ __forceinline__ bool gather_tile(const RowGather &rg, const TileMap &m, int32_t &entry, int &row_tile) {
     const unsigned wg = blockIdx.x + gridDim.x * blockIdx.y;
     const unsigned total = (unsigned)rg.tiles[0] * (unsigned)m.row_tiles, per = (total + XCDS - 1) / XCDS;
     const unsigned idx = (wg % XCDS) * per + wg / XCDS;
     if (wg / XCDS >= per || idx >= total) return false;
-    slot = (int)(idx / (unsigned)m.row_tiles);
-    row_tile = (int)(idx % (unsigned)m.row_tiles);
+    const unsigned slot = idx / (unsigned)m.row_tiles;
+    row_tile = (int)(idx - slot * (unsigned)m.row_tiles);
+    entry = rg.tiles[1 + slot];
+    const int e = entry & ((1 << MOE_EXPERT_BITS) - 1), t = entry >> MOE_EXPERT_BITS;
+    const unsigned tok_tiles = (unsigned)(rg.offsets[e + 1] - rg.offsets[e] + BN - 1) / (unsigned)BN;
+    if (rg.columns && tok_tiles > 1) {
+        int tok_tile;
+        gather_order((unsigned)t * (unsigned)m.row_tiles + (unsigned)row_tile, (unsigned)m.row_tiles, tok_tiles, row_tile, tok_tile);
+        entry = e | (tok_tile << MOE_EXPERT_BITS);
+    }
     return true;
 }
 inline dim3 gather_grid(const TileMap &m, int64_t slots, int threads) {

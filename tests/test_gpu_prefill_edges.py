@@ -241,6 +241,23 @@ def test_expert_groups(dev, orc, wt, counts, n_used):
     check(dev.mul_mat_id(wt, experts, x, ids), orc.mul_mat_id(wt, experts, x, ids, want=("sum_abs",)), "expert groups")
 
 
+# An expert larger than an XCD's L2 has its token tiles in columns of 8: one short tile, a column and one tile, two columns and a short one, none
+@pytest.mark.parametrize("wt,K,N", [(O.Q4_0, 1024, 8000), (O.Q4_K, 2048, 4100)], ids=lambda v: O.TYPE_NAMES.get(v))
+def test_large_experts_with_many_token_tiles(dev, orc, wt, K, N):
+    counts = (3, 520, 0, 1060)
+    rng = np.random.default_rng(K)
+    w = np.stack([np.roll(np.tile(orc.quantize_weights(wt, common.weights_f32(K + e, 100, K)), (-(-N // 100), 1))[:N], e, axis=0) for e in range(4)])
+    assert w[0].nbytes > 4 << 20
+    ids = rng.permutation(np.repeat(np.arange(4), counts)).astype(np.int32).reshape(-1, 1)
+    x = common.activations_f32(K, ids.shape[0], K)
+    y = dev.mul_mat_id(wt, w, x[:, None], ids)[:, 0]
+    for e in (0, 1, 3):
+        of = ids[:, 0] == e
+        if counts[e] > 100:
+            assert y[of].tobytes() == dev.mul_mat(wt, w[e], x[of], split_k=False).tobytes()
+        check(y[of][:50, :150], orc.mul_mat(wt, w[e, :150], x[of][:50], nthreads=8, want=("sum_abs",)), "expert %d" % e)
+
+
 # ---- rows too short to be split: few tokens and expert pairs as near to the 64-bit sums as the GEMV's 8 tokens are ----
 def distance(orc, wt, K, w, x, y):
     """2-norm of y - sum in 64 bits over that of the sum, of the same quantized operands"""

@@ -2,7 +2,8 @@
 // For every grid shape given on stdin ("row_tiles tok_tiles concurrent" per line) it verifies that
 //   * every tile is visited exactly once and workgroups past the last tile get the out-of-range coordinate,
 //   * the eight XCDs (workgroup id modulo 8) get tile counts that differ by at most one stretch remainder,
-//   * the tiles one XCD works on at a time (consecutive stretch positions) stay within a few blocks of the map.
+//   * the tiles one XCD works on at a time (consecutive stretch positions) stay within a few blocks of the map;
+// and of the order of an expert's tiles (gather_order) that it is a bijection with few row tiles in flight.
 // Prints "ok <shapes>" or the first violation; no device code runs.
 #include <cstdio>
 #include <cstdlib>
@@ -61,6 +62,26 @@ int main() {
                            s0, rt, tt, nr, nt, m.sr, m.sc);
                     return 1;
                 }
+            }
+        }
+        // expert groups: a bijection onto an expert's tiles, a stretch of 64 of them over at most one column's token tiles and the next one's
+        std::vector<int> group((size_t)(rt * tt), 0);
+        for (unsigned i0 = 0; i0 < m.tiles; i0 += 64) {
+            std::vector<char> rows((size_t)rt, 0);
+            long nr = 0;
+            for (unsigned i = i0; i < i0 + 64 && i < m.tiles; i++) {
+                int r, t;
+                gather_order(i, (unsigned)rt, (unsigned)tt, r, t);
+                if (r < 0 || r >= rt || t < 0 || t >= tt || group[(size_t)r * tt + t]++) {
+                    printf("expert group %ld x %ld: index %u -> (%d, %d) out of range or taken\n", rt, tt, i, r, t);
+                    return 1;
+                }
+                if (!rows[r]) { rows[r] = 1; nr++; }
+            }
+            const long narrowest = tt % GATHER_COLUMN && i0 / (rt * GATHER_COLUMN) + 2 > tt / GATHER_COLUMN ? tt % GATHER_COLUMN : (long)GATHER_COLUMN;
+            if (nr > 64 / narrowest + 3) {
+                printf("expert group %ld x %ld: 64 tiles from %u on touch %ld row tiles\n", rt, tt, i0, nr);
+                return 1;
             }
         }
         shapes++;
