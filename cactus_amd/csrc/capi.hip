@@ -818,10 +818,10 @@ int chip_mul_mat_id(int type, const void *W, size_t nb01, size_t nb02, int64_t K
         int32_t *offsets = reinterpret_cast<int32_t *>((uint8_t *)workspace + moe_rows_bytes(type, K, rows));
         int32_t *perm = offsets + align16(4 * (size_t)(n_as + 1)) / 4;
         int32_t *tiles = perm + align16(4 * (size_t)pairs) / 4;
-        const int bn = type == T_F16 ? gemm_f16_moe_tile_tokens() : (kq ? gemm_kq_moe_tile_tokens() : gemm_blk32_moe_tile_tokens());
+        const int bn = type == T_F16 ? gemm_f16_moe_tile_tokens() : (kq ? gemm_kq_moe_tile_tokens(type, N, n_as, pairs, lim.compute_units) : gemm_blk32_moe_tile_tokens());
         if (hipError_t e = launch_moe_group(ids, ids_stride, n_used, pairs, n_as, bn, offsets, perm, tiles, st); e != hipSuccess)
             return (int)e;
-        const RowGather rg{perm, offsets, tiles, (int32_t)n_used, (int32_t)ne11, nb02, (size_t)N * nb01 > ((size_t)4 << 20)};
+        const RowGather rg{perm, offsets, tiles, (int32_t)n_used, (int32_t)ne11, nb02, (size_t)N * nb01 > ((size_t)4 << 20), bn};
         // the grid provides a slot for every token tile the list can have; slots past its length exit at once
         const int64_t slots = pairs / bn + n_as;
         if (type == T_F16) return hip_rc(launch_gemm_f16(W, nb01, K, N, workspace, stride, pairs, y, ldy, lim, st, &rg, slots));

@@ -2,12 +2,12 @@
 // lm_ggml_vec_dot_q2_K_q8_K .. _q6_K_q8_K, _iq4_xs_q8_K (reference ggml-cpu/ggml-cpu-quants.c) as driven by
 // lm_ggml_compute_forward_mul_mat (ggml-cpu/ggml-cpu.c:1257-1449).
 //
-// This file holds the choice of the kernel and the staging kernel, which runs Q6_K and Q3_K where there is a tile for at most every CU;
+// This file holds the choice of the kernel and the staging kernel, which runs Q6_K, Q3_K and IQ4_XS where there is a tile for at most every CU;
 // gemm_kr_kernel (gemm_kquant_rows.hip) runs everything else.
 //
 // Per 256-value super-block the reference forms sumi = sum_j sc_j * dot(q_j, a_j) with signed scales per 16 values, and applies d
 // and the activation scale once.  The integer scales are folded into the int8 MFMA operand: Q6_K as the two signed bytes of (q - 32)*sc =
-// 256*hi + lo, sumi = 256*P0 + P1; Q3_K as one plane (4 - q)*sc in -128..124, sumi = -P0.  The planes accumulate in the MFMA's own int32
+// 256*hi + lo, sumi = 256*P0 + P1, as those of code*sc of IQ4_XS; Q3_K as one plane (4 - q)*sc in -128..124, sumi = -P0.  The planes accumulate in the MFMA's own int32
 // accumulator over the 8 k-blocks of a super-block, all sums are exact, and the vector unit works once per super-block and output.
 //
 // Measured for Q6_K with these digits against base-64 digits of the product plus 4064 (16 instead of 10 vector instructions per four weights, and a
@@ -21,6 +21,7 @@
 #include "kernels.h"
 #include "kquant_dev.h"
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <type_traits>
 
@@ -108,6 +109,37 @@ template <> struct KQ<T_Q3_K> {
     __device__ static __forceinline__ int sumi(int p0, int) { return -p0; }
 };
 
+template <> struct KQ<T_IQ4_XS> {
+    static constexpr int BYTES = BYTES_IQ4_XS, NPL = 2;
+    // d | u16 scales_h | scales_l[4] | qs[128]: k-block ib is qs[16 ib ..], low nibbles its first k-half, high nibbles the second.
+    // The two items of a k-block read the same bytes.
+    struct Raw { u32x4 q[2][2]; u32x2 h; uint32_t d; };
+    __device__ static __forceinline__ void fetch(Raw &r, const uint8_t *blk, int x) {
+        const int p = x >> 1;
+        r.h = *reinterpret_cast<const u32x2 *>(blk);
+        r.d = r.h.x & 0xffffu;
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int c = 0; c < 2; c++) r.q[h][c] = *reinterpret_cast<const u32x4_a4 *>(blk + 8 + 16 * (4 * h + p + 2 * c));
+    }
+    __device__ static __forceinline__ void expand(u32x4 (&cell)[NPL][2], const Raw &r, int h, int x) {
+        const int p = x >> 1, hf = x & 1;
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const int ls = iq4_xs_scale(r.h, 4 * h + p + 2 * c);
+            const uint32_t mul = splat16((uint32_t)ls), add = splat16((uint32_t)(128 - 128 * ls));
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                uint32_t hi, lo;
+                byte_digits(iq4_codes((r.q[h][c][i] >> (4 * hf)) & 0x0f0f0f0fu), 0x00ff00ffu, mul, add, hi, lo);
+                cell[0][c][i] = hi; cell[1][c][i] = lo;
+            }
+        }
+    }
+    __device__ static __forceinline__ int sumi(int p0, int p1) { return (p0 << 8) + p1; }
+};
+
 constexpr int KQ_PRODUCERS = 4;               // staging waves per workgroup, one per SIMD
 
 template <int WT, int WR, int WC>
@@ -153,10 +185,10 @@ struct KqCfg {
 // The two kinds of wave run side by side on every SIMD, so operand expansion (vector pipe, LDS writes, memory
 // latency) overlaps the matrix pipe by construction instead of by instruction scheduling.  Nothing in the loops is
 // conditional: loads past the last stage repeat it, and stores that do not apply go to a per-thread dump slot.
-template <int WT, int WR, int WC, int OCC>
+template <int WT, int WR, int WC, int OCC, bool GATHER>
 __global__ __launch_bounds__((WR * WC + KQ_PRODUCERS) * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 void gemm_kq_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64_t N, const uint8_t *__restrict__ ws,
-                    size_t ws_stride, int64_t M, float *__restrict__ y, int64_t ldy, TileMap map, int slice_sb) {
+                    size_t ws_stride, int64_t M, float *__restrict__ y, int64_t ldy, TileMap map, RowGather rg, int slice_sb) {
     using T = KQ<WT>;
     using C = KqCfg<WT, WR, WC>;
     constexpr int TN = KQ_TN;
@@ -166,15 +198,25 @@ void gemm_kq_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64
     // split K: grid row s takes super-blocks sb0 .. of every row
     // and writes its partial tile to slice s of y
     int sb0 = 0, nstages = (int)(K / QK_K) * 2;
-    if (slice_sb > 0) {
+    if (!GATHER && slice_sb > 0) {
         sb0 = (int)blockIdx.y * slice_sb;
         nstages = 2 * min(slice_sb, (int)(K / QK_K) - sb0);
         y += (size_t)blockIdx.y * (size_t)M * (size_t)ldy;
     }
-    const TileCoord tc = xcd_tile(blockIdx.x, map);
-    if (tc.row_tile >= map.row_tiles || tc.tok_tile >= map.tok_tiles) return;        // padding of the tile map
+    TileCoord tc;
+    int32_t entry = 0;
+    if constexpr (GATHER) {
+        if (!gather_tile<C::BN>(rg, map, entry, tc.row_tile)) return;
+        tc.tok_tile = 0;
+    } else {
+        tc = xcd_tile(blockIdx.x, map);
+        if (tc.row_tile >= map.row_tiles || tc.tok_tile >= map.tok_tiles) return;    // padding of the tile map
+    }
+    size_t w_offset;
+    const GatherView gv = resolve_gather<GATHER>(rg, entry, w_offset, M);
+    W += w_offset;
     const int64_t row_base = (int64_t)tc.row_tile * C::BM;
-    const int64_t tok_base = (int64_t)tc.tok_tile * C::BN;
+    const int64_t tok_base = (int64_t)(GATHER ? gv.tok_tile : tc.tok_tile) * C::BN;
     if (tok_base >= M) return;
 
     if (wave >= C::NC) {
@@ -195,9 +237,9 @@ void gemm_kq_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64
         for (int i = 0; i < C::W_PER_T; i++) wsrc[i] = W + (size_t)min(row_base + ((pt + i * C::NPT) >> 2), N - 1) * nb01;
 #pragma unroll
         for (int i = 0; i < C::X_PER_T; i++)
-            xsrc[i] = ws + (size_t)min(tok_base + ((pt + i * C::NPT) >> 3), M - 1) * ws_stride + 16 * ((pt + i * C::NPT) & 7);
+            xsrc[i] = ws + (size_t)gv.act_row(min(tok_base + ((pt + i * C::NPT) >> 3), M - 1)) * ws_stride + 16 * ((pt + i * C::NPT) & 7);
         // activation scale: thread t < BN for token t
-        const uint8_t *ssrc = ws + (size_t)min(tok_base + min(pt, C::BN - 1), M - 1) * ws_stride;
+        const uint8_t *ssrc = ws + (size_t)gv.act_row(min(tok_base + min(pt, C::BN - 1), M - 1)) * ws_stride;
         const int nsb = nstages >> 1;
 
         auto fetch_w = [&](Wts &R, int sb_wanted) {
@@ -354,10 +396,11 @@ void gemm_kq_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64
     for (int c = 0; c < TN; c++) {
         const int64_t tok = tok_base + n0 + c * 32 + l32;
         if (tok >= M) continue;
+        const int64_t orow = gv.out_row(tok);
 #pragma unroll
         for (int g = 0; g < 4; g++) {
             const int64_t row = row_base + r0 + 8 * g + 4 * half;
-            float *dst = y + (size_t)tok * ldy + row;
+            float *dst = y + (size_t)orow * ldy + row;
             if (row + 3 < N && (((uintptr_t)dst) & 15) == 0) {
                 *reinterpret_cast<float4 *>(dst) = make_float4(out[c][4 * g], out[c][4 * g + 1], out[c][4 * g + 2], out[c][4 * g + 3]);
             } else {
@@ -381,18 +424,13 @@ static int kq_slices_for(int64_t K, int64_t N, int64_t M, int64_t cus) {
     const int64_t per = ceil_div(units, s);
     return (int)ceil_div(units, per);                                   // no empty slice
 }
-// Q6_K and Q3_K with at most a 128 x 64 tile for every CU: gemm_kq_kernel, whose staging waves expand a weight once for 128 tokens (us,
-// staged / gemm_kr_kernel: Q6_K 14336 values x 4096 rows at 512 tokens 113 / 128, 201 tokens 66 / 74, 4096 x 4096 at 512 tokens 38.6 / 44; Q3_K
-// 14336 x 4096 at 201 tokens 49 / 53) - unless half of its 128-token tile would be empty and the slices give gemm_kr_kernel a workgroup for
-// every CU (32 tokens: Q6_K 41 / 27, Q3_K 30 / 20).
-static bool kq_staged(int wtype, int64_t K, int64_t N, int64_t M, int64_t cus) {
-    const int64_t tiles = ceil_div(N, (int64_t)128) * ceil_div(M, (int64_t)64);
-    if ((wtype != T_Q6_K && wtype != T_Q3_K) || tiles > cus) return false;
-    return M > 64 || tiles * kq_slices_for(K, N, M, cus) < cus;
-}
-// How gemm_kr_kernel covers a product: k groups of a workgroup (1: four waves that walk the super-blocks in order, two workgroups a CU; 2: eight
-// waves, four on the even and four on the odd super-blocks, one workgroup a CU) and slices of K.  Q3_K .. Q6_K run in one group and the
-// slices above.  Q2_K and IQ4_XS by their number of 128 x 64 tiles:
+// How a product is covered: the staging kernel (groups 0), or gemm_kr_kernel in one or two k groups a workgroup (1: four waves that walk the
+// super-blocks in order, two workgroups a CU; 2: eight waves, four on the even and four on the odd super-blocks, one workgroup a CU); and slices of K.
+// Q3_K .. Q6_K run in the slices above and in one group - or, Q6_K and Q3_K with at most a 128 x 64 tile for every CU, in the staging kernel,
+// which expands a weight once for 128 tokens (us, staged / gemm_kr_kernel: Q6_K 14336 values x 4096 rows at 512 tokens 113 / 128, 201 tokens 66 / 74,
+// 4096 x 4096 at 512 tokens 38.6 / 44; Q3_K 14336 x 4096 at 201 tokens 49 / 53), unless half of its 128-token tile would be empty and the slices
+// give gemm_kr_kernel a workgroup for every CU (32 tokens: Q6_K 41 / 27, Q3_K 30 / 20).
+// Q2_K and IQ4_XS by their number of 128 x 64 tiles:
 //   more tiles than CUs     one group (us, 512 tokens x 4096 values x 4608 rows, one / two groups: Q2_K 36 / 44, IQ4_XS 66 / 72)
 //   above half as many      two groups, so that every SIMD has two waves (4096 rows: Q2_K 29 / 27, IQ4_XS 45 / 42); so too with 2 slices of
 //                           rows above 8192 values (14336 values x 4096 rows at 201 tokens: Q2_K 47 / 42, IQ4_XS 75 / 68)
@@ -401,17 +439,25 @@ static bool kq_staged(int wtype, int64_t K, int64_t N, int64_t M, int64_t cus) {
 //                           rounded up: 96 tiles in 3 slices leave 32 workgroups for a second turn (IQ4_XS 4096 x 4096 at 130 tokens 29 / 31 us
 //                           in 2 / 3).  The slice sum pays for at most 150000 partial outputs a super-block of a row (IQ4_XS 1792 values x
 //                           4096 rows at 64 tokens 21.7 / 16.4 whole / in 4), not for rows of three or less or for two slices of less than 8.
-struct KrPlan { int groups, slices; };
-static KrPlan kr_plan(int wtype, int64_t K, int64_t N, int64_t M, int64_t cus) {
-    if (wtype != T_Q2_K && wtype != T_IQ4_XS) return KrPlan{1, kq_slices_for(K, N, M, cus)};
+//   IQ4_XS, 5 to 11 super-blocks in one or two slices, up to 128 tokens: the staging kernel (us, staged / gemm_kr_kernel: 2304 values x
+//                           8192 rows at 93 tokens 21.5 / 25.9, 1280 x 8192 at 64 16.3 / 19.0; 2560 x 15500 at 127 31.3 / 29.4)
+struct KqPlan { int groups, slices; };
+static KqPlan kq_plan(int wtype, int64_t K, int64_t N, int64_t M, int64_t cus) {
     const int64_t tiles = ceil_div(N, (int64_t)128) * ceil_div(M, (int64_t)64), units = K / QK_K;
-    if (tiles > cus || units == 1) return KrPlan{1, 1};
+    if (wtype != T_Q2_K && wtype != T_IQ4_XS) {
+        const int slices = kq_slices_for(K, N, M, cus);
+        const bool staged = (wtype == T_Q6_K || wtype == T_Q3_K) && tiles <= cus && (M > 64 || tiles * slices < cus);
+        return KqPlan{staged ? 0 : 1, slices};
+    }
+    if (tiles > cus || units == 1) return KqPlan{1, 1};
     const int64_t most = std::max<int64_t>(8, std::min<int64_t>(16, units / 4));
     int64_t s = units < 4 ? 1 : std::min({cus / tiles, units, most, units * 150000 / (M * N)});
-    if (s < (units < 8 ? 3 : 2)) return KrPlan{units < 4 ? 1 : 2, 1};
+    if (s < (units < 8 ? 3 : 2)) s = 1;
+    if (wtype == T_IQ4_XS && s <= 2 && units >= 5 && units < 12 && M > (units < 8 ? 32 : 64) && M <= 128 && M * N <= 1400000) return KqPlan{0, kq_slices_for(K, N, M, cus)};
+    if (s == 1) return KqPlan{units < 4 ? 1 : 2, 1};
     const int64_t per = ceil_div(units, s);
     s = ceil_div(units, per);                                           // no empty slice
-    return KrPlan{s == 2 && units > 32 ? 2 : 1, (int)s};
+    return KqPlan{s == 2 && units > 32 ? 2 : 1, (int)s};
 }
 
 // With few tokens the GEMM's time is its walk over K, whatever the token count, while the GEMV forms pass over the weights once
@@ -462,27 +508,50 @@ bool gemm_kq_supported(int wtype, int64_t K, int64_t N, int64_t n, bool can_spli
 int gemm_kq_slices(int wtype, int64_t K, int64_t N, int64_t n, int compute_units) {
     const int64_t cus = compute_units > 0 ? compute_units : 256;
     if (!gemm_kq_supported(wtype, K, N, n, true)) return 1;
-    return kr_plan(wtype, K, N, n, cus).slices;
+    return kq_plan(wtype, K, N, n, cus).slices;
 }
 
-template <int WT>
+using KqTile = KqCfg<T_Q6_K, 2, 2>;                                          // 64 x 128, 4 + 4 waves
+template <int WT, bool GATHER>
 static hipError_t launch_kq(const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, int64_t M,
-                            float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st, int slices, float *part) {
-    using C = KqCfg<WT, 2, 2>;                                               // 64 x 128, 4 + 4 waves
+                            float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t slots, int slices, float *part) {
+    using C = KqCfg<WT, 2, 2>;
     const size_t lds_bytes = C::TOTAL;
     if ((int64_t)lds_bytes > lim.max_lds_per_block) return hipErrorInvalidValue;
-    auto kfn = gemm_kq_kernel<WT, 2, 2, 2>;
+    auto kfn = gemm_kq_kernel<WT, 2, 2, 2, GATHER>;
     static LdsGrant grant;
     if (hipError_t e = grant_dynamic_lds(kfn, lds_bytes, lim, grant); e != hipSuccess) return e;
-    const TileMap map = make_tile_map(ceil_div(N, C::BM), ceil_div(M, C::BN), 32);      // 32 workgroups run on an XCD at a time
+    const TileMap map = make_tile_map(ceil_div(N, C::BM), GATHER ? 1 : ceil_div(M, C::BN), 32);     // 32 workgroups run on an XCD at a time
     const int slice_sb = slices > 1 ? (int)ceil_div(K / QK_K, (int64_t)slices) : 0;
-    hipLaunchKernelGGL(kfn, dim3(map.grid, (unsigned)slices), dim3(C::NT), lds_bytes, st, (const uint8_t *)W, nb01, K, N,
-                       (const uint8_t *)ws, ws_stride, M, slices > 1 ? part : y, slices > 1 ? N : ldy, map, slice_sb);
+    hipLaunchKernelGGL(kfn, GATHER ? gather_grid(map, slots, C::NT) : dim3(map.grid, (unsigned)slices), dim3(C::NT), lds_bytes, st, (const uint8_t *)W,
+                       nb01, K, N, (const uint8_t *)ws, ws_stride, M, slices > 1 ? part : y, slices > 1 ? N : ldy, map, rg, slice_sb);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     return slices > 1 ? launch_sum_slices(part, slices, M, N, y, ldy, st) : hipSuccess;
 }
 
-int gemm_kq_moe_tile_tokens() { return gemm_kr_tile_tokens(); }
+template <bool GATHER>
+static hipError_t launch_staged_type(int wtype, const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, int64_t M, float *y,
+                                     int64_t ldy, const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t slots, int slices, float *part) {
+    switch (wtype) {
+        case T_Q6_K: return launch_kq<T_Q6_K, GATHER>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, slices, part);
+        case T_Q3_K: return launch_kq<T_Q3_K, GATHER>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, slices, part);
+        case T_IQ4_XS: return launch_kq<T_IQ4_XS, GATHER>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, slots, slices, part);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+// Expert groups of these types with at most a tile for every CU: the staging kernel here too (us, staged / gemm_kr_kernel: Q6_K 13824
+// values x 2928 rows, 2 experts, 144 pairs 97 / 122, 1280 x 800, 4 experts, 232 pairs 19.4 / 22.9; Q3_K 8960 x 280, 2 experts, 242 pairs 52.7 / 55.9;
+// IQ4_XS 7936 x 1384, 4 experts, 396 pairs 65 / 76), whose tiles are 64 rows by 128 pairs.
+// The number of tiles is known on the device only; ids drawn evenly pick n_as * (1 - e^(-pairs / n_as)) experts.
+static bool kq_staged_groups(int wtype, int64_t N, int64_t n_as, int64_t pairs, int64_t cus) {
+    if (wtype != T_Q6_K && wtype != T_Q3_K && wtype != T_IQ4_XS) return false;
+    const float experts = (float)n_as, picked = experts * (1.f - std::exp(-(float)pairs / experts));
+    return (picked + (float)pairs / (float)KqTile::BN) * (float)ceil_div(N, (int64_t)KqTile::BM) <= (float)cus;
+}
+int gemm_kq_moe_tile_tokens(int wtype, int64_t N, int64_t n_as, int64_t pairs, int compute_units) {
+    return kq_staged_groups(wtype, N, n_as, pairs, compute_units > 0 ? compute_units : 256) ? KqTile::BN : gemm_kr_tile_tokens();
+}
 
 hipError_t launch_gemm_kq(int wtype, const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride,
                           int64_t M, float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st, const RowGather *rgp, int64_t n_as,
@@ -491,16 +560,15 @@ hipError_t launch_gemm_kq(int wtype, const void *W, size_t nb01, int64_t K, int6
     if (!gemm_kq_type(wtype)) return hipErrorInvalidValue;
     const RowGather rg = rgp ? *rgp : RowGather{nullptr, nullptr, nullptr, 1, 1, 0};
     const GemmMats mats = one_gemm_mat(W, nb01, N, y, ldy);
-    if (rg.perm) return launch_gemm_kr(1, wtype, mats, K, ws, ws_stride, M, lim, st, rg, n_as, 1, nullptr);
     const int64_t cus = lim.compute_units > 0 ? lim.compute_units : 256;
+    if (rg.perm && rg.tile_tokens == KqTile::BN) return launch_staged_type<true>(wtype, W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as, 1, nullptr);
+    if (rg.perm) return launch_gemm_kr(1, wtype, mats, K, ws, ws_stride, M, lim, st, rg, n_as, 1, nullptr);
     auto room = [&](int slices) {
         return slices <= 1 || (split.part && split.bytes >= (size_t)slices * (size_t)M * (size_t)N * sizeof(float) && (((uintptr_t)split.part) & 15) == 0);
     };
-    KrPlan p = kr_plan(wtype, K, N, M, cus);
-    if (!room(p.slices)) p = KrPlan{2, 1};
-    if (kq_staged(wtype, K, N, M, cus))
-        return wtype == T_Q6_K ? launch_kq<T_Q6_K>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, p.slices, split.part)
-                               : launch_kq<T_Q3_K>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, p.slices, split.part);
+    KqPlan p = kq_plan(wtype, K, N, M, cus);
+    if (!room(p.slices)) p = KqPlan{p.groups > 0 && (wtype == T_Q2_K || wtype == T_IQ4_XS) ? 2 : p.groups, 1};
+    if (p.groups == 0) return launch_staged_type<false>(wtype, W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, 0, p.slices, split.part);
     return launch_gemm_kr(p.groups, wtype, mats, K, ws, ws_stride, M, lim, st, rg, n_as, p.slices, split.part);
 }
 
@@ -512,8 +580,8 @@ bool gemm_kq_group_applicable(int wtype, int64_t K, const GemmMats &mats, int64_
     if (mats.count < 2 || !gemm_kq_type(wtype)) return false;
     for (int i = 0; i < mats.count; i++) {
         const int64_t N = mats.m[i].N;
-        const KrPlan p = kr_plan(wtype, K, N, n, cus);
-        if (!gemm_kq_supported(wtype, K, N, n, false) || p.slices != 1 || p.groups != 1 || kq_staged(wtype, K, N, n, cus)) return false;
+        const KqPlan p = kq_plan(wtype, K, N, n, cus);
+        if (!gemm_kq_supported(wtype, K, N, n, false) || p.slices != 1 || p.groups != 1) return false;
         if (gemm_kr_rows_in_reach(mats.m[i].nb01) < 32) return false;
     }
     return true;

@@ -283,14 +283,6 @@ template <> struct KR<T_IQ4_XS> {
     __device__ static __forceinline__ Hdr hdr(const u32x4 *row, int) { return Hdr{*reinterpret_cast<const u32x2 *>(row)}; }
     static constexpr int KA(int q) { return 2 * q; }
     static constexpr int KB(int q) { return 2 * q + 1; }
-    // four code indices (one per byte) -> code point + 128 of kvalues_iq4nl (reference ggml-common.h), 1..241
-    __device__ static __forceinline__ uint32_t lookup4(uint32_t idx) {
-        constexpr uint32_t F = 0x80808080u, T0 = 0xbfad9881u ^ F, T1 = 0xf6eaddcfu ^ F, T2 = 0x26190d01u ^ F, T3 = 0x71594535u ^ F;
-        const uint32_t sel = idx & 0x07070707u;
-        const uint32_t lo = __builtin_amdgcn_perm(T1, T0, sel), hi = __builtin_amdgcn_perm(T3, T2, sel);
-        const uint32_t m = ((idx >> 3) & 0x01010101u) * 0xffu;
-        return (lo & ~m) | (hi & m);
-    }
     struct Raw { u32x2 q[4]; };
     template <int Q> __device__ static __forceinline__ Raw load(const u32x4 *row, int) {
         Raw r;
@@ -306,14 +298,13 @@ template <> struct KR<T_IQ4_XS> {
 #pragma unroll
         for (int e = 0; e < 2; e++) {
             const int ib = 2 * Q + e;
-            const uint32_t nib = (h.h.y >> (4 * ib)) & 15u, top = (h.h.x >> (16 + 2 * ib)) & 3u;
-            const int ls = (int)(nib | (top << 4)) - 32;
+            const int ls = iq4_xs_scale(h.h, ib);
             const uint32_t mul = splat16((uint32_t)ls), add = splat16((uint32_t)(128 - 128 * ls));
             const uint32_t w[4] = {r.q[2 * e].x, r.q[2 * e].y, r.q[2 * e + 1].x, r.q[2 * e + 1].y};
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 uint32_t hi, lo;
-                byte_digits(lookup4((w[i] >> (4 * hf)) & 0x0f0f0f0fu), 0x00ff00ffu, mul, add, hi, lo);
+                byte_digits(iq4_codes((w[i] >> (4 * hf)) & 0x0f0f0f0fu), 0x00ff00ffu, mul, add, hi, lo);
                 c[e][0][i] = hi; c[e][1][i] = lo;
             }
         }

@@ -131,6 +131,7 @@ struct RowGather {
     int32_t n_used, ne11;
     size_t nb02;
     bool columns;                              // an expert's token tiles in columns (gather_tile)
+    int32_t tile_tokens;                       // what the list was built for
 };
 struct GatherView {                // resolved once per workgroup
     const int32_t *list;           // this expert's pairs, or nullptr
@@ -422,7 +423,7 @@ bool       moe_gemm_ahead(int wtype, int64_t K, int64_t N, int64_t n_as, int64_t
 hipError_t launch_moe_group(const int32_t *ids, int64_t ids_stride, int64_t n_used, int64_t pairs, int64_t n_as,
                             int tile_tokens, int32_t *offsets, int32_t *perm, int32_t *tiles, hipStream_t st);
 int        gemm_blk32_moe_tile_tokens();
-int        gemm_kq_moe_tile_tokens();
+int        gemm_kq_moe_tile_tokens(int wtype, int64_t N, int64_t n_as, int64_t pairs, int compute_units);
 int        gemm_f16_moe_tile_tokens();
 
 }  // namespace chip

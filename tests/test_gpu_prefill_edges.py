@@ -57,10 +57,10 @@ def random_rows(wt, rng, N, nsb):
 
 
 # (K, N, n): one super-block; ragged tiles; K split over workgroups with uneven slices; the GEMV passes that 9 tokens take on few
-# short rows; 128 x 128 tiles; many tokens, few rows; the GEMM at the fewest tokens it is taken from
+# short rows; 128 x 128 tiles; many tokens, few rows; the GEMM at the fewest tokens it is taken from; the staging kernel
 @pytest.mark.parametrize("wt", LOW_BIT, ids=lambda t: O.TYPE_NAMES[t])
 @pytest.mark.parametrize("K,N,n", [(256, 5, 41), (1024, 131, 65), (2304, 131, 70), (4096, 300, 9), (512, 4100, 1030), (768, 33, 1100),
-                                   (14336, 70, 9)])
+                                   (14336, 70, 9), (2304, 8200, 70), (1280, 8100, 33)])
 def test_low_bit_kquant_gemm(dev, orc, wt, K, N, n):
     rng = np.random.default_rng(K + N + wt)
     w = random_rows(wt, rng, N, K // 256)
@@ -239,6 +239,20 @@ def test_expert_groups(dev, orc, wt, counts, n_used):
     experts = np.stack([orc.quantize_weights(wt, common.weights_f32(wt + e, N, K)) for e in range(len(counts))])
     x = common.activations_f32(wt, n_tokens, K).reshape(n_tokens, 1, K)
     check(dev.mul_mat_id(wt, experts, x, ids), orc.mul_mat_id(wt, experts, x, ids, want=("sum_abs",)), "expert groups")
+
+
+# Few tiles of these types run in the staging kernel (64 rows x 128 pairs), the same rows inside a large matrix in the other one
+@pytest.mark.parametrize("wt", (O.Q6_K, O.Q3_K, O.IQ4_XS), ids=lambda t: O.TYPE_NAMES[t])
+def test_staged_expert_groups_equal_the_row_kernel(dev, orc, wt):
+    K, N, counts = 768, 70, (1, 64, 0, 65, 128, 129, 300)
+    rng = np.random.default_rng(wt)
+    w = np.stack([orc.quantize_weights(wt, common.weights_f32(wt + e, N, K)) for e in range(len(counts))])
+    ids = rng.permutation(np.repeat(np.arange(len(counts)), counts)).astype(np.int32).reshape(-1, 1)
+    x = common.activations_f32(wt, ids.shape[0], K)[:, None]
+    y = dev.mul_mat_id(wt, w, x, ids)
+    check(y, orc.mul_mat_id(wt, w, x, ids, want=("sum_abs",)), "staged groups")
+    large = np.concatenate([np.tile(w, (1, 70, 1)), w], axis=1)
+    assert np.ascontiguousarray(dev.mul_mat_id(wt, large, x, ids)[:, :, -N:]).tobytes() == y.tobytes()
 
 
 # An expert larger than an XCD's L2 has its token tiles in columns of 8: one short tile, a column and one tile, two columns and a short one, none
