@@ -812,7 +812,7 @@ int chip_mul_mat_id(int type, const void *W, size_t nb01, size_t nb02, int64_t K
     hipStream_t st = (hipStream_t)stream;
 
     const bool kq = gemm_kq_type(type);
-    if (moe_group_supported(n_as, pairs) && moe_gemm_ahead(type, K, N, n_as, pairs)) {
+    if (moe_group_supported(n_as, pairs) && moe_gemm_ahead(type, K, N, chip_row_size(type, K), n_as, pairs)) {
         rc = chip_mul_mat_prepare(type, K, x, ldx, rows, workspace, workspace_bytes, stream);
         if (rc) return rc;
         int32_t *offsets = reinterpret_cast<int32_t *>((uint8_t *)workspace + moe_rows_bytes(type, K, rows));

@@ -419,7 +419,7 @@ hipError_t launch_rope(const float *x, const int32_t *pos, const float *freq_fac
 // moe_group.hip: counting sort of MUL_MAT_ID's (token, slot) pairs by expert into offsets[n_as + 1] / perm[pairs].
 // tiles[0] = number of token tiles, tiles[1 + i] = expert | tile << 12 for tiles of `tile_tokens` pairs.
 bool       moe_group_supported(int64_t n_as, int64_t pairs);
-bool       moe_gemm_ahead(int wtype, int64_t K, int64_t N, int64_t n_as, int64_t pairs);      // the GEMM by expert groups against a GEMV per pair
+bool       moe_gemm_ahead(int wtype, int64_t K, int64_t N, size_t row_bytes, int64_t n_as, int64_t pairs);      // the GEMM by expert groups against a GEMV per pair
 hipError_t launch_moe_group(const int32_t *ids, int64_t ids_stride, int64_t n_used, int64_t pairs, int64_t n_as,
                             int tile_tokens, int32_t *offsets, int32_t *perm, int32_t *tiles, hipStream_t st);
 int        gemm_blk32_moe_tile_tokens();

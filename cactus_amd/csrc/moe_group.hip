@@ -4,6 +4,7 @@
 // (atomic cursors); no output depends on it, since every output row is computed on its own.
 #include "dev_common.h"
 #include "kernels.h"
+#include <algorithm>
 #include <cmath>
 
 namespace chip {
@@ -111,22 +112,27 @@ hipError_t launch_moe_group(const int32_t *ids, int64_t ids_stride, int64_t n_us
 }
 
 // MUL_MAT_ID: the pairs grouped by expert and run through the GEMM of the weight type, or a GEMV per pair?  Both times estimated in us, with
-// terms fitted to 40 measured products of each type (6 to 520 pairs, 8 to 128 experts, 512 to 14336 values, at most 0.5 GB of experts; one in ten
-// off by more than 10 to 20 per cent):
-//   GEMV   a pair costs its rows by the 4096 values of one of them; that pairs share an expert buys nothing
+// terms fitted to 40 measured products of each type and checked against 14500 others (16 to 4095 pairs, 2 to 400 experts, 256 to 14336 values, at most 1 GB
+// of experts that no cache holds):
+//   GEMV   a pair costs its rows by the 4096 values of one of them; that pairs share an expert buys nothing.  From 64 pairs on not faster than
+//          8 TB/s, which large experts come to (Q8_0 3072 values x 1024 rows, 32 experts, 156 pairs 69, 42 without this term; GEMM 38); fewer
+//          pairs share the caches (Q8_0 2048 x 3584, 8 experts, 32 pairs 29, 38 with it)
 //   GEMM   quantizer, grouping and launch, a walk over K, and the tiles by the 512 that the chip runs at a time.  With ids drawn evenly
 //          n_as * (1 - e^(-pairs / n_as)) experts are picked, and a single pair has its row tiles walked whole
+// Where both are close the choice is the one on the safer side of the estimates (nine in ten within 20 per cent, the worst 40 to 80): the GEMV below 64
+// pairs and for Q2_K, Q3_K and IQ4_XS, else the GEMM.
 // (us, GEMV / GEMM: Q4_K 2048 values x 768 rows, 128 experts, 64 pairs 17 / 26, 128 pairs 28.5 / 28.2; 768 x 2048 64 pairs 34 / 24; 4096 x
-// 14336, 8 experts, 16 pairs 63 / 70, 32 pairs 105 / 69; Q8_0 2048 x 768, 128 experts, 256 pairs 46 / 54; 14336 x 4096, 8 experts, 32 pairs
-// 198 / 135.  A limit of 64 pairs for all was 18 per cent above the better of the two on average for Q4_K, this is 0.4; the worst of all
-// 500 products 34 per cent.)  F16 stays with the limit: its GEMV's time is that of the experts' bytes, which the terms do not hold.
-bool moe_gemm_ahead(int wtype, int64_t K, int64_t N, int64_t n_as, int64_t pairs) {
+// 14336, 8 experts, 16 pairs 63 / 70, 32 pairs 105 / 69; Q4_0 2560 x 12214, 12 experts, 32 pairs 71 / 96; Q8_0 1024 x 3676, 28 experts, 32 pairs
+// 30 / 45.  Of the 14500 calls 3 per cent take the slower one by more than 5 per cent, and 7 calls by 5 to 15 per cent where the line at 64 pairs
+// takes the faster; that line takes the slower one by more than 5 per cent in 15 per cent of them.)  F16 stays with the line: its GEMV's time is that of the experts' bytes.
+bool moe_gemm_ahead(int wtype, int64_t K, int64_t N, size_t row_bytes, int64_t n_as, int64_t pairs) {
     const int64_t forced = tune("CHIP_MOE_MIN", 0);
     if (forced > 0) return pairs >= forced;
     if (wtype == T_F16 || gemv_max_tokens(wtype, K, DeviceLimits{256, 160 * 1024}) < 1) return pairs >= MOE_FEW_PAIRS;
     if (pairs < 16 || pairs >= 4096) return pairs >= 16;
     if (pairs < MOE_FEW_PAIRS && (wtype == T_Q4_1 || wtype == T_Q5_1)) return false;    // one chain of additions, twice as far off as the GEMV's lanes
     struct { float pair, walk, turn, ends; } c;                         // pair: per 1024 rows x 4096 values; the others per super-block, per tile
+    const bool low_bit = wtype == T_Q3_K || wtype == T_Q2_K || wtype == T_IQ4_XS;
     switch (wtype) {
         case T_Q4_K:   c = {0.235f, 0.92f, 1.25f, 3.5f}; break;
         case T_Q5_K:   c = {0.365f, 1.10f, 1.50f, 4.0f}; break;
@@ -142,9 +148,12 @@ bool moe_gemm_ahead(int wtype, int64_t K, int64_t N, int64_t n_as, int64_t pairs
         default:       c = {0.380f, 1.07f, 1.05f, 2.1f};                // IQ4_NL
     }
     const float n_pairs = (float)pairs, experts = (float)n_as, units = (float)K / 256.f;
-    const float gemv = 6.5f + c.pair * n_pairs * (float)N / 1024.f * (float)ceil_div(K, (int64_t)4096);
+    const float pair_bytes = (float)N * (float)row_bytes;
+    const bool few = pairs < MOE_FEW_PAIRS;
+    const float gemv = 6.5f + n_pairs * std::max(c.pair * (float)N / 1024.f * (float)ceil_div(K, (int64_t)4096), few ? 0.f : pair_bytes / 8e6f);
     const float tiles = (experts * (1.f - std::exp(-n_pairs / experts)) + n_pairs / 64.f) * (float)ceil_div(N, (int64_t)(gemm_kq_type(wtype) ? 128 : 64));
-    return 10.f + c.walk * units + tiles / 512.f * (c.turn * units + c.ends) < gemv;
+    const float gemm = 10.f + c.walk * units + tiles / 512.f * (c.turn * units + c.ends);
+    return gemm * (few ? 1.15f : low_bit ? 1.05f : 0.95f) < gemv;
 }
 
 }  // namespace chip

@@ -32,6 +32,37 @@ def launches(dev, call):
     return count.value
 
 
+def mul_mat_id_launches(dev, wt, K, N, n_as, n_used, n_tokens):
+    """Of an expert matmul: 3 (quantizer, grouping, GEMM) where its pairs are grouped, fewer where each is a GEMV."""
+    L, row = dev.lib, dev.row_size(wt, K)
+    rng = np.random.default_rng(K + N)
+    dW = dev.alloc(n_as * N * row)
+    dev.check(L.chip_memset(dW.ptr, 0, n_as * N * row, None))
+    dx = dev.to_device(common.activations_f32(K, n_tokens, K))
+    ids = dev.to_device(np.stack([rng.permutation(n_as)[:n_used] for _ in range(n_tokens)]).astype(np.int32))
+    dy = dev.alloc(n_tokens * n_used * N * 4)
+    wsz = L.chip_mul_mat_id_workspace_size(wt, K, n_as, n_used, n_tokens, 1)
+    ws = dev.alloc(wsz)
+    return launches(dev, lambda st: L.chip_mul_mat_id(wt, dW.ptr, row, N * row, K, N, n_as, dx.ptr, K, 1, ids.ptr, n_used, n_used, n_tokens,
+                                                      dy.ptr, N, ws.ptr, wsz, st))
+
+
+def group_launches(dev, members, K, n):
+    """Of chip_mul_mat_group over members [(type, rows), ...]."""
+    import cactus_amd as ca
+    L = dev.lib
+    arr, keep, wsz = (ca.Mat * len(members))(), [dev.to_device(common.activations_f32(K, n, K))], 0
+    for i, (wt, N) in enumerate(members):
+        row = dev.row_size(wt, K)
+        dW, dy = dev.alloc(N * row), dev.alloc(n * N * 4)
+        dev.check(L.chip_memset(dW.ptr, 0, N * row, None))
+        keep += [dW, dy]
+        arr[i] = ca.Mat(wt, dW.ptr, row, N, dy.ptr, N, None, 0)
+        wsz = max(wsz, L.chip_mul_mat_workspace_size_n(wt, K, N, n))
+    ws = dev.alloc(wsz)
+    return launches(dev, lambda st: L.chip_mul_mat_group(arr, len(members), K, keep[0].ptr, K, n, ws.ptr, wsz, st))
+
+
 def mul_mat_launches(dev, wt, W, x, split_k=True):
     n, K = x.shape
     N, L = W.shape[0], dev.lib
@@ -60,17 +91,18 @@ def test_split_k_takes_three_launches_whatever_the_rows(dev, orc, wt, N):
 @pytest.mark.parametrize("K,N,n_as,n_used,n_tokens,gemm", [(2048, 768, 128, 8, 8, False), (1024, 256, 64, 2, 32, False), (2048, 768, 128, 8, 192, True),
                                                            (512, 2048, 32, 4, 100, True), (1024, 256, 8, 8, 40, True), (512, 70, 5, 2, 90, False), (512, 70, 5, 2, 700, True)])
 def test_low_bit_expert_matmul_takes_the_gemm_where_it_is_ahead(dev, wt, K, N, n_as, n_used, n_tokens, gemm):
-    L, row = dev.lib, dev.row_size(wt, K)
-    rng = np.random.default_rng(K + N)
-    dW = dev.alloc(n_as * N * row)
-    dev.check(L.chip_memset(dW.ptr, 0, n_as * N * row, None))
-    dx = dev.to_device(common.activations_f32(K, n_tokens, K))
-    ids = dev.to_device(np.stack([rng.permutation(n_as)[:n_used] for _ in range(n_tokens)]).astype(np.int32))
-    dy = dev.alloc(n_tokens * n_used * N * 4)
-    wsz = L.chip_mul_mat_id_workspace_size(wt, K, n_as, n_used, n_tokens, 1)
-    ws = dev.alloc(wsz)
-    assert launches(dev, lambda st: L.chip_mul_mat_id(wt, dW.ptr, row, N * row, K, N, n_as, dx.ptr, K, 1, ids.ptr, n_used, n_used, n_tokens,
-                                                      dy.ptr, N, ws.ptr, wsz, st)) == (3 if gemm else 2)
+    assert mul_mat_id_launches(dev, wt, K, N, n_as, n_used, n_tokens) == (3 if gemm else 2)
+
+
+# us, GEMV / GEMM: 69 / 38, 172 / 104, 30 / 45, 71 / 96, 23 / 28, 11 / 13, 17 / 26, 105 / 69, 63 / 70, 29 / 36, 26 / 33; F16 below and from 64 pairs on
+@pytest.mark.parametrize("wt,K,N,n_as,n_used,n_tokens,gemm", [
+    (O.Q8_0, 3072, 1024, 32, 4, 39, True), (O.Q8_0, 3584, 768, 128, 2, 225, True), (O.Q8_0, 1024, 3676, 28, 8, 4, False),
+    (O.Q4_0, 2560, 12214, 12, 8, 4, False), (O.Q5_K, 1536, 3328, 32, 8, 2, False), (O.Q4_K, 512, 2048, 8, 4, 4, False),
+    (O.Q4_K, 2048, 768, 128, 8, 8, False), (O.Q4_K, 4096, 14336, 8, 2, 16, True), (O.Q4_K, 4096, 14336, 8, 2, 8, False),
+    (O.Q8_0, 2048, 3584, 8, 4, 8, False), (O.IQ4_XS, 3072, 106, 12, 1, 506, False),
+    (O.F16, 512, 300, 8, 3, 21, False), (O.F16, 512, 300, 8, 4, 16, True)])
+def test_expert_matmul_takes_the_gemm_where_it_is_ahead(dev, wt, K, N, n_as, n_used, n_tokens, gemm):
+    assert (mul_mat_id_launches(dev, wt, K, N, n_as, n_used, n_tokens) == 3) == gemm
 
 
 # long rows with a short last stage, no room to split K: quantizer and six GEMV passes while they are ahead of the GEMM's walk
