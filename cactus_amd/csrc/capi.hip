@@ -388,11 +388,14 @@ static int mmv_min_tokens(int type, int64_t K, int64_t N) {
            : ((type == T_Q4_K || type == T_Q5_K || type == T_Q4_0) && N * K < (32LL << 20)) ? (type == T_Q4_0 ? 8 : 7)
            : (type == T_Q4_K && K > 13312) ? 7 : MMV_MIN_TOKENS;
 }
+// The matrix-core GEMVs reach a tile's 16 rows by 32-bit offsets from the first: rows further apart go through the dot-product GEMV.
+static bool mmv_rows_in_reach(size_t nb01) { return nb01 <= ((size_t)1 << 28); }
 // Two Q4_K / Q5_K matrices of one shape on the same rows at 5..8 tokens (ffn_gate and ffn_up): true when each alone would
 // take one launch of the matrix-core GEMV whatever the workspace size - they then run as one launch in which every
 // workgroup, after its tiles of the first matrix, takes the same tiles of the second (the activation image is built once;
 // every tile is computed as in a launch of its own: the same bits).
-static bool mmv_pair_applicable(int type, int64_t K, int64_t N, int64_t n, const DeviceLimits &lim) {
+static bool mmv_pair_applicable(int type, size_t nb01, int64_t K, int64_t N, int64_t n, const DeviceLimits &lim) {
+    if (!mmv_rows_in_reach(nb01)) return false;
     if (n < 5 || n > 8 || !(type == T_Q4_K || type == T_Q5_K) || tune("CHIP_MMV_PAIR", 1) == 0) return false;
     if (gemm_kq_supported(type, K, N, n, false) || gemm_kq_supported(type, K, N, n, true)) return false;
     return n >= mmv_min_tokens(type, K, N) && n <= mmv_q4k_max_tokens(type, K, N, lim);
@@ -439,7 +442,7 @@ static int mul_mat_run(int type, const void *W, size_t nb01, int64_t K, int64_t 
 
     // 5 tokens or more: integer sums on the matrix cores, up to 16 tokens per pass over the weights
     const int mmv_min = mmv_min_tokens(type, K, N);
-    const int mgroup = (n >= mmv_min) ? mmv_max_tokens(type, K, N, lim) : 0;
+    const int mgroup = (n >= mmv_min && mmv_rows_in_reach(nb01)) ? mmv_max_tokens(type, K, N, lim) : 0;
     if (mgroup > 0) {
         for (int64_t t0 = 0; t0 < n; t0 += mgroup) {
             const int nt = (int)((n - t0 < mgroup) ? n - t0 : mgroup);
@@ -541,7 +544,7 @@ int chip_mul_mat_pair(int type, const void *W1, const void *W2, size_t nb01, int
         return hip_rc(launch_gemv_fused_pair(type, W1, W2, nb01, K, N, x, ldx, (int)n, workspace,
                                              act_stride(chip_vec_dot_type(type), K), y1, y2, ldy, lim, (hipStream_t)stream));
     if (int rc = chip_mul_mat_prepare(type, K, x, ldx, n, workspace, workspace_bytes, stream); rc) return rc;
-    if (mmv_pair_applicable(type, K, N, n, lim))
+    if (mmv_pair_applicable(type, nb01, K, N, n, lim))
         return hip_rc(launch_mmv_q4k(type, W1, nb01, K, N, workspace, act_stride(chip_vec_dot_type(type), K), (int)n, y1, ldy, lim,
                                      (hipStream_t)stream, W2, y2));
     const GroupMat gm[2] = {{type, W1, nb01, N, y1, ldy, nullptr, 0}, {type, W2, nb01, N, y2, ldy, nullptr, 0}};
@@ -724,7 +727,7 @@ static int mul_mat_group(const chip_mat *mats, int count, int64_t K, const float
     if (live == 2) {                                                   // ffn_gate and ffn_up at 5..8 tokens
         const GroupMat &a = gm[0], &b = gm[1];
         const bool twins = a.wtype == b.wtype && a.N == b.N && a.nb01 == b.nb01 && a.ldy == b.ldy && !a.t16 && !b.t16;
-        if (twins && mmv_pair_applicable(a.wtype, K, a.N, n, lim))
+        if (twins && mmv_pair_applicable(a.wtype, a.nb01, K, a.N, n, lim))
             return hip_rc(launch_mmv_q4k(a.wtype, a.W, a.nb01, K, a.N, workspace, stride, (int)n, a.y, a.ldy, lim, st, b.W, b.y));
     }
     if (int rc = run_members(gm, live, K, n, workspace, workspace_bytes, lim, stream); rc) return rc;

@@ -102,11 +102,12 @@ def test_kquant_row_gemm(dev, orc, wt, K, N, n):
 
 
 # Rows so far apart that a tile spans more than 2^32 bytes, and more than 2^32 bytes apart each: (type, stride, rows, tokens).  One whole tile
-# and a ragged one; K split (3584 values at 20 tokens); rows that lie alone
+# and a ragged one; K split (3584 values at 20 tokens); rows that lie alone; 8 to 12 tokens, which the matrix-core GEMVs take of closer rows
 @pytest.mark.parametrize("wt,K,stride,N,n", [(O.Q4_K, 512, 140 << 20, 40, 70), (O.Q2_K, 3584, 150 << 20, 33, 20), (O.IQ4_XS, 256, (4 << 30) + 64, 3, 60),
-                                             (O.Q5_K, 3584, (2 << 30) + 16, 5, 80)],
+                                             (O.Q5_K, 3584, (2 << 30) + 16, 5, 80), (O.Q4_K, 512, 300 << 20, 20, 8), (O.Q5_K, 512, 300 << 20, 20, 16),
+                                             (O.Q4_0, 512, 300 << 20, 20, 9), (O.Q8_0, 512, 300 << 20, 20, 12)],
                          ids=lambda v: O.TYPE_NAMES[v] if isinstance(v, int) and v in O.TYPE_NAMES else None)
-def test_kquant_rows_far_apart(dev, orc, wt, K, stride, N, n):
+def test_rows_far_apart(dev, orc, wt, K, stride, N, n):
     L = dev.lib
     w = orc.quantize_weights(wt, common.weights_f32(K + N, N, K))
     x = common.activations_f32(K + n, n, K)
