@@ -111,6 +111,20 @@ hipError_t launch_moe_group(const int32_t *ids, int64_t ids_stride, int64_t n_us
     return hipGetLastError();
 }
 
+// Few pairs of long rows stay with the GEMV, whose lanes share the additions that the GEMM makes in one chain of K / 256 (error, relative 2-norm
+// x 1e8, GEMV / GEMM: Q4_K 4096 values 12.7 / 10.2, 8192 12.6 / 12.2, 14336 12.8 / 15.1; Q6_K 2048 7.2 / 5.9, 4096 7.7 / 8.0, 14336 8.3 / 13.2;
+// Q2_K 4096 11.0 / 8.6, 8192 10.7 / 11.5; Q5_K as Q4_K, Q3_K and IQ4_XS as Q6_K).  The types with a minimum per 32 values as well, at every length;
+// the other block-32 types have sums of their own for this.
+static bool few_pairs_as_near(int wtype, int64_t K) {
+    switch (wtype) {
+        case T_Q4_1: case T_Q5_1: return false;
+        case T_Q4_K: case T_Q5_K: return K <= 8192;
+        case T_Q2_K: return K <= 4096;
+        case T_Q6_K: case T_Q3_K: case T_IQ4_XS: return K < 4096;
+        default: return true;
+    }
+}
+
 // MUL_MAT_ID: the pairs grouped by expert and run through the GEMM of the weight type, or a GEMV per pair?  Both times estimated in us, with
 // terms fitted to 40 measured products of each type and checked against 14500 others (16 to 4095 pairs, 2 to 400 experts, 256 to 14336 values, at most 1 GB
 // of experts that no cache holds):
@@ -130,7 +144,8 @@ bool moe_gemm_ahead(int wtype, int64_t K, int64_t N, size_t row_bytes, int64_t n
     if (forced > 0) return pairs >= forced;
     if (wtype == T_F16 || gemv_max_tokens(wtype, K, DeviceLimits{256, 160 * 1024}) < 1) return pairs >= MOE_FEW_PAIRS;
     if (pairs < 16 || pairs >= 4096) return pairs >= 16;
-    if (pairs < MOE_FEW_PAIRS && (wtype == T_Q4_1 || wtype == T_Q5_1)) return false;    // one chain of additions, twice as far off as the GEMV's lanes
+    const bool few = pairs < MOE_FEW_PAIRS;
+    if (few && !few_pairs_as_near(wtype, K)) return false;
     struct { float pair, walk, turn, ends; } c;                         // pair: per 1024 rows x 4096 values; the others per super-block, per tile
     const bool low_bit = wtype == T_Q3_K || wtype == T_Q2_K || wtype == T_IQ4_XS;
     switch (wtype) {
@@ -149,7 +164,6 @@ bool moe_gemm_ahead(int wtype, int64_t K, int64_t N, size_t row_bytes, int64_t n
     }
     const float n_pairs = (float)pairs, experts = (float)n_as, units = (float)K / 256.f;
     const float pair_bytes = (float)N * (float)row_bytes;
-    const bool few = pairs < MOE_FEW_PAIRS;
     const float gemv = 6.5f + n_pairs * std::max(c.pair * (float)N / 1024.f * (float)ceil_div(K, (int64_t)4096), few ? 0.f : pair_bytes / 8e6f);
     const float tiles = (experts * (1.f - std::exp(-n_pairs / experts)) + n_pairs / 64.f) * (float)ceil_div(N, (int64_t)(gemm_kq_type(wtype) ? 128 : 64));
     const float gemm = 10.f + c.walk * units + tiles / 512.f * (c.turn * units + c.ends);

@@ -308,6 +308,21 @@ def test_block32_few_expert_pairs_as_near_as_the_gemv(dev, orc, wt, K):
     assert distance(orc, wt, K, rows, x[:, 0], y) <= 1.1 * distance(orc, wt, K, rows, x[:, 0], gemv)
 
 
+# 60 pairs of 4 experts (grouped up to some length of the rows) against the same tokens three at a time (a GEMV per pair)
+@pytest.mark.parametrize("K", (3840, 4096, 8448))
+@pytest.mark.parametrize("wt", (O.Q4_K, O.Q5_K, O.Q6_K) + LOW_BIT, ids=lambda t: O.TYPE_NAMES[t])
+def test_kquant_few_expert_pairs_as_near_as_the_gemv(dev, orc, wt, K):
+    N, n_as, n_used, n = 5000, 4, 4, 15
+    w = np.tile(orc.quantize_weights(wt, common.weights_f32(K, 250, K)), (n_as * N // 250, 1)).reshape(n_as, N, -1)
+    x = common.activations_f32(K, n, K).reshape(n, 1, K)
+    ids = np.tile(np.arange(4, dtype=np.int32), (n, 1))
+    y = dev.mul_mat_id(wt, w, x, ids)[:, :, :100].reshape(n, -1)
+    gemv = np.concatenate([dev.mul_mat_id(wt, w, x[i:i + 3], ids[i:i + 3]) for i in range(0, n, 3)])[:, :, :100].reshape(n, -1)
+    assert (y.tobytes() != gemv.tobytes()) == (K <= {O.Q4_K: 8192, O.Q5_K: 8192, O.Q2_K: 4096}.get(wt, 3840))
+    rows = w[0, :100]
+    assert distance(orc, wt, K, rows, x[:, 0], y[:, :100]) <= 1.1 * distance(orc, wt, K, rows, x[:, 0], gemv[:, :100])
+
+
 # K in eight slices of one super-block (Q2_K, IQ4_XS) and in two of four: no further off than rows walked whole (8192 outputs: within 1 per cent)
 @pytest.mark.parametrize("wt", LOW_BIT, ids=lambda t: O.TYPE_NAMES[t])
 def test_slices_of_k_as_near_as_whole_rows(dev, orc, wt):
