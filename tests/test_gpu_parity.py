@@ -12,6 +12,7 @@ import functools
 
 import common
 import oracle as O
+from test_gpu_routes import mul_mat_id_launches
 
 
 @functools.lru_cache(maxsize=12)
@@ -871,11 +872,12 @@ def test_mul_mat_id_is_mul_mat_on_the_chosen_expert(dev, orc):
 
 
 @pytest.mark.parametrize("wt", O.WEIGHT_TYPES, ids=lambda t: O.TYPE_NAMES[t])
-@pytest.mark.parametrize("n_tokens,ne11,n_as", [(16, 1, 8), (50, 4, 6), (130, 1, 32)])
-def test_mul_mat_id_prefill_grouped_by_expert(dev, orc, wt, n_tokens, ne11, n_as):
-    """64 (token, slot) pairs and more: grouped by expert on the device and run through the GEMMs.  Uneven loads: one
-    expert gets a pair from every token, some get none."""
-    K, N, n_used = 512, 150, 4
+@pytest.mark.parametrize("n_tokens,ne11,n_as,N,grouped", [(16, 1, 8, 150, False), (16, 1, 8, 1500, True), (50, 4, 6, 400, True), (130, 1, 32, 150, True)])
+def test_mul_mat_id_prefill_grouped_by_expert(dev, orc, wt, n_tokens, ne11, n_as, N, grouped):
+    """Many (token, slot) pairs: grouped by expert on the device and run through the GEMMs, but for 64 pairs on few rows, a GEMV each (F16:
+    grouped from 64 pairs on).  Uneven loads: one expert gets a pair from every token, some get none."""
+    K, n_used = 512, 4
+    assert (mul_mat_id_launches(dev, wt, K, N, n_as, n_used, n_tokens) == 3) == (grouped or wt == O.F16)
     rng = np.random.default_rng(900 + wt + n_tokens)
     W = np.stack([orc.quantize_weights(wt, common.weights_f32(900 + wt + e, N, K)) for e in range(n_as)])
     x = common.activations_f32(901 + wt, n_tokens * ne11, K).reshape(n_tokens, ne11, K)
@@ -889,7 +891,8 @@ def test_mul_mat_id_prefill_grouped_by_expert(dev, orc, wt, n_tokens, ne11, n_as
 def test_mul_mat_id_grouped_matches_pairwise_and_skips_bad_ids(dev, orc):
     """The grouped GEMM path and the pair-by-pair GEMV path agree within the tolerance on the same inputs (first 15
     tokens alone take the GEMV path), and an id outside [0, n_as) leaves exactly its own output row unwritten."""
-    wt, K, N, n_as, n_used, n_tokens = O.Q4_K, 1024, 96, 8, 4, 40
+    wt, K, N, n_as, n_used, n_tokens = O.Q4_K, 1024, 400, 8, 4, 40
+    assert mul_mat_id_launches(dev, wt, K, N, n_as, n_used, n_tokens) == 3 and mul_mat_id_launches(dev, wt, K, N, n_as, n_used, 15) == 2
     W, x, ids = moe_case(orc, wt, K, N, n_as, n_used, n_tokens, 1, 77)
     ids[7, 2] = n_as + 5
     ids[9, 0] = -1

@@ -6,6 +6,7 @@ import pytest
 
 import common
 import oracle as O
+from test_gpu_routes import group_launches, mul_mat_id_launches, mul_mat_launches
 
 pytestmark = pytest.mark.gpu
 
@@ -99,6 +100,23 @@ def test_kquant_row_gemm(dev, orc, wt, K, N, n):
     ref = orc.mul_mat(wt, w[rows], x[toks], nthreads=8, want=("sum_abs",))
     check(y[np.ix_(toks, rows)], ref, "k-quant row gemm")
     assert np.isfinite(y).all()
+
+
+# K in eight slices of seven super-blocks that give each CU a workgroup of this kernel, tokens one past its 32-token walk and one short of it
+@pytest.mark.parametrize("n", (31, 33))
+@pytest.mark.parametrize("wt", (O.Q6_K, O.Q3_K), ids=lambda t: O.TYPE_NAMES[t])
+def test_kquant_row_gemm_over_slices(dev, orc, wt, n):
+    K, N = 14336, 4096
+    w = np.tile(orc.quantize_weights(wt, common.weights_f32(wt, 128, K)), (N // 128, 1))
+    w[4001] = w[3]
+    x = common.activations_f32(K + n, n, K)
+    assert mul_mat_launches(dev, wt, w, x) == 3
+    y = dev.mul_mat(wt, w, x)
+    ref = orc.mul_mat(wt, w[:128], x, nthreads=8, want=("sum_abs",))
+    check(y[:, :128], ref, "slices")
+    same = np.tile(y[:, :128], (1, N // 128))
+    same[:, 4001] = y[:, 3]
+    assert y.tobytes() == same.tobytes()
 
 
 # Rows so far apart that a tile spans more than 2^32 bytes, and more than 2^32 bytes apart each: (type, stride, rows, tokens).  One whole tile
@@ -199,10 +217,10 @@ def test_f16_gemm_stage_counts(dev, orc, K, N, n):
 
 # ---- matrices on one activation whose tiles share a launch: the bits of each by itself ----
 # (type, K, rows of each, n): one row tile and a ragged one, 64 x 64 tiles; more row tiles than CUs; a first member of one row; two
-# super-blocks and one of another type between; a K that is no multiple of a stage
+# super-blocks and one of another type between; a K that is no multiple of a stage; Q6_K and Q3_K in the staging kernel (a launch each) and beside it
 @pytest.mark.parametrize("wt,K,rows,n", [(O.Q4_0, 960, (960, 320, 320), 133), (O.Q8_0, 192, (1, 65, 130, 64), 70), (O.Q5_1, 256, (8200, 8190), 130),
-                                         (O.Q4_K, 1024, (129, 128, 1), 140), (O.Q5_K, 512, (4100, 4100), 260), (O.Q6_K, 256, (300, 70), 65),
-                                         (O.Q3_K, 512, (200, 1030), 129), (O.Q2_K, 768, (33, 500), 200)],
+                                         (O.Q4_K, 1024, (129, 128, 1), 140), (O.Q5_K, 512, (4100, 4100), 260), (O.Q6_K, 256, (300, 70), 65), (O.Q6_K, 256, (4200, 4106), 520),
+                                         (O.Q3_K, 512, (200, 1030), 129), (O.Q3_K, 512, (4200, 4106), 520), (O.Q2_K, 768, (33, 500), 200)],
                          ids=lambda v: O.TYPE_NAMES[v] if isinstance(v, int) and v in O.TYPE_NAMES else None)
 def test_grouped_gemms_equal_single_calls(dev, orc, wt, K, rows, n):
     rng = np.random.default_rng(K + n)
@@ -213,6 +231,8 @@ def test_grouped_gemms_equal_single_calls(dev, orc, wt, K, rows, n):
         rows = (rows[0], 64, rows[1])
     ws = [(t, orc.quantize_weights(t, common.weights_f32(K + N + i, N, K))) for i, (t, N) in enumerate(zip(types, rows))]
     x = common.activations_f32(K + n, n, K)
+    staged = wt in (O.Q6_K, O.Q3_K) and rows[0] < 4000
+    assert group_launches(dev, [(t, W.shape[0]) for t, W in ws], K, n) == 1 + (len(ws) if staged else len(set(types)))
     ys = dev.mul_mat_group(ws, x)
     for i, ((t, W), y) in enumerate(zip(ws, ys)):
         assert y.tobytes() == dev.mul_mat(t, W, x).tobytes(), i
@@ -233,13 +253,34 @@ def test_grouped_gemms_equal_single_calls(dev, orc, wt, K, rows, n):
                          ids=("tile edges", "320 experts", "8400 pairs"))
 @pytest.mark.parametrize("wt", (O.Q4_K, O.Q6_K, O.Q4_0, O.F16), ids=lambda t: O.TYPE_NAMES[t])
 def test_expert_groups(dev, orc, wt, counts, n_used):
-    K, N = 256, 70
+    K, N = 256, 130
     rng = np.random.default_rng(wt + len(counts))
     ids = rng.permutation(np.repeat(np.arange(len(counts)), counts)).astype(np.int32).reshape(-1, n_used)
     n_tokens = ids.shape[0]
+    assert mul_mat_id_launches(dev, wt, K, N, len(counts), n_used, n_tokens) == 3
     experts = np.stack([orc.quantize_weights(wt, common.weights_f32(wt + e, N, K)) for e in range(len(counts))])
     x = common.activations_f32(wt, n_tokens, K).reshape(n_tokens, 1, K)
     check(dev.mul_mat_id(wt, experts, x, ids), orc.mul_mat_id(wt, experts, x, ids, want=("sum_abs",)), "expert groups")
+
+
+# Ids that name no expert, among the pairs that the grouping keeps in registers (the first 8192) and behind them: their rows are not written
+@pytest.mark.parametrize("wt", (O.Q4_K, O.Q4_0, O.F16), ids=lambda t: O.TYPE_NAMES[t])
+def test_expert_groups_skip_ids_out_of_range(dev, orc, wt):
+    K, N, n_as, n_used, n_tokens = 256, 130, 5, 2, 4300
+    rng = np.random.default_rng(wt)
+    ids = rng.integers(0, n_as, (n_tokens, n_used)).astype(np.int32)
+    at = np.array([0, 63, 1024, 8191, 8192, 8193, 8500, 2 * n_tokens - 1])
+    bad = np.zeros(2 * n_tokens, bool)
+    bad[at] = True
+    ok = ids.copy()
+    ids.reshape(-1)[at] = [-1, n_as, 2 ** 31 - 1, -2 ** 31, n_as, -1, 4096, n_as + 5]
+    assert mul_mat_id_launches(dev, wt, K, N, n_as, n_used, n_tokens) == 3
+    experts = np.stack([orc.quantize_weights(wt, common.weights_f32(wt + e, N, K)) for e in range(n_as)])
+    x = common.activations_f32(wt, n_tokens, K).reshape(n_tokens, 1, K)
+    y = dev.mul_mat_id(wt, experts, x, ids).reshape(-1, N)
+    ref = orc.mul_mat_id(wt, experts, x, ok, want=("sum_abs",))
+    assert np.isnan(y[bad]).all() and np.isfinite(y[~bad]).all()
+    check(y[~bad], {k: ref[k].reshape(-1, N)[~bad] for k in ("y", "sum_abs")}, "bad ids")
 
 
 # Few tiles of these types run in the staging kernel (64 rows x 128 pairs), the same rows inside a large matrix in the other one
@@ -358,10 +399,12 @@ def test_block32_short_rows_of_few_tokens(dev, orc, wt, K, N, n):
     check(dev.mul_mat(wt, w, x), orc.mul_mat(wt, w, x, nthreads=8, want=("sum_abs",)), "%d tokens" % n)
 
 
-# ---- 15 pairs (a GEMV each), 16 pairs of long rows on few experts (grouped), 130 pairs on many experts with few rows (a GEMV each) ----
-@pytest.mark.parametrize("n_tokens,n_used,n_as,K,N", [(15, 1, 2, 4096, 2000), (8, 2, 2, 4096, 2000), (65, 2, 64, 512, 24)])
+# ---- 15 and 16 pairs (a GEMV each), 16 pairs of many short rows (grouped), 130 pairs on many experts with few rows (a GEMV each) ----
+@pytest.mark.parametrize("n_tokens,n_used,n_as,K,N,grouped", [(15, 1, 2, 4096, 2000, False), (8, 2, 2, 4096, 2000, False), (15, 1, 4, 256, 4000, False),
+                                                              (4, 4, 4, 256, 4000, True), (65, 2, 64, 512, 24, False)])
 @pytest.mark.parametrize("wt", (O.Q4_K, O.Q3_K, O.Q4_0), ids=lambda t: O.TYPE_NAMES[t])
-def test_expert_matmul_of_few_pairs(dev, orc, wt, n_tokens, n_used, n_as, K, N):
+def test_expert_matmul_of_few_pairs(dev, orc, wt, n_tokens, n_used, n_as, K, N, grouped):
+    assert (mul_mat_id_launches(dev, wt, K, N, n_as, n_used, n_tokens) == 3) == grouped
     rng = np.random.default_rng(n_tokens + wt)
     experts = np.stack([orc.quantize_weights(wt, common.weights_f32(wt + e, N, K)) for e in range(n_as)])
     x = common.activations_f32(wt, n_tokens, K).reshape(n_tokens, 1, K)
