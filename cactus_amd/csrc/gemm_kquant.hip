@@ -475,10 +475,13 @@ static int64_t gemm_kq_min_tokens(int wtype, int64_t K, int64_t N, bool can_spli
 }
 
 // Q3_K, Q2_K and IQ4_XS: the dot-product GEMV passes of 8 tokens, whose time grows with the tokens, against the GEMM, whose time
-// below 128 tokens does not.  A token count alone does not part them (GEMV / GEMM, us, split K: IQ4_XS 8192 x 8192 at 12
-// tokens 36 / 43, 1024 x 14336 at 9 tokens 20 / 19; Q2_K 1024 x 4096 at 10 tokens 12 / 14, 4096 x 4096 at 9 tokens 16 / 15;
-// unsplit: IQ4_XS 748 x 7168 at 32 tokens 34 / 58, 4096 x 1024 at 25 tokens 32 / 14), so both times are estimated, in us, with terms
-// fitted to 5000 measured products (to 13 and 9 per cent for nine in ten of them):
+// below 128 tokens does not.  A token count alone does not part them (GEMV / GEMM, us, rows x values, split K: Q3_K 300 x 2816
+// at 10 tokens 11 / 14, 4096 x 4096 at 9 tokens 15 / 14, 1024 x 14336 at 9 tokens 19 / 14; IQ4_XS 1024 x 4096 at 10 tokens 12 / 13, 8192 x 8192 at 12
+// tokens 37 / 27; unsplit: IQ4_XS 748 x 7168 at 32 tokens 33 / 48, 4096 x 1024 at 25 tokens 31 / 13), so both times are estimated, in us.
+// The terms of the GEMM were fitted to the staging kernel in the slices of kq_slices_for, which Q2_K and IQ4_XS only rarely run in now: for them
+// they are an upper bound, and the GEMM is taken late rather than early.  Of 5100 products (9 to 200 tokens, values x rows, GEMV / GEMM)
+// the slower one is taken by more than 5 per cent in 1 per cent of Q3_K (2048 x 290 at 10 tokens 11.3 / 14.2), 4 of Q2_K (8192 x 9071 at 14 tokens
+// 46 / 22) and 6 of IQ4_XS (9984 x 10019 at 14 tokens 60 / 34), nearly always the GEMV:
 //   GEMV   a launch per pass, then per token the rounds of 1024 rows (four a CU) and of 4096 values of a row
 //   GEMM   quantizer and launch (and slice sum), then the super-blocks a workgroup walks times the rounds of 256 workgroups; split K
 //          has most of the weights in flight at once and pays for their bytes too

@@ -19,8 +19,8 @@
 // four waves of a k group (global_load_lds, double buffered), so a super-block needs one barrier and everything it waits for was
 // requested a whole super-block earlier.
 //
-// Bound: the vector instructions and MFMAs of a SIMD do not overlap (403 and 34 per super-block and wave for Q4_K; 62 % + 42 % of the cycles
-// by the counters, 16384 rows x 4096 values x 1024 tokens), LDS is 27 % busy without bank conflicts.  Reading operands a step ahead took
+// Bound: the vector instructions and MFMAs of a SIMD do not overlap (403 and 34 per super-block and wave for Q4_K; 62 % + 40 % of the cycles
+// by the counters, ffn_gate + ffn_up of 14336 rows x 4096 values at 512 tokens), LDS is 25 % busy, 2 % of it bank conflicts (Q6_K: 22 %).  Reading operands a step ahead took
 // a quarter off the first form, in which every read was waited for at once; widening d and dmin once instead
 // of in a half-rate v_fma_mix per output and full-rate v_bitop3 in place of v_and_or / v_bfi another 3 %.
 // Measured against the staging kernel (Q4_K, Q5_K: the single-plane kernel) that ran these before, us for values x rows: Q4_K 512 tokens
@@ -77,7 +77,8 @@ __device__ __forceinline__ u32x4 i16x8_to_f16(const u32x4 &v) {
     return c;
 }
 // Per weight type.  A super-block is fetched as NCH 16-byte chunks (the last one ends with the super-block, so it may overlap the
-// one before) and kept in LDS as STRIDE cells of a row, STRIDE odd so that 16 rows' cells of one index fall into different banks.
+// one before) and kept in LDS in that order, NCH cells a row.  Where NCH is odd, 16 rows' cells of one index fall into different banks; for Q6_K (14
+// cells) and Q2_K (6) two of them share one.
 // Lane (row, hf) reads its share back: hdr() what all items need, load<Q>() the 16-value k-half hf of k-blocks KA(Q) and KB(Q), which
 // expand<Q>() turns into MFMA operand cells [k-block][plane].
 template <int WT> struct KR;
@@ -332,10 +333,9 @@ struct KrCfg {
     static constexpr size_t FB_BYTES = T::NF16 > 0 ? (size_t)BN * 32 : 0;
     static constexpr size_t OFF_SX = OFF_FB + 4 * KS * FB_BYTES;          // [j % 4][k group] f32 [token]: activation scale
     static constexpr size_t OFF_ROW = OFF_SX + 4 * KS * (size_t)BN * 4;   // i32 [token]: output row (expert groups)
-    static constexpr size_t TOTAL0 = OFF_ROW + (size_t)BN * 4;
+    static constexpr size_t TOTAL = OFF_ROW + (size_t)BN * 4;
     // the other k groups' partial outputs take the place of the operands at the end
     static_assert((size_t)(KS - 1) * 4 * TN * 16 * 256 <= OFF_SX, "partial outputs lie in front of the output rows");
-    static constexpr size_t TOTAL = TOTAL0;
 };
 
 __device__ __forceinline__ void kr_load16_into_lds(const uint8_t *base, uint32_t off, uint32_t lds_addr) {

@@ -1474,7 +1474,7 @@ int backend_graph_compute(lm_ggml_backend_t backend, lm_ggml_cgraph *cgraph) {
         int members[CHIP_GROUP_MAX];
         bool aliased[CHIP_GROUP_MAX] = {false, false, false, false};
         int n_members = 1;
-        if ((n <= 4 || n == 8) && fusion_enabled()) {      // the token counts chip_mul_mat_group has a one-launch form for
+        if ((n <= 4 || n == 8) && fusion_enabled()) {      // quantizer included; from 17 tokens on chip_mul_mat_group joins only GEMMs, and the rows are shared through c->quantized here
             bool slots_free = true;
             for (int slot : grouped) slots_free = slots_free && slot < 0;
             // A SILU held back for its MUL reads the gate projection's result only when that MUL runs, after this node:

@@ -120,9 +120,9 @@ __device__ __forceinline__ GemmMat pick_gemm_mat(const GemmMats &t, int &row_til
 }
 
 // Row gather of LM_GGML_OP_MUL_MAT_ID for the GEMM kernels (reference ggml-cpu/ggml-cpu.c:1460-1710 groups the (token,
-// slot) pairs by expert the same way: matrix_rows / matrix_row_counts).  With perm set, blockIdx.y walks a list of
-// token tiles built on the device: entry i = expert | tile << 12 says "pairs perm[offsets[e] + tile * BN ...] of expert
-// e"; entries past tiles[-1] (the count, stored in front of the list) do not exist.  The expert's matrix is
+// slot) pairs by expert the same way: matrix_rows / matrix_row_counts).  With perm set, the grid covers a list of
+// token tiles built on the device (int8 GEMMs: gather_tile; F16: blockIdx.y is the entry): entry i = expert | tile << 12 says "pairs
+// perm[offsets[e] + tile * BN ...] of expert e"; the count stands in front of the list.  The expert's matrix is
 // W + e * nb02; pair p reads activation row (p / n_used) * ne11 + (p % n_used) % ne11 and writes output row p.
 // perm == nullptr: plain MUL_MAT.
 constexpr int MOE_EXPERT_BITS = 12;
@@ -346,8 +346,8 @@ hipError_t launch_gemm_kq_group(int wtype, const GemmMats &mats, int64_t K, cons
                                 hipStream_t st);
 // Expert matmuls of fewer pairs than this are a GEMV per pair, unless the grouped GEMM is both ahead and as near to the 64-bit sums
 constexpr int64_t MOE_FEW_PAIRS = 64;
-// In the three GEMM launchers: with rg, n_as is the number of token-tile slots the grid provides in y (an upper bound
-// of the tile list's length) and n is the number of pairs; gemm_*_moe_tile_tokens gives the tile height the list must be built for.
+// In the three GEMM launchers: with rg, n_as is the number of token-tile slots the grid provides (an upper bound
+// of the tile list's length; F16: in y) and n is the number of pairs; gemm_*_moe_tile_tokens gives the tile height the list must be built for.
 
 // ops.hip: RMS_NORM, ADD, MUL, SILU over F32 rows (ldb = 0 broadcasts one row of b over all rows of a).
 // LM_GGML_OP_MUL_MAT with a batched, strided F16 src0 (the attention matmuls over the KV cache):

@@ -13,13 +13,14 @@ def splits_k(lib, t, K, N, n):
     return lib.chip_mul_mat_workspace_size_n(t, K, N, n) > lib.chip_mul_mat_workspace_size(t, K, n)
 
 
-# Measured on either side of the rule (us, GEMV passes / GEMM): the low-bit types take the GEMM, with K split, only where it is ahead
+# On either side of the rule (us, GEMV passes / GEMM): the low-bit types take the GEMM, with K split, where it is estimated to be ahead.  The estimate
+# is late for Q2_K and IQ4_XS: some of their GEMV cases here are faster through the GEMM by now
 @pytest.mark.parametrize("t,K,N,n,gemm", [
-    (ca.IQ4_XS, 4096, 1024, 10, False), (ca.IQ4_XS, 8192, 8192, 12, False), (ca.IQ4_XS, 2048, 692, 9, False),        # 12 / 17, 36 / 43, 12 / 16
-    (ca.IQ4_XS, 14336, 1024, 12, True), (ca.IQ4_XS, 4096, 4096, 17, True),                                           # 23 / 19, 24 / 18
-    (ca.Q3_K, 2816, 300, 10, False), (ca.Q3_K, 3840, 612, 9, False), (ca.Q3_K, 4096, 4096, 9, True), (ca.Q3_K, 14336, 1024, 9, True),
-    (ca.Q3_K, 14336, 70, 9, True), (ca.Q2_K, 14336, 70, 9, True), (ca.IQ4_XS, 14336, 70, 9, True),
-    (ca.Q2_K, 2304, 280, 11, False), (ca.Q2_K, 4096, 1024, 10, False), (ca.Q2_K, 4096, 4096, 12, True)])
+    (ca.IQ4_XS, 4096, 1024, 10, False), (ca.IQ4_XS, 8192, 8192, 12, False), (ca.IQ4_XS, 2048, 692, 9, False),        # 12 / 13, 37 / 27, 11 / 11
+    (ca.IQ4_XS, 14336, 1024, 12, True), (ca.IQ4_XS, 4096, 4096, 17, True),                                           # 22 / 17, 24 / 15
+    (ca.Q3_K, 2816, 300, 10, False), (ca.Q3_K, 3840, 612, 9, False), (ca.Q3_K, 4096, 4096, 9, True), (ca.Q3_K, 14336, 1024, 9, True),    # 11 / 14, 12 / 14, 15 / 14, 19 / 14
+    (ca.Q3_K, 14336, 70, 9, True), (ca.Q2_K, 14336, 70, 9, True), (ca.IQ4_XS, 14336, 70, 9, True),                              # 18 / 13, 18 / 12, 18 / 16
+    (ca.Q2_K, 2304, 280, 11, False), (ca.Q2_K, 4096, 1024, 10, False), (ca.Q2_K, 4096, 4096, 12, True)])                          # 12 / 11, 12 / 11, 17 / 12
 def test_low_bit_types_take_the_gemm_where_it_is_ahead(lib, t, K, N, n, gemm):
     assert splits_k(lib, t, K, N, n) == gemm
     assert splits_k(lib, t, K, N, 70)
