@@ -440,7 +440,9 @@ static int kq_slices_for(int64_t K, int64_t N, int64_t M, int64_t cus) {
 //                           in 2 / 3).  The slice sum pays for at most 150000 partial outputs a super-block of a row (IQ4_XS 1792 values x
 //                           4096 rows at 64 tokens 21.7 / 16.4 whole / in 4), not for rows of three or less or for two slices of less than 8.
 //   IQ4_XS, 5 to 11 super-blocks in one or two slices, up to 128 tokens: the staging kernel (us, staged / gemm_kr_kernel: 2304 values x
-//                           8192 rows at 93 tokens 21.5 / 25.9, 1280 x 8192 at 64 16.3 / 19.0; 2560 x 15500 at 127 31.3 / 29.4)
+//                           8192 rows at 93 tokens 21.5 / 25.9, 1280 x 8192 at 64 16.3 / 19.0; 2560 x 15500 at 127 31.3 / 29.4); 2 and 3 up
+//                           to 96 tokens on at most 1000000 outputs, 600000 where the other kernel has one token tile (768 x 3788 at 52 11.7 / 12.8,
+//                           512 x 11088 at 65 10.7 / 11.9; 512 x 14373 at 60 12.2 / 11.5, 512 x 13107 at 86 13.5 / 12.2)
 struct KqPlan { int groups, slices; };
 static KqPlan kq_plan(int wtype, int64_t K, int64_t N, int64_t M, int64_t cus) {
     const int64_t tiles = ceil_div(N, (int64_t)128) * ceil_div(M, (int64_t)64), units = K / QK_K;
@@ -453,6 +455,7 @@ static KqPlan kq_plan(int wtype, int64_t K, int64_t N, int64_t M, int64_t cus) {
     const int64_t most = std::max<int64_t>(8, std::min<int64_t>(16, units / 4));
     int64_t s = units < 4 ? 1 : std::min({cus / tiles, units, most, units * 150000 / (M * N)});
     if (s < (units < 8 ? 3 : 2)) s = 1;
+    if (wtype == T_IQ4_XS && units < 4 && M <= 96 && M * N <= (M > 64 ? 1000000 : 600000)) return KqPlan{0, 1};
     if (wtype == T_IQ4_XS && s <= 2 && units >= 5 && units < 12 && M > (units < 8 ? 32 : 64) && M <= 128 && M * N <= 1400000) return KqPlan{0, kq_slices_for(K, N, M, cus)};
     if (s == 1) return KqPlan{units < 4 ? 1 : 2, 1};
     const int64_t per = ceil_div(units, s);
@@ -584,7 +587,8 @@ bool gemm_kq_group_applicable(int wtype, int64_t K, const GemmMats &mats, int64_
     for (int i = 0; i < mats.count; i++) {
         const int64_t N = mats.m[i].N;
         const KqPlan p = kq_plan(wtype, K, N, n, cus);
-        if (!gemm_kq_supported(wtype, K, N, n, false) || p.slices != 1 || p.groups != 1) return false;
+        // (IQ4_XS of 2 and 3 super-blocks: alone in the staging kernel, together faster in one launch; the same bits)
+        if (!gemm_kq_supported(wtype, K, N, n, false) || p.slices != 1 || !(p.groups == 1 || (wtype == T_IQ4_XS && K < 4 * QK_K))) return false;
         if (gemm_kr_rows_in_reach(mats.m[i].nb01) < 32) return false;
     }
     return true;

@@ -61,7 +61,7 @@ def random_rows(wt, rng, N, nsb):
 # short rows; 128 x 128 tiles; many tokens, few rows; the GEMM at the fewest tokens it is taken from; the staging kernel
 @pytest.mark.parametrize("wt", LOW_BIT, ids=lambda t: O.TYPE_NAMES[t])
 @pytest.mark.parametrize("K,N,n", [(256, 5, 41), (1024, 131, 65), (2304, 131, 70), (4096, 300, 9), (512, 4100, 1030), (768, 33, 1100),
-                                   (14336, 70, 9), (2304, 8200, 70), (1280, 8100, 33)])
+                                   (14336, 70, 9), (2304, 8200, 70), (1280, 8100, 33), (512, 300, 96), (768, 131, 33)])
 def test_low_bit_kquant_gemm(dev, orc, wt, K, N, n):
     rng = np.random.default_rng(K + N + wt)
     w = random_rows(wt, rng, N, K // 256)
@@ -220,7 +220,7 @@ def test_f16_gemm_stage_counts(dev, orc, K, N, n):
 # super-blocks and one of another type between; a K that is no multiple of a stage; Q6_K and Q3_K in the staging kernel (a launch each) and beside it
 @pytest.mark.parametrize("wt,K,rows,n", [(O.Q4_0, 960, (960, 320, 320), 133), (O.Q8_0, 192, (1, 65, 130, 64), 70), (O.Q5_1, 256, (8200, 8190), 130),
                                          (O.Q4_K, 1024, (129, 128, 1), 140), (O.Q5_K, 512, (4100, 4100), 260), (O.Q6_K, 256, (300, 70), 65), (O.Q6_K, 256, (4200, 4106), 520),
-                                         (O.Q3_K, 512, (200, 1030), 129), (O.Q3_K, 512, (4200, 4106), 520), (O.Q2_K, 768, (33, 500), 200)],
+                                         (O.Q3_K, 512, (200, 1030), 129), (O.Q3_K, 512, (4200, 4106), 520), (O.Q2_K, 768, (33, 500), 200), (O.IQ4_XS, 768, (256, 65, 130), 41)],
                          ids=lambda v: O.TYPE_NAMES[v] if isinstance(v, int) and v in O.TYPE_NAMES else None)
 def test_grouped_gemms_equal_single_calls(dev, orc, wt, K, rows, n):
     rng = np.random.default_rng(K + n)
