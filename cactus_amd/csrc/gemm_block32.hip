@@ -28,6 +28,7 @@
 #include "dev_common.h"
 #include "act_layout.h"
 #include "kernels.h"
+#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
@@ -667,6 +668,48 @@ static int blk32_slices_for(int64_t K, int64_t N, int64_t M, int64_t cus) {
     return (int)ceil_div(units, per);                                   // no empty slice
 }
 
+// Few output tiles: gemm_blk32_few_kernel, whose ks waves a workgroup share the K of a 32 x 32 tile, or the staged walk of this file, whichever
+// is estimated ahead, in us of a launch.  Fitted to 707 products of 256 to 14336 values x 320 to 14336 rows at 17 to 512 tokens (11 and 19 per cent
+// of spread); the walk is left where it is more than 15 per cent slower: 1.21 x over all of them, 16 more than 2 per cent slower than before, the
+// worst 1.12 x (14336 values x 2048 rows at 133 tokens).  us, walk / few: Q4_0 960 x 960 at 133 tokens 9.3 / 5.5, 2560 x 960 13.3 / 8.4, 4096 x 4096 at 17
+// 12.1 / 9.0, at 128 20.8 / 14.5, 2048 x 2048 at 512 20.9 / 14.7; Q5_0 2048 x 2048 at 40 13.9 / 7.4; 14336 x 4096 at 32 25.0 / 25.4 and stays.
+//   few    a launch; the turns of 8 waves a CU, each the fetch of a first chunk and then its chunks of 256 values, as long as a load takes or as
+//          the vector work of the waves of a CU
+//   walk   a launch; the turns of the workgroups a CU holds, each the fetch of a first stage and then its stages; the slice sum
+// It depends on the sizes alone, not on the room in the workspace: the same bits alone and in a group.  At most 64 tiles of rows of 4096 values
+// and more also split the K of the 8 waves over two workgroups (Q4_0 8192 x 320 at 64 tokens 12.0 walk, 12.6 / 10.9 in one / two; 4096 x 320 8.4 / 8.8).
+struct FewPlan { int ks, slices; };              // ks 0: the walk
+static float blk32_walk_us(int wtype, int64_t K, int64_t N, int64_t M, int64_t cus) {
+    const int slices = blk32_slices_for(K, N, M, cus);
+    const int64_t g128 = ceil_div(N, (int64_t)128) * ceil_div(M, (int64_t)128), g64x128 = ceil_div(N, (int64_t)64) * ceil_div(M, (int64_t)128);
+    int64_t wgs = ceil_div(N, (int64_t)64) * ceil_div(M, (int64_t)64) * slices, per_cu = 3;
+    float stage = 0.59f;                                                 // 64 x 64 tiles
+    if (slices == 1 && blk32_near(wtype, K, N, M)) stage = 0.65f;
+    else if (slices == 1 && 2 * g128 >= 3 * cus) { wgs = g128; per_cu = 2; stage = 2.04f; }
+    else if (slices == 1 && 2 * g64x128 >= 3 * cus) { wgs = g64x128; per_cu = 2; stage = 0.95f; }
+    const int64_t turns = wgs / (per_cu * cus), rest = wgs % (per_cu * cus);
+    const float stages = (float)ceil_div(ceil_div(K, (int64_t)(32 * GEMM_KB)), (int64_t)slices);
+    float t = 1.8f + (float)turns * (3.6f + stages * stage * (float)per_cu);
+    if (rest) t += 3.6f + stages * std::max(0.59f, stage * std::max(1.f, (float)rest / (float)cus));
+    return slices > 1 ? t + 2.7f + 0.9e-6f * (float)N * (float)M * (float)slices : t;
+}
+static FewPlan blk32_few_plan(int wtype, int64_t K, int64_t N, int64_t M, size_t nb01, int64_t cus) {
+    const int64_t tiles = ceil_div(N, (int64_t)32) * ceil_div(M, (int64_t)32);
+    if (K < 256 || tiles > 65536 || nb01 > ((size_t)1 << 27)) return FewPlan{0, 1};           // (rows within 32-bit reach)
+    float best = blk32_walk_us(wtype, K, N, M, cus) / 1.15f;
+    FewPlan plan{0, 1};
+    for (int ks = 2; ks <= 8; ks *= 2) {
+        const int slices = ks == 8 && tiles <= 64 && K >= 4096 ? 2 : 1;
+        const int64_t wgs = tiles * slices, turn = cus * (8 / ks), turns = wgs / turn, rest = wgs % turn;
+        const float chunks = (float)ceil_div(2 * ceil_div(ceil_div(K / 64, (int64_t)slices), (int64_t)ks), (int64_t)8);
+        float t = 2.04f + (float)turns * (1.8f + chunks * 2.62f);
+        if (rest) t += 1.8f + chunks * std::max(1.72f, 0.328f * std::max((float)ks, (float)(rest * ks) / (float)cus));
+        if (slices > 1) t += 3.8f + 0.9e-6f * (float)N * (float)M * (float)slices;
+        if (t < best) { best = t; plan = FewPlan{ks, slices}; }
+    }
+    return plan;
+}
+
 template <int WT, int TM, int TN, int WR, int WC, int OCC, bool GATHER, bool NEAR = false, bool TAIL = false>
 static hipError_t launch_direct(GemmMats mats, int64_t K, const void *ws, size_t ws_stride, int64_t M, const DeviceLimits &lim, hipStream_t st,
                                 const RowGather &rg, int64_t n_as, int slices = 1, float *part = nullptr) {
@@ -696,6 +739,15 @@ template <int WT>
 static hipError_t launch_type(const GemmMats &mats, int64_t K, const void *ws, size_t ws_stride, int64_t M, const DeviceLimits &lim, hipStream_t st,
                               const RowGather &rg, int64_t n_as, SplitK split) {
     const int64_t cus = lim.compute_units > 0 ? lim.compute_units : 256;
+    if (!rg.perm) {                                                      // (the members of a group have the plan of the first)
+        const GemmMat &m = mats.m[0];
+        FewPlan few = blk32_few_plan(WT, K, m.N, M, m.nb01, cus);
+        if (const int f = (int)tune("CHIP_BLK32_FEW", 0); f) few = FewPlan{f % 10 == 9 ? 0 : f % 10, f / 100 + 1};
+        const bool near = blk32_near(WT, K, m.N, M);
+        if (few.slices > 1 && !(split.part && split.bytes >= (size_t)few.slices * (size_t)M * (size_t)m.N * sizeof(float) && (((uintptr_t)split.part) & 15) == 0))
+            few.slices = 1;
+        if (few.ks > 0) return launch_gemm_blk32_few(WT, few.ks, near, mats, K, ws, ws_stride, M, lim, st, few.slices, split.part);
+    }
     if (!rg.perm && split.part) {
         const int64_t N = mats.m[0].N;
         const int slices = blk32_slices_for(K, N, M, cus);
@@ -757,10 +809,14 @@ hipError_t launch_gemm_blk32(int wtype, const void *W, size_t nb01, int64_t K, i
 // 320 rows 31 -> 13, ffn_gate + ffn_up of 2560 rows 23 -> 14; 512 tokens x 4096 values x 14336 rows twice 195 -> 185).
 bool gemm_blk32_group_applicable(int wtype, int64_t K, const GemmMats &mats, int64_t n, int compute_units) {
     if (mats.count < 2) return false;
-    for (int i = 0; i < mats.count; i++)
-        if (!gemm_blk32_supported(wtype, K, mats.m[i].N, n, false) || gemm_blk32_slices(wtype, K, mats.m[i].N, n, compute_units) != 1 ||
-            blk32_near(wtype, K, mats.m[i].N, n) != blk32_near(wtype, K, mats.m[0].N, n))
+    const int64_t cus = compute_units > 0 ? compute_units : 256;
+    const FewPlan first = blk32_few_plan(wtype, K, mats.m[0].N, n, mats.m[0].nb01, cus);
+    for (int i = 0; i < mats.count; i++) {
+        const FewPlan few = blk32_few_plan(wtype, K, mats.m[i].N, n, mats.m[i].nb01, cus);
+        if (few.ks != first.ks || few.slices != 1 || (few.ks == 0 && gemm_blk32_slices(wtype, K, mats.m[i].N, n, compute_units) != 1) ||
+            !gemm_blk32_supported(wtype, K, mats.m[i].N, n, false) || blk32_near(wtype, K, mats.m[i].N, n) != blk32_near(wtype, K, mats.m[0].N, n))
             return false;
+    }
     return true;
 }
 hipError_t launch_gemm_blk32_group(int wtype, const GemmMats &mats, int64_t K, const void *ws, size_t ws_stride, int64_t n, const DeviceLimits &lim,

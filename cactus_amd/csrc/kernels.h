@@ -295,6 +295,9 @@ hipError_t launch_mmv_q6k(const void *W, size_t nb01, int64_t K, int64_t N, cons
 hipError_t launch_mmv(int wtype, const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride,
                       int n, float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st);
 
+// gemm_block32_few.hip: the same product for few output tiles, in tiles of 32 rows x 32 tokens whose K is shared by ks waves (K >= 256).
+hipError_t launch_gemm_blk32_few(int wtype, int ks, bool near, const GemmMats &mats, int64_t K, const void *ws, size_t ws_stride, int64_t M, const DeviceLimits &lim,
+                                 hipStream_t st, int slices = 1, float *part = nullptr);
 // gemm_block32.hip: int8-MFMA prefill GEMM over weights in 32-value blocks with one fp16 scale (Q4_0, Q8_0, Q5_0,
 // IQ4_NL), activations in the split Q8_0 workspace layout.  _supported includes the token count from which it pays.
 // Split K: with fewer output tiles than the machine holds workgroups, K is cut into slices that run as

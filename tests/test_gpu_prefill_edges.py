@@ -410,3 +410,21 @@ def test_expert_matmul_of_few_pairs(dev, orc, wt, n_tokens, n_used, n_as, K, N, 
     x = common.activations_f32(wt, n_tokens, K).reshape(n_tokens, 1, K)
     ids = np.stack([rng.permutation(n_as)[:n_used] for _ in range(n_tokens)]).astype(np.int32)
     check(dev.mul_mat_id(wt, experts, x, ids), orc.mul_mat_id(wt, experts, x, ids, want=("sum_abs",)), "few pairs")
+
+
+# ---- few output tiles of block-32 rows: waves that share the K of a tile.  (K, N, n): one chunk of 256 values; chunks that start early (10, 14 and 30
+# blocks); one row, one row more than a tile, 19 tokens and two tiles of tokens; more rows than a turn of workgroups; K over two workgroups too ----
+@pytest.mark.parametrize("K,N,n", [(256, 33, 49), (320, 31, 64), (448, 1, 48), (960, 65, 33), (960, 2100, 50), (2112, 97, 19), (4096, 4100, 33), (4096, 40, 66)])
+@pytest.mark.parametrize("wt", (O.Q4_0, O.Q8_0, O.Q5_0, O.IQ4_NL, O.Q4_1, O.Q5_1), ids=lambda t: O.TYPE_NAMES[t])
+def test_block32_few_tiles(dev, orc, wt, K, N, n):
+    rng = np.random.default_rng(K + N + wt)
+    w = np.tile(orc.quantize_weights(wt, common.weights_f32(K + N, min(N, 150), K)), (-(-N // 150), 1))[:N]
+    x = common.activations_f32(K + n, n, K)
+    x[2] *= 2e-3                                  # scales that are subnormal in fp16, and below its smallest
+    x[3] *= 1e-9
+    x[5] = -np.abs(x[5])
+    if K == 2112:
+        assert mul_mat_launches(dev, wt, w, x) == 2          # the walk would split K and add the slices
+    y = dev.mul_mat(wt, w, x)
+    rows = np.unique(np.concatenate([[0, N - 1], rng.choice(N, min(N, 100), replace=False)]))
+    check(y[:, rows], orc.mul_mat(wt, w[rows], x, nthreads=8, want=("sum_abs",)), "few tiles")
