@@ -676,7 +676,8 @@ static int blk32_slices_for(int64_t K, int64_t N, int64_t M, int64_t cus) {
 //   few    a launch; the turns of 8 waves a CU, each the fetch of a first chunk and then its chunks of 256 values, as long as a load takes or as
 //          the vector work of the waves of a CU
 //   walk   a launch; the turns of the workgroups a CU holds, each the fetch of a first stage and then its stages; the slice sum
-// It depends on the sizes alone, not on the room in the workspace: the same bits alone and in a group.  At most 64 tiles of rows of 4096 values
+// A caller without room for the slices that the walk would be cut into keeps the order of one walk over K, whatever the tile (room: the caller has it;
+// a group is planned without, so that its members have the bits of their single calls).  At most 64 tiles of rows of 4096 values
 // and more also split the K of the 8 waves over two workgroups (Q4_0 8192 x 320 at 64 tokens 12.0 walk, 12.6 / 10.9 in one / two; 4096 x 320 8.4 / 8.8).
 struct FewPlan { int ks, slices; };              // ks 0: the walk
 static float blk32_walk_us(int wtype, int64_t K, int64_t N, int64_t M, int64_t cus) {
@@ -693,9 +694,10 @@ static float blk32_walk_us(int wtype, int64_t K, int64_t N, int64_t M, int64_t c
     if (rest) t += 3.6f + stages * std::max(0.59f, stage * std::max(1.f, (float)rest / (float)cus));
     return slices > 1 ? t + 2.7f + 0.9e-6f * (float)N * (float)M * (float)slices : t;
 }
-static FewPlan blk32_few_plan(int wtype, int64_t K, int64_t N, int64_t M, size_t nb01, int64_t cus) {
+static FewPlan blk32_few_plan(int wtype, int64_t K, int64_t N, int64_t M, size_t nb01, int64_t cus, bool room) {
     const int64_t tiles = ceil_div(N, (int64_t)32) * ceil_div(M, (int64_t)32);
     if (K < 256 || tiles > 65536 || nb01 > ((size_t)1 << 27)) return FewPlan{0, 1};           // (rows within 32-bit reach)
+    if (!room && blk32_slices_for(K, N, M, cus) > 1) return FewPlan{0, 1};
     float best = blk32_walk_us(wtype, K, N, M, cus) / 1.15f;
     FewPlan plan{0, 1};
     for (int ks = 2; ks <= 8; ks *= 2) {
@@ -741,7 +743,7 @@ static hipError_t launch_type(const GemmMats &mats, int64_t K, const void *ws, s
     const int64_t cus = lim.compute_units > 0 ? lim.compute_units : 256;
     if (!rg.perm) {                                                      // (the members of a group have the plan of the first)
         const GemmMat &m = mats.m[0];
-        FewPlan few = blk32_few_plan(WT, K, m.N, M, m.nb01, cus);
+        FewPlan few = blk32_few_plan(WT, K, m.N, M, m.nb01, cus, split.part != nullptr);
         if (const int f = (int)tune("CHIP_BLK32_FEW", 0); f) few = FewPlan{f % 10 == 9 ? 0 : f % 10, f / 100 + 1};
         const bool near = blk32_near(WT, K, m.N, M);
         if (few.slices > 1 && !(split.part && split.bytes >= (size_t)few.slices * (size_t)M * (size_t)m.N * sizeof(float) && (((uintptr_t)split.part) & 15) == 0))
@@ -810,9 +812,9 @@ hipError_t launch_gemm_blk32(int wtype, const void *W, size_t nb01, int64_t K, i
 bool gemm_blk32_group_applicable(int wtype, int64_t K, const GemmMats &mats, int64_t n, int compute_units) {
     if (mats.count < 2) return false;
     const int64_t cus = compute_units > 0 ? compute_units : 256;
-    const FewPlan first = blk32_few_plan(wtype, K, mats.m[0].N, n, mats.m[0].nb01, cus);
+    const FewPlan first = blk32_few_plan(wtype, K, mats.m[0].N, n, mats.m[0].nb01, cus, false);
     for (int i = 0; i < mats.count; i++) {
-        const FewPlan few = blk32_few_plan(wtype, K, mats.m[i].N, n, mats.m[i].nb01, cus);
+        const FewPlan few = blk32_few_plan(wtype, K, mats.m[i].N, n, mats.m[i].nb01, cus, false);
         if (few.ks != first.ks || few.slices != 1 || (few.ks == 0 && gemm_blk32_slices(wtype, K, mats.m[i].N, n, compute_units) != 1) ||
             !gemm_blk32_supported(wtype, K, mats.m[i].N, n, false) || blk32_near(wtype, K, mats.m[i].N, n) != blk32_near(wtype, K, mats.m[0].N, n))
             return false;
