@@ -7,6 +7,7 @@
 #include <math.h>
 #include "kernels.h"
 
+#include <algorithm>
 #include <atomic>
 #include <cstdio>
 #include <cstring>
@@ -395,7 +396,7 @@ static bool mmv_rows_in_reach(size_t nb01) { return nb01 <= ((size_t)1 << 28); }
 // workgroup, after its tiles of the first matrix, takes the same tiles of the second (the activation image is built once;
 // every tile is computed as in a launch of its own: the same bits).
 static bool mmv_pair_applicable(int type, size_t nb01, int64_t K, int64_t N, int64_t n, const DeviceLimits &lim) {
-    if (!mmv_rows_in_reach(nb01)) return false;
+    if (!mmv_rows_in_reach(nb01) || kq_few_plan(type, nb01, K, N, n, false, lim.compute_units).ks > 0) return false;
     if (n < 5 || n > 8 || !(type == T_Q4_K || type == T_Q5_K) || tune("CHIP_MMV_PAIR", 1) == 0) return false;
     if (gemm_kq_supported(type, K, N, n, false) || gemm_kq_supported(type, K, N, n, true)) return false;
     return n >= mmv_min_tokens(type, K, N) && n <= mmv_q4k_max_tokens(type, K, N, lim);
@@ -410,6 +411,14 @@ int chip_mul_mat_run_ws(int type, const void *W, size_t nb01, int64_t K, int64_t
                         float *y, int64_t ldy, void *stream) {
     if (workspace_bytes < chip_mul_mat_workspace_size(type, K, n)) return CHIP_ENOMEM;
     return mul_mat_run(type, W, nb01, K, N, n, workspace, workspace_bytes, y, ldy, stream);
+}
+// K is split only with room for every slice's partial output behind the activation rows
+static SplitK split_room(int type, int64_t K, int64_t N, int64_t n, const void *workspace, size_t workspace_bytes, const DeviceLimits &lim) {
+    const size_t act = act_rows_bytes(type, K, n);
+    if (workspace_bytes <= act) return SplitK{nullptr, 0};
+    const SplitK split{reinterpret_cast<float *>((uint8_t *)const_cast<void *>(workspace) + act), workspace_bytes - act};
+    const int slices = split_slices(type, K, N, n, lim.compute_units);
+    return slices > 1 && split.bytes >= (size_t)slices * (size_t)n * (size_t)N * sizeof(float) ? split : SplitK{nullptr, 0};
 }
 // workspace_bytes: what the caller says lies behind `workspace` (0 = the activation rows only, no room for split-K partials)
 static int mul_mat_run(int type, const void *W, size_t nb01, int64_t K, int64_t N, int64_t n, const void *workspace,
@@ -426,13 +435,10 @@ static int mul_mat_run(int type, const void *W, size_t nb01, int64_t K, int64_t 
     const size_t stride = act_stride(chip_vec_dot_type(type), K);
     hipStream_t st = (hipStream_t)stream;
 
-    SplitK split{nullptr, 0};
-    if (const size_t act = act_rows_bytes(type, K, n); workspace_bytes > act)
-        split = SplitK{reinterpret_cast<float *>((uint8_t *)const_cast<void *>(workspace) + act), workspace_bytes - act};
-    // K is split only with room for every slice's partial output behind the activation rows
-    const int want_slices = split.part ? split_slices(type, K, N, n, lim.compute_units) : 1;
-    const bool can_split = want_slices > 1 && split.bytes >= (size_t)want_slices * (size_t)n * (size_t)N * sizeof(float);
-    if (!can_split) split = SplitK{nullptr, 0};
+    const SplitK split = split_room(type, K, N, n, workspace, workspace_bytes, lim);
+    const bool can_split = split.part != nullptr;
+    if (const KqFew f = kq_few_plan(type, nb01, K, N, n, can_split, lim.compute_units); f.ks > 0)
+        return hip_rc(launch_gemm_kq_few(f, &type, one_gemm_mat(W, nb01, N, y, ldy), K, workspace, stride, n, lim, st));
     if (gemm_blk32_supported(type, K, N, n, can_split))
         return hip_rc(launch_gemm_blk32(type, W, nb01, K, N, workspace, stride, n, y, ldy, lim, st, nullptr, 1, split));
     if (type == T_F16 && gemm_f16_supported(K, N, n))
@@ -500,9 +506,44 @@ int chip_mul_mat_noalloc(int type, const void *W, size_t nb01, int64_t K, int64_
     return chip_mul_mat(type, W, nb01, K, N, x, ldx, n, y, ldy, sp, NOALLOC_SCRATCH_BYTES, stream);
 }
 
+static KqFew few_for(const GroupMat &m, int64_t K, int64_t n, const void *workspace, size_t workspace_bytes, const DeviceLimits &lim) {
+    return kq_few_plan(m.wtype, m.nb01, K, m.N, n, split_room(m.wtype, K, m.N, n, workspace, workspace_bytes, lim).part != nullptr, lim.compute_units);
+}
+// Every member in gemm_kq_few_kernel by itself, with one number of waves, and no more than two types: one launch with the bits of the single calls.
+static bool few_group(const GroupMat *gm, int live, int64_t K, int64_t n, const void *workspace, size_t workspace_bytes, const DeviceLimits &lim,
+                      KqFew &f, int *types, GemmMats &mats) {
+    mats = GemmMats{};
+    f = KqFew{1, n > 16 ? 2 : 1, 0};
+    if (live > GEMM_MATS_MAX) return false;
+    const int lo = std::min_element(gm, gm + live, [](const GroupMat &a, const GroupMat &b) { return a.wtype < b.wtype; })->wtype;
+    int hi = lo;
+    for (int i = 0; i < live; i++) {
+        const KqFew m = few_for(gm[i], K, n, workspace, workspace_bytes, lim);
+        if (m.ks == 0 || (f.ks > 0 && m.ks != f.ks)) return false;
+        f.ks = m.ks;
+        f.rt = std::max(f.rt, m.rt);
+        if (gm[i].wtype != lo) {
+            if (hi != lo && gm[i].wtype != hi) return false;
+            hi = gm[i].wtype;
+        }
+    }
+    if (hi != lo) f.rt = 1;
+    for (int t : {lo, hi})
+        for (int i = 0; i < live; i++)
+            if (gm[i].wtype == t && mats.count < live) {
+                types[mats.count] = t;
+                mats.m[mats.count++] = GemmMat{(const uint8_t *)gm[i].W, gm[i].nb01, gm[i].N, gm[i].y, gm[i].ldy};
+            }
+    return true;
+}
 // The members [0, live) of a group over prepared rows, each as chip_mul_mat_run would; those of one type that the GEMM takes, and whose
 // tiles it runs faster together, in one launch.
 static int run_members(const GroupMat *gm, int live, int64_t K, int64_t n, void *workspace, size_t workspace_bytes, const DeviceLimits &lim, void *stream) {
+    KqFew few;
+    int types[GEMM_MATS_MAX];
+    GemmMats all;
+    if (live > 1 && few_group(gm, live, K, n, workspace, workspace_bytes, lim, few, types, all))
+        return hip_rc(launch_gemm_kq_few(few, types, all, K, workspace, act_stride(chip_vec_dot_type(types[0]), K), n, lim, (hipStream_t)stream));
     unsigned done = 0;
     for (int i = 0; i < live; i++) {
         if (done >> i & 1) continue;
@@ -516,7 +557,11 @@ static int run_members(const GroupMat *gm, int live, int64_t K, int64_t n, void 
             }
         const size_t stride = act_stride(chip_vec_dot_type(type), K);
         hipError_t e = hipErrorNotSupported;
-        if (mats.count > 1 && gemm_blk32_group_applicable(type, K, mats, n, lim.compute_units))
+        bool any_few = false;
+        for (int j = i; j < live; j++) any_few |= (set >> j & 1) && few_for(gm[j], K, n, workspace, workspace_bytes, lim).ks > 0;
+        if (mats.count > 1 && any_few)
+            ;                                                            // each by itself
+        else if (mats.count > 1 && gemm_blk32_group_applicable(type, K, mats, n, lim.compute_units))
             e = launch_gemm_blk32_group(type, mats, K, workspace, stride, n, lim, (hipStream_t)stream);
         else if (mats.count > 1 && gemm_kq_group_applicable(type, K, mats, n, lim.compute_units))
             e = launch_gemm_kq_group(type, mats, K, workspace, stride, n, lim, (hipStream_t)stream);

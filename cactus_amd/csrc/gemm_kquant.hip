@@ -517,6 +517,89 @@ int gemm_kq_slices(int wtype, int64_t K, int64_t N, int64_t n, int compute_units
     return kq_plan(wtype, K, N, n, cus).slices;
 }
 
+// gemm_kq_few_kernel against whatever else would run the product: both times are estimated, in us, and it is taken where it is ahead by 7 per cent.
+// Fitted to 12500 products (512 to 14336 values, 256 to 20000 rows, 5 to 300 tokens; each with up to five forms of this kernel), which it is within 7 per
+// cent of (the others within 5 to 10; the matrix-core GEMVs 23).  Over the same products: 5 to 8 tokens 1.28 x, 9 to 16 1.78, 17 to 32 1.56, 33 to
+// 64 1.42, to 128 1.32, to 300 1.20; the best form that there is would be 1 to 2 per cent faster still; one product in 110 is more than 3 per cent slower.
+//   fixed, turn   launch, first loads and the sum of the waves; once more per turn of the workgroups that fit the device
+//   walk          a super-block of one wave after the other
+//   work, cu      vector instructions: super-blocks per SIMD, on average and on the busiest CU
+struct FewForm { int rt, tt, ks; float fixed, turn, walk, work, cu; };
+static constexpr FewForm kFewForms[] = {
+    {1, 1, 4, 2.764f, 0.553f, 0.249f, 0.235f, 0.377f}, {1, 1, 8, 2.582f, 0.780f, 0.071f, 0.159f, 0.483f}, {1, 1, 16, 1.795f, 1.679f, 0.111f, 0.173f, 0.473f},
+    {2, 1, 2, 0.f, 3.677f, 0.607f, 0.370f, 0.780f},    {2, 1, 4, 0.f, 3.803f, 0.390f, 0.415f, 0.643f},    {1, 2, 4, 3.117f, 1.037f, 0.252f, 0.169f, 0.517f},
+    {1, 2, 8, 2.062f, 1.785f, 0.090f, 0.156f, 0.640f}, {2, 2, 2, 4.216f, 0.818f, 0.843f, 0.206f, 0.788f}, {2, 2, 4, 4.119f, 0.896f, 0.487f, 0.274f, 0.798f},
+    {2, 2, 8, 2.349f, 1.802f, 0.438f, 0.211f, 1.005f}};
+// a type's share of the walk and the work; the GEMMs: fixed, slices of K, a walk's super-block, a turn, super-blocks per workgroup slot, the walk of a
+// second token tile, a million partial outputs; the dot-product GEMV: a pass, its rounds of 1024 rows, then per token parts of 4096 values, those times the
+// rounds, and the same per pass; the matrix-core GEMV: a pass, its steps of 16 rows a CU, 1e4 values per pass, 1e5 per token, steps per 10 tokens
+struct KqTimes { float few, gemm[7], gemv[5], mmv[5]; };
+static const KqTimes &kq_times(int wtype) {
+    static const KqTimes q4k{0.936f, {2.946f, 2.733f, 0.783f, 2.216f, 1.611f, 0.353f, 1.469f}, {3.178f, 0.f, 0.108f, 0.132f, 0.f}, {5.602f, 0.f, 0.f, 2.018f, 0.785f}};
+    static const KqTimes q5k{1.206f, {1.790f, 2.643f, 1.163f, 3.531f, 1.524f, 0.357f, 1.793f}, {3.051f, 0.f, 0.120f, 0.118f, 0.211f}, {5.714f, 0.093f, 0.f, 2.391f, 0.836f}};
+    static const KqTimes q6k{1.284f, {2.948f, 2.387f, 1.055f, 2.261f, 1.456f, 0.231f, 2.027f}, {3.437f, 0.207f, 0.126f, 0.105f, 0.075f}, {}};
+    static const KqTimes q3k{0.887f, {2.393f, 2.177f, 0.744f, 2.435f, 1.179f, 0.251f, 1.955f}, {3.182f, 0.271f, 0.135f, 0.093f, 0.120f}, {}};
+    static const KqTimes q2k{0.85f, {4.631f, 2.364f, 0.616f, 0.f, 1.671f, 0.321f, 1.015f}, {3.041f, 0.218f, 0.140f, 0.114f, 0.f}, {}};
+    static const KqTimes iq4{1.348f, {5.142f, 2.518f, 1.090f, 0.f, 2.777f, 0.418f, 0.816f}, {2.961f, 0.232f, 0.146f, 0.107f, 0.017f}, {}};
+    switch (wtype) {
+        case T_Q4_K: return q4k;
+        case T_Q5_K: return q5k;
+        case T_Q6_K: return q6k;
+        case T_Q3_K: return q3k;
+        case T_Q2_K: return q2k;
+        default:     return iq4;
+    }
+}
+static float few_estimate(const FewForm &f, int wtype, int64_t K, int64_t N, int64_t n, int64_t cus) {
+    const int64_t units = K / QK_K, blocks = ceil_div(N, (int64_t)(16 * f.rt)) * ceil_div(n, (int64_t)(16 * f.tt));
+    const int simd = f.rt * f.tt == 1 ? 4 : f.rt * f.tt == 2 ? 3 : 2;                    // waves a SIMD's registers hold
+    const int64_t slots = cus * std::max<int64_t>(1, std::min(160 * 1024 / (gemm_kq_few_stretch(wtype, f.rt, f.tt) * f.ks), 4 * simd / f.ks));
+    const float turns = (float)ceil_div(blocks, slots);
+    return f.fixed + f.turn * turns + kq_times(wtype).few * (f.walk * turns * (float)ceil_div(units, (int64_t)f.ks) + f.work * (float)(blocks * units) / (float)(4 * cus) +
+                                                             f.cu * (float)(ceil_div(blocks, cus) * units) / 4.f);
+}
+// the GEMM, the matrix-core GEMV (Q4_K, Q5_K) or the dot-product GEMV, whichever a caller with room for partial outputs would reach
+static float others_estimate(int wtype, int64_t K, int64_t N, int64_t n, const KqPlan &p, int64_t cus) {
+    const KqTimes &t = kq_times(wtype);
+    const bool four = wtype == T_Q4_K || wtype == T_Q5_K;
+    const int64_t units = K / QK_K;
+    if (four ? n >= gemm_kq_min_tokens(wtype, K, N, p.slices > 1) : n >= 9) {
+        const int64_t per = ceil_div(ceil_div(units, (int64_t)p.slices), (int64_t)(p.groups == 2 ? 2 : 1));
+        const int64_t tiles = p.groups == 0 ? ceil_div(N, (int64_t)64) * ceil_div(n, (int64_t)128) : ceil_div(N, (int64_t)128) * ceil_div(n, (int64_t)64);
+        const float turns = (float)ceil_div(tiles * p.slices, cus * (p.groups == 1 ? 2 : 1)), walk = turns * (float)per;
+        return t.gemm[0] + (p.slices > 1 ? t.gemm[1] + t.gemm[6] * (float)p.slices * (float)(N * n) * 1e-6f : 0.f) + (t.gemm[2] + (n > 32 ? t.gemm[5] : 0.f)) * walk +
+               t.gemm[3] * turns + t.gemm[4] * (float)(tiles * units) / (float)(2 * cus);
+    }
+    if (four && n >= (N * K >= (32LL << 20) ? 5 : 7)) {
+        const float passes = (float)ceil_div(n, (int64_t)(K <= 6144 ? 16 : 8)), steps = (float)ceil_div(ceil_div(ceil_div(N, (int64_t)16), cus) * units, (int64_t)8);
+        return passes * (t.mmv[0] + t.mmv[1] * steps + t.mmv[2] * 1e-4f * (float)K) + (float)n * (t.mmv[3] * 1e-5f * (float)K + t.mmv[4] * 0.1f * steps);
+    }
+    const float passes = (float)ceil_div(n, (int64_t)8), rounds = (float)ceil_div(N, (int64_t)1024), parts = (float)ceil_div(K, (int64_t)4096);
+    return passes * (t.gemv[0] + t.gemv[1] * rounds + t.gemv[4] * parts * rounds) + (float)n * parts * (t.gemv[2] + t.gemv[3] * rounds);
+}
+// Forms of 32 tokens above 16 tokens.  Rows of two super-blocks up to 32 tokens, of three there for the types without a matrix-core GEMV, from four on
+// otherwise: K is what the waves share.  Above 32 tokens a caller without room for slices of K keeps the order of one walk over it.  Products that
+// are known to run in slices of K and a slice sum stay there: long rows on many rows (us, slices / this, 14336 values x 4096 rows at 32 tokens: Q4_K 19.8
+// / 18.9, Q6_K 23.9 / 20.8, Q3_K 19.6 / 16.8) and a few rows above 64 tokens.  Up to 320 tokens, where the estimates were fitted.
+KqFew kq_few_plan(int wtype, size_t nb01, int64_t K, int64_t N, int64_t n, bool can_split, int compute_units) {
+    if (!gemm_kq_type(wtype) || n < 5 || n > 320 || N < 1 || K % QK_K != 0 || nb01 > ((size_t)1 << 28)) return KqFew{0, 0, 0};
+    const int64_t cus = compute_units > 0 ? compute_units : 256, units = K / QK_K, forced = tune("CHIP_KQ_FEW", -1);
+    if (forced > 0) return units >= forced % 100 ? KqFew{(int)(forced / 1000), (int)(forced / 100 % 10), (int)(forced % 100)} : KqFew{0, 0, 0};
+    const bool four = wtype == T_Q4_K || wtype == T_Q5_K;
+    if (forced == 0 || units < (n <= 32 ? 2 : 4) || (units == 3 && four) || tune("CHIP_GEMM_MIN_TOKENS", 0) > 0) return KqFew{0, 0, 0};
+    const KqPlan p = kq_plan(wtype, K, N, n, cus);
+    if (n > 32 && p.slices > 1 && !can_split) return KqFew{0, 0, 0};
+    if (p.slices > 1 && ((n > 16 && K > 8192 && N > 2048) || (n > 64 && N < 320))) return KqFew{0, 0, 0};
+    KqFew best{0, 0, 0};
+    float least = 0.93f * others_estimate(wtype, K, N, n, p, cus);
+    for (const FewForm &f : kFewForms) {
+        // (one row tile of long rows over few waves: 1.3 x as long as estimated for Q2_K 14336 values x 4096 rows at 72 tokens)
+        if (f.tt != (n > 16 ? 2 : 1) || f.ks > units || (f.rt == 1 && f.tt == 2 && f.ks == 4 && K > 8192 && n > 32)) continue;
+        if (const float e = few_estimate(f, wtype, K, N, n, cus); e < least) { least = e; best = KqFew{f.rt, f.tt, f.ks}; }
+    }
+    return best;
+}
+
 using KqTile = KqCfg<T_Q6_K, 2, 2>;                                          // 64 x 128, 4 + 4 waves
 template <int WT, bool GATHER>
 static hipError_t launch_kq(const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, int64_t M,

@@ -337,6 +337,14 @@ hipError_t launch_gemm_kq(int wtype, const void *W, size_t nb01, int64_t K, int6
 // gemm_kquant_rows.hip: the same product by waves that expand their own rows; groups: 1 or 2 k groups a workgroup, slices: parts of K
 hipError_t launch_gemm_kr(int groups, int wtype, const GemmMats &mats, int64_t K, const void *ws, size_t ws_stride, int64_t n,
                           const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t slots, int slices, float *part);
+// gemm_kquant_few.hip: the same product for few tokens, in tiles of 16 rt rows x 16 tt tokens (rt, tt: 1 or 2) whose K is shared by ks waves (no more than K
+// has super-blocks, at most 16, and 8 where rt or tt is 2).  kq_few_plan: ks 0 where another kernel is taken; can_split: the caller's workspace
+// has room for slices of K.  What a product's bits depend on is ks.
+struct KqFew { int rt, tt, ks; };
+KqFew      kq_few_plan(int wtype, size_t nb01, int64_t K, int64_t N, int64_t n, bool can_split, int compute_units);
+int        gemm_kq_few_stretch(int wtype, int rt, int tt);                // bytes of LDS a wave takes
+hipError_t launch_gemm_kq_few(KqFew f, const int *types, const GemmMats &mats, int64_t K, const void *ws, size_t ws_stride, int64_t n, const DeviceLimits &lim,
+                              hipStream_t st);
 int        gemm_kr_tile_tokens();
 int64_t    gemm_kr_rows_in_reach(size_t nb01);
 // Several matrices of one type on the same rows in one launch.  _applicable: every member alone would take the GEMM, unsplit; its

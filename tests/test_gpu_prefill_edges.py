@@ -375,6 +375,38 @@ def test_slices_of_k_as_near_as_whole_rows(dev, orc, wt):
     assert distance(orc, wt, K, w, x, slices) <= 1.03 * distance(orc, wt, K, w, x, whole)
 
 
+# ---- K-quants, 5 to 40 tokens: tiles of 16 or 32 rows and tokens whose super-blocks are shared by waves ----
+# (K, N, n): one row and two super-blocks, a wave each; ragged rows and more waves than a row has left over; 16 and 17 tokens; a second token tile of one
+# token; an odd number of super-blocks over eight waves; more row tiles than a turn of workgroups; more waves than 48 KB of local memory serve
+@pytest.mark.parametrize("wt", (O.Q4_K, O.Q5_K, O.Q6_K) + LOW_BIT, ids=lambda t: O.TYPE_NAMES[t])
+@pytest.mark.parametrize("K,N,n", [(512, 1, 9), (1280, 33, 16), (1280, 47, 17), (1024, 130, 33), (2816, 300, 40), (1024, 20000, 9), (14336, 4000, 9)])
+def test_kquant_few_tokens(dev, orc, wt, K, N, n):
+    w = np.tile(orc.quantize_weights(wt, common.weights_f32(K + N, min(N, 200), K)), (-(-N // 200), 1))[:N]
+    x = common.activations_f32(K + n, n, K)
+    x[3] = 0
+    assert mul_mat_launches(dev, wt, w, x) == 2
+    y = dev.mul_mat(wt, w, x)
+    assert y.tobytes() == dev.mul_mat(wt, w, x).tobytes() and np.array_equal(y[:, 200:], y[:, :max(N - 200, 0)] if N < 400 else y[:, :-200])
+    rows = np.unique(np.concatenate([np.arange(min(N, 60)), [N - 1]]))
+    check(y[:, rows], orc.mul_mat(wt, w[rows], x, nthreads=8, want=("sum_abs",)), "few tokens")
+    gemv = np.concatenate([dev.mul_mat(wt, w, x[i:i + 4]) for i in range(0, n, 4)])
+    if len(rows) > 40:                        # (2-norms of some hundred outputs: within a tenth)
+        assert distance(orc, wt, K, w[rows], x, y[:, rows]) <= 1.1 * distance(orc, wt, K, w[rows], x, gemv[:, rows])
+
+
+# members of one and of two types, in any order: one launch behind the quantizer, the bits of the single calls
+@pytest.mark.parametrize("types", [(O.Q4_K, O.Q4_K, O.Q6_K), (O.Q6_K, O.Q3_K), (O.IQ4_XS, O.Q2_K, O.IQ4_XS), (O.Q5_K, O.Q4_K), (O.Q5_K, O.Q5_K, O.Q5_K)],
+                         ids=lambda ts: "-".join(O.TYPE_NAMES[t] for t in ts))
+@pytest.mark.parametrize("n", (9, 20))
+def test_kquant_few_tokens_in_a_group(dev, orc, types, n):
+    K = 1024
+    ws = [(t, orc.quantize_weights(t, common.weights_f32(K + i, N, K))) for i, (t, N) in enumerate(zip(types, (200, 33, 129)))]
+    x = common.activations_f32(K + n, n, K)
+    assert group_launches(dev, [(t, w.shape[0]) for t, w in ws], K, n) == 2
+    for (t, w), y in zip(ws, dev.mul_mat_group(ws, x)):
+        assert y.tobytes() == dev.mul_mat(t, w, x).tobytes(), O.TYPE_NAMES[t]
+
+
 # an infinite weight scale gives infinities, not NaN, also where the roundings of the sum are kept
 @pytest.mark.parametrize("wt", (O.Q4_0, O.Q8_0, O.Q5_0, O.IQ4_NL), ids=lambda t: O.TYPE_NAMES[t])
 def test_block32_few_tokens_with_an_infinite_scale(dev, orc, wt):
