@@ -582,7 +582,7 @@ static float others_estimate(int wtype, int64_t K, int64_t N, int64_t n, const K
 // are known to run in slices of K and a slice sum stay there: long rows on many rows (us, slices / this, 14336 values x 4096 rows at 32 tokens: Q4_K 19.8
 // / 18.9, Q6_K 23.9 / 20.8, Q3_K 19.6 / 16.8) and a few rows above 64 tokens.  Up to 320 tokens, where the estimates were fitted.
 KqFew kq_few_plan(int wtype, size_t nb01, int64_t K, int64_t N, int64_t n, bool can_split, int compute_units) {
-    if (!gemm_kq_type(wtype) || n < 5 || n > 320 || N < 1 || K % QK_K != 0 || nb01 > ((size_t)1 << 28)) return KqFew{0, 0, 0};
+    if (!gemm_kq_type(wtype) || n < 5 || n > 1200 || N < 1 || K % QK_K != 0 || nb01 > ((size_t)1 << 28)) return KqFew{0, 0, 0};
     const int64_t cus = compute_units > 0 ? compute_units : 256, units = K / QK_K, forced = tune("CHIP_KQ_FEW", -1);
     if (forced > 0) return units >= forced % 100 ? KqFew{(int)(forced / 1000), (int)(forced / 100 % 10), (int)(forced % 100)} : KqFew{0, 0, 0};
     const bool four = wtype == T_Q4_K || wtype == T_Q5_K;
