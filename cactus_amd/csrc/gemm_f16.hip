@@ -19,16 +19,16 @@ namespace chip {
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
-constexpr int F16_KG = 4;                     // 16-value k-groups per LDS stage
+constexpr int F16_KG = 4;                     // 16-value k-groups per LDS stage (or twice as many: KG)
 
-template <int TM, int TN, int WR, int WC>
+template <int TM, int TN, int WR, int WC, int KG = F16_KG>
 struct F16Cfg {
     static constexpr int NW = WR * WC, NT = NW * 64;
     static constexpr int BM = 32 * TM * WR;                        // weight rows per workgroup
     static constexpr int BN = 32 * TN * WC;                        // tokens per workgroup
-    // plane stride 2 mod 16 cells: the staging threads of one wave spread over the bank groups
-    static constexpr int A_PLANE = BM + 2, B_PLANE = BN + 2;
-    static constexpr int CELLS = F16_KG * 2;                       // 16-byte cells per row and stage
+    static constexpr int CELLS = KG * 2;                           // 16-byte cells per row and stage
+    // plane stride 2 (16 cells: 1) mod 16 cells: the staging threads of one wave spread over the bank groups
+    static constexpr int A_PLANE = BM + 16 / CELLS, B_PLANE = BN + 16 / CELLS;
     static constexpr size_t OFF_A = 0;
     static constexpr size_t OFF_B = OFF_A + (size_t)CELLS * A_PLANE * 16;
     static constexpr size_t STAGE = OFF_B + (size_t)CELLS * B_PLANE * 16;
@@ -46,9 +46,8 @@ struct F16Cfg {
 enum F16Mode { F16_PLAIN, F16_EXPERTS, F16_BATCH };
 // AHEAD: stages whose loads are in flight, each in a register set of its own.  With few tiles the kernel is bound by the latency
 // of its loads: a stage's 4 (16) MFMAs a wave end long before the next stage's weights have come from HBM.  One stage ahead -> AHEAD
-// (us, a different 4096 x 4096 F16 matrix each call, which no cache holds): 64 x 64 tiles, AHEAD 3: 64 tokens 38.4 -> 26.6, 201
-// tokens 41.3 -> 30.0, 512 tokens 61.7 -> 45.2 (AHEAD 2: 29.8, 33.3, 44.6; AHEAD 4 at three workgroups a CU: 26.0, 28.7, 45.8;
-// at four it spills: 66.9, 70.7, 111); 128 tokens of 14336 x 4096: 179 -> 106.  128 x 128 tiles, AHEAD 2: 1024 tokens 83.8 -> 66.6.
+// (us, a different 4096 x 4096 F16 matrix each call, which no cache holds): 64 x 64 tiles, AHEAD 2: 64 tokens 38.4 -> 29.8, 201
+// tokens 41.3 -> 33.3, 512 tokens 61.7 -> 44.6.  128 x 128 tiles, AHEAD 2: 1024 tokens 83.8 -> 66.6.
 // More workgroups a CU cover each other's loads, and the deeper prefetch then only crowds the caches (launch_gemm_f16).
 __device__ __forceinline__ u32x4 round8_f16(const float4 a, const float4 b) {
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
@@ -60,12 +59,12 @@ __device__ __forceinline__ u32x4 round8_f16(const float4 a, const float4 b) {
     return r;
 }
 
-template <int TM, int TN, int WR, int WC, int OCC, F16Mode MODE, bool XF32, int AHEAD>
+template <int TM, int TN, int WR, int WC, int OCC, F16Mode MODE, bool XF32, int AHEAD, int KG>
 __global__ __launch_bounds__(WR *WC * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 void gemm_f16_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int64_t N, const uint8_t *__restrict__ ws,
                      size_t ws_stride, int64_t M, float *__restrict__ y, int64_t ldy, TileMap map, RowGather rg, F16Batch fb) {
     static_assert(!XF32 || MODE == F16_BATCH, "fp32 activation rows come with the attention mode");
-    using C = F16Cfg<TM, TN, WR, WC>;
+    using C = F16Cfg<TM, TN, WR, WC, KG>;
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -96,9 +95,10 @@ void gemm_f16_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int6
     if (tok_base >= M) return;
     // The attention mode also takes K that is not a multiple of the 64-value stage (n_kv cache positions, a multiple of 8):
     // cells of the last stage that lie past K are zeroed on both sides.
-    constexpr bool KTAIL = MODE == F16_BATCH;
-    const int nstages = (int)(KTAIL ? ceil_div(K, (int64_t)(16 * F16_KG)) : K / (16 * F16_KG));
-    constexpr int STAGE_BYTES = 16 * F16_KG * 2;                   // bytes of one row per stage
+    // (as are those of a last stage that 64 values are left for, KG = 8)
+    constexpr bool KTAIL = MODE == F16_BATCH || KG > F16_KG;
+    const int nstages = (int)(KTAIL ? ceil_div(K, (int64_t)(16 * KG)) : K / (16 * KG));
+    constexpr int STAGE_BYTES = 16 * KG * 2;                   // bytes of one row per stage
     static_assert(C::NT % C::CELLS == 0, "a thread's items all have the same cell index");
     const int my_cell = tid % C::CELLS;
 
@@ -127,7 +127,7 @@ void gemm_f16_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int6
     auto fetch = [&](auto set, int stage) {
         auto &wq = wqs[decltype(set)::value]; auto &xq = xqs[decltype(set)::value]; auto &xf = xfs[decltype(set)::value];
         bool &live = lives[decltype(set)::value];
-        live = !KTAIL || (int64_t)stage * (16 * F16_KG) + 8 * my_cell < K;
+        live = !KTAIL || (int64_t)stage * (16 * KG) + 8 * my_cell < K;
         const size_t off = live ? (size_t)stage * STAGE_BYTES : 0;                   // a dead cell re-reads stage 0 (in bounds) and is zeroed
 #pragma unroll
         for (int i = 0; i < C::W_PER_T; i++) wq[i] = *reinterpret_cast<const u32x4 *>(wsrc[i] + off);
@@ -178,7 +178,7 @@ void gemm_f16_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int6
         const f16x8 *A = reinterpret_cast<const f16x8 *>(lds + (size_t)buf * C::STAGE + C::OFF_A);
         const f16x8 *B = reinterpret_cast<const f16x8 *>(lds + (size_t)buf * C::STAGE + C::OFF_B);
 #pragma unroll
-        for (int g = 0; g < F16_KG; g++) {
+        for (int g = 0; g < KG; g++) {
             f16x8 af[TM], bf[TN];
 #pragma unroll
             for (int a = 0; a < TM; a++) af[a] = A[(g * 2 + half) * C::A_PLANE + (wr * TM + a) * 32 + l32];
@@ -395,13 +395,14 @@ static hipError_t launch_f16_direct(const void *W, size_t nb01, int64_t K, int64
 // rows must be 16-byte aligned (the weight alignment rule of the C-ABI) and K a multiple of the 64-value stage
 bool gemm_f16_supported(int64_t K, int64_t N, int64_t n) { return K >= 64 && K % (16 * F16_KG) == 0 && N >= 1 && n >= 32; }
 
-template <int TM, int TN, int WR, int WC, int OCC, F16Mode MODE, bool XF32 = false, int AHEAD = 1>
+template <int TM, int TN, int WR, int WC, int OCC, F16Mode MODE, bool XF32 = false, int AHEAD = 1, int KG = F16_KG>
 static hipError_t launch_f16(const void *W, size_t nb01, int64_t K, int64_t N, const void *ws, size_t ws_stride, int64_t M,
                              float *y, int64_t ldy, const DeviceLimits &lim, hipStream_t st, const RowGather &rg, int64_t n_as,
                              const F16Batch &fb = F16Batch{1, 0, 0, nullptr, 0, 0, 1}) {
-    using C = F16Cfg<TM, TN, WR, WC>;
+    using C = F16Cfg<TM, TN, WR, WC, KG>;
     const size_t lds_bytes = 2 * C::STAGE;
-    auto kfn = gemm_f16_kernel<TM, TN, WR, WC, OCC, MODE, XF32, AHEAD>;
+    if ((int64_t)lds_bytes > lim.max_lds_per_block) return hipErrorInvalidValue;
+    auto kfn = gemm_f16_kernel<TM, TN, WR, WC, OCC, MODE, XF32, AHEAD, KG>;
     static LdsGrant grant;
     if (hipError_t e = grant_dynamic_lds(kfn, lds_bytes, lim, grant); e != hipSuccess) return e;
     TileMap map = make_tile_map(ceil_div(N, C::BM), MODE == F16_PLAIN ? ceil_div(M, C::BN) : 1, 32 * (4 * OCC / C::NW > 0 ? 4 * OCC / C::NW : 1));
@@ -458,17 +459,21 @@ hipError_t launch_gemm_f16(const void *W, size_t nb01, int64_t K, int64_t N, con
     const int64_t cus = lim.compute_units > 0 ? lim.compute_units : 256;
     if (rg.perm) return launch_f16<1, 1, 2, 2, 4, F16_EXPERTS>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);      // expert groups: 64 x 64 tiles
     // Stages ahead, by the workgroups a CU runs (400 drawn products, median of the times against the other depth): 128 x 128, one
-    // a CU: 2 (1 is 14 % slower), more: 1 (3 % faster than 2 for K > 2048, the same below); 64 x 64, up to one and a half a CU: 3, more: 2
-    // (up to 2 a CU 1 %, from 2.5 a CU 3 % faster than 3; 1 is 5 to 35 % slower up to 2.5 a CU and no faster beyond).
+    // a CU: 2 (1 is 14 % slower), more: 1 (3 % faster than 2 for K > 2048, the same below); 64 x 64: 2 (1 is 5 to 35 % slower up to 2.5 a CU and no
+    // faster beyond).  Up to one and a half workgroups of 64 x 64 a CU a stage is 128 values: its loads, reads, MFMAs and barrier, which follow each
+    // other, come half as often.  Over 800 products 1.05 to 1.07 x against 64 values two or three ahead; at two a CU 2 % slower where a cache holds
+    // the matrix, from 2.5 on 4 % in any case.  Up to half a workgroup a CU 64 x 32 tiles, twice as many: 1.13 x.  us, 64 values two or three ahead -> now,
+    // 4096 x 4096 that no cache holds at 64 tokens 31.6 -> 26.4, 201 31.6 -> 28.2, 300 36.9 -> 34.5; 14336 x 4096 at 201 80.6 -> 75.9.
     const int64_t g128 = ceil_div(N, 128) * ceil_div(M, 128), g256 = ceil_div(N, 256) * ceil_div(M, 256), g64 = ceil_div(N, 64) * ceil_div(M, 64);
     const int cfg = (int)tune("CHIP_GEMM_F16_CFG", 2 * g256 >= cus && K >= 4 * BIG_K && n_as == 1 ? 9 : g128 >= cus ? 0 : 1);
     switch (cfg) {
         case 0:                                                                                                         // 128 x 128, 4 waves
             if (g128 > cus) return launch_f16<2, 2, 2, 2, 2, F16_PLAIN, false, 1>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
             return launch_f16<2, 2, 2, 2, 2, F16_PLAIN, false, 2>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
-        case 1:                                                                                                         // 64 x 64, 4 waves
-            if (2 * g64 > 3 * cus) return launch_f16<1, 1, 2, 2, 4, F16_PLAIN, false, 2>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
-            return launch_f16<1, 1, 2, 2, 4, F16_PLAIN, false, 3>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
+        case 1:                                                                                                         // 64 x 64, 4 waves; 64 x 32, 2 waves
+            if (2 * g64 <= cus) return launch_f16<1, 1, 2, 1, 2, F16_PLAIN, false, 2, 8>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
+            if (2 * g64 <= 3 * cus) return launch_f16<1, 1, 2, 2, 2, F16_PLAIN, false, 2, 8>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
+            return launch_f16<1, 1, 2, 2, 4, F16_PLAIN, false, 2>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
         case 9: return launch_f16_direct(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st);                             // 256 x 256, 4 waves, direct to LDS
         default: return hipErrorInvalidValue;
     }

@@ -215,6 +215,18 @@ def test_f16_gemm_stage_counts(dev, orc, K, N, n):
     check(y[np.ix_(toks, rows)], ref, "F16 gemm, %d stages" % (K // 64))
 
 
+# (K, N, n): 64 x 32 tiles with one token in the last, and two stages of 128 values; 64 x 64 tiles of one to two workgroups a CU; more
+@pytest.mark.parametrize("K,N,n", [(256, 70, 33), (1280, 1030, 97), (768, 2050, 520), (512, 8200, 333)])
+def test_f16_gemm_by_the_tiles_a_cu_gets(dev, orc, K, N, n):
+    rng = np.random.default_rng(K + N)
+    w = orc.quantize_weights(O.F16, common.weights_f32(K + N, N, K))
+    x = common.activations_f32(K + n, n, K)
+    y = dev.mul_mat(O.F16, w, x)
+    rows = np.unique(np.concatenate([[0, N - 1], rng.choice(N, 60, replace=False)]))
+    toks = np.unique(np.concatenate([[0, n - 1], rng.choice(n, 30, replace=False)]))
+    check(y[np.ix_(toks, rows)], orc.mul_mat(O.F16, w[rows], x[toks], nthreads=8, want=("sum_abs",)), "F16 gemm")
+
+
 # ---- matrices on one activation whose tiles share a launch: the bits of each by itself ----
 # (type, K, rows of each, n): one row tile and a ragged one, 64 x 64 tiles; more row tiles than CUs; a first member of one row; two
 # super-blocks and one of another type between; a K that is no multiple of a stage; Q6_K and Q3_K in the staging kernel (a launch each) and beside it
