@@ -426,10 +426,14 @@ static int kq_slices_for(int64_t K, int64_t N, int64_t M, int64_t cus) {
 }
 // How a product is covered: the staging kernel (groups 0), or gemm_kr_kernel in one or two k groups a workgroup (1: four waves that walk the
 // super-blocks in order, two workgroups a CU; 2: eight waves, four on the even and four on the odd super-blocks, one workgroup a CU); and slices of K.
-// Q3_K .. Q6_K run in the slices above and in one group - or, Q6_K and Q3_K with at most a 128 x 64 tile for every CU, in the staging kernel,
+// Q3_K .. Q6_K run in the slices above, mostly in one group - or, Q6_K and Q3_K with at most a 128 x 64 tile for every CU, in the staging kernel,
 // which expands a weight once for 128 tokens (us, staged / gemm_kr_kernel: Q6_K 14336 values x 4096 rows at 512 tokens 113 / 128, 201 tokens 66 / 74,
 // 4096 x 4096 at 512 tokens 38.6 / 44; Q3_K 14336 x 4096 at 201 tokens 49 / 53), unless half of its 128-token tile would be empty and the slices
 // give gemm_kr_kernel a workgroup for every CU (32 tokens: Q6_K 41 / 27, Q3_K 30 / 20).
+// Rows above 2048 values whose workgroups fit the CUs take two groups a workgroup where one would leave a CU four waves (us, one / two groups: Q4_K unsplit
+// 4096 x 4096 at 512 tokens 32.8 / 28.3, 14336 rows at 64 27.8 / 25.0; Q5_K 36.9 / 32.3; over 700 products 1.12 x, none slower; up to 2048 values 1.01
+// x and one group stays) or where the staging kernel's tiles come to a second turn (Q6_K 1.57 x, Q3_K 1.84 x over 44 products: 128-token tiles
+// that are half empty); Q3_K above 128 tokens on half the CUs and more in any case (14336 x 4096 at 201 tokens 42.3 / 40.3 without the quantizer; 1.05 x).
 // Q2_K and IQ4_XS by their number of 128 x 64 tiles:
 //   more tiles than CUs     one group (us, 512 tokens x 4096 values x 4608 rows, one / two groups: Q2_K 36 / 44, IQ4_XS 66 / 72)
 //   above half as many      two groups, so that every SIMD has two waves (4096 rows: Q2_K 29 / 27, IQ4_XS 45 / 42); so too with 2 slices of
@@ -449,7 +453,11 @@ static KqPlan kq_plan(int wtype, int64_t K, int64_t N, int64_t M, int64_t cus) {
     if (wtype != T_Q2_K && wtype != T_IQ4_XS) {
         const int slices = kq_slices_for(K, N, M, cus);
         const bool staged = (wtype == T_Q6_K || wtype == T_Q3_K) && tiles <= cus && (M > 64 || tiles * slices < cus);
-        return KqPlan{staged ? 0 : 1, slices};
+        const bool fits = units > 8 && tiles * slices <= cus;
+        const bool two = fits && (wtype == T_Q4_K || wtype == T_Q5_K ? slices == 1
+                                                                     : staged && (ceil_div(N, (int64_t)64) * ceil_div(M, (int64_t)128) * slices > cus ||
+                                                                                  (wtype == T_Q3_K && M > 128 && 2 * tiles * slices >= cus)));
+        return KqPlan{two ? 2 : staged ? 0 : 1, slices};
     }
     if (tiles > cus || units == 1) return KqPlan{1, 1};
     const int64_t most = std::max<int64_t>(8, std::min<int64_t>(16, units / 4));
@@ -656,29 +664,40 @@ hipError_t launch_gemm_kq(int wtype, const void *W, size_t nb01, int64_t K, int6
         return slices <= 1 || (split.part && split.bytes >= (size_t)slices * (size_t)M * (size_t)N * sizeof(float) && (((uintptr_t)split.part) & 15) == 0);
     };
     KqPlan p = kq_plan(wtype, K, N, M, cus);
-    if (!room(p.slices)) p = KqPlan{p.groups > 0 && (wtype == T_Q2_K || wtype == T_IQ4_XS) ? 2 : p.groups, 1};
+    // (unsplit for want of room: in the groups that more tokens of the same rows take, whose sums are added in the same order)
+    if (!room(p.slices)) p = KqPlan{wtype == T_Q2_K || wtype == T_IQ4_XS ? (p.groups > 0 ? 2 : 0) : wtype != T_Q6_K && K > 8 * QK_K ? 2 : p.groups, 1};
     if (p.groups == 0) return launch_staged_type<false>(wtype, W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, 0, p.slices, split.part);
     return launch_gemm_kr(p.groups, wtype, mats, K, ws, ws_stride, M, lim, st, rg, n_as, p.slices, split.part);
 }
 
 // Members that run unsplit by themselves: the same bits, fewer launches and one set of tiles (us, ffn_gate + ffn_up, Q4_K
 // of 4096 values x 14336 rows at 512 tokens, whose 896 tiles each leave a quarter of the second turn idle: 2 x 93.5 -> 164; wq + wk + wv of 1024
-// values x 1024 + 256 + 256 rows at 128 tokens 36 -> 13).
+// values x 1024 + 256 + 256 rows at 128 tokens 36 -> 13).  Q4_K and Q5_K that alone take two groups a workgroup run in one where their tiles together
+// are more than the CUs, whose sums are then added in one chain (2 x 6912 rows x 2560 values at 200 tokens 35.4, in two groups 39.4).
+static int kq_group_groups(int wtype, int64_t K, const GemmMats &mats, int64_t n, int64_t cus) {
+    if (wtype == T_Q2_K || wtype == T_IQ4_XS || kq_plan(wtype, K, mats.m[0].N, n, cus).groups != 2) return 1;
+    int64_t tiles = 0;
+    for (int i = 0; i < mats.count; i++) tiles += ceil_div(mats.m[i].N, (int64_t)128) * ceil_div(n, (int64_t)64);
+    return (wtype == T_Q4_K || wtype == T_Q5_K) && tiles > cus ? 1 : 2;
+}
 bool gemm_kq_group_applicable(int wtype, int64_t K, const GemmMats &mats, int64_t n, int compute_units) {
     const int64_t cus = compute_units > 0 ? compute_units : 256;
     if (mats.count < 2 || !gemm_kq_type(wtype)) return false;
+    const int groups = kq_group_groups(wtype, K, mats, n, cus);
     for (int i = 0; i < mats.count; i++) {
         const int64_t N = mats.m[i].N;
         const KqPlan p = kq_plan(wtype, K, N, n, cus);
         // (IQ4_XS of 2 and 3 super-blocks: alone in the staging kernel, together faster in one launch; the same bits)
-        if (!gemm_kq_supported(wtype, K, N, n, false) || p.slices != 1 || !(p.groups == 1 || (wtype == T_IQ4_XS && K < 4 * QK_K))) return false;
+        if (!gemm_kq_supported(wtype, K, N, n, false) || p.slices != 1 || 
+            !(p.groups == groups || (p.groups == 2 && (wtype == T_Q4_K || wtype == T_Q5_K)) || (wtype == T_IQ4_XS && K < 4 * QK_K))) return false;
         if (gemm_kr_rows_in_reach(mats.m[i].nb01) < 32) return false;
     }
     return true;
 }
 hipError_t launch_gemm_kq_group(int wtype, const GemmMats &mats, int64_t K, const void *ws, size_t ws_stride, int64_t n, const DeviceLimits &lim,
                                 hipStream_t st) {
-    return launch_gemm_kr(1, wtype, mats, K, ws, ws_stride, n, lim, st, RowGather{nullptr, nullptr, nullptr, 1, 1, 0}, 1, 1, nullptr);
+    const int groups = kq_group_groups(wtype, K, mats, n, lim.compute_units > 0 ? lim.compute_units : 256);
+    return launch_gemm_kr(groups, wtype, mats, K, ws, ws_stride, n, lim, st, RowGather{nullptr, nullptr, nullptr, 1, 1, 0}, 1, 1, nullptr);
 }
 
 }  // namespace chip

@@ -387,8 +387,7 @@ template <int WT>
 hipError_t launch_kr_groups(int groups, const GemmMats &mats, int64_t K, const void *ws, size_t ws_stride, int64_t M, const DeviceLimits &lim,
                             hipStream_t st, const RowGather &rg, int64_t slots, int slices, float *part) {
     if (rg.perm) return launch_kr<WT, 2, 1, 2, true>(mats, K, ws, ws_stride, M, lim, st, rg, slots, 1, nullptr);   // expert groups
-    if constexpr (WT == T_Q2_K || WT == T_IQ4_XS)
-        if (groups == 2) return launch_kr<WT, 2, 2, 2, false>(mats, K, ws, ws_stride, M, lim, st, rg, slots, slices, part);
+    if (groups == 2) return launch_kr<WT, 2, 2, 2, false>(mats, K, ws, ws_stride, M, lim, st, rg, slots, slices, part);
     return launch_kr<WT, 2, 1, 2, false>(mats, K, ws, ws_stride, M, lim, st, rg, slots, slices, part);
 }
 
