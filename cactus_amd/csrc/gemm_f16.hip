@@ -462,7 +462,9 @@ hipError_t launch_gemm_f16(const void *W, size_t nb01, int64_t K, int64_t N, con
     // a CU: 2 (1 is 14 % slower), more: 1 (3 % faster than 2 for K > 2048, the same below); 64 x 64: 2 (1 is 5 to 35 % slower up to 2.5 a CU and no
     // faster beyond).  Up to one and a half workgroups of 64 x 64 a CU a stage is 128 values: its loads, reads, MFMAs and barrier, which follow each
     // other, come half as often.  Over 800 products 1.05 to 1.07 x against 64 values two or three ahead; at two a CU 2 % slower where a cache holds
-    // the matrix, from 2.5 on 4 % in any case.  Up to half a workgroup a CU 64 x 32 tiles, twice as many: 1.13 x.  us, 64 values two or three ahead -> now,
+    // the matrix, from 2.5 on 4 % in any case.  Up to half a workgroup a CU 64 x 32 tiles, twice as many: 1.13 x.  One or two token tiles stay with 64
+    // values three ahead on half to one workgroup a CU (2048 values x 8120 rows at 83 tokens 15.7 against 17.3), and rows up to 1280 values on a quarter to a
+    // half (768 x 7845 at 43 tokens 7.1 against 9.0): a CU's one workgroup has few loads in flight there, or too few stages to win back a fill.  us, 64 values two or three ahead -> now,
     // 4096 x 4096 that no cache holds at 64 tokens 31.6 -> 26.4, 201 31.6 -> 28.2, 300 36.9 -> 34.5; 14336 x 4096 at 201 80.6 -> 75.9.
     const int64_t g128 = ceil_div(N, 128) * ceil_div(M, 128), g256 = ceil_div(N, 256) * ceil_div(M, 256), g64 = ceil_div(N, 64) * ceil_div(M, 64);
     const int cfg = (int)tune("CHIP_GEMM_F16_CFG", 2 * g256 >= cus && K >= 4 * BIG_K && n_as == 1 ? 9 : g128 >= cus ? 0 : 1);
@@ -471,8 +473,9 @@ hipError_t launch_gemm_f16(const void *W, size_t nb01, int64_t K, int64_t N, con
             if (g128 > cus) return launch_f16<2, 2, 2, 2, 2, F16_PLAIN, false, 1>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
             return launch_f16<2, 2, 2, 2, 2, F16_PLAIN, false, 2>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
         case 1:                                                                                                         // 64 x 64, 4 waves; 64 x 32, 2 waves
-            if (2 * g64 <= cus) return launch_f16<1, 1, 2, 1, 2, F16_PLAIN, false, 2, 8>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
-            if (2 * g64 <= 3 * cus) return launch_f16<1, 1, 2, 2, 2, F16_PLAIN, false, 2, 8>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
+            if (2 * g64 <= cus && !(M <= 128 && K <= 1280 && 4 * g64 > cus)) return launch_f16<1, 1, 2, 1, 2, F16_PLAIN, false, 2, 8>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
+            if (2 * g64 <= 3 * cus && !(M <= 128 && g64 <= cus)) return launch_f16<1, 1, 2, 2, 2, F16_PLAIN, false, 2, 8>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
+            if (2 * g64 <= 3 * cus) return launch_f16<1, 1, 2, 2, 4, F16_PLAIN, false, 3>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
             return launch_f16<1, 1, 2, 2, 4, F16_PLAIN, false, 2>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
         case 9: return launch_f16_direct(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st);                             // 256 x 256, 4 waves, direct to LDS
         default: return hipErrorInvalidValue;
