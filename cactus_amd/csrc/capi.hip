@@ -517,17 +517,19 @@ static bool few_group(const GroupMat *gm, int live, int64_t K, int64_t n, const 
     if (live > GEMM_MATS_MAX) return false;
     const int lo = std::min_element(gm, gm + live, [](const GroupMat &a, const GroupMat &b) { return a.wtype < b.wtype; })->wtype;
     int hi = lo;
+    bool far = false;                                                    // a member whose rows forms of 32 rows do not reach (kq_few_plan)
     for (int i = 0; i < live; i++) {
         const KqFew m = few_for(gm[i], K, n, workspace, workspace_bytes, lim);
         if (m.ks == 0 || (f.ks > 0 && m.ks != f.ks)) return false;
         f.ks = m.ks;
         f.rt = std::max(f.rt, m.rt);
+        far |= gemm_kr_rows_in_reach(gm[i].nb01) < 32;
         if (gm[i].wtype != lo) {
             if (hi != lo && gm[i].wtype != hi) return false;
             hi = gm[i].wtype;
         }
     }
-    if (hi != lo) f.rt = 1;
+    if (hi != lo || far) f.rt = 1;
     for (int t : {lo, hi})
         for (int i = 0; i < live; i++)
             if (gm[i].wtype == t && mats.count < live) {

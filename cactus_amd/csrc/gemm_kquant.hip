@@ -590,9 +590,12 @@ static float others_estimate(int wtype, int64_t K, int64_t N, int64_t n, const K
 // are known to run in slices of K and a slice sum stay there: long rows on many rows (us, slices / this, 14336 values x 4096 rows at 32 tokens: Q4_K 19.8
 // / 18.9, Q6_K 23.9 / 20.8, Q3_K 19.6 / 16.8) and a few rows above 64 tokens.  Up to 320 tokens, where the estimates were fitted.
 KqFew kq_few_plan(int wtype, size_t nb01, int64_t K, int64_t N, int64_t n, bool can_split, int compute_units) {
-    if (!gemm_kq_type(wtype) || n < 5 || n > 1200 || N < 1 || K % QK_K != 0 || nb01 > ((size_t)1 << 28)) return KqFew{0, 0, 0};
+    if (!gemm_kq_type(wtype) || n < 5 || n > 1200 || N < 1 || K % QK_K != 0) return KqFew{0, 0, 0};
+    // rows that the kernel's 32-bit offsets reach from a tile's first: forms of 32 rows where all of them are, none where not even 16 are
+    const int64_t reach = gemm_kr_rows_in_reach(nb01);
+    if (reach < 16) return KqFew{0, 0, 0};
     const int64_t cus = compute_units > 0 ? compute_units : 256, units = K / QK_K, forced = tune("CHIP_KQ_FEW", -1);
-    if (forced > 0) return units >= forced % 100 ? KqFew{(int)(forced / 1000), (int)(forced / 100 % 10), (int)(forced % 100)} : KqFew{0, 0, 0};
+    if (forced > 0) return units >= forced % 100 && reach >= 16 * (forced / 1000) ? KqFew{(int)(forced / 1000), (int)(forced / 100 % 10), (int)(forced % 100)} : KqFew{0, 0, 0};
     const bool four = wtype == T_Q4_K || wtype == T_Q5_K;
     if (forced == 0 || units < (n <= 32 ? 2 : 4) || (units == 3 && four) || tune("CHIP_GEMM_MIN_TOKENS", 0) > 0) return KqFew{0, 0, 0};
     const KqPlan p = kq_plan(wtype, K, N, n, cus);
@@ -603,7 +606,7 @@ KqFew kq_few_plan(int wtype, size_t nb01, int64_t K, int64_t N, int64_t n, bool 
     for (const FewForm &f : kFewForms) {
         // A wave adds up at most eight super-blocks: no longer a chain than the walks and slices of K that ran before (relative error x 1e8, before / this:
         // Q4_K 14336 values at 9 tokens 14.3 / 8.3, 8192 at 40 9.5 / 8.2; Q3_K 8192 at 40 7.5 / 5.5).
-        if (f.tt != (n > 16 ? 2 : 1) || f.ks > units || units > 8 * f.ks) continue;
+        if (f.tt != (n > 16 ? 2 : 1) || f.ks > units || units > 8 * f.ks || reach < 16 * f.rt) continue;
         if (const float e = few_estimate(f, wtype, K, N, n, cus); e < least) { least = e; best = KqFew{f.rt, f.tt, f.ks}; }
     }
     return best;

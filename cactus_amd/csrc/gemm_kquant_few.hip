@@ -51,7 +51,7 @@ __device__ __forceinline__ void few_tile(uint8_t *lds, int stretch, const GemmMa
     const int tokens = (int)min((int64_t)C::BN, M - tok_base), nsb = (int)(K / QK_K);
     uint8_t *const own = lds + wave * stretch;
 
-    // (offsets of 32 bits from the tile's first row and first token: kq_few_plan)
+    // (offsets of 32 bits from the tile's first row and first token: kq_few_plan, and few_group for members that share a launch, see to it)
     const uint8_t *const w0 = mat.W + (size_t)row_base * mat.nb01, *const x0 = ws + (size_t)tok_base * ws_stride;
     uint32_t woff[C::NLD], wdst[C::NLD], xoff[C::NX];
 #pragma unroll

@@ -120,10 +120,13 @@ def test_kquant_row_gemm_over_slices(dev, orc, wt, n):
 
 
 # Rows so far apart that a tile spans more than 2^32 bytes, and more than 2^32 bytes apart each: (type, stride, rows, tokens).  One whole tile
-# and a ragged one; K split (3584 values at 20 tokens); rows that lie alone; 8 to 12 tokens, which the matrix-core GEMVs take of closer rows
+# and a ragged one; K split (3584 values at 20 tokens); rows that lie alone; 8 to 12 tokens, which the matrix-core GEMVs take of closer rows; 8 to 24
+# tokens, which tiles of 32 rows take of closer rows, 2^32 bytes from a tile's first row to its last and just below that of a tile of 16
 @pytest.mark.parametrize("wt,K,stride,N,n", [(O.Q4_K, 512, 140 << 20, 40, 70), (O.Q2_K, 3584, 150 << 20, 33, 20), (O.IQ4_XS, 256, (4 << 30) + 64, 3, 60),
                                              (O.Q5_K, 3584, (2 << 30) + 16, 5, 80), (O.Q4_K, 512, 300 << 20, 20, 8), (O.Q5_K, 512, 300 << 20, 20, 16),
-                                             (O.Q4_0, 512, 300 << 20, 20, 9), (O.Q8_0, 512, 300 << 20, 20, 12)],
+                                             (O.Q4_0, 512, 300 << 20, 20, 9), (O.Q8_0, 512, 300 << 20, 20, 12),
+                                             (O.Q4_K, 512, 140 << 20, 40, 8), (O.Q4_K, 512, 250 << 20, 40, 16), (O.Q6_K, 512, 250 << 20, 40, 12),
+                                             (O.Q4_K, 512, 140 << 20, 40, 24), (O.Q3_K, 1024, 140 << 20, 40, 40), (O.IQ4_XS, 1024, 270 << 20, 20, 12)],
                          ids=lambda v: O.TYPE_NAMES[v] if isinstance(v, int) and v in O.TYPE_NAMES else None)
 def test_rows_far_apart(dev, orc, wt, K, stride, N, n):
     L = dev.lib
@@ -145,6 +148,25 @@ def test_rows_far_apart(dev, orc, wt, K, stride, N, n):
         y = dy.download(np.float32, 2 * n * N).reshape(2, n, N)
         check(y[0], ref, "rows far apart")
         assert np.isnan(y[1]).all() or y[1].tobytes() == y[0].tobytes()
+
+
+# The same rows beside a matrix that alone takes tiles of 32 rows, in one launch: 16 rows a tile for both
+def test_rows_far_apart_in_a_group(dev, orc):
+    import cactus_amd as ca
+    L, wt, K, n, stride, N, near = dev.lib, O.Q4_K, 2048, 24, 140 << 20, 40, 8000
+    w = orc.quantize_weights(wt, common.weights_f32(3, 160, K))
+    x = common.activations_f32(4, n, K)
+    dW, dV, dx, dy = dev.alloc((N - 1) * stride + w.shape[1]), dev.to_device(np.tile(w, (near // 160, 1))), dev.to_device(x), dev.alloc(n * (N + near) * 4)
+    for r in range(N):
+        dW.upload(w[r], r * stride)
+    mats = (ca.Mat * 2)(ca.Mat(wt, dW.ptr, stride, N, dy.ptr, N, None, 0), ca.Mat(wt, dV.ptr, w.shape[1], near, dy.ptr + 4 * n * N, near, None, 0))
+    wsz = max(L.chip_mul_mat_workspace_size_n(wt, K, m, n) for m in (N, near))
+    ws = dev.alloc(wsz)
+    dev.check(L.chip_mul_mat_group(mats, 2, K, dx.ptr, K, n, ws.ptr, wsz, None))
+    dev.sync()
+    y = dy.download(np.float32, n * (N + near))
+    check(y[:n * N].reshape(n, N), orc.mul_mat(wt, w[:N], x, nthreads=8, want=("sum_abs",)), "far member")
+    assert np.array_equal(y[n * N:].reshape(n, -1, 160)[:, :, :N], np.repeat(y[:n * N].reshape(n, 1, N), near // 160, axis=1))
 
 
 @pytest.mark.parametrize("wt", LOW_BIT, ids=lambda t: O.TYPE_NAMES[t])
