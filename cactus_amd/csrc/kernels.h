@@ -348,7 +348,7 @@ hipError_t launch_gemm_kq_few(KqFew f, const int *types, const GemmMats &mats, i
 int        gemm_kr_tile_tokens();
 int64_t    gemm_kr_rows_in_reach(size_t nb01);
 // Several matrices of one type on the same rows in one launch.  _applicable: every member alone would take the GEMM, unsplit; its
-// outputs have the same bits (Q4_K and Q5_K of more than 2048 values: to a rounding of the sums, gemm_kquant.hip).
+// outputs have the same bits.
 bool       gemm_blk32_group_applicable(int wtype, int64_t K, const GemmMats &mats, int64_t n, int compute_units);
 hipError_t launch_gemm_blk32_group(int wtype, const GemmMats &mats, int64_t K, const void *ws, size_t ws_stride, int64_t n, const DeviceLimits &lim,
                                    hipStream_t st);

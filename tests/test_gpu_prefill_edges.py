@@ -1,12 +1,14 @@
 """GPU parity of the prefill kernels at the sizes where their staging ends unevenly: short last stages, ragged tiles, small
 and large shapes of each dispatch rule.  Against the CPU oracle, within 1e-5 * sum |terms| per output (the summation order is
 all that differs), as the other matmul tests."""
+import re
+
 import numpy as np
 import pytest
 
 import common
 import oracle as O
-from test_gpu_routes import group_launches, mul_mat_id_launches, mul_mat_launches
+from test_gpu_routes import group_kernels, group_launches, mul_mat_id_launches, mul_mat_launches
 
 pytestmark = pytest.mark.gpu
 
@@ -280,6 +282,23 @@ def test_grouped_gemms_equal_single_calls(dev, orc, wt, K, rows, n):
     pick = np.unique(np.concatenate([[0, W.shape[0] - 1], rng.choice(W.shape[0], min(W.shape[0], 100), replace=False)]))
     ref = orc.mul_mat(ws[-1][0], W[pick], x[toks], nthreads=8, want=("sum_abs",))
     check(ys[-1][np.ix_(toks, pick)], ref, "last member")
+
+
+# Q4_K and Q5_K above 2048 values, in one k group and in two: members share a launch only in the number that each has alone
+@pytest.mark.parametrize("wt,K,rows,n,groups", [(O.Q4_K, 2560, (6912, 6912), 200, (1,)), (O.Q5_K, 2304, (3000, 2900), 260, (2,)), (O.Q5_K, 2304, (3000, 6000), 260, (2, 1)),
+                                                (O.Q5_K, 2304, (6000, 3000), 260, (1, 2)), (O.Q4_K, 4096, (4096, 4096), 512, (1,))],
+                         ids=lambda v: O.TYPE_NAMES[v] if isinstance(v, int) and v in O.TYPE_NAMES else None)
+def test_joined_k_groups_equal_single_calls(dev, orc, wt, K, rows, n, groups):
+    q = orc.quantize_weights(wt, common.weights_f32(K + n, 101, K))
+    ws = [np.roll(np.tile(q, (-(-N // 101), 1))[:N], i, axis=0) for i, N in enumerate(rows)]
+    x = common.activations_f32(K + n, n, K)
+    names = [k for k in group_kernels(dev, [(wt, N) for N in rows], K, n) if "gemm_kr_kernel" in k]
+    assert [int(re.search(r"gemm_kr_kernelILi%dELi2ELi(\d)E" % wt, k)[1]) for k in names] == list(groups)
+    for w, y in zip(ws, dev.mul_mat_group([(wt, w) for w in ws], x)):
+        assert y.tobytes() == dev.mul_mat(wt, w, x).tobytes()
+    if rows[0] == rows[1]:
+        y1, y2 = dev.mul_mat_pair(wt, ws[0], ws[1], x)
+        assert y1.tobytes() == dev.mul_mat(wt, ws[0], x).tobytes() and y2.tobytes() == dev.mul_mat(wt, ws[1], x).tobytes()
 
 
 # ---- expert groups: pairs of each expert around a tile of 64, more experts than a turn of the scan takes, more pairs than are kept in registers ----

@@ -16,9 +16,14 @@ def dev():
     return cactus_amd.Device(0)
 
 
-def launches(dev, call):
-    """Kernel launches of call(stream), which is made once before it is recorded (a kernel's first launch raises its LDS limit)."""
+class NodeParams(C.Structure):
+    _fields_ = [("block", C.c_uint * 3), ("extra", C.c_void_p), ("func", C.c_void_p), ("grid", C.c_uint * 3), ("params", C.c_void_p), ("shared", C.c_uint)]
+
+
+def kernels(dev, call):
+    """Names (mangled) of the kernels of call(stream), which is made once before it is recorded (a kernel's first launch raises its LDS limit)."""
     hip = C.CDLL("libamdhip64.so")
+    hip.hipKernelNameRefByPtr.restype = C.c_char_p
     st, graph, count = C.c_void_p(), C.c_void_p(), C.c_size_t()
     dev.check(dev.lib.chip_stream_create(C.byref(st)))
     dev.check(call(st))
@@ -27,9 +32,19 @@ def launches(dev, call):
     rc = call(st)
     assert hip.hipStreamEndCapture(st, C.byref(graph)) == 0 and rc == 0
     assert hip.hipGraphGetNodes(graph, None, C.byref(count)) == 0
+    nodes, names = (C.c_void_p * count.value)(), []
+    assert hip.hipGraphGetNodes(graph, nodes, C.byref(count)) == 0
+    for node in nodes:
+        p = NodeParams()
+        assert hip.hipGraphKernelNodeGetParams(C.c_void_p(node), C.byref(p)) == 0
+        names.append(hip.hipKernelNameRefByPtr(C.c_void_p(p.func), st).decode())
     hip.hipGraphDestroy(graph)
     dev.check(dev.lib.chip_stream_destroy(st))
-    return count.value
+    return names
+
+
+def launches(dev, call):
+    return len(kernels(dev, call))
 
 
 def mul_mat_id_launches(dev, wt, K, N, n_as, n_used, n_tokens):
@@ -47,7 +62,7 @@ def mul_mat_id_launches(dev, wt, K, N, n_as, n_used, n_tokens):
                                                       dy.ptr, N, ws.ptr, wsz, st))
 
 
-def group_launches(dev, members, K, n):
+def group_kernels(dev, members, K, n):
     """Of chip_mul_mat_group over members [(type, rows), ...]."""
     import cactus_amd as ca
     L = dev.lib
@@ -60,16 +75,24 @@ def group_launches(dev, members, K, n):
         arr[i] = ca.Mat(wt, dW.ptr, row, N, dy.ptr, N, None, 0)
         wsz = max(wsz, L.chip_mul_mat_workspace_size_n(wt, K, N, n))
     ws = dev.alloc(wsz)
-    return launches(dev, lambda st: L.chip_mul_mat_group(arr, len(members), K, keep[0].ptr, K, n, ws.ptr, wsz, st))
+    return kernels(dev, lambda st: L.chip_mul_mat_group(arr, len(members), K, keep[0].ptr, K, n, ws.ptr, wsz, st))
 
 
-def mul_mat_launches(dev, wt, W, x, split_k=True):
+def group_launches(dev, members, K, n):
+    return len(group_kernels(dev, members, K, n))
+
+
+def mul_mat_kernels(dev, wt, W, x, split_k=True):
     n, K = x.shape
     N, L = W.shape[0], dev.lib
     dW, dx, dy = dev.to_device(W), dev.to_device(x), dev.alloc(n * N * 4)
     wsz = L.chip_mul_mat_workspace_size_n(wt, K, N, n) if split_k else L.chip_mul_mat_workspace_size(wt, K, n)
     ws = dev.alloc(wsz)
-    return launches(dev, lambda st: L.chip_mul_mat(wt, dW.ptr, W.shape[1], K, N, dx.ptr, K, n, dy.ptr, N, ws.ptr, wsz, st))
+    return kernels(dev, lambda st: L.chip_mul_mat(wt, dW.ptr, W.shape[1], K, N, dx.ptr, K, n, dy.ptr, N, ws.ptr, wsz, st))
+
+
+def mul_mat_launches(dev, wt, W, x, split_k=True):
+    return len(mul_mat_kernels(dev, wt, W, x, split_k))
 
 
 # quantizer, GEMM over slices of K, slice sum; rows in fours, and one, two and three rows in a token's last group
