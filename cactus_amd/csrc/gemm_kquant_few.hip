@@ -6,14 +6,16 @@
 // end: it loads its rows' packed bytes and its tokens' quants in memory order, a super-block ahead of the one it multiplies, turns them round
 // through a stretch of LDS of its own, with no barrier, and expands its lanes' operands in registers (kquant_rows_dev.h; what the digit planes
 // are: gemm_kquant_rows.hip).  A v_mfma_i32_16x16x64_i8 covers two k-blocks: lane (x, g) holds the k-half g % 2 of a k-block of item (H, g / 2), for rows
-// and tokens alike.  The waves' sums meet in LDS once and are added as doubles: chains of K / 256 / ks additions, no further from the 64-bit sums than the
-// GEMV's (test_kquant_few_tokens).
+// and tokens alike.  A super-block's integers are scaled and added in 64 bits, and so are the waves' sums, which meet in LDS once: a result is its sum
+// rounded once.  (In 32 bits the kernel is 1 to 3 per cent faster, 7.7 against 7.8 us for Q6_K 4096 values x 4096 rows at 8 tokens, but rows of two super-blocks were up
+// to 1.16 x as far from the 64-bit sums as the GEMV's, and Q2_K and IQ4_XS 1.07 x as far as slices of K; 2-norm of the error over that of the sums, 512
+// values at 15 tokens, GEMV / 32 bits / 64: Q3_K 4.0e-8 / 4.5e-8 / 2.7e-8.)
 //
 // Bound: the issue of vector instructions (some 200 per super-block of 16 rows x 16 tokens, over half of them the expansion) at two to four waves a
 // SIMD, and the tokens' quants, 4 KB for the 1.3 to 3.4 KB of 16 rows: tiles of 32 rows halve those where there are rows enough.  us, what ran before /
-// this, 8 tokens (a GEMV): Q6_K 4096 values x 4096 rows 9.6 / 7.5, 14336 x 4096 20.4 / 16.4, 4096 x 32000 39 / 29; Q4_K 1024 x 3072 7.6 / 4.0,
-// 14336 x 4096 14.1 / 11.4; 32 tokens (the GEMM, in slices of K): Q4_K 4096 x 4096 13.9 / 8.2, x 14336 27.5 / 18.7, 2048 x 768 11.1 / 5.0; 64 tokens Q4_K 4096 x 4096
-// 16.4 / 11.0.  16 rows rather than 32 a tile because 4096 rows are then a workgroup for every CU; more waves than super-blocks have nothing to share.
+// this, 8 tokens (a GEMV): Q6_K 4096 values x 4096 rows 9.6 / 7.8, 14336 x 4096 20.0 / 16.7, 4096 x 32000 37 / 31; Q4_K 1024 x 3072 7.7 / 4.1; 32
+// tokens (the GEMM, in slices of K): Q4_K 4096 x 4096 13.8 / 8.3, x 14336 27.0 / 18.7, 2048 x 768 11.2 / 5.1; 64 tokens Q4_K 4096 x 4096
+// 16.1 / 11.1.  16 rows rather than 32 a tile because 4096 rows are then a workgroup for every CU; more waves than super-blocks have nothing to share.
 #include "dev_common.h"
 #include "act_layout.h"
 #include "kernels.h"
@@ -36,7 +38,7 @@ struct KfCfg {
     static constexpr int ROW = T::NCH | 1;                                // cells a row takes in LDS: 16 rows' cells of one index in different banks
     // a wave's stretch: rows, tokens' quants ([token][16 cells], swizzled), their scales, their block sums as fp16 ([token][16])
     static constexpr int OFF_X = BM * ROW * 16, OFF_D = OFF_X + BN * 256, OFF_S = OFF_D + BN * 4, WAVE = OFF_S + (T::NF16 ? BN * 32 : 0);
-    static_assert(WAVE % 16 == 0 && WAVE >= BM * BN * 4, "a wave's sums take the place of its operands");
+    static_assert(WAVE % 16 == 0 && WAVE >= BM * BN * 8, "a wave's sums take the place of its operands");
 };
 
 // One tile; `stretch`: bytes of LDS a wave has.
@@ -93,11 +95,7 @@ __device__ __forceinline__ void few_tile(uint8_t *lds, int stretch, const GemmMa
     const u32x4 *const row = reinterpret_cast<const u32x4 *>(own) + x * C::ROW;           // and 16 rows on per tile of rows
     // cell 2 * k-block + k-half of the lane's token; the bits that H and the second k-block add are not set in it
     const uint32_t b_lane = (uint32_t)C::OFF_X + (uint32_t)x * 256u + 16u * (uint32_t)((2 * (3 - T::NEXT) * p + hf) ^ x);
-    f32x4 out[RT][TT];
-#pragma unroll
-    for (int r = 0; r < RT; r++)
-#pragma unroll
-        for (int c = 0; c < TT; c++) out[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    double out[RT][TT][4] = {};
 
     Load k;
     load(k, wave);                                                                       // (ks <= nsb: launch_few)
@@ -106,37 +104,33 @@ __device__ __forceinline__ void few_tile(uint8_t *lds, int stretch, const GemmMa
         if (sb + ks < nsb) load(k, sb + ks);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        typename T::Hdr h[RT];
-#pragma unroll
-        for (int r = 0; r < RT; r++) h[r] = T::hdr(row + 16 * r * C::ROW, hf);
         i32x4 P[T::NPL][RT][TT];
 #pragma unroll
         for (int H = 0; H < 2; H++) {
-            u32x4 a[2][TT];
-#pragma unroll
-            for (int e = 0; e < 2; e++)
-#pragma unroll
-                for (int c = 0; c < TT; c++)
-                    a[e][c] = *reinterpret_cast<const u32x4 *>(own + c * 4096 + (b_lane ^ (uint32_t)(16 * (8 * H + 2 * T::NEXT * e))));
+            // Q5_K reads its header for each half and for the fold: held over all it would not fit the registers
+            if constexpr (WT == T_Q5_K) asm volatile("" ::: "memory");
 #pragma unroll
             for (int r = 0; r < RT; r++) {
                 u32x4 w[2][T::NPL];
-                T::expand(T::load(row + 16 * r * C::ROW, H, p, hf), h[r], H, p, hf, w);
+                T::expand(T::load(row + 16 * r * C::ROW, H, p, hf), T::hdr(row + 16 * r * C::ROW, hf), H, p, hf, w);
 #pragma unroll
                 for (int e = 0; e < 2; e++)
 #pragma unroll
-                    for (int c = 0; c < TT; c++)
+                    for (int c = 0; c < TT; c++) {
+                        const u32x4 a = *reinterpret_cast<const u32x4 *>(own + c * 4096 + (b_lane ^ (uint32_t)(16 * (8 * H + 2 * T::NEXT * e))));
 #pragma unroll
                         for (int pl = 0; pl < T::NPL; pl++)
-                            P[pl][r][c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, a[e][c]), __builtin_bit_cast(i32x4, w[e][pl]),
+                            P[pl][r][c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, a), __builtin_bit_cast(i32x4, w[e][pl]),
                                                                                 H == 0 && e == 0 ? i32x4{0, 0, 0, 0} : P[pl][r][c], 0, 0, 0);
+                    }
             }
         }
-        // fold, as the reference does once per super-block: out += dx * (d * float(sumi) - dmin * summ)
+        // fold, as the reference does once per super-block: out += dx * (d * sumi - dmin * summ)
 #pragma unroll
         for (int r = 0; r < RT; r++) {
-            float d = h2f(T::scales(h[r])), dmin = h2f(T::scales(h[r]) >> 16);
-            asm volatile("" : "+v"(d), "+v"(dmin));                        // widened once: as halves they would make the multiply-adds half-rate mixed ones
+            if constexpr (WT == T_Q5_K) asm volatile("" ::: "memory");
+            const uint32_t scales = T::scales(T::hdr(row + 16 * r * C::ROW, hf));
+            const double d = h2f(scales), dmin = h2f(scales >> 16);
 #pragma unroll
             for (int c = 0; c < TT; c++) {
                 f32x4 F = {0.f, 0.f, 0.f, 0.f};
@@ -148,7 +142,7 @@ __device__ __forceinline__ void few_tile(uint8_t *lds, int stretch, const GemmMa
 #pragma unroll
                 for (int v = 0; v < 4; v++) {
                     const float f[2] = {F[v], 0.f};
-                    out[r][c][v] = __builtin_fmaf(T::value(P[0][r][c][v], P[T::NPL - 1][r][c][v], f, d, dmin), dx[v], out[r][c][v]);
+                    out[r][c][v] = __builtin_fma(T::value(P[0][r][c][v], P[T::NPL - 1][r][c][v], f, d, dmin), (double)dx[v], out[r][c][v]);
                 }
             }
         }
@@ -156,7 +150,7 @@ __device__ __forceinline__ void few_tile(uint8_t *lds, int stretch, const GemmMa
         __builtin_amdgcn_wave_barrier();
     }
     // register v of tile (r, c) is token 16 c + 4 g + v, the lane's x its row 16 r + x
-    float *const part = reinterpret_cast<float *>(own);
+    double *const part = reinterpret_cast<double *>(own);
 #pragma unroll
     for (int r = 0; r < RT; r++)
 #pragma unroll
@@ -166,7 +160,7 @@ __device__ __forceinline__ void few_tile(uint8_t *lds, int stretch, const GemmMa
     __syncthreads();
     for (int e = threadIdx.x; e < 256 * RT * TT; e += (int)blockDim.x) {
         double o = 0.;
-        for (int w = 0; w < ks; w++) o += (double)reinterpret_cast<const float *>(lds + w * stretch)[e];
+        for (int w = 0; w < ks; w++) o += reinterpret_cast<const double *>(lds + w * stretch)[e];
         const int tile = e >> 8, t = 16 * (tile / RT) + 4 * ((e & 63) >> 4) + ((e >> 6) & 3);
         const int64_t r = row_base + 16 * (tile % RT) + (e & 15);
         if (t < tokens && r < N) mat.y[(size_t)(tok_base + t) * mat.ldy + r] = (float)o;

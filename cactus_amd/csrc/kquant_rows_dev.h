@@ -43,11 +43,14 @@ __device__ __forceinline__ u32x4 i16x8_to_f16(const u32x4 &v) {
     }
     return c;
 }
+__device__ __forceinline__ float mul_add(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double mul_add(double a, double b, double c) { return __builtin_fma(a, b, c); }
 // Per weight type.  A super-block is fetched as NCH 16-byte chunks (the last one ends with the super-block, so it may overlap the
 // one before) and kept in LDS in that order, NCH cells a row.  Where NCH is odd, 16 rows' cells of one index fall into different banks; for Q6_K (14
 // cells) and Q2_K (6) two of them share one.
 // A lane reads its share back: hdr() what all items need, load() the 16-value k-half hf of the two k-blocks of item (H, p), NEXT apart in half H of
 // the super-block (kr_k_block), which expand() turns into MFMA operand cells [k-block][plane].  H is known at compile time; p and hf may be the lane's.
+// value() is the super-block's d * sumi - dmin * summ, in 32 or in 64 bits.
 template <int WT> struct KR;
 
 template <> struct KR<T_Q4_K> {
@@ -81,8 +84,8 @@ template <> struct KR<T_Q4_K> {
         return u32x2{f16_pair(mn & 0xffu, mn & 0xffu), f16_pair(mn >> 8, mn >> 8)};
     }
     __device__ static __forceinline__ uint32_t scales(const Hdr &h) { return h.h.x; }
-    __device__ static __forceinline__ float value(int p0, int p1, const float (&f)[2], float d, float dmin) {
-        return __builtin_fmaf(-dmin, f[0], d * (float)((p0 << 3) + p1));
+    template <typename R> __device__ static __forceinline__ R value(int p0, int p1, const float (&f)[2], R d, R dmin) {
+        return mul_add(-dmin, (R)f[0], d * (R)((p0 << 3) + p1));
     }
 };
 
@@ -122,8 +125,8 @@ template <> struct KR<T_Q5_K> {
         return u32x2{f16_pair(mn & 0xffu, mn & 0xffu), f16_pair(mn >> 8, mn >> 8)};
     }
     __device__ static __forceinline__ uint32_t scales(const Hdr &h) { return h.h.x; }
-    __device__ static __forceinline__ float value(int p0, int p1, const float (&f)[2], float d, float dmin) {
-        return __builtin_fmaf(-dmin, f[0], d * (float)((p0 << 8) + p1));
+    template <typename R> __device__ static __forceinline__ R value(int p0, int p1, const float (&f)[2], R d, R dmin) {
+        return mul_add(-dmin, (R)f[0], d * (R)((p0 << 8) + p1));
     }
 };
 
@@ -161,7 +164,7 @@ template <> struct KR<T_Q6_K> {
     }
     __device__ static __forceinline__ u32x4 f16_cell(const Hdr &, int, int) { return u32x4{0u, 0u, 0u, 0u}; }
     __device__ static __forceinline__ uint32_t scales(const Hdr &h) { return h.d; }
-    __device__ static __forceinline__ float value(int p0, int p1, const float (&)[2], float d, float) { return d * (float)((p0 << 8) + p1); }
+    template <typename R> __device__ static __forceinline__ R value(int p0, int p1, const float (&)[2], R d, R) { return d * (R)((p0 << 8) + p1); }
 };
 
 template <> struct KR<T_Q3_K> {
@@ -205,7 +208,7 @@ template <> struct KR<T_Q3_K> {
     }
     __device__ static __forceinline__ u32x4 f16_cell(const Hdr &, int, int) { return u32x4{0u, 0u, 0u, 0u}; }
     __device__ static __forceinline__ uint32_t scales(const Hdr &h) { return h.d; }
-    __device__ static __forceinline__ float value(int p0, int, const float (&)[2], float d, float) { return d * (float)-p0; }
+    template <typename R> __device__ static __forceinline__ R value(int p0, int, const float (&)[2], R d, R) { return d * (R)-p0; }
 };
 
 template <> struct KR<T_Q2_K> {
@@ -243,8 +246,8 @@ template <> struct KR<T_Q2_K> {
         return u32x2{f16_pair(w & 0xffu, (w >> 8) & 0xffu), f16_pair((w >> 16) & 0xffu, w >> 24)};
     }
     __device__ static __forceinline__ uint32_t scales(const Hdr &h) { return h.dd; }
-    __device__ static __forceinline__ float value(int p0, int, const float (&f)[2], float d, float dmin) {
-        return __builtin_fmaf(-dmin, f[0], d * (float)p0);
+    template <typename R> __device__ static __forceinline__ R value(int p0, int, const float (&f)[2], R d, R dmin) {
+        return mul_add(-dmin, (R)f[0], d * (R)p0);
     }
 };
 
@@ -285,7 +288,7 @@ template <> struct KR<T_IQ4_XS> {
     }
     __device__ static __forceinline__ u32x4 f16_cell(const Hdr &, int, int) { return u32x4{0u, 0u, 0u, 0u}; }
     __device__ static __forceinline__ uint32_t scales(const Hdr &h) { return h.h.x & 0xffffu; }
-    __device__ static __forceinline__ float value(int p0, int p1, const float (&)[2], float d, float) { return d * (float)((p0 << 8) + p1); }
+    template <typename R> __device__ static __forceinline__ R value(int p0, int p1, const float (&)[2], R d, R) { return d * (R)((p0 << 8) + p1); }
 };
 
 // k-block e (0, 1) of item (H, p)
