@@ -244,11 +244,11 @@ void gemm_blk32_few_kernel(GemmMats mats, int64_t K, const uint8_t *__restrict__
             // a pair's products behind the sums of the one before: all at once they do not fit the registers
             if (p > 0) asm volatile("" : "+v"(acc), "+v"(q.c0), "+v"(q.c1));
             const uint32_t live = 4 * H + 2 * p >= lo && 4 * H + 2 * p < hi ? 0xffffffffu : 0u;       // (lo and hi are even)
-            const uint32_t dx = dx4[2 * H + p];
+            const uint32_t dx = dx4[2 * H + p] & live;                                  // (both factors: a block that does not count may have an infinite one)
             const i32x16 D0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, a[0]), __builtin_bit_cast(i32x4, q.c0), magic, 0, 0, 0);
             const f32x16 P0 = scales(dx & first, q.d0 & first & live);
             if constexpr (T::HAS_MIN) {                                             // m[r][b] * s[t][b]: fp16 factors on both sides
-                const uint32_t s = reinterpret_cast<const u32x4 *>(own + C::OFF_S)[l32][2 * H + p];
+                const uint32_t s = reinterpret_cast<const u32x4 *>(own + C::OFF_S)[l32][2 * H + p] & live;
                 acc = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(f16x4, u32x2{half ? 0u : s, 0u}),
                                                            __builtin_bit_cast(f16x4, u32x2{half ? 0u : q.m & live, 0u}), acc, 0, 0, 0);
             }

@@ -496,6 +496,26 @@ def test_block32_few_tokens_with_an_infinite_scale(dev, orc, wt):
     assert np.isfinite(np.delete(y, (5, 7), axis=1)).all()
 
 
+# ... and so does an infinite activation scale (values above 127 * 65504) or block sum (32 values that add up to more than 65504), whichever wave has the block
+@pytest.mark.parametrize("K,n", [(768, 20), (1344, 80)])
+@pytest.mark.parametrize("wt", (O.Q4_0, O.Q8_0, O.Q5_0, O.IQ4_NL, O.Q4_1, O.Q5_1), ids=lambda t: O.TYPE_NAMES[t])
+def test_block32_few_tokens_with_an_infinite_activation_scale(dev, orc, wt, K, n):
+    N = 70
+    w = orc.quantize_weights(wt, common.weights_f32(K + N, N, K))
+    x = common.activations_f32(K + n, n, K)
+    blocks = K // 32
+    for t in range(blocks // 2):
+        x[t, 64 * t + 5] = 1e7 if t % 2 else -1e7
+    x[n - 2, 320:352] = 3000.0
+    if n == 80:
+        assert "gemm_blk32_few_kernel" in mul_mat_kernels(dev, wt, w, x)[1]
+    aq = orc.quantize_activation(O.VEC_DOT_TYPE[wt], x)
+    ref = np.array([[orc.vec_dot_exact(wt, K, r, a)[0] for r in w] for a in aq])
+    y = dev.mul_mat(wt, w, x)
+    assert not np.isfinite(ref[:blocks // 2]).any() and np.isinf(ref).any() and np.isinf(ref[n - 2]).any() == (wt in (O.Q4_1, O.Q5_1))
+    assert np.array_equal(np.where(np.isfinite(ref), 0, ref), np.where(np.isfinite(y), 0, y), equal_nan=True)
+
+
 # ---- the GEMM from 17 tokens on, from 25 with few rows of 1536 values and more; the token in front of each line; a type with a minimum: GEMV passes ----
 @pytest.mark.parametrize("K,N,n", [(256, 33, 17), (960, 130, 16), (960, 130, 17), (1472, 70, 31), (1536, 130, 24), (1536, 130, 25), (1920, 2049, 17)])
 @pytest.mark.parametrize("wt", (O.Q4_0, O.Q8_0, O.Q5_1, O.IQ4_NL), ids=lambda t: O.TYPE_NAMES[t])
