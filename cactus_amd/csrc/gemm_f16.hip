@@ -94,9 +94,8 @@ void gemm_f16_kernel(const uint8_t *__restrict__ W, size_t nb01, int64_t K, int6
     }
     if (tok_base >= M) return;
     // The attention mode also takes K that is not a multiple of the 64-value stage (n_kv cache positions, a multiple of 8):
-    // cells of the last stage that lie past K are zeroed on both sides.
-    // (as are those of a last stage that 64 values are left for, KG = 8)
-    constexpr bool KTAIL = MODE == F16_BATCH || KG > F16_KG;
+    // cells of the last stage that lie past K are zeroed on both sides.  Elsewhere K is whole stages (launch_gemm_f16).
+    constexpr bool KTAIL = MODE == F16_BATCH;
     const int nstages = (int)(KTAIL ? ceil_div(K, (int64_t)(16 * KG)) : K / (16 * KG));
     constexpr int STAGE_BYTES = 16 * KG * 2;                   // bytes of one row per stage
     static_assert(C::NT % C::CELLS == 0, "a thread's items all have the same cell index");
@@ -468,13 +467,14 @@ hipError_t launch_gemm_f16(const void *W, size_t nb01, int64_t K, int64_t N, con
     // 4096 x 4096 that no cache holds at 64 tokens 31.6 -> 26.4, 201 31.6 -> 28.2, 300 36.9 -> 34.5; 14336 x 4096 at 201 80.6 -> 75.9.
     const int64_t g128 = ceil_div(N, 128) * ceil_div(M, 128), g256 = ceil_div(N, 256) * ceil_div(M, 256), g64 = ceil_div(N, 64) * ceil_div(M, 64);
     const int cfg = (int)tune("CHIP_GEMM_F16_CFG", 2 * g256 >= cus && K >= 4 * BIG_K && n_as == 1 ? 9 : g128 >= cus ? 0 : 1);
+    const bool whole = K % 128 == 0;                                     // stages of 128 values
     switch (cfg) {
         case 0:                                                                                                         // 128 x 128, 4 waves
             if (g128 > cus) return launch_f16<2, 2, 2, 2, 2, F16_PLAIN, false, 1>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
             return launch_f16<2, 2, 2, 2, 2, F16_PLAIN, false, 2>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
         case 1:                                                                                                         // 64 x 64, 4 waves; 64 x 32, 2 waves
-            if (2 * g64 <= cus && !(M <= 128 && K <= 1280 && 4 * g64 > cus)) return launch_f16<1, 1, 2, 1, 2, F16_PLAIN, false, 2, 8>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
-            if (2 * g64 <= 3 * cus && !(M <= 128 && g64 <= cus)) return launch_f16<1, 1, 2, 2, 2, F16_PLAIN, false, 2, 8>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
+            if (whole && 2 * g64 <= cus && !(M <= 128 && K <= 1280 && 4 * g64 > cus)) return launch_f16<1, 1, 2, 1, 2, F16_PLAIN, false, 2, 8>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
+            if (whole && 2 * g64 <= 3 * cus && !(M <= 128 && g64 <= cus)) return launch_f16<1, 1, 2, 2, 2, F16_PLAIN, false, 2, 8>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
             if (2 * g64 <= 3 * cus) return launch_f16<1, 1, 2, 2, 4, F16_PLAIN, false, 3>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
             return launch_f16<1, 1, 2, 2, 4, F16_PLAIN, false, 2>(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st, rg, n_as);
         case 9: return launch_f16_direct(W, nb01, K, N, ws, ws_stride, M, y, ldy, lim, st);                             // 256 x 256, 4 waves, direct to LDS
