@@ -696,7 +696,7 @@ static float blk32_walk_us(int wtype, int64_t K, int64_t N, int64_t M, int64_t c
 }
 static FewPlan blk32_few_plan(int wtype, int64_t K, int64_t N, int64_t M, size_t nb01, int64_t cus, bool room) {
     const int64_t tiles = ceil_div(N, (int64_t)32) * ceil_div(M, (int64_t)32);
-    if (K < 256 || tiles > 65536 || nb01 > ((size_t)1 << 27)) return FewPlan{0, 1};           // (rows within 32-bit reach)
+    if (K < 256 || tiles > 65536 || nb01 > ((size_t)1 << 27) || K > ((int64_t)1 << 26)) return FewPlan{0, 1};    // (rows and tokens within 32-bit reach)
     if (!room && blk32_slices_for(K, N, M, cus) > 1) return FewPlan{0, 1};
     float best = blk32_walk_us(wtype, K, N, M, cus) / 1.15f;
     FewPlan plan{0, 1};
