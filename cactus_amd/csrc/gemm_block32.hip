@@ -670,11 +670,12 @@ static int blk32_slices_for(int64_t K, int64_t N, int64_t M, int64_t cus) {
 
 // Few output tiles: gemm_blk32_few_kernel, whose ks waves a workgroup share the K of a 32 x 32 tile, or the staged walk of this file, whichever
 // is estimated ahead, in us of a launch.  Fitted to 707 products of 256 to 14336 values x 320 to 14336 rows at 17 to 512 tokens (11 and 19 per cent
-// of spread); the walk is left where it is more than 15 per cent slower: 1.21 x over all of them, 16 more than 2 per cent slower than before, the
-// worst 1.12 x (14336 values x 2048 rows at 133 tokens).  us, walk / few: Q4_0 960 x 960 at 133 tokens 9.3 / 5.5, 2560 x 960 13.3 / 8.4, 4096 x 4096 at 17
-// 12.1 / 9.0, at 128 20.8 / 14.5, 2048 x 2048 at 512 20.9 / 14.7; Q5_0 2048 x 2048 at 40 13.9 / 7.4; 14336 x 4096 at 32 25.0 / 25.4 and stays.
+// of spread); the walk is left where it is more than 15 per cent slower.  Over 800 others (512 to 14336 values, 256 to 16384 rows, 5 to 1100 tokens) 1.12 x,
+// none more than 3 per cent slower than before; of products drawn where the tiles half fill the device one in 25 is, the worst 1.2 x.  us, walk / few:
+// Q4_0 960 x 960 at 133 tokens 9.3 / 5.5, 2560 x 960 13.3 / 8.4, 4096 x 4096 at 17 12.1 / 9.0, at 128 20.8 / 14.5, 2048 x 2048 at 512 20.9 / 14.7; Q5_0 2048 x 2048 at 40 13.9 / 7.4; 14336 x 4096 at 32 25.0 / 25.4 and stays.
 //   few    a launch; the turns of 8 waves a CU, each the fetch of a first chunk and then its chunks of 256 values, as long as a load takes or as
-//          the vector work of the waves of a CU
+//          the vector work of the waves of a CU (halfway between the average and the busiest CU: by the average alone one product in 110 was more than
+//          5 per cent slower than the walk, Q8_0 4352 x 4828 at 35 tokens 19.3 / 21.9)
 //   walk   a launch; the turns of the workgroups a CU holds, each the fetch of a first stage and then its stages; the slice sum
 // A caller without room for the slices that the walk would be cut into keeps the order of one walk over K, whatever the tile (room: the caller has it;
 // a group is planned without, so that its members have the bits of their single calls).  At most 64 tiles of rows of 4096 values
@@ -705,7 +706,7 @@ static FewPlan blk32_few_plan(int wtype, int64_t K, int64_t N, int64_t M, size_t
         const int64_t wgs = tiles * slices, turn = cus * (8 / ks), turns = wgs / turn, rest = wgs % turn;
         const float chunks = (float)ceil_div(2 * ceil_div(ceil_div(K / 64, (int64_t)slices), (int64_t)ks), (int64_t)8);
         float t = 2.04f + (float)turns * (1.8f + chunks * 2.62f);
-        if (rest) t += 1.8f + chunks * std::max(1.72f, 0.328f * std::max((float)ks, (float)(rest * ks) / (float)cus));
+        if (rest) t += 1.8f + chunks * std::max(1.72f, 0.328f * std::max((float)ks, 0.5f * ((float)(rest * ks) / (float)cus + (float)(ceil_div(rest, cus) * ks))));
         if (slices > 1) t += 3.8f + 0.9e-6f * (float)N * (float)M * (float)slices;
         if (t < best) { best = t; plan = FewPlan{ks, slices}; }
     }

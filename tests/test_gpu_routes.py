@@ -135,6 +135,14 @@ def test_unsplit_short_last_stage_takes_the_gemm_where_it_is_ahead(dev, orc, wt,
     assert mul_mat_launches(dev, wt, wq, common.activations_f32(6, n, 8256), split_k=False) == count
 
 
+# 300 to 330 tiles of long rows (us, walk in slices of K / tiles shared by waves: 32.9 / 36.6, 34.7 / 38.0, 19.3 / 21.9), and fewer
+@pytest.mark.parametrize("wt,K,N,n,walk", [(O.Q5_0, 9600, 1288, 254, True), (O.IQ4_NL, 9600, 401, 732, True), (O.Q8_0, 4352, 4828, 35, True),
+                                           (O.Q8_0, 2176, 4828, 35, False), (O.Q5_0, 1920, 1288, 254, False)])
+def test_block32_products_that_half_fill_the_device_stay_in_the_walk(dev, wt, K, N, n, walk):
+    names = mul_mat_kernels(dev, wt, np.zeros((N, dev.row_size(wt, K)), np.uint8), common.activations_f32(1, n, K))
+    assert len(names) == (3 if walk else 2) and ("gemm_blk32_kernel" if walk else "gemm_blk32_few_kernel") in names[1]
+
+
 # kqv of more than 128 columns per KV head: one launch of the GEMM with the 256 bytes it asks for, the same bits whatever lies behind
 # them, and nothing written there; one launch of the dot-product kernel without a workspace
 @pytest.mark.parametrize("hd,nh,nkv,n,kv", [(128, 8, 2, 70, 264), (64, 6, 3, 133, 1064), (256, 4, 1, 65, 520), (96, 8, 4, 80, 136)])
