@@ -12,7 +12,7 @@ import functools
 
 import common
 import oracle as O
-from test_gpu_routes import mul_mat_id_launches
+from test_gpu_routes import mul_mat_id_launches, mul_mat_kernels
 
 
 @functools.lru_cache(maxsize=12)
@@ -725,10 +725,11 @@ def exact_q8_K_inputs(rng, n, K):
 
 
 @pytest.mark.parametrize("wt", KQ_TYPES + B32_TYPES, ids=lambda t: O.TYPE_NAMES[t])
-@pytest.mark.parametrize("K,N,n", [(4096, 300, 64), (2304, 131, 70), (14336, 200, 128), (4096, 8000, 50)])
+@pytest.mark.parametrize("K,N,n", [(4096, 300, 64), (2304, 131, 70), (14336, 200, 128), (4096, 8000, 50), (4352, 301, 130)])
 def test_gemm_split_k_vs_oracle(dev, orc, wt, K, N, n):
     """Few tokens on a matrix with few row tiles: K is cut into slices run by separate workgroups and a second kernel adds
-    the partial outputs in slice order (uneven slices at K = 2304; N = 131 is no multiple of the adder's four rows).
+    the partial outputs in slice order (uneven slices at K = 2304 and 4352; N = 131 and 301 are no multiples of the adder's four rows),
+    or the waves of a workgroup share it (4096 values: the K-quants but Q6_K at 50 tokens, and the 32-value blocks; those also at 2304).
     Against the oracle, against the unsplit GEMM, and the same bits on a second run."""
     import cactus_amd as ca
     print("split-k gemm", O.TYPE_NAMES[wt], "K", K, "N", N, "n", n, flush=True)
@@ -736,6 +737,9 @@ def test_gemm_split_k_vs_oracle(dev, orc, wt, K, N, n):
     assert dev.lib.chip_mul_mat_workspace_size_n(wt, K, N, n) > act                   # this case does split
     wq = quantized_weights(wt, K + N, N, K)
     x = common.activations_f32(K + n, n, K)
+    names = mul_mat_kernels(dev, wt, wq, x)
+    if n >= 128 or (wt in KQ_TYPES and n == 70):
+        assert len(names) == 3 and "_few_" not in names[1] and "sum_slices_kernel" in names[2]
     ref = orc.mul_mat(wt, wq, x, nthreads=8, want=("sum_abs",))
     y = dev.mul_mat(wt, wq, x)
     check_outputs(y, ref["y"], ref["sum_abs"], "split-k gemm")

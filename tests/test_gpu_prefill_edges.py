@@ -63,7 +63,7 @@ def random_rows(wt, rng, N, nsb):
 # short rows; 128 x 128 tiles; many tokens, few rows; the GEMM at the fewest tokens it is taken from; the staging kernel
 @pytest.mark.parametrize("wt", LOW_BIT, ids=lambda t: O.TYPE_NAMES[t])
 @pytest.mark.parametrize("K,N,n", [(256, 5, 41), (1024, 131, 65), (2304, 131, 70), (4096, 300, 9), (512, 4100, 1030), (768, 33, 1100),
-                                   (14336, 70, 9), (2304, 8200, 70), (1280, 8100, 33), (512, 300, 96), (768, 131, 33)])
+                                   (14336, 70, 9), (2304, 8200, 70), (1280, 8100, 33), (512, 300, 96), (768, 131, 33), (2304, 12000, 70)])
 def test_low_bit_kquant_gemm(dev, orc, wt, K, N, n):
     rng = np.random.default_rng(K + N + wt)
     w = random_rows(wt, rng, N, K // 256)
@@ -72,6 +72,8 @@ def test_low_bit_kquant_gemm(dev, orc, wt, K, N, n):
     x[4] = 127.0
     x[5] = -127.0
     x[4:6, ::256] = -127.0
+    if N == 12000:
+        assert ("gemm_kq_kernel" in mul_mat_kernels(dev, wt, w, x)[1]) == (wt != O.Q2_K)
     y = dev.mul_mat(wt, w, x)
     rows = np.unique(np.concatenate([[0, 1, 2, 3, N - 1], rng.choice(N, min(N, 200), replace=False)]))
     toks = np.unique(np.concatenate([[0, 3, 4, 5, n - 1], rng.choice(n, min(n, 64), replace=False)]))
@@ -80,9 +82,10 @@ def test_low_bit_kquant_gemm(dev, orc, wt, K, N, n):
 
 
 # The GEMM whose waves expand their own rows, (K, N, n): two workgroups a CU, ragged rows and tokens; two k groups over an odd number
-# of super-blocks; uneven slices and a last tile of one token; two k groups in two slices of different length
+# of super-blocks; uneven slices and a last tile of one token (at 33 tokens by waves that share a tile); two k groups in two slices of different
+# length (Q2_K, IQ4_XS; unsplit Q4_K and Q5_K) and unsplit
 @pytest.mark.parametrize("wt", (O.Q4_K, O.Q5_K, O.Q6_K) + LOW_BIT, ids=lambda t: O.TYPE_NAMES[t])
-@pytest.mark.parametrize("K,N,n", [(512, 4200, 1100), (1280, 4100, 260), (2816, 131, 33), (8448, 4100, 130)])
+@pytest.mark.parametrize("K,N,n", [(512, 4200, 1100), (1280, 4100, 260), (2816, 131, 33), (8448, 4100, 130), (2816, 131, 65), (8448, 4100, 200)])
 def test_kquant_row_gemm(dev, orc, wt, K, N, n):
     rng = np.random.default_rng(K + N + wt)
     w = rng.integers(0, 256, (N, K // 256, O.BLOCK_BYTES[wt]), dtype=np.uint8)
@@ -96,6 +99,13 @@ def test_kquant_row_gemm(dev, orc, wt, K, N, n):
     x[3] = 0
     x[4] = 127.0
     x[5] = -127.0
+    names = mul_mat_kernels(dev, wt, w, x)
+    staged = wt in (O.Q6_K, O.Q3_K)
+    if N == 131:
+        assert ("gemm_kq_few" if n == 33 else "gemm_kq_kernel" if staged else "gemm_kr_kernel") in names[1] and len(names) == (2 if n == 33 else 3)
+    elif K == 8448 and not (staged and n == 130):
+        groups = 1 if n == 200 and wt in (O.Q4_K, O.Q5_K) else 2
+        assert ("gemm_kq_kernel" if wt == O.Q6_K else "gemm_kr_kernelILi%dELi2ELi%dE" % (wt, groups)) in names[1]
     y = dev.mul_mat(wt, w, x)
     rows = np.unique(np.concatenate([[0, 1, 2, 3, N - 1], rng.choice(N, min(N, 150), replace=False)]))
     toks = np.unique(np.concatenate([[0, 3, 4, 5, n - 1], rng.choice(n, min(n, 48), replace=False)]))
@@ -417,18 +427,22 @@ def test_kquant_few_expert_pairs_as_near_as_the_gemv(dev, orc, wt, K):
     assert distance(orc, wt, K, rows, x[:, 0], y[:, :100]) <= 1.1 * distance(orc, wt, K, rows, x[:, 0], gemv[:, :100])
 
 
-# K in eight slices of one super-block (Q2_K, IQ4_XS) and in two of four: no further off than rows walked whole (8192 outputs: within 1 per cent)
+# K in eight slices of one super-block (Q2_K, IQ4_XS) and in two of four: no further off than rows walked whole (9216 outputs: within 1 per cent).  At 64
+# tokens eight waves share it
+@pytest.mark.parametrize("n", (64, 72))
 @pytest.mark.parametrize("wt", LOW_BIT, ids=lambda t: O.TYPE_NAMES[t])
-def test_slices_of_k_as_near_as_whole_rows(dev, orc, wt):
-    K, N, n = 2048, 128, 64
+def test_slices_of_k_as_near_as_whole_rows(dev, orc, wt, n):
+    K, N = 2048, 128
     w = orc.quantize_weights(wt, common.weights_f32(K + N, N, K))
     x = common.activations_f32(K + n, n, K)
+    names = mul_mat_kernels(dev, wt, w, x)
+    assert "gemm_kq_few_kernel" in names[1] if n == 64 else "sum_slices_kernel" in names[2]
     whole, slices = dev.mul_mat(wt, w, x, split_k=False), dev.mul_mat(wt, w, x)
     assert slices.tobytes() != whole.tobytes()
     assert distance(orc, wt, K, w, x, slices) <= 1.03 * distance(orc, wt, K, w, x, whole)
 
 
-# ---- K-quants, 5 to 40 tokens: tiles of 16 or 32 rows and tokens whose super-blocks are shared by waves ----
+# ---- K-quants of few tokens: tiles of 16 or 32 rows and tokens whose super-blocks are shared by waves ----
 # (K, N, n): one row and two super-blocks, a wave each; ragged rows and more waves than a row has left over; 16 and 17 tokens; a second token tile of one
 # token; an odd number of super-blocks over eight waves; more row tiles than a turn of workgroups; more waves than 48 KB of local memory serve
 @pytest.mark.parametrize("wt", (O.Q4_K, O.Q5_K, O.Q6_K) + LOW_BIT, ids=lambda t: O.TYPE_NAMES[t])
@@ -479,6 +493,22 @@ def test_kquant_few_tokens_in_a_group(dev, orc, types, n):
     assert group_launches(dev, [(t, w.shape[0]) for t, w in ws], K, n) == 2
     for (t, w), y in zip(ws, dev.mul_mat_group(ws, x)):
         assert y.tobytes() == dev.mul_mat(t, w, x).tobytes(), O.TYPE_NAMES[t]
+
+
+# members that take tiles of 16 and of 32 rows alone: of 32 for all of one type, of 16 where there are two types
+@pytest.mark.parametrize("types,kernel", [((O.Q4_K,) * 3, "gemm_kq_few_kernelILi12ELi2ELi2E"), ((O.Q3_K,) * 3, "gemm_kq_few_kernelILi11ELi2ELi2E"),
+                                          ((O.Q4_K, O.Q6_K, O.Q6_K), "gemm_kq_few_two_kernelILi12ELi14ELi2E")], ids=("one type", "Q3_K", "two types"))
+def test_kquant_few_tokens_in_a_group_of_tall_and_short_tiles(dev, orc, types, kernel):
+    K, n, rows = 2304, 40, (2001, 2107, 33)
+    q = [orc.quantize_weights(t, common.weights_f32(K + i, 50, K)) for i, t in enumerate(types)]
+    ws = [(t, np.tile(w, (-(-N // 50), 1))[:N]) for t, w, N in zip(types, q, rows)]
+    x = common.activations_f32(K, n, K)
+    for (t, w), rt in zip(ws, (1, 2, 1)):
+        assert "gemm_kq_few_kernelILi%dELi%dELi2E" % (t, rt) in mul_mat_kernels(dev, t, w, x)[1]
+    names = group_kernels(dev, [(t, w.shape[0]) for t, w in ws], K, n)
+    assert len(names) == 2 and kernel in names[1]
+    for (t, w), y in zip(ws, dev.mul_mat_group(ws, x)):
+        assert y.tobytes() == dev.mul_mat(t, w, x).tobytes(), w.shape
 
 
 # an infinite weight scale gives infinities, not NaN, also where the roundings of the sum are kept
