@@ -610,7 +610,7 @@ KqFew kq_few_plan(int wtype, size_t nb01, int64_t K, int64_t N, int64_t n, bool 
     KqFew best{0, 0, 0};
     float least = 0.93f * others_estimate(wtype, K, N, n, p, cus);
     for (const FewForm &f : kFewForms) {
-        // (at most eight super-blocks a wave: longer rows take the next form of more waves, or none, as in the fit)
+        // (at most eight super-blocks a wave: a chain of eight additions at most, gemm_kquant_few.hip)
         if (f.tt != (n > 16 ? 2 : 1) || f.ks > units || units > 8 * f.ks || reach < 16 * f.rt) continue;
         if (const float e = few_estimate(f, wtype, K, N, n, cus); e < least) { least = e; best = KqFew{f.rt, f.tt, f.ks}; }
     }

@@ -6,14 +6,16 @@
 // end: it loads its rows' packed bytes and its tokens' quants in memory order, a super-block ahead of the one it multiplies, turns them round
 // through a stretch of LDS of its own, with no barrier, and expands its lanes' operands in registers (kquant_rows_dev.h; what the digit planes
 // are: gemm_kquant_rows.hip).  A v_mfma_i32_16x16x64_i8 covers two k-blocks: lane (x, g) holds the k-half g % 2 of a k-block of item (H, g / 2), for rows
-// and tokens alike.  A super-block's integers are scaled and added in 64 bits, and so are the waves' sums, which meet in LDS once: a result is its sum
-// rounded once.  (In 32 bits the kernel is 1 to 3 per cent faster, 7.7 against 7.8 us for Q6_K 4096 values x 4096 rows at 8 tokens, but rows of two super-blocks were up
-// to 1.16 x as far from the 64-bit sums as the GEMV's, and Q2_K and IQ4_XS 1.07 x as far as slices of K; 2-norm of the error over that of the sums, 512
-// values at 15 tokens, GEMV / 32 bits / 64: Q3_K 4.0e-8 / 4.5e-8 / 2.7e-8.)
+// and tokens alike.  The waves' sums meet in LDS once and are added as doubles.  A wave scales and adds its super-blocks in 32 bits, at most eight of
+// them (kq_few_plan), no further from the 64-bit sums than the GEMV, the walks and the slices of K that ran before (2-norm of the error over 239 random
+// products of Q4_K, Q5_K, Q6_K and Q3_K, 1024 to 14336 values at 5 to 300 tokens: 0.80 of theirs on average, 1.05 at most, where the sample is good for
+// 0.03); but rows of up to three super-blocks, and Q2_K and IQ4_XS, whose slices were short chains added as doubles, in 64 bits, a result rounded once:
+// in 32 bits they were up to 1.16 and 1.07 x as far (512 values at 15 tokens, GEMV / 32 bits / 64: Q3_K 4.0e-8 / 4.5e-8 / 2.7e-8).  64 bits
+// take 1.025 x the time (83 products of Q2_K and IQ4_XS; so does the product in 32 bits added in 64).
 //
-// Bound: the issue of vector instructions (some 200 per super-block of 16 rows x 16 tokens, over half of them the expansion) at two to four waves a
-// SIMD, and the tokens' quants, 4 KB for the 1.3 to 3.4 KB of 16 rows: tiles of 32 rows halve those where there are rows enough.  us, what ran before /
-// this, 8 tokens (a GEMV): Q6_K 4096 values x 4096 rows 9.6 / 7.8, 14336 x 4096 20.0 / 16.7, 4096 x 32000 37 / 31; Q4_K 1024 x 3072 7.7 / 4.1; 32
+// Bound: the issue of vector instructions (by the counters 230 per super-block of 16 rows x 16 tokens for Q4_K, 280 to 300 for Q6_K, over half of them the expansion) at two
+// to four waves a SIMD, and the tokens' quants, 4 KB for the 1.3 to 3.4 KB of 16 rows: tiles of 32 rows halve those where there are rows enough.  us, what ran
+// before / this, 8 tokens (a GEMV): Q6_K 4096 values x 4096 rows 9.6 / 7.7, 14336 x 4096 20.0 / 16.5, 4096 x 32000 37 / 31; Q4_K 1024 x 3072 7.7 / 4.1; 32
 // tokens (the GEMM, in slices of K): Q4_K 4096 x 4096 13.8 / 8.3, x 14336 27.0 / 18.7, 2048 x 768 11.2 / 5.1; 64 tokens Q4_K 4096 x 4096
 // 16.1 / 11.1.  16 rows rather than 32 a tile because 4096 rows are then a workgroup for every CU; more waves than super-blocks have nothing to share.
 #include "dev_common.h"
@@ -30,6 +32,10 @@ namespace {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 
+// Rows of up to three super-blocks, and Q2_K and IQ4_XS of any length, are scaled and added in 64 bits.
+constexpr int FEW_SHORT = 3;
+constexpr bool few_always_wide(int wt) { return wt == T_Q2_K || wt == T_IQ4_XS; }
+
 template <int WT, int RT, int TT>
 struct KfCfg {
     using T = KR<WT>;
@@ -41,12 +47,13 @@ struct KfCfg {
     static_assert(WAVE % 16 == 0 && WAVE >= BM * BN * 8, "a wave's sums take the place of its operands");
 };
 
-// One tile; `stretch`: bytes of LDS a wave has.
-template <int WT, int RT, int TT>
+// One tile; `stretch`: bytes of LDS a wave has.  WIDE: super-blocks are scaled and added in 64 bits.
+template <int WT, int RT, int TT, bool WIDE>
 __device__ __forceinline__ void few_tile(uint8_t *lds, int stretch, const GemmMat &mat, int row_tile, int tok_tile, int64_t K,
                                          const uint8_t *__restrict__ ws, size_t ws_stride, int64_t M) {
     using T = KR<WT>;
     using C = KfCfg<WT, RT, TT>;
+    using real = std::conditional_t<WIDE, double, float>;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ks = (int)blockDim.x >> 6;
     const int x = lane & 15, g = lane >> 4, hf = g & 1, p = g >> 1;
     const int64_t N = mat.N, row_base = (int64_t)row_tile * C::BM, tok_base = (int64_t)tok_tile * C::BN;
@@ -95,7 +102,7 @@ __device__ __forceinline__ void few_tile(uint8_t *lds, int stretch, const GemmMa
     const u32x4 *const row = reinterpret_cast<const u32x4 *>(own) + x * C::ROW;           // and 16 rows on per tile of rows
     // cell 2 * k-block + k-half of the lane's token; the bits that H and the second k-block add are not set in it
     const uint32_t b_lane = (uint32_t)C::OFF_X + (uint32_t)x * 256u + 16u * (uint32_t)((2 * (3 - T::NEXT) * p + hf) ^ x);
-    double out[RT][TT][4] = {};
+    real out[RT][TT][4] = {};
 
     Load k;
     load(k, wave);                                                                       // (ks <= nsb: launch_few)
@@ -104,23 +111,35 @@ __device__ __forceinline__ void few_tile(uint8_t *lds, int stretch, const GemmMa
         if (sb + ks < nsb) load(k, sb + ks);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
+        // (beside 64-bit sums the headers of all row tiles and a half's quants would not fit the registers: they are read where they are used)
+        typename T::Hdr held[RT];
+        auto hdr = [&](int r) { return WIDE ? T::hdr(row + 16 * r * C::ROW, hf) : held[r]; };
+        auto quants = [&](int H, int e, int c) { return *reinterpret_cast<const u32x4 *>(own + c * 4096 + (b_lane ^ (uint32_t)(16 * (8 * H + 2 * T::NEXT * e)))); };
+        if constexpr (!WIDE)
+#pragma unroll
+            for (int r = 0; r < RT; r++) held[r] = T::hdr(row + 16 * r * C::ROW, hf);
         i32x4 P[T::NPL][RT][TT];
 #pragma unroll
         for (int H = 0; H < 2; H++) {
-            // Q5_K reads its header for each half and for the fold: held over all it would not fit the registers
-            if constexpr (WT == T_Q5_K) asm volatile("" ::: "memory");
+            if constexpr (WT == T_Q5_K && WIDE) asm volatile("" ::: "memory");            // its header again for each half and for the fold
+            u32x4 a[2][TT];
+            if constexpr (!WIDE)
+#pragma unroll
+                for (int e = 0; e < 2; e++)
+#pragma unroll
+                    for (int c = 0; c < TT; c++) a[e][c] = quants(H, e, c);
 #pragma unroll
             for (int r = 0; r < RT; r++) {
                 u32x4 w[2][T::NPL];
-                T::expand(T::load(row + 16 * r * C::ROW, H, p, hf), T::hdr(row + 16 * r * C::ROW, hf), H, p, hf, w);
+                T::expand(T::load(row + 16 * r * C::ROW, H, p, hf), hdr(r), H, p, hf, w);
 #pragma unroll
                 for (int e = 0; e < 2; e++)
 #pragma unroll
                     for (int c = 0; c < TT; c++) {
-                        const u32x4 a = *reinterpret_cast<const u32x4 *>(own + c * 4096 + (b_lane ^ (uint32_t)(16 * (8 * H + 2 * T::NEXT * e))));
+                        if constexpr (WIDE) a[e][c] = quants(H, e, c);
 #pragma unroll
                         for (int pl = 0; pl < T::NPL; pl++)
-                            P[pl][r][c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, a), __builtin_bit_cast(i32x4, w[e][pl]),
+                            P[pl][r][c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, a[e][c]), __builtin_bit_cast(i32x4, w[e][pl]),
                                                                                 H == 0 && e == 0 ? i32x4{0, 0, 0, 0} : P[pl][r][c], 0, 0, 0);
                     }
             }
@@ -128,9 +147,10 @@ __device__ __forceinline__ void few_tile(uint8_t *lds, int stretch, const GemmMa
         // fold, as the reference does once per super-block: out += dx * (d * sumi - dmin * summ)
 #pragma unroll
         for (int r = 0; r < RT; r++) {
-            if constexpr (WT == T_Q5_K) asm volatile("" ::: "memory");
-            const uint32_t scales = T::scales(T::hdr(row + 16 * r * C::ROW, hf));
-            const double d = h2f(scales), dmin = h2f(scales >> 16);
+            if constexpr (WT == T_Q5_K && WIDE) asm volatile("" ::: "memory");
+            const uint32_t scales = T::scales(hdr(r));
+            real d = h2f(scales), dmin = h2f(scales >> 16);
+            if constexpr (!WIDE) asm volatile("" : "+v"(d), "+v"(dmin));   // widened once: as halves they would make the multiply-adds half-rate mixed ones
 #pragma unroll
             for (int c = 0; c < TT; c++) {
                 f32x4 F = {0.f, 0.f, 0.f, 0.f};
@@ -142,7 +162,7 @@ __device__ __forceinline__ void few_tile(uint8_t *lds, int stretch, const GemmMa
 #pragma unroll
                 for (int v = 0; v < 4; v++) {
                     const float f[2] = {F[v], 0.f};
-                    out[r][c][v] = __builtin_fma(T::value(P[0][r][c][v], P[T::NPL - 1][r][c][v], f, d, dmin), (double)dx[v], out[r][c][v]);
+                    out[r][c][v] = mul_add(T::value(P[0][r][c][v], P[T::NPL - 1][r][c][v], f, d, dmin), (real)dx[v], out[r][c][v]);
                 }
             }
         }
@@ -150,7 +170,7 @@ __device__ __forceinline__ void few_tile(uint8_t *lds, int stretch, const GemmMa
         __builtin_amdgcn_wave_barrier();
     }
     // register v of tile (r, c) is token 16 c + 4 g + v, the lane's x its row 16 r + x
-    double *const part = reinterpret_cast<double *>(own);
+    real *const part = reinterpret_cast<real *>(own);
 #pragma unroll
     for (int r = 0; r < RT; r++)
 #pragma unroll
@@ -160,7 +180,7 @@ __device__ __forceinline__ void few_tile(uint8_t *lds, int stretch, const GemmMa
     __syncthreads();
     for (int e = threadIdx.x; e < 256 * RT * TT; e += (int)blockDim.x) {
         double o = 0.;
-        for (int w = 0; w < ks; w++) o += reinterpret_cast<const double *>(lds + w * stretch)[e];
+        for (int w = 0; w < ks; w++) o += (double)reinterpret_cast<const real *>(lds + w * stretch)[e];
         const int tile = e >> 8, t = 16 * (tile / RT) + 4 * ((e & 63) >> 4) + ((e >> 6) & 3);
         const int64_t r = row_base + 16 * (tile % RT) + (e & 15);
         if (t < tokens && r < N) mat.y[(size_t)(tok_base + t) * mat.ldy + r] = (float)o;
@@ -170,19 +190,19 @@ __device__ __forceinline__ void few_tile(uint8_t *lds, int stretch, const GemmMa
 constexpr int few_waves(int rt, int tt) { return rt * tt == 1 ? 16 : 8; }               // most waves of a workgroup
 #define KQ_FEW_BOUNDS(RT, TT) __launch_bounds__(64 * few_waves(RT, TT)) __attribute__((amdgpu_waves_per_eu((RT) * (TT) == 1 ? 4 : (RT) * (TT) == 2 ? 3 : 2)))
 
-template <int WT, int RT, int TT>
+template <int WT, int RT, int TT, bool WIDE>
 __global__ KQ_FEW_BOUNDS(RT, TT)
 void gemm_kq_few_kernel(GemmMats mats, int64_t K, const uint8_t *__restrict__ ws, size_t ws_stride, int64_t M, TileMap map) {
     extern __shared__ __align__(16) uint8_t lds[];
     TileCoord tc = xcd_tile(blockIdx.x, map);
     if (tc.row_tile >= map.row_tiles || tc.tok_tile >= map.tok_tiles) return;            // padding of the tile map
     const GemmMat mat = pick_gemm_mat(mats, tc.row_tile);
-    few_tile<WT, RT, TT>(lds, KfCfg<WT, RT, TT>::WAVE, mat, tc.row_tile, tc.tok_tile, K, ws, ws_stride, M);
+    few_tile<WT, RT, TT, WIDE>(lds, KfCfg<WT, RT, TT>::WAVE, mat, tc.row_tile, tc.tok_tile, K, ws, ws_stride, M);
 }
 
 // matrices of two types on the same rows: the row tiles from `second` on are of type WB
 template <int WA, int WB, int TT> constexpr int few_two_stretch() { return KfCfg<WA, 1, TT>::WAVE > KfCfg<WB, 1, TT>::WAVE ? KfCfg<WA, 1, TT>::WAVE : KfCfg<WB, 1, TT>::WAVE; }
-template <int WA, int WB, int TT>
+template <int WA, int WB, int TT, bool SHORT>
 __global__ KQ_FEW_BOUNDS(1, TT)
 void gemm_kq_few_two_kernel(GemmMats mats, int second, int64_t K, const uint8_t *__restrict__ ws, size_t ws_stride, int64_t M, TileMap map) {
     extern __shared__ __align__(16) uint8_t lds[];
@@ -191,29 +211,29 @@ void gemm_kq_few_two_kernel(GemmMats mats, int second, int64_t K, const uint8_t 
     constexpr int STRETCH = few_two_stretch<WA, WB, TT>();
     const bool of_b = tc.row_tile >= second;
     const GemmMat mat = pick_gemm_mat(mats, tc.row_tile);
-    if (of_b) few_tile<WB, 1, TT>(lds, STRETCH, mat, tc.row_tile, tc.tok_tile, K, ws, ws_stride, M);
-    else few_tile<WA, 1, TT>(lds, STRETCH, mat, tc.row_tile, tc.tok_tile, K, ws, ws_stride, M);
+    if (of_b) few_tile<WB, 1, TT, SHORT || few_always_wide(WB)>(lds, STRETCH, mat, tc.row_tile, tc.tok_tile, K, ws, ws_stride, M);
+    else few_tile<WA, 1, TT, SHORT || few_always_wide(WA)>(lds, STRETCH, mat, tc.row_tile, tc.tok_tile, K, ws, ws_stride, M);
 }
 
 struct FewCall { GemmMats mats; int64_t K; const void *ws; size_t ws_stride; int64_t M; const DeviceLimits &lim; hipStream_t st; int ks; };
 
-template <int WT, int RT, int TT>
+template <int WT, int RT, int TT, bool WIDE>
 hipError_t launch_few(FewCall c) {
     using C = KfCfg<WT, RT, TT>;
     const size_t bytes = (size_t)c.ks * C::WAVE;
     if (c.ks < 1 || c.ks > few_waves(RT, TT) || c.ks > c.K / QK_K || (int64_t)bytes > c.lim.max_lds_per_block) return hipErrorInvalidValue;
-    auto kfn = gemm_kq_few_kernel<WT, RT, TT>;
+    auto kfn = gemm_kq_few_kernel<WT, RT, TT, WIDE>;
     static LdsGrant grant;
     if (hipError_t e = grant_dynamic_lds(kfn, bytes, c.lim, grant); e != hipSuccess) return e;
     const TileMap map = make_tile_map(number_row_tiles(c.mats, C::BM), ceil_div(c.M, (int64_t)C::BN), 32 * std::max(1, 16 / c.ks));
     hipLaunchKernelGGL(kfn, dim3(map.grid), dim3(64 * c.ks), bytes, c.st, c.mats, c.K, (const uint8_t *)c.ws, c.ws_stride, c.M, map);
     return hipGetLastError();
 }
-template <int WA, int WB, int TT>
+template <int WA, int WB, int TT, bool SHORT>
 hipError_t launch_two(FewCall c, int first_b) {
     const size_t bytes = (size_t)c.ks * few_two_stretch<WA, WB, TT>();
     if (c.ks < 1 || c.ks > few_waves(1, TT) || c.ks > c.K / QK_K || (int64_t)bytes > c.lim.max_lds_per_block) return hipErrorInvalidValue;
-    auto kfn = gemm_kq_few_two_kernel<WA, WB, TT>;
+    auto kfn = gemm_kq_few_two_kernel<WA, WB, TT, SHORT>;
     static LdsGrant grant;
     if (hipError_t e = grant_dynamic_lds(kfn, bytes, c.lim, grant); e != hipSuccess) return e;
     const TileMap map = make_tile_map(number_row_tiles(c.mats, 16), ceil_div(c.M, (int64_t)(16 * TT)), 32 * std::max(1, 16 / c.ks));
@@ -221,14 +241,24 @@ hipError_t launch_two(FewCall c, int first_b) {
     return hipGetLastError();
 }
 
+template <int WT, bool WIDE>
+hipError_t launch_few_form(int rt, int tt, const FewCall &c) {
+    if (rt == 1) return tt == 1 ? launch_few<WT, 1, 1, WIDE>(c) : launch_few<WT, 1, 2, WIDE>(c);
+    return tt == 1 ? launch_few<WT, 2, 1, WIDE>(c) : launch_few<WT, 2, 2, WIDE>(c);
+}
+bool few_short(const FewCall &c) { return c.K <= FEW_SHORT * QK_K; }
 template <int WT>
 hipError_t launch_few_type(int rt, int tt, const FewCall &c) {
-    if (rt == 1) return tt == 1 ? launch_few<WT, 1, 1>(c) : launch_few<WT, 1, 2>(c);
-    return tt == 1 ? launch_few<WT, 2, 1>(c) : launch_few<WT, 2, 2>(c);
+    if (few_always_wide(WT) || few_short(c)) return launch_few_form<WT, true>(rt, tt, c);
+    return launch_few_form<WT, few_always_wide(WT)>(rt, tt, c);
+}
+template <int WA, int WB, int TT>
+hipError_t launch_two_form(const FewCall &c, int first_b) {
+    return few_short(c) ? launch_two<WA, WB, TT, true>(c, first_b) : launch_two<WA, WB, TT, false>(c, first_b);
 }
 template <int WA, int WB>
 hipError_t launch_two_types(int tt, const FewCall &c, int first_b) {
-    if constexpr (WA < WB) return tt == 1 ? launch_two<WA, WB, 1>(c, first_b) : launch_two<WA, WB, 2>(c, first_b);
+    if constexpr (WA < WB) return tt == 1 ? launch_two_form<WA, WB, 1>(c, first_b) : launch_two_form<WA, WB, 2>(c, first_b);
     return hipErrorInvalidValue;
 }
 template <int WA>
