@@ -430,13 +430,10 @@ static int kq_slices_for(int64_t K, int64_t N, int64_t M, int64_t cus) {
 // which expands a weight once for 128 tokens (us, staged / gemm_kr_kernel: Q6_K 14336 values x 4096 rows at 512 tokens 113 / 128, 201 tokens 66 / 74,
 // 4096 x 4096 at 512 tokens 38.6 / 44; Q3_K 14336 x 4096 at 201 tokens 49 / 53), unless half of its 128-token tile would be empty and the slices
 // give gemm_kr_kernel a workgroup for every CU (32 tokens: Q6_K 41 / 27, Q3_K 30 / 20).
-// Rows above 2048 values take two groups a workgroup, Q4_K and Q5_K unsplit on up to half a workgroup a CU (us, one / two groups: Q4_K 4096 values x 14414
-// rows at 50 tokens 30.8 / 27.4, Q5_K 11520 x 4245 at 181 89 / 80; two such matrices in one launch 33.2 / 31.2 and 90 / 82; over 45 products 1.15 x and 1.07 x,
-// none slower, three in one launch 0.9 x from a third of a workgroup a CU on).  Not above half, where two groups are 1.03 to 1.13 x ahead alone but
-// two such matrices together 1.08 to 1.22 x behind (Q4_K 4352 x 6424 at 244 tokens 50.3 / 56.3): a member of a joined call has the bits of its own call.
-// Up to 2048 values 1.01 x, and one group stays.  The others where the staging kernel's tiles come to a second turn (Q6_K 1.57 x, Q3_K 1.84 x
-// over 44 products: 128-token tiles that are half empty); Q3_K above 128 tokens on half the CUs and more in any case (14336 x 4096 at 201 tokens 42.3 / 40.3
-// without the quantizer; 1.05 x).
+// Rows above 2048 values whose workgroups fit the CUs take two groups a workgroup where one would leave a CU four waves (us, one / two groups: Q4_K unsplit
+// 4096 x 4096 at 512 tokens 32.8 / 28.3, 14336 rows at 64 27.8 / 25.0; Q5_K 36.9 / 32.3; over 700 products 1.12 x, none slower; up to 2048 values 1.01
+// x and one group stays) or where the staging kernel's tiles come to a second turn (Q6_K 1.57 x, Q3_K 1.84 x over 44 products: 128-token tiles
+// that are half empty); Q3_K above 128 tokens on half the CUs and more in any case (14336 x 4096 at 201 tokens 42.3 / 40.3 without the quantizer; 1.05 x).
 // Q2_K and IQ4_XS by their number of 128 x 64 tiles:
 //   more tiles than CUs     one group (us, 512 tokens x 4096 values x 4608 rows, one / two groups: Q2_K 36 / 44, IQ4_XS 66 / 72)
 //   above half as many      two groups, so that every SIMD has two waves (4096 rows: Q2_K 29 / 27, IQ4_XS 45 / 42); so too with 2 slices of
@@ -457,7 +454,7 @@ static KqPlan kq_plan(int wtype, int64_t K, int64_t N, int64_t M, int64_t cus) {
         const int slices = kq_slices_for(K, N, M, cus);
         const bool staged = (wtype == T_Q6_K || wtype == T_Q3_K) && tiles <= cus && (M > 64 || tiles * slices < cus);
         const bool fits = units > 8 && tiles * slices <= cus;
-        const bool two = fits && (wtype == T_Q4_K || wtype == T_Q5_K ? slices == 1 && 2 * tiles <= cus
+        const bool two = fits && (wtype == T_Q4_K || wtype == T_Q5_K ? slices == 1
                                                                      : staged && (ceil_div(N, (int64_t)64) * ceil_div(M, (int64_t)128) * slices > cus ||
                                                                                   (wtype == T_Q3_K && M > 128 && 2 * tiles * slices >= cus)));
         return KqPlan{two ? 2 : staged ? 0 : 1, slices};
@@ -576,11 +573,8 @@ static float others_estimate(int wtype, int64_t K, int64_t N, int64_t n, const K
     const int64_t units = K / QK_K;
     if (four ? n >= gemm_kq_min_tokens(wtype, K, N, p.slices > 1) : n >= 9) {
         const int64_t tiles = p.groups == 0 ? ceil_div(N, (int64_t)64) * ceil_div(n, (int64_t)128) : ceil_div(N, (int64_t)128) * ceil_div(n, (int64_t)64);
-        // (estimated in two groups up to a workgroup a CU: above half of that kq_plan leaves them out for the sake of joined members, and those are further ahead
-        // of this kernel than one alone: three of Q4_K 4608 values x 4452 rows at 213 tokens 51 us in one launch, 77 in this kernel)
-        const bool two = p.groups == 2 || (four && p.slices == 1 && units > 8 && tiles <= cus);
-        const int64_t per = ceil_div(ceil_div(units, (int64_t)p.slices), (int64_t)(two ? 2 : 1));
-        const float turns = (float)ceil_div(tiles * p.slices, cus * (p.groups == 0 || two ? 1 : 2)), walk = turns * (float)per;
+        const int64_t per = ceil_div(ceil_div(units, (int64_t)p.slices), (int64_t)(p.groups == 2 ? 2 : 1));
+        const float turns = (float)ceil_div(tiles * p.slices, cus * (p.groups == 1 ? 2 : 1)), walk = turns * (float)per;
         return t.gemm[0] + (p.slices > 1 ? t.gemm[1] + t.gemm[6] * (float)p.slices * (float)(N * n) * 1e-6f : 0.f) + (t.gemm[2] + (n > 32 ? t.gemm[5] : 0.f)) * walk +
                t.gemm[3] * turns + t.gemm[4] * (float)(tiles * units) / (float)(2 * cus);
     }
@@ -679,30 +673,53 @@ hipError_t launch_gemm_kq(int wtype, const void *W, size_t nb01, int64_t K, int6
     return launch_gemm_kr(p.groups, wtype, mats, K, ws, ws_stride, M, lim, st, rg, n_as, p.slices, split.part);
 }
 
-// Members that run unsplit by themselves, in the number of k groups that each takes alone: the same bits, fewer launches and one set of tiles (us, ffn_gate +
-// ffn_up, Q4_K of 4096 values x 14336 rows at 512 tokens, whose 896 tiles each leave a quarter of the second turn idle: 2 x 93.5 -> 164; wq + wk + wv of 1024
-// values x 1024 + 256 + 256 rows at 128 tokens 36 -> 13).
+// Members that run unsplit by themselves: the same bits, fewer launches and one set of tiles (us, ffn_gate + ffn_up, Q4_K
+// of 4096 values x 14336 rows at 512 tokens, whose 896 tiles each leave a quarter of the second turn idle: 2 x 93.5 -> 164; wq + wk + wv of 1024
+// values x 1024 + 256 + 256 rows at 128 tokens 36 -> 13).  A member is added up in the k groups that it has alone: all in the same number; or, Q4_K and
+// Q5_K whose tiles together are more than the CUs, where one group is ahead (Q4_K 4352 values x 6424 rows twice at 244 tokens 50.3 us, in two 56.3), all in
+// one, which walks the even super-blocks of those that alone have two and then the odd ones.  That walk fetches the lines that two super-blocks share
+// twice: over 33 groups of two and three matrices 0.96 x the speed of the walk in order, which would add in another order (Q4_K 2816 values x 8213 rows
+// twice at 171 tokens 32.1 / 34.0 us, 5120 x 3676 three times at 462 83.7 / 96.1).
 // The k groups that a member alone runs in, 0: the staging kernel.  (IQ4_XS of 2 and 3 super-blocks: alone in the staging kernel, together
 // faster in one launch; the same bits)
 static int kq_own_groups(int wtype, int64_t K, int64_t N, int64_t n, int64_t cus) {
     return wtype == T_IQ4_XS && K < 4 * QK_K ? 1 : kq_plan(wtype, K, N, n, cus).groups;
 }
+// the k groups of the launch, 0: members that do not share one; even_odd is set where one group stands for two
+static int kq_group_groups(int wtype, int64_t K, GemmMats &mats, int64_t n, int64_t cus) {
+    const bool four = wtype == T_Q4_K || wtype == T_Q5_K;
+    int64_t tiles = 0;
+    int least = 2, most = 0;
+    for (int i = 0; i < mats.count; i++) {
+        const int own = kq_own_groups(wtype, K, mats.m[i].N, n, cus);
+        mats.m[i].even_odd = four && own == 2;
+        least = std::min(least, own);
+        most = std::max(most, own);
+        tiles += ceil_div(mats.m[i].N, (int64_t)128) * ceil_div(n, (int64_t)64);
+    }
+    if (least == 0 || (least != most && !four) || (least == 2 && (wtype == T_Q2_K || wtype == T_IQ4_XS))) return 0;
+    if (least == 1 || (four && tiles > cus)) return 1;
+    for (int i = 0; i < mats.count; i++) mats.m[i].even_odd = false;
+    return 2;
+}
 bool gemm_kq_group_applicable(int wtype, int64_t K, const GemmMats &mats, int64_t n, int compute_units) {
     const int64_t cus = compute_units > 0 ? compute_units : 256;
     if (mats.count < 2 || !gemm_kq_type(wtype)) return false;
-    const int groups = kq_own_groups(wtype, K, mats.m[0].N, n, cus);
-    if (groups == 0 || (groups == 2 && (wtype == T_Q2_K || wtype == T_IQ4_XS))) return false;
+    GemmMats t = mats;
+    if (kq_group_groups(wtype, K, t, n, cus) == 0) return false;
     for (int i = 0; i < mats.count; i++) {
         const int64_t N = mats.m[i].N;
-        if (!gemm_kq_supported(wtype, K, N, n, false) || kq_plan(wtype, K, N, n, cus).slices != 1 || kq_own_groups(wtype, K, N, n, cus) != groups) return false;
+        if (!gemm_kq_supported(wtype, K, N, n, false) || kq_plan(wtype, K, N, n, cus).slices != 1) return false;
         if (gemm_kr_rows_in_reach(mats.m[i].nb01) < 32) return false;
     }
     return true;
 }
 hipError_t launch_gemm_kq_group(int wtype, const GemmMats &mats, int64_t K, const void *ws, size_t ws_stride, int64_t n, const DeviceLimits &lim,
                                 hipStream_t st) {
-    const int groups = kq_own_groups(wtype, K, mats.m[0].N, n, lim.compute_units > 0 ? lim.compute_units : 256);
-    return launch_gemm_kr(groups, wtype, mats, K, ws, ws_stride, n, lim, st, RowGather{nullptr, nullptr, nullptr, 1, 1, 0}, 1, 1, nullptr);
+    GemmMats t = mats;
+    const int groups = kq_group_groups(wtype, K, t, n, lim.compute_units > 0 ? lim.compute_units : 256);
+    if (groups == 0) return hipErrorInvalidValue;
+    return launch_gemm_kr(groups, wtype, t, K, ws, ws_stride, n, lim, st, RowGather{nullptr, nullptr, nullptr, 1, 1, 0}, 1, 1, nullptr);
 }
 
 }  // namespace chip

@@ -58,6 +58,9 @@ struct KrCfg {
     static constexpr size_t OFF_SX = OFF_FB + 4 * KS * FB_BYTES;          // [j % 4][k group] f32 [token]: activation scale
     static constexpr size_t OFF_ROW = OFF_SX + 4 * KS * (size_t)BN * 4;   // i32 [token]: output row (expert groups)
     static constexpr size_t TOTAL = OFF_ROW + (size_t)BN * 4;
+    // EVEN_ODD: as many of a lane's 16 TN sums as leave room for two workgroups a CU wait here, [wave][sum][lane]; the rest in registers
+    static constexpr int ROOM = (80 * 1024 - (int)TOTAL) / (NW * 256), WAIT = ROOM < 0 ? 0 : ROOM < 16 * TN ? ROOM : 16 * TN;
+    static constexpr size_t TOTAL_EVEN_ODD = TOTAL + (size_t)WAIT * NW * 256;
     // the other k groups' partial outputs take the place of the operands at the end
     static_assert((size_t)(KS - 1) * 4 * TN * 16 * 256 <= OFF_SX, "partial outputs lie in front of the output rows");
 };
@@ -72,7 +75,9 @@ __device__ __forceinline__ void kr_load16_into_lds(const uint8_t *src, uint32_t 
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_addr) : "memory");
 }
 
-template <int WT, int TN, int KS, int OCC, bool GATHER>
+// EVEN_ODD: matrices with even_odd set are walked over their even super-blocks and then over the odd ones; in between the sums wait in LDS and registers
+// (in y they took 11 to 17 us of a launch of 30 to 130).
+template <int WT, int TN, int KS, int OCC, bool GATHER, bool EVEN_ODD>
 __global__ __launch_bounds__(4 * KS * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
 void gemm_kr_kernel(GemmMats mats, int64_t K, const uint8_t *__restrict__ ws, size_t ws_stride, int64_t M, TileMap map, RowGather rg,
                     int slice_sb) {
@@ -98,6 +103,12 @@ void gemm_kr_kernel(GemmMats mats, int64_t K, const uint8_t *__restrict__ ws, si
         if (tc.row_tile >= map.row_tiles || tc.tok_tile >= map.tok_tiles) return;        // padding of the tile map
     }
     const GemmMat mat = GATHER ? mats.m[0] : pick_gemm_mat(mats, tc.row_tile);
+    const int evens = EVEN_ODD && mat.even_odd ? (nsb + 1) / 2 : nsb;     // super-blocks in front of the turn to the odd ones
+    auto nth = [&](int i) {                                              // the i-th super-block of the walk (past the end: the last)
+        i = min(i, nsb - 1);
+        if constexpr (EVEN_ODD) return evens == nsb ? i : i < evens ? 2 * i : 2 * (i - evens) + 1;
+        return i;
+    };
     const int64_t N = mat.N, ldy = mat.ldy;
     const size_t nb01 = mat.nb01;
     float *__restrict__ y = mat.y;
@@ -125,7 +136,7 @@ void gemm_kr_kernel(GemmMats mats, int64_t K, const uint8_t *__restrict__ ws, si
     u32x4 *const raw_lds = reinterpret_cast<u32x4 *>(lds + C::RAW * wave);
     u32x4 raw[C::NLD];
     auto fetch_w = [&](int sb_wanted) {
-        const uint8_t *p = wbase + (size_t)min(sb_wanted, nsb - 1) * T::BYTES;
+        const uint8_t *p = wbase + (size_t)nth(sb_wanted) * T::BYTES;
 #pragma unroll
         for (int t = 0; t < C::NLD; t++) raw[t] = *reinterpret_cast<const typename T::chunk_t *>(p + woff[t]);
     };
@@ -147,7 +158,7 @@ void gemm_kr_kernel(GemmMats mats, int64_t K, const uint8_t *__restrict__ ws, si
         else boff[j] = (uint32_t)min(t, tokens - 1) * (uint32_t)ws_stride + cell;
     }
     auto issue_x = [&](int sb_wanted, int buf) {
-        const size_t o = (size_t)min(sb_wanted, nsb - 1) * QK_K;
+        const size_t o = (size_t)nth(sb_wanted) * QK_K;
         const uint32_t dst = lds0 + (uint32_t)(C::OFF_B + (size_t)(buf * KS + grp) * C::B_BYTES) + (uint32_t)(wr * C::B_PER_W) * 1024u;
 #pragma unroll
         for (int j = 0; j < C::B_PER_W; j++) {
@@ -162,7 +173,7 @@ void gemm_kr_kernel(GemmMats mats, int64_t K, const uint8_t *__restrict__ ws, si
     float xs;
     u32x4 bs;
     auto fetch_s = [&](int sb_wanted) {
-        const int sb = min(sb_wanted, nsb - 1);
+        const int sb = nth(sb_wanted);
         xs = reinterpret_cast<const float *>(ssrc)[sb];
         if constexpr (T::NF16 > 0) bs = *reinterpret_cast<const u32x4 *>(bssrc + (size_t)sb * 32);
     };
@@ -179,6 +190,19 @@ void gemm_kr_kernel(GemmMats mats, int64_t K, const uint8_t *__restrict__ ws, si
     for (int c = 0; c < TN; c++)
 #pragma unroll
         for (int v = 0; v < 16; v++) out[c][v] = 0.f;
+
+    // at the turn to the odd super-blocks
+    float kept[EVEN_ODD ? 16 * TN - C::WAIT : 1] = {};
+    float *const waiting = reinterpret_cast<float *>(lds + C::TOTAL) + wave * C::WAIT * 64 + lane;
+    auto turn = [&]() {
+#pragma unroll
+        for (int i = 0; i < 16 * TN; i++) {
+            float &o = out[i / 16][i % 16];
+            if (i < C::WAIT) waiting[i * 64] = o;
+            else kept[i - C::WAIT] = o;
+            o = 0.f;
+        }
+    };
 
     // This wave's 32 rows against the first 32*NTL of the tile's tokens.  Activations are the MFMA's first operand: register v of tile c
     // is token 32 c + 8 (v / 4) + 4 half + v % 4, the lane's l32 its row.
@@ -318,7 +342,12 @@ void gemm_kr_kernel(GemmMats mats, int64_t K, const uint8_t *__restrict__ ws, si
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (!last) T::expand(r0, h, 0, 0, half, cc);
         };
-        for (int it = 0; it + 1 < nit; it++) iteration(it, std::false_type{});
+        int it = 0;
+        if constexpr (EVEN_ODD) {
+            for (; it < evens && it + 1 < nit; it++) iteration(it, std::false_type{});
+            if (evens < nsb) turn();
+        }
+        for (; it + 1 < nit; it++) iteration(it, std::false_type{});
         iteration(nit - 1, std::true_type{});
         __syncthreads();
     };
@@ -343,6 +372,10 @@ void gemm_kr_kernel(GemmMats mats, int64_t K, const uint8_t *__restrict__ ws, si
 #pragma unroll
                 for (int v = 0; v < 16; v++) out[c][v] += part[(((g - 1) * 4 + wr) * TN * 16 + c * 16 + v) * 64 + lane];
     }
+    if constexpr (EVEN_ODD)
+        if (evens < nsb)
+#pragma unroll
+            for (int i = 0; i < 16 * TN; i++) out[i / 16][i % 16] += i < C::WAIT ? waiting[i * 64] : kept[i < C::WAIT ? 0 : i - C::WAIT];
     const int64_t row = row_base + l32;
     if (row >= N) return;
 #pragma unroll
@@ -358,26 +391,27 @@ void gemm_kr_kernel(GemmMats mats, int64_t K, const uint8_t *__restrict__ ws, si
         }
 }
 
-template <int WT, int TN, int KS, int OCC, bool GATHER>
+template <int WT, int TN, int KS, int OCC, bool GATHER, bool EVEN_ODD = false>
 hipError_t launch_kr(GemmMats mats, int64_t K, const void *ws, size_t ws_stride, int64_t M, const DeviceLimits &lim, hipStream_t st,
                      const RowGather &rg, int64_t slots, int slices, float *part) {
     using C = KrCfg<WT, TN, KS>;
-    if ((int64_t)C::TOTAL > lim.max_lds_per_block) return hipErrorInvalidValue;
-    auto kfn = gemm_kr_kernel<WT, TN, KS, OCC, GATHER>;
+    constexpr size_t LDS = EVEN_ODD ? C::TOTAL_EVEN_ODD : C::TOTAL;
+    if ((int64_t)LDS > lim.max_lds_per_block) return hipErrorInvalidValue;
+    auto kfn = gemm_kr_kernel<WT, TN, KS, OCC, GATHER, EVEN_ODD>;
     static LdsGrant grant;                                               // one per kernel instantiation
-    if (hipError_t e = grant_dynamic_lds(kfn, C::TOTAL, lim, grant); e != hipSuccess) return e;
-    const int per_cu = (int)(160 * 1024 / C::TOTAL) > 0 ? (int)(160 * 1024 / C::TOTAL) : 1;
+    if (hipError_t e = grant_dynamic_lds(kfn, LDS, lim, grant); e != hipSuccess) return e;
+    const int per_cu = (int)(160 * 1024 / LDS) > 0 ? (int)(160 * 1024 / LDS) : 1;
     const int64_t row_tiles = number_row_tiles(mats, KR_ROWS);
     if constexpr (GATHER) {
         const TileMap map = make_tile_map(row_tiles, 1, 32 * per_cu);
-        hipLaunchKernelGGL(kfn, gather_grid(map, slots, C::NT), dim3(C::NT), C::TOTAL, st, mats, K, (const uint8_t *)ws, ws_stride, M, map, rg, 0);
+        hipLaunchKernelGGL(kfn, gather_grid(map, slots, C::NT), dim3(C::NT), LDS, st, mats, K, (const uint8_t *)ws, ws_stride, M, map, rg, 0);
         return hipGetLastError();
     } else {
         const TileMap map = make_tile_map(row_tiles, ceil_div(M, C::BN), 32 * per_cu);
         const GemmMat out = mats.m[0];
         const int slice_sb = slices > 1 ? (int)ceil_div(K / QK_K, (int64_t)slices) : 0;
         if (slices > 1) { mats.m[0].y = part; mats.m[0].ldy = out.N; }                  // (one matrix)
-        hipLaunchKernelGGL(kfn, dim3(map.grid, (unsigned)slices), dim3(C::NT), C::TOTAL, st, mats, K, (const uint8_t *)ws, ws_stride, M, map, rg, slice_sb);
+        hipLaunchKernelGGL(kfn, dim3(map.grid, (unsigned)slices), dim3(C::NT), LDS, st, mats, K, (const uint8_t *)ws, ws_stride, M, map, rg, slice_sb);
         if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
         return slices > 1 ? launch_sum_slices(part, slices, M, out.N, out.y, out.ldy, st, WT == T_Q2_K || WT == T_IQ4_XS) : hipSuccess;
     }
@@ -388,6 +422,9 @@ hipError_t launch_kr_groups(int groups, const GemmMats &mats, int64_t K, const v
                             hipStream_t st, const RowGather &rg, int64_t slots, int slices, float *part) {
     if (rg.perm) return launch_kr<WT, 2, 1, 2, true>(mats, K, ws, ws_stride, M, lim, st, rg, slots, 1, nullptr);   // expert groups
     if (groups == 2) return launch_kr<WT, 2, 2, 2, false>(mats, K, ws, ws_stride, M, lim, st, rg, slots, slices, part);
+    if constexpr (WT == T_Q4_K || WT == T_Q5_K)
+        for (int i = 0; i < mats.count; i++)
+            if (mats.m[i].even_odd) return launch_kr<WT, 2, 1, 2, false, true>(mats, K, ws, ws_stride, M, lim, st, rg, slots, slices, part);
     return launch_kr<WT, 2, 1, 2, false>(mats, K, ws, ws_stride, M, lim, st, rg, slots, slices, part);
 }
 

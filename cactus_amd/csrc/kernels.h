@@ -91,7 +91,8 @@ __host__ __device__ __forceinline__ TileCoord xcd_tile(unsigned wg, const TileMa
 // Up to four matrices of one type over the same activation rows in one GEMM launch: their row tiles are numbered one matrix after the
 // other, first[i] is the number of matrix i's first one.  A plain product is a table of one.
 constexpr int GEMM_MATS_MAX = 4;
-struct GemmMat { const uint8_t *W; size_t nb01; int64_t N; float *y; int64_t ldy; };
+// even_odd (gemm_kr_kernel): the sums of two k groups from one - the even super-blocks' first, the odd ones' added to them.
+struct GemmMat { const uint8_t *W; size_t nb01; int64_t N; float *y; int64_t ldy; bool even_odd = false; };
 struct GemmMats { GemmMat m[GEMM_MATS_MAX]; int first[GEMM_MATS_MAX]; int count; };
 inline GemmMats one_gemm_mat(const void *W, size_t nb01, int64_t N, float *y, int64_t ldy) {
     GemmMats t{};

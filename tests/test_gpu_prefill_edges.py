@@ -1,8 +1,6 @@
 """GPU parity of the prefill kernels at the sizes where their staging ends unevenly: short last stages, ragged tiles, small
 and large shapes of each dispatch rule.  Against the CPU oracle, within 1e-5 * sum |terms| per output (the summation order is
 all that differs), as the other matmul tests."""
-import re
-
 import numpy as np
 import pytest
 
@@ -83,7 +81,7 @@ def test_low_bit_kquant_gemm(dev, orc, wt, K, N, n):
 
 # The GEMM whose waves expand their own rows, (K, N, n): two workgroups a CU, ragged rows and tokens; two k groups over an odd number
 # of super-blocks; uneven slices and a last tile of one token (at 33 tokens by waves that share a tile); two k groups in two slices of different
-# length (Q2_K, IQ4_XS; unsplit Q4_K and Q5_K) and unsplit
+# length (Q2_K, IQ4_XS) and unsplit
 @pytest.mark.parametrize("wt", (O.Q4_K, O.Q5_K, O.Q6_K) + LOW_BIT, ids=lambda t: O.TYPE_NAMES[t])
 @pytest.mark.parametrize("K,N,n", [(512, 4200, 1100), (1280, 4100, 260), (2816, 131, 33), (8448, 4100, 130), (2816, 131, 65), (8448, 4100, 200)])
 def test_kquant_row_gemm(dev, orc, wt, K, N, n):
@@ -104,8 +102,7 @@ def test_kquant_row_gemm(dev, orc, wt, K, N, n):
     if N == 131:
         assert ("gemm_kq_few" if n == 33 else "gemm_kq_kernel" if staged else "gemm_kr_kernel") in names[1] and len(names) == (2 if n == 33 else 3)
     elif K == 8448 and not (staged and n == 130):
-        groups = 1 if n == 200 and wt in (O.Q4_K, O.Q5_K) else 2
-        assert ("gemm_kq_kernel" if wt == O.Q6_K else "gemm_kr_kernelILi%dELi2ELi%dE" % (wt, groups)) in names[1]
+        assert ("gemm_kq_kernel" if wt == O.Q6_K else "gemm_kr_kernelILi%dELi2ELi2E" % wt) in names[1]
     y = dev.mul_mat(wt, w, x)
     rows = np.unique(np.concatenate([[0, 1, 2, 3, N - 1], rng.choice(N, min(N, 150), replace=False)]))
     toks = np.unique(np.concatenate([[0, 3, 4, 5, n - 1], rng.choice(n, min(n, 48), replace=False)]))
@@ -294,16 +291,22 @@ def test_grouped_gemms_equal_single_calls(dev, orc, wt, K, rows, n):
     check(ys[-1][np.ix_(toks, pick)], ref, "last member")
 
 
-# Q4_K and Q5_K above 2048 values, in one k group and in two: members share a launch only in the number that each has alone
-@pytest.mark.parametrize("wt,K,rows,n,groups", [(O.Q4_K, 2560, (6912, 6912), 200, (1,)), (O.Q5_K, 2304, (3000, 2900), 260, (2,)), (O.Q5_K, 2304, (3000, 6000), 260, (2, 1)),
-                                                (O.Q5_K, 2304, (6000, 3000), 260, (1, 2)), (O.Q4_K, 4096, (4096, 4096), 512, (1,))],
+# Q4_K and Q5_K above 2048 values, whose members run in one k group and in two alone: one launch in two groups, or in one that adds as two do where that is what
+# a member has alone (an odd number of super-blocks, a last tile of four tokens, ragged rows)
+@pytest.mark.parametrize("wt,K,rows,n,alone,joined", [(O.Q4_K, 2560, (6912, 6912), 200, (2, 2), "1ELi2ELb0ELb1E"), (O.Q5_K, 2304, (3000, 2900), 260, (2, 2), "2ELi2ELb0ELb0E"),
+                                                      (O.Q5_K, 2304, (3000, 5990), 260, (2, 2), "1ELi2ELb0ELb1E"), (O.Q4_K, 2304, (3000, 8001), 260, (2, 1), "1ELi2ELb0ELb1E"),
+                                                      (O.Q4_K, 2304, (8001, 2, 3000), 260, (1, 0, 2), None), (O.Q5_K, 2304, (8001, 3000), 260, (1, 2), "1ELi2ELb0ELb1E"),
+                                                      (O.Q4_K, 4096, (4096, 4096), 512, (2, 2), "1ELi2ELb0ELb1E"), (O.Q4_K, 2304, (8001, 9000), 260, (1, 1), "1ELi2ELb0ELb0E")],
                          ids=lambda v: O.TYPE_NAMES[v] if isinstance(v, int) and v in O.TYPE_NAMES else None)
-def test_joined_k_groups_equal_single_calls(dev, orc, wt, K, rows, n, groups):
+def test_joined_k_groups_equal_single_calls(dev, orc, wt, K, rows, n, alone, joined):
     q = orc.quantize_weights(wt, common.weights_f32(K + n, 101, K))
     ws = [np.roll(np.tile(q, (-(-N // 101), 1))[:N], i, axis=0) for i, N in enumerate(rows)]
     x = common.activations_f32(K + n, n, K)
-    names = [k for k in group_kernels(dev, [(wt, N) for N in rows], K, n) if "gemm_kr_kernel" in k]
-    assert [int(re.search(r"gemm_kr_kernelILi%dELi2ELi(\d)E" % wt, k)[1]) for k in names] == list(groups)
+    for w, groups in zip(ws, alone):
+        assert groups == 0 or "gemm_kr_kernelILi%dELi2ELi%dELi2ELb0ELb0E" % (wt, groups) in mul_mat_kernels(dev, wt, w, x)[1]
+    names = group_kernels(dev, [(wt, N) for N in rows], K, n)
+    if joined is not None:
+        assert len(names) == 2 and "gemm_kr_kernelILi%dELi2ELi%s" % (wt, joined) in names[1]
     for w, y in zip(ws, dev.mul_mat_group([(wt, w) for w in ws], x)):
         assert y.tobytes() == dev.mul_mat(wt, w, x).tobytes()
     if rows[0] == rows[1]:
