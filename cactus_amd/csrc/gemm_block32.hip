@@ -676,6 +676,9 @@ static int blk32_slices_for(int64_t K, int64_t N, int64_t M, int64_t cus) {
 //   few    a launch; the turns of 8 waves a CU, each the fetch of a first chunk and then its chunks of 256 values, as long as a load takes or as
 //          the vector work of the waves of a CU (halfway between the average and the busiest CU: by the average alone one product in 110 was more than
 //          5 per cent slower than the walk, Q8_0 4352 x 4828 at 35 tokens 19.3 / 21.9)
+//          Not for more tiles than the device holds workgroups of two waves, nor for more than 16 chunks a wave, where the estimate is short of what either
+//          takes (us, walk / few: Q8_0 7168 x 7543 at 1042 tokens 274 / 337, Q5_0 12800 x 4687 at 778 281 / 296; Q5_1 9984 x 6009 at 89 47.5 / 56.5, IQ4_NL
+//          9472 x 6334 at 82 46.2 / 53.6)
 //   walk   a launch; the turns of the workgroups a CU holds, each the fetch of a first stage and then its stages; the slice sum
 // A caller without room for the slices that the walk would be cut into keeps the order of one walk over K, whatever the tile (room: the caller has it;
 // a group is planned without, so that its members have the bits of their single calls).  At most 64 tiles of rows of 4096 values
@@ -698,13 +701,14 @@ static float blk32_walk_us(int wtype, int64_t K, int64_t N, int64_t M, int64_t c
 static FewPlan blk32_few_plan(int wtype, int64_t K, int64_t N, int64_t M, size_t nb01, int64_t cus, bool room) {
     const int64_t tiles = ceil_div(N, (int64_t)32) * ceil_div(M, (int64_t)32);
     if (K < 256 || tiles > 65536 || nb01 > ((size_t)1 << 27) || K > ((int64_t)1 << 26)) return FewPlan{0, 1};    // (rows and tokens within 32-bit reach)
-    if (!room && blk32_slices_for(K, N, M, cus) > 1) return FewPlan{0, 1};
+    if (tiles > 4 * cus || (!room && blk32_slices_for(K, N, M, cus) > 1)) return FewPlan{0, 1};
     float best = blk32_walk_us(wtype, K, N, M, cus) / 1.15f;
     FewPlan plan{0, 1};
     for (int ks = 2; ks <= 8; ks *= 2) {
         const int slices = ks == 8 && tiles <= 64 && K >= 4096 ? 2 : 1;
         const int64_t wgs = tiles * slices, turn = cus * (8 / ks), turns = wgs / turn, rest = wgs % turn;
         const float chunks = (float)ceil_div(2 * ceil_div(ceil_div(K / 64, (int64_t)slices), (int64_t)ks), (int64_t)8);
+        if (chunks > 16) continue;
         float t = 2.04f + (float)turns * (1.8f + chunks * 2.62f);
         if (rest) t += 1.8f + chunks * std::max(1.72f, 0.328f * std::max((float)ks, 0.5f * ((float)(rest * ks) / (float)cus + (float)(ceil_div(rest, cus) * ks))));
         if (slices > 1) t += 3.8f + 0.9e-6f * (float)N * (float)M * (float)slices;

@@ -135,12 +135,19 @@ def test_unsplit_short_last_stage_takes_the_gemm_where_it_is_ahead(dev, orc, wt,
     assert mul_mat_launches(dev, wt, wq, common.activations_f32(6, n, 8256), split_k=False) == count
 
 
-# 300 to 330 tiles of long rows (us, walk in slices of K / tiles shared by waves: 32.9 / 36.6, 34.7 / 38.0, 19.3 / 21.9), and fewer
+# 300 to 330 tiles of long rows (us, walk in slices of K / tiles shared by waves: 32.9 / 36.6, 34.7 / 38.0, 19.3 / 21.9), and fewer; 564 tiles of rows
+# that are long for two waves (47.5 / 56.5)
 @pytest.mark.parametrize("wt,K,N,n,walk", [(O.Q5_0, 9600, 1288, 254, True), (O.IQ4_NL, 9600, 401, 732, True), (O.Q8_0, 4352, 4828, 35, True),
-                                           (O.Q8_0, 2176, 4828, 35, False), (O.Q5_0, 1920, 1288, 254, False)])
+                                           (O.Q8_0, 2176, 4828, 35, False), (O.Q5_0, 1920, 1288, 254, False), (O.Q5_1, 9984, 6009, 89, True)])
 def test_block32_products_that_half_fill_the_device_stay_in_the_walk(dev, wt, K, N, n, walk):
     names = mul_mat_kernels(dev, wt, np.zeros((N, dev.row_size(wt, K)), np.uint8), common.activations_f32(1, n, K))
     assert len(names) == (3 if walk else 2) and ("gemm_blk32_kernel" if walk else "gemm_blk32_few_kernel") in names[1]
+
+
+# more 32 x 32 tiles than a device full of two-wave workgroups (us, walk / tiles shared by waves: 274 / 337)
+def test_block32_products_of_many_tiles_stay_in_the_walk(dev):
+    names = mul_mat_kernels(dev, O.Q8_0, np.zeros((7543, dev.row_size(O.Q8_0, 7168)), np.uint8), common.activations_f32(1, 1042, 7168))
+    assert len(names) == 2 and "gemm_blk32_kernel" in names[1]
 
 
 # kqv of more than 128 columns per KV head: one launch of the GEMM with the 256 bytes it asks for, the same bits whatever lies behind
