@@ -588,7 +588,10 @@ static float others_estimate(int wtype, int64_t K, int64_t N, int64_t n, const K
 // Forms of 32 tokens above 16 tokens.  Rows of two super-blocks up to 32 tokens, of three there for the types without a matrix-core GEMV, from four on
 // otherwise: K is what the waves share.  Above 32 tokens a caller without room for slices of K keeps the order of one walk over it.  Products that
 // are known to run in slices of K and a slice sum stay there: long rows on many rows (us, slices / this, 14336 values x 4096 rows at 32 tokens: Q4_K 19.8
-// / 18.9, Q6_K 23.9 / 20.8, Q3_K 19.6 / 16.8) and a few rows above 64 tokens.  Up to 320 tokens, where the estimates were fitted.
+// / 18.9, Q6_K 23.9 / 20.8, Q3_K 19.6 / 16.8) and a few rows above 64 tokens.  So do Q6_K and Q3_K above 32 tokens whose tiles in the staging kernel come to
+// two thirds and three quarters of the CUs, where 39 products are 0.96 x its speed (Q6_K 1024 values x 11884 rows at 49 tokens 11.6 / 13.4, 3328 x 16161
+// at 47 26.8 / 29.2; Q3_K 1536 x 13500 at 33 11.4 / 13.5; just below 38 are 1.07 x).  Up to 1200 tokens: beyond the 300 of the fit the estimates
+// are extrapolated (1464 products of 300 to 1200 tokens 1.17 x).
 KqFew kq_few_plan(int wtype, size_t nb01, int64_t K, int64_t N, int64_t n, bool can_split, int compute_units) {
     if (!gemm_kq_type(wtype) || n < 5 || n > 1200 || N < 1 || K % QK_K != 0) return KqFew{0, 0, 0};
     // rows that the kernel's 32-bit offsets reach from a tile's first: forms of 32 rows where all of them are, none where not even 16 are
@@ -601,6 +604,8 @@ KqFew kq_few_plan(int wtype, size_t nb01, int64_t K, int64_t N, int64_t n, bool 
     const KqPlan p = kq_plan(wtype, K, N, n, cus);
     if (n > 32 && p.slices > 1 && !can_split) return KqFew{0, 0, 0};
     if (p.slices > 1 && ((n > 16 && K > 8192 && N > 2048) || (n > 64 && N < 320))) return KqFew{0, 0, 0};
+    if (const int64_t staged = ceil_div(N, (int64_t)64) * ceil_div(n, (int64_t)128); p.groups == 0 && p.slices == 1 && n > 32 &&
+        (wtype == T_Q6_K ? 3 * staged >= 2 * cus : wtype == T_Q3_K && 4 * staged >= 3 * cus)) return KqFew{0, 0, 0};
     KqFew best{0, 0, 0};
     float least = 0.93f * others_estimate(wtype, K, N, n, p, cus);
     for (const FewForm &f : kFewForms) {

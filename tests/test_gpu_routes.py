@@ -144,6 +144,15 @@ def test_block32_products_that_half_fill_the_device_stay_in_the_walk(dev, wt, K,
     assert len(names) == (3 if walk else 2) and ("gemm_blk32_kernel" if walk else "gemm_blk32_few_kernel") in names[1]
 
 
+# Q6_K and Q3_K above 32 tokens by the workgroups that the staging kernel has, on either side of the rule and at 32 tokens (us, staging / tiles shared by
+# waves: 11.6 / 13.4, 26.8 / 29.2, 11.4 / 13.5)
+@pytest.mark.parametrize("wt,K,N,n,staged", [(O.Q6_K, 1024, 11884, 49, True), (O.Q6_K, 3328, 16161, 47, True), (O.Q3_K, 1536, 13500, 33, True), (O.Q6_K, 1024, 10880, 49, False),
+                                             (O.Q6_K, 1024, 10881, 49, True), (O.Q3_K, 2048, 12224, 40, False), (O.Q3_K, 2048, 12225, 40, True), (O.Q3_K, 1536, 13500, 32, False)])
+def test_kquant_products_that_fill_the_staging_kernel_stay_there(dev, wt, K, N, n, staged):
+    names = mul_mat_kernels(dev, wt, np.zeros((N, dev.row_size(wt, K)), np.uint8), common.activations_f32(1, n, K))
+    assert len(names) == 2 and ("gemm_kq_kernel" if staged else "gemm_kq_few_kernel") in names[1]
+
+
 # more 32 x 32 tiles than a device full of two-wave workgroups (us, walk / tiles shared by waves: 274 / 337)
 def test_block32_products_of_many_tiles_stay_in_the_walk(dev):
     names = mul_mat_kernels(dev, O.Q8_0, np.zeros((7543, dev.row_size(O.Q8_0, 7168)), np.uint8), common.activations_f32(1, 1042, 7168))
