@@ -14,8 +14,9 @@
 // chunk's eight are, and the chunks' sums are added; the waves' in 64 bits.  Relative 2-norm of the error against 64-bit sums, walk / this / NEAR:
 // Q4_0 960 values 1.0e-7 / 5.9e-8 / 4.9e-8, 14336 values 1.3e-7 / 8.0e-8 / 4.9e-8.
 //
-// Bound: the issue of vector instructions, some 400 per chunk and wave (two per result, the unpacking, the sums), at two waves a SIMD: 3.3 us a
-// chunk of 8 waves on a CU, 1.4 to 1.7 us one of a wave alone, of which 0.7 us is the load.  Registers (210 to 250) hold a third wave off.  Loading operands straight from
+// Bound: the issue of vector instructions, by the counters some 450 per chunk and wave (two per result, the unpacking, the sums) and 350 a wave to start and
+// to add up, at two waves a SIMD: 2.1 us a chunk of 8 waves on a CU (Q4_0 4096 rows at 64 tokens 17.2 us for 8192 values, 21.4 for 12288).  Registers (210 to
+// 250) hold a third wave off.  Loading operands straight from
 // global memory, a lane its own row's, took twice as long: 32 rows a load instruction cost some 160 clocks of the CU's address unit.  us,
 // gemm_blk32_kernel / this, values x rows: Q4_0 960 x 960 at 133 tokens 9.3 / 5.5, 4096 x 4096 at 17 12.1 / 9.0, 2048 x 2048 at 512 20.9 / 14.7.
 #include "dev_common.h"

@@ -13,7 +13,7 @@
 // in 32 bits they were up to 1.16 and 1.07 x as far (512 values at 15 tokens, GEMV / 32 bits / 64: Q3_K 4.0e-8 / 4.5e-8 / 2.7e-8).  64 bits
 // take 1.025 x the time (83 products of Q2_K and IQ4_XS; so does the product in 32 bits added in 64).
 //
-// Bound: the issue of vector instructions (by the counters 230 per super-block of 16 rows x 16 tokens for Q4_K, 280 to 300 for Q6_K, over half of them the expansion) at two
+// Bound: the issue of vector instructions (by the counters 214 per super-block of 16 rows x 16 tokens for Q4_K, 267 to 291 for Q6_K, over half of them the expansion) at two
 // to four waves a SIMD, and the tokens' quants, 4 KB for the 1.3 to 3.4 KB of 16 rows: tiles of 32 rows halve those where there are rows enough.  us, what ran
 // before / this, 8 tokens (a GEMV): Q6_K 4096 values x 4096 rows 9.6 / 7.7, 14336 x 4096 20.0 / 16.5, 4096 x 32000 37 / 31; Q4_K 1024 x 3072 7.7 / 4.1; 32
 // tokens (the GEMM, in slices of K): Q4_K 4096 x 4096 13.8 / 8.3, x 14336 27.0 / 18.7, 2048 x 768 11.2 / 5.1; 64 tokens Q4_K 4096 x 4096

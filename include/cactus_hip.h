@@ -186,7 +186,7 @@ CHIP_API int chip_mul_mat_pair_silu_mul(int type, const void *W1, const void *W2
  * its result rounded to fp16 at y_f16_t[row * ld16 + token], as chip_mul_mat_store_t.  Every output equals, bit for bit,
  * what chip_mul_mat (chip_mul_mat_store_t) returns for that member alone - except at exactly 8 tokens when the members
  * together stream at most 24 MB: they then run as one launch of the dot-product GEMV over the quantized rows, while a
- * member alone may take the matrix-core GEMV, which adds its partial sums in another order (same tolerance against the
+ * member alone may take a matrix-core kernel, which adds its partial sums in another order (same tolerance against the
  * reference, not the same bits).  The workspace must hold
  * chip_mul_mat_workspace_size(type, K, n) bytes for the members' activation format. */
 #define CHIP_GROUP_MAX 4
