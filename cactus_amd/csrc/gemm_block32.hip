@@ -670,15 +670,17 @@ static int blk32_slices_for(int64_t K, int64_t N, int64_t M, int64_t cus) {
 
 // Few output tiles: gemm_blk32_few_kernel, whose ks waves a workgroup share the K of a 32 x 32 tile, or the staged walk of this file, whichever
 // is estimated ahead, in us of a launch.  Fitted to 707 products of 256 to 14336 values x 320 to 14336 rows at 17 to 512 tokens (11 and 19 per cent
-// of spread); the walk is left where it is more than 15 per cent slower.  Over 800 others (512 to 14336 values, 256 to 16384 rows, 5 to 1100 tokens) 1.12 x,
-// none more than 3 per cent slower than before; of products drawn where the tiles half fill the device one in 25 is, the worst 1.2 x.  us, walk / few:
+// of spread); the walk is left where it is more than 15 per cent slower, of the types but IQ4_NL 10 where there are more tiles than CUs.  Over 934 products of
+// 257 to 1024 tiles 1.22 x, one in 90 more than 3 per cent slower than the walk (IQ4_NL 4352 x 9584 at 60 tokens 1.15 x), one in 20 left to it that would be
+// more than 3 per cent ahead.  us, walk / few:
 // Q4_0 960 x 960 at 133 tokens 9.3 / 5.5, 2560 x 960 13.3 / 8.4, 4096 x 4096 at 17 12.1 / 9.0, at 128 20.8 / 14.5, 2048 x 2048 at 512 20.9 / 14.7; Q5_0 2048 x 2048 at 40 13.9 / 7.4; 14336 x 4096 at 32 25.0 / 25.4 and stays.
 //   few    a launch; the turns of 8 waves a CU, each the fetch of a first chunk and then its chunks of 256 values, as long as a load takes or as
 //          the vector work of the waves of a CU (halfway between the average and the busiest CU: by the average alone one product in 110 was more than
 //          5 per cent slower than the walk, Q8_0 4352 x 4828 at 35 tokens 19.3 / 21.9)
 //          Not for more tiles than the device holds workgroups of two waves, nor for more than 16 chunks a wave, where the estimate is short of what either
 //          takes (us, walk / few: Q8_0 7168 x 7543 at 1042 tokens 274 / 337, Q5_0 12800 x 4687 at 778 281 / 296; Q5_1 9984 x 6009 at 89 47.5 / 56.5, IQ4_NL
-//          9472 x 6334 at 82 46.2 / 53.6)
+//          9472 x 6334 at 82 46.2 / 53.6); nor by two waves for Q8_0 at 33 to 64 tokens where the walk, which then reads the rows once, is not cut (10 products 0.96 x,
+//          768 x 11600 at 46 9.1 / 10.1)
 //   walk   a launch; the turns of the workgroups a CU holds, each the fetch of a first stage and then its stages; the slice sum
 // A caller without room for the slices that the walk would be cut into keeps the order of one walk over K, whatever the tile (room: the caller has it;
 // a group is planned without, so that its members have the bits of their single calls).  At most 64 tiles of rows of 4096 values
@@ -702,13 +704,13 @@ static FewPlan blk32_few_plan(int wtype, int64_t K, int64_t N, int64_t M, size_t
     const int64_t tiles = ceil_div(N, (int64_t)32) * ceil_div(M, (int64_t)32);
     if (K < 256 || tiles > 65536 || nb01 > ((size_t)1 << 27) || K > ((int64_t)1 << 26)) return FewPlan{0, 1};    // (rows and tokens within 32-bit reach)
     if (tiles > 4 * cus || (!room && blk32_slices_for(K, N, M, cus) > 1)) return FewPlan{0, 1};
-    float best = blk32_walk_us(wtype, K, N, M, cus) / 1.15f;
+    float best = blk32_walk_us(wtype, K, N, M, cus) / (tiles > cus && wtype != T_IQ4_NL ? 1.1f : 1.15f);
     FewPlan plan{0, 1};
     for (int ks = 2; ks <= 8; ks *= 2) {
         const int slices = ks == 8 && tiles <= 64 && K >= 4096 ? 2 : 1;
         const int64_t wgs = tiles * slices, turn = cus * (8 / ks), turns = wgs / turn, rest = wgs % turn;
         const float chunks = (float)ceil_div(2 * ceil_div(ceil_div(K / 64, (int64_t)slices), (int64_t)ks), (int64_t)8);
-        if (chunks > 16) continue;
+        if (chunks > 16 || (wtype == T_Q8_0 && ks == 2 && M > 32 && M <= 64 && blk32_slices_for(K, N, M, cus) == 1)) continue;
         float t = 2.04f + (float)turns * (1.8f + chunks * 2.62f);
         if (rest) t += 1.8f + chunks * std::max(1.72f, 0.328f * std::max((float)ks, 0.5f * ((float)(rest * ks) / (float)cus + (float)(ceil_div(rest, cus) * ks))));
         if (slices > 1) t += 3.8f + 0.9e-6f * (float)N * (float)M * (float)slices;

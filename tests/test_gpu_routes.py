@@ -138,10 +138,18 @@ def test_unsplit_short_last_stage_takes_the_gemm_where_it_is_ahead(dev, orc, wt,
 # 300 to 330 tiles of long rows (us, walk in slices of K / tiles shared by waves: 32.9 / 36.6, 34.7 / 38.0, 19.3 / 21.9), and fewer; 564 tiles of rows
 # that are long for two waves (47.5 / 56.5)
 @pytest.mark.parametrize("wt,K,N,n,walk", [(O.Q5_0, 9600, 1288, 254, True), (O.IQ4_NL, 9600, 401, 732, True), (O.Q8_0, 4352, 4828, 35, True),
-                                           (O.Q8_0, 2176, 4828, 35, False), (O.Q5_0, 1920, 1288, 254, False), (O.Q5_1, 9984, 6009, 89, True)])
+                                           (O.Q8_0, 2176, 4828, 35, False), (O.Q5_0, 1920, 1288, 254, False), (O.Q5_1, 9984, 6009, 89, True),
+                                           (O.Q4_0, 4352, 2736, 243, False), (O.IQ4_NL, 4352, 2736, 243, True)])
 def test_block32_products_that_half_fill_the_device_stay_in_the_walk(dev, wt, K, N, n, walk):
     names = mul_mat_kernels(dev, wt, np.zeros((N, dev.row_size(wt, K)), np.uint8), common.activations_f32(1, n, K))
     assert len(names) == (3 if walk else 2) and ("gemm_blk32_kernel" if walk else "gemm_blk32_few_kernel") in names[1]
+
+
+# a tile of 64 tokens reads the rows once, two of 32 twice: Q8_0 by two waves (us, walk / tiles shared by waves: 9.1 / 10.1)
+@pytest.mark.parametrize("wt,n,walk", [(O.Q8_0, 46, True), (O.Q8_0, 33, True), (O.Q8_0, 32, False), (O.Q4_0, 46, False)])
+def test_block32_products_of_two_token_tiles(dev, wt, n, walk):
+    names = mul_mat_kernels(dev, wt, np.zeros((11600, dev.row_size(wt, 768)), np.uint8), common.activations_f32(1, n, 768))
+    assert len(names) == 2 and ("gemm_blk32_kernel" if walk else "gemm_blk32_few_kernel") in names[1]
 
 
 # Q6_K and Q3_K above 32 tokens by the workgroups that the staging kernel has, on either side of the rule and at 32 tokens (us, staging / tiles shared by
